@@ -136,7 +136,7 @@ struct LaunchTimer {
 // ---------------------------------------------------------------- prims ----
 // Exclusive scan of n int32 values into out[0..n] (out[n] = total).
 void scan_i32_to_i64(Context &c, const int *in, long long *out, long n);
-// the same over up to four arrays, in one launch where they suit the
+// the same over up to five arrays, in one launch where they suit the
 // single-pass scan
 struct ScanJob {
   const int *in;

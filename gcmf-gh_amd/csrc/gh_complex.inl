@@ -11,18 +11,24 @@
 // intersection into the union.
 //
 // Here one wave takes one pair of complex polygons:
-//   1. the lanes build the node lists (every ring its own cycle), classify
-//      every source edge of every ring of P against every source edge of
-//      every ring of Q (intersect(), polyclip.h:60-179) and write the
-//      non-zero records, each P edge's in Q order, at scanned offsets;
-//   2. lane 0 replays the records in the reference's loop order (P ring, P
-//      edge, Q ring, Q edge; polyclip.h:200-277), inserting vertices by alpha
-//      with the reference's tie rule (polygon.h:101-113), so the lists are
-//      the reference's;
-//   3. lane 0 labels and traces over all components (label_trace_multi) and
-//      cleans the result up (polyclip.h:791-807).
-// Pairs of this kind are few and small next to the single-ring batches, so
-// the sequential part runs on one lane per pair.
+//   1. the lanes classify every source edge of every ring of P against every
+//      source edge of every ring of Q (intersect(), polyclip.h:60-179), 64
+//      Q edges at a time held one per lane and read by readlane, and write
+//      the non-zero records, each P edge's in Q order, at scanned offsets;
+//   2. a pair in general position whose arrays fit the launch's LDS
+//      (complex_fast) is spliced, labelled, traced and cleaned up by the
+//      whole wave in LDS;
+//   3. every other pair is replayed by lane 0 in global memory: the records
+//      in the reference's loop order (P ring, P edge, Q ring, Q edge;
+//      polyclip.h:200-277), inserting vertices by alpha with the reference's
+//      tie rule (polygon.h:101-113), then label_trace_multi over all
+//      components and the clean-up (polyclip.h:791-807).
+//
+// What bounds it: dependent accesses, one pair at a time.  On one MI355X 300
+// pairs of 120 vertices took 881 us in the clip launch when lane 0 replayed
+// every pair from global memory and each lane read every Q edge by itself
+// (another 144 us in the counting launch); see complex_fast for what it
+// takes now.
 
 constexpr int kComplexW = 64;
 
@@ -396,9 +402,150 @@ struct ComplexArgs {
   unsigned long long *bad;  // pairs whose parts lie outside the layers
 };
 
-__global__ void __launch_bounds__(kComplexW)
+// The rings of both sides of a pair (at most 64 each), by a block's first
+// wave: off[s][r]
+// the first vertex of ring r counted over side s's rings, src[s][r] its first
+// vertex in the layer.
+struct ComplexRings {
+  int off[2][65];
+  long src[2][64];
+};
+
+__device__ __forceinline__ void complex_rings(const ComplexArgs &a, const ComplexPair &cp,
+                                              ComplexRings &R) {
+  const int lane = threadIdx.x;
+  for (int side = 0; side < 2 && lane < kComplexW; side++) {
+    const int r0 = side ? cp.o0 : cp.b0, rn = side ? cp.on : cp.bn;
+    long s = 0;
+    int n = 0;
+    if (lane < rn)
+      ring_of(side ? a.oVNum : a.bVNum, side ? a.oVPSNum : a.bVPSNum, r0 + lane, s, n);
+    int tot;
+    const int pre = grp_scan<kComplexW>(n, tot);
+    if (lane < rn) {
+      R.off[side][lane] = pre;
+      R.src[side][lane] = s;
+    }
+    if (lane == 0) R.off[side][rn] = tot;
+  }
+  __syncthreads();
+}
+
+// ring of vertex v of a side with rn rings
+__device__ __forceinline__ int ring_at(const int *off, int rn, int v) {
+  int r = 0;
+  while (r + 1 < rn && v >= off[r + 1]) r++;
+  return r;
+}
+
+struct ComplexSide {
+  const double *C;
+  const int *off;
+  const long *src;
+  int rn;
+  // original coordinates of vertex v, which lies in ring r
+  __device__ __forceinline__ pt orig(int v, int r) const {
+    return ld(C, src[r] + (v - off[r]));
+  }
+  // the vertex after v on its ring r
+  __device__ __forceinline__ int next(int v, int r) const {
+    return v + 1 == off[r + 1] ? off[r] : v + 1;
+  }
+};
+
+__device__ __forceinline__ ComplexSide complex_side(const ComplexArgs &a, const ComplexPair &cp,
+                                                    const ComplexRings &R, int side) {
+  return ComplexSide{side ? a.oCoords : a.bCoords, R.off[side], R.src[side],
+                     side ? cp.on : cp.bn};
+}
+
+// Whether one parameter of the edge pair lies well outside [-eps, 1 - eps),
+// so that itype() is 0: with the ends of one edge strictly on one side of the
+// other's line, a = A1 / (A1 - A2) is at least 1 - 2^-53 when |A1| >
+// |A1 - A2| and below -1e-6 (1 - 2^-50) when it is negative and |A1| > 1e-6
+// |A1 - A2|, and no type takes such a parameter.
+__device__ __forceinline__ bool edges_apart(pt P1, pt P2, pt Q1, pt Q2) {
+  const double AP1 = triA(P1, Q1, Q2), AP2 = triA(P2, Q1, Q2), dP = AP1 - AP2;
+  const double AQ1 = triA(Q1, P1, P2), AQ2 = triA(Q2, P1, P2), dQ = AQ1 - AQ2;
+  const bool sP = (AP1 > 0 && AP2 > 0) || (AP1 < 0 && AP2 < 0);
+  const bool sQ = (AQ1 > 0 && AQ2 > 0) || (AQ1 < 0 && AQ2 < 0);
+  return fabs(dP) > kGhEps &&
+         ((sP && fabs(AP1) > 1e-6 * fabs(dP)) || (sQ && fabs(AQ1) > 1e-6 * fabs(dQ)));
+}
+
+// edge v of a side in the frame nrm
+__device__ __forceinline__ void complex_edge(const ComplexSide &S, int v, const double nrm[3],
+                                             pt &A, pt &B) {
+  const int r = ring_at(S.off, S.rn, v);
+  const pt a = S.orig(v, r), b = S.orig(S.next(v, r), r);
+  A = pt{(a.x - nrm[0]) * nrm[2], (a.y - nrm[1]) * nrm[2]};
+  B = pt{(b.x - nrm[0]) * nrm[2], (b.y - nrm[1]) * nrm[2]};
+}
+
+// Every P edge against every Q edge, by a block of nw waves: f(p, q, type,
+// alpha, beta) for the non-zero types.  Wave w takes the w-th of every nw
+// chunks of kCxChunk Q edges, held one per lane and read by readlane, four at
+// a time for independent chains; a lane holds one P edge.  With nw = 1 each
+// P edge's calls come in Q order, from lane p % 64.
+constexpr int kCxChunk = 16;
+template <class F>
+__device__ __forceinline__ void complex_records(const ComplexSide &P, const ComplexSide &Q,
+                                                const double nrm[3], int nw, F &&f) {
+  const int lane = __lane_id(), nP = P.off[P.rn], nQ = Q.off[Q.rn];
+  const int w = threadIdx.x >> 6;
+  for (int p0 = 0; p0 < nP; p0 += 64) {
+    const int p = p0 + lane;
+    pt P1{0.0, 0.0}, P2{0.0, 0.0};
+    if (p < nP) complex_edge(P, p, nrm, P1, P2);
+    for (int q0 = w * kCxChunk; q0 < nQ; q0 += nw * kCxChunk) {
+      pt A{0.0, 0.0}, B{0.0, 0.0};
+      if (lane < kCxChunk && q0 + lane < nQ) complex_edge(Q, q0 + lane, nrm, A, B);
+      const int m = min(kCxChunk, nQ - q0);
+      for (int l = 0; l < m; l += 4) {
+        bool apart[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const pt Q1{lane_d(A.x, l + u), lane_d(A.y, l + u)};
+          const pt Q2{lane_d(B.x, l + u), lane_d(B.y, l + u)};
+          apart[u] = p >= nP || l + u >= m || edges_apart(P1, P2, Q1, Q2);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          if (!__ballot(!apart[u])) continue;
+          const pt Q1{lane_d(A.x, l + u), lane_d(A.y, l + u)};
+          const pt Q2{lane_d(B.x, l + u), lane_d(B.y, l + u)};
+          if (apart[u]) continue;
+          double al, be;
+          const int t = itype(P1, P2, Q1, Q2, al, be);
+          if (t != 0) f(p, q0 + l + u, t, al, be);
+        }
+      }
+    }
+  }
+}
+
+// the most LDS a pair's arrays may take (a block's default limit): pairs of
+// up to about 1500 vertices
+constexpr long kComplexLds = 65536 - 4096;
+
+// bytes of LDS complex_fast needs for a pair of n vertices in nr rings with
+// R intersection records (LDS arrays each rounded up to 16 bytes)
+__host__ __device__ constexpr long complex_fast_bytes(long n, long nr, long R) {
+  return 36 * n + 160 * R + 48 * nr + 32 * 16;
+}
+
+// One block per pair: the frame, then the number of intersection records and
+// with it the pair's capacities; the edges (p, q) of the first kCxHits
+// records, in any order, at hits, so that the clip classifies only those
+// again.  need[0]: the largest complex_fast_bytes of the launch's pairs that
+// are at most ldsMax.  Four waves share a pair's edge pairs, since a call's
+// few hundred pairs leave most SIMDs empty otherwise.
+constexpr int kCxSetup = 256;
+constexpr int kCxHits = 64;
+__global__ void __launch_bounds__(kCxSetup)
     k_complex_setup(long M, ComplexArgs a, int *nodeCap, int *compCap, int *rings,
-                    int *edgesP) {
+                    int *edgesP, int *recCnt, int *swapped, unsigned long long *need,
+                    long ldsMax, int2 *hits) {
   const long k = blockIdx.x;
   if (k >= M) return;
   const int lane = threadIdx.x;
@@ -409,48 +556,44 @@ __global__ void __launch_bounds__(kComplexW)
     if (lane == 0) {
       a.status[k] = GH_DISJOINT;
       atomicAdd(a.bad, 1ULL);
-      rings[k] = edgesP[k] = nodeCap[k] = compCap[k] = 0;
+      rings[k] = edgesP[k] = nodeCap[k] = compCap[k] = recCnt[k] = swapped[k] = 0;
     }
     return;
   }
+  __shared__ ComplexRings R;
+  __shared__ int nHits;
+  if (lane == 0) nHits = 0;
+  const bool few = cp.bn <= 64 && cp.on <= 64;
+  if (few) complex_rings(a, cp, R);
   double m[2][4];
   long long nv[2] = {0, 0};
   bool emptyRing = false;
-  for (int side = 0; side < 2; side++) {
-    const int r0 = side ? cp.o0 : cp.b0, rn = side ? cp.on : cp.bn;
-    const double *C = side ? a.oCoords : a.bCoords;
-    const int *vn = side ? a.oVNum : a.bVNum;
-    const long *vp = side ? a.oVPSNum : a.bVPSNum;
+  for (int side = 0; side < 2 && few; side++) {
+    const ComplexSide S = complex_side(a, cp, R, side);
+    nv[side] = S.off[S.rn];
+    for (int r = 0; r < S.rn; r++) emptyRing |= S.off[r + 1] - S.off[r] < 1;
     double x0 = INFINITY, y0 = INFINITY, x1 = -INFINITY, y1 = -INFINITY;
-    for (int r = r0; r < r0 + rn; r++) {
-      long s;
-      int n;
-      ring_of(vn, vp, r, s, n);
-      emptyRing |= n < 1;
-      nv[side] += n > 0 ? n : 0;
-      for (int i = lane; i < n; i += kComplexW) {
-        const double x = C[2 * (s + i)], y = C[2 * (s + i) + 1];
-        x0 = fmin(x0, x);
-        y0 = fmin(y0, y);
-        x1 = fmax(x1, x);
-        y1 = fmax(y1, y);
-      }
+    for (int v = lane; v < S.off[S.rn]; v += kCxSetup) {
+      const pt c = S.orig(v, ring_at(S.off, S.rn, v));
+      x0 = fmin(x0, c.x);
+      y0 = fmin(y0, c.y);
+      x1 = fmax(x1, c.x);
+      y1 = fmax(y1, c.y);
     }
-    pgrp_minmax<kComplexW>(x0, x1);
-    pgrp_minmax<kComplexW>(y0, y1);
+    pgrp_minmax<kCxSetup>(x0, x1);
+    pgrp_minmax<kCxSetup>(y0, y1);
     m[side][0] = x0;
     m[side][1] = y0;
     m[side][2] = x1;
     m[side][3] = y1;
   }
-  if (lane != 0) return;
   int st = GH_OK;
-  const bool apart = m[0][0] > m[1][2] || m[0][2] < m[1][0] || m[0][1] > m[1][3] ||
-                     m[0][3] < m[1][1];
-  if (nv[0] < 1 || nv[1] < 1 || cp.bn > 64 || cp.on > 64 || emptyRing) st = GH_DISJOINT;
+  const bool apart = few && (m[0][0] > m[1][2] || m[0][2] < m[1][0] || m[0][1] > m[1][3] ||
+                     m[0][3] < m[1][1]);
+  if (!few || nv[0] < 1 || nv[1] < 1 || emptyRing) st = GH_DISJOINT;
   if (apart && !a.unionOp) st = GH_DISJOINT;
-  double cx = 0.0, cy = 0.0, s = 1.0;
-  if (a.normalize & 1) {
+  double nrm[3] = {0.0, 0.0, 1.0};
+  if (st == GH_OK && (a.normalize & 1)) {
     double b[4];
     if (apart) {  // the joint MBR (a union only)
       b[0] = fmin(m[0][0], m[1][0]);
@@ -464,99 +607,43 @@ __global__ void __launch_bounds__(kComplexW)
       b[3] = m[1][3] < m[0][3] ? m[1][3] : m[0][3];
     }
     const double w = b[2] - b[0], h = b[3] - b[1], e = w > h ? w : h;
-    cx = b[0];
-    cy = b[1];
-    s = e > 0.0 ? 1.0 / e : 1.0;
+    nrm[0] = b[0];
+    nrm[1] = b[1];
+    nrm[2] = e > 0.0 ? 1.0 / e : 1.0;
     if (a.normalize & 4) {
       const double rr = sqrt((double)nv[0] * (double)nv[1]) / 1024.0;
       double f = 1.0;
       while (f < rr) f *= 2.0;
-      s *= f;
+      nrm[2] *= f;
     }
   }
-  a.status[k] = st;
-  a.norm[3 * k] = cx;
-  a.norm[3 * k + 1] = cy;
-  a.norm[3 * k + 2] = s;
-  rings[k] = st == GH_OK ? cp.bn + cp.on : 0;
-  edgesP[k] = st == GH_OK ? (int)nv[0] : 0;
-  // the node and component capacities need the intersection count
-  // (k_complex_count adds it)
-  nodeCap[k] = st == GH_OK ? (int)(nv[0] + nv[1]) + 4 * (cp.bn + cp.on) + 16 : 0;
-  compCap[k] = st == GH_OK ? cp.bn + cp.on + 8 : 0;
-}
-
-// the side's vertex i (over its rings in order) in the pair's frame and
-// original coordinates; sEdge lists the rings' first global vertex and
-// ring lengths are read from VNum
-struct RingWalk {
-  const double *C;
-  const int *vn;
-  const long *vp;
-  int r0, rn;
-};
-
-// records of P edge e (global over P's rings) against every Q edge, in Q
-// order; f(qEdge, type, alpha, beta) for the non-zero types
-template <class F>
-__device__ void complex_edge_records(const RingWalk &P, int pr, int pi, const RingWalk &Q,
-                                     const double *nrm, F &&f) {
-  long ps;
-  int pn;
-  ring_of(P.vn, P.vp, pr, ps, pn);
-  const double cx = nrm[0], cy = nrm[1], s = nrm[2];
-  auto tf = [&](double x, double y) { return pt{(x - cx) * s, (y - cy) * s}; };
-  const pt P1 = tf(P.C[2 * (ps + pi)], P.C[2 * (ps + pi) + 1]);
-  const int pj = pi + 1 == pn ? 0 : pi + 1;
-  const pt P2 = tf(P.C[2 * (ps + pj)], P.C[2 * (ps + pj) + 1]);
-  int qe = 0;
-  for (int qr = Q.r0; qr < Q.r0 + Q.rn; qr++) {
-    long qs;
-    int qn;
-    ring_of(Q.vn, Q.vp, qr, qs, qn);
-    for (int qi = 0; qi < qn; qi++, qe++) {
-      const int qj = qi + 1 == qn ? 0 : qi + 1;
-      const pt Q1 = tf(Q.C[2 * (qs + qi)], Q.C[2 * (qs + qi) + 1]);
-      const pt Q2 = tf(Q.C[2 * (qs + qj)], Q.C[2 * (qs + qj) + 1]);
-      double al, be;
-      const int t = itype(P1, P2, Q1, Q2, al, be);
-      if (t != 0) f(qe, t, al, be);
-    }
+  if (lane == 0) {
+    a.status[k] = st;
+    a.norm[3 * k] = nrm[0];
+    a.norm[3 * k + 1] = nrm[1];
+    a.norm[3 * k + 2] = nrm[2];
+    swapped[k] = 0;
   }
-}
-
-__device__ __forceinline__ void complex_walks(const ComplexArgs &a, const ComplexPair &cp,
-                                              RingWalk &P, RingWalk &Q) {
-  P = RingWalk{a.bCoords, a.bVNum, a.bVPSNum, cp.b0, cp.bn};
-  Q = RingWalk{a.oCoords, a.oVNum, a.oVPSNum, cp.o0, cp.on};
-}
-
-// intersection records per pair (for the capacities)
-__global__ void __launch_bounds__(kComplexW)
-    k_complex_count(long M, ComplexArgs a, int *recCnt, int *nodeCap, int *compCap) {
-  const long k = blockIdx.x;
-  if (k >= M) return;
-  if (a.status[k] != GH_OK) {
-    if (threadIdx.x == 0) recCnt[k] = 0;
-    return;
-  }
-  const ComplexPair cp = complex_pair(a.parts, k);
-  RingWalk P, Q;
-  complex_walks(a, cp, P, Q);
   int cnt = 0;
-  for (int pr = P.r0; pr < P.r0 + P.rn; pr++) {
-    const int pn = P.vn[pr] - 1;
-    for (int pi = threadIdx.x; pi < pn; pi += kComplexW)
-      complex_edge_records(P, pr, pi, Q, a.norm + 3 * k,
-                           [&](int, int, double, double) { cnt++; });
+  if (st == GH_OK) {
+    complex_records(complex_side(a, cp, R, 0), complex_side(a, cp, R, 1), nrm, kCxSetup / 64,
+                    [&](int p, int q, int, double, double) {
+                      const int i = atomicAdd(&nHits, 1);
+                      if (i < kCxHits) hits[k * kCxHits + i] = make_int2(p, q);
+                    });
+    __syncthreads();
+    cnt = nHits;
   }
-  cnt = grp_sum<kComplexW>(cnt);
-  if (threadIdx.x == 0) {
-    recCnt[k] = cnt;
-    // two nodes per record, two more per split pair, and the result
-    nodeCap[k] += 4 * cnt;
-    compCap[k] += cnt;
-  }
+  if (lane != 0) return;
+  const int nr = cp.bn + cp.on;
+  recCnt[k] = cnt;
+  rings[k] = st == GH_OK ? nr : 0;
+  edgesP[k] = st == GH_OK ? (int)nv[0] : 0;
+  // two nodes per record, two more per split pair, and the result
+  nodeCap[k] = st == GH_OK ? (int)(nv[0] + nv[1]) + 4 * nr + 16 + 4 * cnt : 0;
+  compCap[k] = st == GH_OK ? nr + 8 + cnt : 0;
+  const long b = complex_fast_bytes(nv[0] + nv[1], nr, cnt);
+  if (st == GH_OK && b <= ldsMax) atomicMax(need, (unsigned long long)b);
 }
 
 struct ComplexWork {
@@ -567,7 +654,7 @@ struct ComplexWork {
   double *opn, *opo;
   int *onext, *oprev, *ocompRoot;
   int *roots;             // [ring total] ring start nodes
-  int *recQ, *recT;       // [records] Q edge and type
+  int *recP, *recQ, *recT;  // [records] P edge, Q edge and type
   double *recA, *recB;    // [records] alpha, beta
   int *edgeRec;           // [P edges + M] per-P-edge record offsets within the pair
   int *outNComp, *outNVerts, *compLen;
@@ -575,8 +662,303 @@ struct ComplexWork {
   int cleanup;
 };
 
+// The winding of the segment P0 -> P1 about R (polygon::pointInPoly,
+// polygon.h:427-448)
+__device__ __forceinline__ int seg_wind(pt P0, pt P1, pt R) {
+  if ((P0.y < R.y) == (P1.y < R.y)) return 0;
+  const int w = 2 * (P1.y > P0.y) - 1;
+  if (P0.x >= R.x)
+    return P1.x > R.x || (triA(P0, P1, R) > 0) == (P1.y > P0.y) ? w : 0;
+  return P1.x > R.x && (triA(P0, P1, R) > 0) == (P1.y > P0.y) ? w : 0;
+}
+
+// Splicing, labelling, tracing and clean-up of one pair in general position,
+// by one wave in LDS.  General position: every record is of type 1 (both
+// edges crossed inside) and every crossing is labelled CROSSING, so that no
+// source vertex carries a link, links are mutual, and steps 2, 5 and 6 of
+// the labelling have nothing to do.  Then
+//   - the list of a ring is its source vertices, each followed by its edge's
+//     crossings by alpha (a later record before an earlier one on ties,
+//     polygon.h:101-113), so a crossing's place in its side's list is (its
+//     edge) + (its rank among the side's crossings) + 1, and rings own
+//     contiguous ranges of the crossings;
+//   - step 4 starts at the ring's first vertex and alternates, so a
+//     crossing's enex is the start status and its rank's parity;
+//   - createResult goes from crossing to crossing: lane 0 walks those (a few
+//     per pair) and notes the segments, and all lanes write the vertices.
+// Returns false, having written nothing but xy, when the pair is not in
+// general position (lane 0's replay then takes it).
+// All accesses but the layer's coordinates and the result are to LDS.
+//
+// Measured on one MI355X (set-up and count, then clip): 300 pairs of 120
+// vertices 6 + 144 + 881 -> 34 + 57 us, the unions of 7 pairs 6 + 96 + 769 ->
+// 31 + 53 us.  With one wave and no edges_apart the set-up took 78 us, and
+// the clip, counting and classifying by itself, 197.
+struct FastRecs {  // the pair's records, in LDS
+  int *er, *rp, *rq;  // [nP + 1] offsets per P edge; P and Q edge per record
+  double *al, *be;
+};
+
+__device__ bool complex_fast(const ComplexSide &P, const ComplexSide &Q, int nRec,
+                             const FastRecs &rec, const double *pn,
+                             Arena &ar, bool U, int cleanup, long long cap, long long capComp,
+                             double *xy, int *clenOut, int *outComps, int *outVerts) {
+  const int lane = threadIdx.x;
+  const int nP = P.off[P.rn], nQ = Q.off[Q.rn], nS = nP + nQ;
+  const int rn[2] = {P.rn, Q.rn}, nR = P.rn + Q.rn;
+  // every take below fits: the caller checked complex_fast_bytes
+  int *qo = ar.take<int>(nQ + 1, nullptr);
+  int *ord[2] = {ar.take<int>(nRec, nullptr), ar.take<int>(nRec, nullptr)};
+  int *inv[2] = {ar.take<int>(nRec, nullptr), ar.take<int>(nRec, nullptr)};
+  // -- each edge's records by alpha (P) and beta (Q)
+  for (int i = lane; i <= nQ; i += kComplexW) qo[i] = 0;
+  __syncthreads();
+  for (int r = lane; r < nRec; r += kComplexW) atomicAdd(&qo[rec.rq[r]], 1);
+  __syncthreads();
+  grp_scan_range<kComplexW, int>(nQ, [&](int q) { return qo[q]; },
+                                 [&](int q, int pre, int) { qo[q] = pre; });
+  __syncthreads();
+  for (int r = lane; r < nRec; r += kComplexW) ord[1][atomicAdd(&qo[rec.rq[r]], 1)] = r;
+  __syncthreads();
+  // qo[q] is now the end of edge q's run
+  for (int q = lane; q < nQ; q += kComplexW) {
+    const int b = q ? qo[q - 1] : 0, z = qo[q];
+    for (int i = b + 1; i < z; i++) {
+      const int r = ord[1][i];
+      const double v = rec.be[r];
+      int j = i - 1;
+      while (j >= b && (rec.be[ord[1][j]] > v || (rec.be[ord[1][j]] == v && ord[1][j] < r))) {
+        ord[1][j + 1] = ord[1][j];
+        j--;
+      }
+      ord[1][j + 1] = r;
+    }
+  }
+  for (int p = lane; p < nP; p += kComplexW) {
+    const int b = rec.er[p], z = rec.er[p + 1];
+    for (int i = b; i < z; i++) {
+      const double v = rec.al[i];
+      int j = i - 1;
+      while (j >= b && rec.al[ord[0][j]] >= v) {
+        ord[0][j + 1] = ord[0][j];
+        j--;
+      }
+      ord[0][j + 1] = i;
+    }
+  }
+  __syncthreads();
+  for (int j = lane; j < nRec; j += kComplexW) {
+    inv[0][ord[0][j]] = j;
+    inv[1][ord[1][j]] = j;
+  }
+  // first crossing of edge e of a side
+  auto first = [&](int s, int e) { return s ? (e ? qo[e - 1] : 0) : rec.er[e]; };
+  auto edge_of = [&](int s, int r) { return s ? rec.rq[r] : rec.rp[r]; };
+  // a node: a source vertex of P or (from nP) of Q, or (from nS) a record's
+  // crossing
+  auto src = [&](int s, int v) { return (s ? nP : 0) + v; };
+  // -- the lists, each ring's crossings and each crossing's ring
+  int *lst[2] = {ar.take<int>(nP + nRec, nullptr), ar.take<int>(nQ + nRec, nullptr)};
+  int *crng[2] = {ar.take<int>(nRec, nullptr), ar.take<int>(nRec, nullptr)};
+  int *rc[2] = {ar.take<int>(P.rn + 1, nullptr), ar.take<int>(Q.rn + 1, nullptr)};
+  int *in = ar.take<int>(nR, nullptr);
+  int *vis = ar.take<int>(nRec, nullptr);
+  __syncthreads();
+  for (int s = 0; s < 2; s++) {
+    const ComplexSide &S = s ? Q : P;
+    const int n = s ? nQ : nP;
+    for (int v = lane; v < n; v += kComplexW) {
+      const int f = first(s, v);
+      lst[s][v + f] = src(s, v);
+    }
+    for (int j = lane; j < nRec; j += kComplexW) {
+      const int r = ord[s][j], e = edge_of(s, r);
+      lst[s][e + 1 + j] = nS + r;
+      crng[s][j] = ring_at(S.off, S.rn, e);
+    }
+    for (int r = lane; r <= rn[s]; r += kComplexW)
+      rc[s][r] = S.off[r] < n ? first(s, S.off[r]) : nRec;
+  }
+  for (int j = lane; j < nRec; j += kComplexW) vis[j] = 0;
+  __syncthreads();
+  // -- labels (polyclip.h:343-397), every one CROSSING, and an even number
+  // of crossings on every ring (else the statuses do not alternate round it)
+  bool slow = false;
+  for (int r = lane; r < nRec; r += kComplexW) {
+    int nb[2][2];  // the nodes before and after the crossing on both lists
+    for (int s = 0; s < 2; s++) {
+      const ComplexSide &S = s ? Q : P;
+      const int e = edge_of(s, r), j = inv[s][r], b = first(s, e);
+      const int z = s ? qo[e] : rec.er[e + 1];
+      nb[s][0] = j > b ? nS + ord[s][j - 1] : src(s, e);
+      nb[s][1] = j + 1 < z ? nS + ord[s][j + 1] : src(s, S.next(e, crng[s][j]));
+    }
+    const pt Pm = ld(pn, nb[0][0]), I = ld(pn, nS + r), Pp = ld(pn, nb[0][1]);
+    int t[2];
+    for (int d = 0; d < 2; d++) {
+      const int q = nb[1][d];  // linked to a P neighbour: the same crossing
+      t[d] = rel_pos(q >= nS && q == nb[0][0], q >= nS && q == nb[0][1], ld(pn, q), Pm, I, Pp);
+    }
+    if (!((t[0] == 0 && t[1] == 1) || (t[0] == 1 && t[1] == 0))) slow = true;
+  }
+  for (int s = 0; s < 2; s++)
+    for (int r = lane; r < rn[s]; r += kComplexW)
+      if ((rc[s][r + 1] - rc[s][r]) & 1) slow = true;
+  if (grp_any<kComplexW>(slow)) return false;
+  // -- every ring's first vertex inside the other polygon (steps 3.5 and 4)
+  for (int g = 0; g < nR; g++) {
+    const int s = g >= P.rn ? 1 : 0, o = 1 - s;
+    const ComplexSide &S = s ? Q : P, &O = o ? Q : P;
+    const pt X = ld(pn, src(s, S.off[g - (s ? P.rn : 0)]));
+    const int n = o ? nQ : nP;
+    int w = 0;
+    for (int v = lane; v < n; v += kComplexW) {
+      const int ring = ring_at(O.off, O.rn, v);
+      const int b = first(o, v), z = o ? qo[v] : rec.er[v + 1];
+      pt A = ld(pn, src(o, v));
+      for (int j = b; j < z; j++) {
+        const pt B = ld(pn, nS + ord[o][j]);
+        w += seg_wind(A, B, X);
+        A = B;
+      }
+      w += seg_wind(A, ld(pn, src(o, O.next(v, ring))), X);
+    }
+    w = grp_sum<kComplexW>(w);
+    if (lane == 0) in[g] = w & 1;
+  }
+  // -- createResult (polyclip.h:743-783): the segments, in order.  The
+  // departures from the crossings form cycles, so there are at most two
+  // segments per record, and one per ring without crossings.
+  const int maxSeg = 2 * nRec + nR;
+  int *so = ar.take<int>(maxSeg + 1, nullptr);  // first output position
+  int *sp = ar.take<int>(maxSeg, nullptr);      // first list position
+  int *sx = ar.take<int>(maxSeg, nullptr);      // component and direction
+  int *sr = ar.take<int>(maxSeg, nullptr);      // side and ring
+  const int maxComp = nRec + nR;
+  int *compRoot = ar.take<int>(maxComp, nullptr), *clen = ar.take<int>(maxComp, nullptr);
+  __shared__ int sh[3];
+  __syncthreads();
+  if (lane == 0) {
+    int ns = 0, nc = 0, tot = 0;
+    bool fits = true;
+    auto ring_list = [&](int s, int r, int &b, int &len) {
+      const ComplexSide &S = s ? Q : P;
+      b = S.off[r] + rc[s][r];
+      len = S.off[r + 1] + rc[s][r + 1] - b;
+    };
+    auto put = [&](int s, int r, bool fwd, int p, int len) {
+      if (ns >= maxSeg) {
+        fits = false;
+        return;
+      }
+      so[ns] = tot;
+      sp[ns] = p;
+      sx[ns] = 2 * nc + (fwd ? 1 : 0);
+      sr[ns] = 64 * s + r;
+      ns++;
+      tot += len;
+    };
+    for (int g = 0; g < nR; g++) {  // step 3.5: rings without crossings
+      const int s = g >= P.rn ? 1 : 0, r = g - (s ? P.rn : 0);
+      if (rc[s][r + 1] != rc[s][r] || (in[g] != 0) == U) continue;
+      int b, len;
+      ring_list(s, r, b, len);
+      compRoot[nc] = tot;
+      clen[nc] = len;
+      put(s, r, true, b, len);
+      nc++;
+    }
+    for (int c0 = 0; c0 < nRec && fits; c0++) {
+      if (vis[ord[0][c0]]) continue;
+      vis[ord[0][c0]] = 1;
+      const int start = tot;
+      int s = 0, j = c0;
+      while (fits) {
+        const int r = crng[s][j], lo = rc[s][r], hi = rc[s][r + 1];
+        int b, len;
+        ring_list(s, r, b, len);
+        const int st0 = in[(s ? P.rn : 0) + r] ? EXIT : ENTRY;
+        const int enex = ((j - lo) & 1) ? (st0 == ENTRY ? EXIT : ENTRY) : st0;
+        const bool fwd = (enex == ENTRY) != U;
+        const int j2 = fwd ? (j + 1 == hi ? lo : j + 1) : (j == lo ? hi - 1 : j - 1);
+        const int p = edge_of(s, ord[s][j]) + 1 + j, r2 = ord[s][j2];
+        const int p2 = edge_of(s, r2) + 1 + j2;
+        int d = fwd ? p2 - p : p - p2;
+        if (d <= 0) d += len;
+        int q = fwd ? p + 1 : p - 1;
+        if (q >= b + len) q -= len;
+        if (q < b) q += len;
+        put(s, r, fwd, q, d);
+        vis[r2] = 1;
+        if (s == 0 && j2 == c0) break;
+        s = 1 - s;
+        j = inv[s][r2];
+        if (s == 0 && j == c0) break;
+      }
+      if (nc < maxComp) {
+        compRoot[nc] = start;
+        clen[nc] = tot - start;
+      }
+      nc++;
+    }
+    so[ns] = tot;
+    if (tot > nS + 2 * nRec || tot > cap || nc > maxComp || nc > capComp) fits = false;
+    sh[0] = ns;
+    sh[1] = nc;
+    sh[2] = fits ? tot : -1;
+  }
+  __syncthreads();
+  const int ns = sh[0], nc = sh[1], tot = sh[2];
+  if (tot < 0) return false;
+  // -- the result vertices
+  int *omap = ar.take<int>(nS + 2 * nRec, nullptr), *cw = ar.take<int>(nS + 2 * nRec, nullptr);
+  for (int w = lane; w < tot; w += kComplexW) {
+    int a = 0, z = ns;  // the segment with so[a] <= w < so[a + 1]
+    while (z - a > 1) {
+      const int m = (a + z) >> 1;
+      if (so[m] <= w) a = m;
+      else z = m;
+    }
+    const int s = sr[a] >> 6, r = sr[a] & 63;
+    const ComplexSide &S = s ? Q : P;
+    const int b = S.off[r] + rc[s][r], len = S.off[r + 1] + rc[s][r + 1] - b;
+    int q = (sx[a] & 1) ? sp[a] + (w - so[a]) : sp[a] - (w - so[a]);
+    if (q >= b + len) q -= len;
+    if (q < b) q += len;
+    const int v = lst[s][q];
+    omap[w] = v;
+    cw[w] = sx[a] >> 1;
+    pt o;
+    if (v < nS) {
+      o = S.orig(v - (s ? nP : 0), r);
+    } else {  // (1 - alpha) P1 + alpha P2 in the original coordinates
+      const int e = rec.rp[v - nS], pr = ring_at(P.off, P.rn, e);
+      const double al = rec.al[v - nS];
+      const pt A = P.orig(e, pr), B = P.orig(P.next(e, pr), pr);
+      o = pt{(1.0 - al) * A.x + al * B.x, (1.0 - al) * A.y + al * B.y};
+    }
+    st(xy, w, o);
+  }
+  __syncthreads();
+  OutBuf O;
+  O.n = tot;
+  O.ncomp = nc;
+  O.compRoot = compRoot;
+  if (cleanup) {
+    int *sc = ar.take<int>(3 * nc + tot, nullptr);
+    grp_cleanup_compact<kComplexW>(O, xy, clen, cw, sc, pn, omap, 0);
+    __syncthreads();
+  }
+  for (int c = lane; c < O.ncomp; c += kComplexW) clenOut[c] = clen[c];
+  if (lane == 0) {
+    *outComps = O.ncomp;
+    *outVerts = O.n;
+  }
+  return true;
+}
+
 __global__ void __launch_bounds__(kComplexW)
-    k_complex_clip(long M, ComplexArgs a, ComplexWork w) {
+    k_complex_clip(long M, ComplexArgs a, ComplexWork w, const int2 *hits, int ldsBytes) {
   const long k = blockIdx.x;
   if (k >= M) return;
   const int lane = threadIdx.x;
@@ -588,8 +970,100 @@ __global__ void __launch_bounds__(kComplexW)
     return;
   }
   const ComplexPair cp = complex_pair(a.parts, k);
-  RingWalk P, Q;
-  complex_walks(a, cp, P, Q);
+  __shared__ ComplexRings R;
+  complex_rings(a, cp, R);
+  const ComplexSide P = complex_side(a, cp, R, 0), Q = complex_side(a, cp, R, 1);
+  const int nP = P.off[P.rn], nQ = Q.off[Q.rn], base = nP + nQ, nSrcP = nP;
+  const double nrm[3] = {a.norm[3 * k], a.norm[3 * k + 1], a.norm[3 * k + 2]};
+  const long long rb = a.recOff[k], nRec = a.recOff[k + 1] - rb;
+  // -- the records: in LDS when the pair fits there, else in the pair's
+  // global region
+  extern __shared__ __align__(16) char complex_lds[];
+  const bool fits = complex_fast_bytes(base, cp.bn + cp.on, nRec) <= ldsBytes;
+  Arena ar{fits ? complex_lds : nullptr, ldsBytes};
+  int *er = ar.take<int>(nSrcP + 1, w.edgeRec + a.edgeOff[k] + k);
+  int *recP = ar.take<int>(nRec, w.recP + rb), *recQ = ar.take<int>(nRec, w.recQ + rb);
+  int *recT = ar.take<int>(nRec, w.recT + rb);
+  double *recA = ar.take<double>(nRec, w.recA + rb), *recB = ar.take<double>(nRec, w.recB + rb);
+  for (int e = lane; e <= nSrcP; e += kComplexW) er[e] = 0;
+  __syncthreads();
+  bool plain = true;  // every record of type 1
+  auto scan_er = [&] {
+    __syncthreads();
+    const int tot = grp_scan_range<kComplexW, int>(
+        nSrcP, [&](int e) { return er[e]; }, [&](int e, int pre, int) { er[e] = pre; });
+    if (lane == 0) er[nSrcP] = tot;
+    __syncthreads();
+  };
+  if (nRec <= kCxHits) {
+    // the set-up's hits, one per lane, ranked by (P edge, Q edge)
+    const int2 h = lane < nRec ? hits[k * kCxHits + lane] : make_int2(0x7fffffff, 0);
+    int o = 0;
+    for (int l = 0; l < (int)nRec; l++) {
+      const int p = __builtin_amdgcn_readlane(h.x, l), q = __builtin_amdgcn_readlane(h.y, l);
+      o += p < h.x || (p == h.x && q < h.y) ? 1 : 0;
+    }
+    if (lane < nRec) {
+      pt P1, P2, Q1, Q2;
+      complex_edge(P, h.x, nrm, P1, P2);
+      complex_edge(Q, h.y, nrm, Q1, Q2);
+      double al, be;
+      const int t = itype(P1, P2, Q1, Q2, al, be);
+      recP[o] = h.x;
+      recQ[o] = h.y;
+      recT[o] = t;
+      recA[o] = al;
+      recB[o] = be;
+      plain = t == 1;
+      atomicAdd(&er[h.x], 1);
+    }
+    scan_er();
+  } else {
+    complex_records(P, Q, nrm, 1, [&](int p, int, int, double, double) { er[p]++; });
+    scan_er();
+    int p0 = -1, o = 0;  // the lane's P edge and its next record
+    complex_records(P, Q, nrm, 1, [&](int p, int q, int t, double al, double be) {
+      if (p != p0) {
+        p0 = p;
+        o = er[p];
+      }
+      recP[o] = p;
+      recQ[o] = q;
+      recT[o] = t;
+      recA[o] = al;
+      recB[o] = be;
+      o++;
+      plain = plain && t == 1;
+    });
+    __syncthreads();
+  }
+  double *xy = w.xyTmp + 2 * a.nodeOff[k];
+  int *clen = w.compLen + a.compOff[k];
+  if (fits && !grp_any<kComplexW>(!plain)) {
+    double *pn = ar.take<double>(2 * (base + nRec), nullptr);
+    for (int v = lane; v < base; v += kComplexW) {
+      const bool onQ = v >= nP;
+      const ComplexSide &S = onQ ? Q : P;
+      const int i = onQ ? v - nP : v;
+      const pt o = S.orig(i, ring_at(S.off, S.rn, i));
+      st(pn, v, pt{(o.x - nrm[0]) * nrm[2], (o.y - nrm[1]) * nrm[2]});
+    }
+    __syncthreads();
+    for (int r = lane; r < nRec; r += kComplexW) {
+      const int e = recP[r];
+      const pt P1 = ld(pn, e), P2 = ld(pn, P.next(e, ring_at(P.off, P.rn, e)));
+      const double al = recA[r];
+      st(pn, base + r, pt{(1.0 - al) * P1.x + al * P2.x, (1.0 - al) * P1.y + al * P2.y});
+    }
+    __syncthreads();
+    if (complex_fast(P, Q, (int)nRec, FastRecs{er, recP, recQ, recA, recB}, pn, ar,
+                     a.unionOp != 0, w.cleanup, a.nodeOff[k + 1] - a.nodeOff[k],
+                     a.compOff[k + 1] - a.compOff[k], xy, clen, w.outNComp + k,
+                     w.outNVerts + k))
+      return;
+    __syncthreads();
+  }
+  // -- lane 0's replay: the source nodes, ring by ring (P's rings, then Q's)
   const long long nb0 = a.nodeOff[k], cap = a.nodeOff[k + 1] - nb0;
   Nodes N;
   N.pn = w.npn + 2 * nb0;
@@ -603,80 +1077,27 @@ __global__ void __launch_bounds__(kComplexW)
   N.cap = (int)cap;
   double *alpha = w.nalpha + nb0;
   int *roots = w.roots + a.ringOff[k];
-  const double *nrm = a.norm + 3 * k;
-  // -- source nodes, ring by ring (P's rings, then Q's)
-  int base = 0;
-  for (int side = 0; side < 2; side++) {
-    const RingWalk &R = side ? Q : P;
-    for (int r = R.r0; r < R.r0 + R.rn; r++) {
-      long s;
-      int n;
-      ring_of(R.vn, R.vp, r, s, n);
-      for (int i = lane; i < n; i += kComplexW) {
-        const double x = R.C[2 * (s + i)], y = R.C[2 * (s + i) + 1];
-        const int v = base + i;
-        st(N.pn, v, pt{(x - nrm[0]) * nrm[2], (y - nrm[1]) * nrm[2]});
-        st(N.po, v, pt{x, y});
-        N.next[v] = base + (i + 1 == n ? 0 : i + 1);
-        N.prev[v] = base + (i == 0 ? n - 1 : i - 1);
-        N.nb[v] = -1;
-        N.fl[v] = F_SRC;
-        N.lab[v] = L_NONE;
-        N.enex[v] = NEITHER;
-        alpha[v] = -2.0;
-      }
-      if (lane == 0) roots[(side ? cp.bn : 0) + (r - R.r0)] = base;
-      base += n;
-    }
+  for (int v = lane; v < base; v += kComplexW) {
+    const bool onQ = v >= nP;
+    const ComplexSide &S = onQ ? Q : P;
+    const int sb = onQ ? nP : 0, i = v - sb, r = ring_at(S.off, S.rn, i);
+    const pt o = S.orig(i, r);
+    st(N.pn, v, pt{(o.x - nrm[0]) * nrm[2], (o.y - nrm[1]) * nrm[2]});
+    st(N.po, v, o);
+    N.next[v] = sb + S.next(i, r);
+    N.prev[v] = sb + (i == S.off[r] ? S.off[r + 1] - 1 : i - 1);
+    N.nb[v] = -1;
+    N.fl[v] = F_SRC;
+    N.lab[v] = L_NONE;
+    N.enex[v] = NEITHER;
+    alpha[v] = -2.0;
   }
-  const int nSrcP = (int)(a.edgeOff[k + 1] - a.edgeOff[k]);
+  for (int r = lane; r < P.rn + Q.rn; r += kComplexW)
+    roots[r] = r < P.rn ? P.off[r] : nP + Q.off[r - P.rn];
   N.n = base;
-  // -- records of every P edge, in Q order, at the edge's scanned offset
-  int *er = w.edgeRec + a.edgeOff[k] + k;  // nSrcP + 1 entries
-  const long long rb = a.recOff[k];
-  {
-    int e0 = 0;
-    for (int pr = P.r0; pr < P.r0 + P.rn; pr++) {
-      const int pn = P.vn[pr] - 1;
-      for (int pi = lane; pi < pn; pi += kComplexW) {
-        int cnt = 0;
-        complex_edge_records(P, pr, pi, Q, nrm, [&](int, int, double, double) { cnt++; });
-        er[e0 + pi] = cnt;
-      }
-      e0 += pn;
-    }
-    __syncthreads();
-    if (lane == 0) {  // exclusive scan of the per-edge counts
-      int run = 0;
-      for (int e = 0; e < nSrcP; e++) {
-        const int c = er[e];
-        er[e] = run;
-        run += c;
-      }
-      er[nSrcP] = run;
-    }
-    __syncthreads();
-    e0 = 0;
-    for (int pr = P.r0; pr < P.r0 + P.rn; pr++) {
-      const int pn = P.vn[pr] - 1;
-      for (int pi = lane; pi < pn; pi += kComplexW) {
-        long long o = rb + er[e0 + pi];
-        complex_edge_records(P, pr, pi, Q, nrm, [&](int qe, int t, double al, double be) {
-          w.recQ[o] = qe;
-          w.recT[o] = t;
-          w.recA[o] = al;
-          w.recB[o] = be;
-          o++;
-        });
-      }
-      e0 += pn;
-    }
-    __syncthreads();
-  }
+  __syncthreads();
   if (lane != 0) return;
   // -- the insertions in the reference's loop order (polyclip.h:200-277)
-  const int nSrcQ = base - nSrcP;
-  (void)nSrcQ;
   auto insert = [&](int V, int curr, double al) {  // insertVertex, polygon.h:101-113
     do {
       curr = N.next[curr];
@@ -698,9 +1119,8 @@ __global__ void __launch_bounds__(kComplexW)
     while (!(N.fl[two] & F_SRC)) two = N.next[two];
     const pt P1 = P_(N, one), P2 = P_(N, two), P1o = ld(N.po, one), P2o = ld(N.po, two);
     for (int j = er[e]; j < er[e + 1]; j++) {
-      const long long o = rb + j;
-      const int q1 = nSrcP + w.recQ[o], t = w.recT[o];
-      const double al = w.recA[o], be = w.recB[o];
+      const int q1 = nSrcP + recQ[j], t = recT[j];
+      const double al = recA[j], be = recB[j];
       const pt Q1 = P_(N, q1), Q1o = ld(N.po, q1);
       int IP, IQ;
       switch (t) {
@@ -783,8 +1203,6 @@ __global__ void __launch_bounds__(kComplexW)
     w.outNVerts[k] = 0;
     return;
   }
-  double *xy = w.xyTmp + 2 * nb0;
-  int *clen = w.compLen + a.compOff[k];
   int nc = 0, nv = 0;
   for (int c = 0; c < O.ncomp; c++) {
     int r = O.compRoot[c];
@@ -821,8 +1239,10 @@ void clip_complex(Context &c, const JoinInputs &in, const int *parts, long M,
   a.unionOp = unionOp ? 1 : 0;
   a.B = in.B;
   a.O = in.O;
-  a.bad = wsT<unsigned long long>(c, "cx_bad", 1);
-  fill_i32(c, (int *)a.bad, 0, 2);
+  // [0] bad parts, [1] LDS the fast path needs, [2, 6) status counts
+  unsigned long long *ctr = wsT<unsigned long long>(c, "cx_counters", 6);
+  a.bad = ctr;
+  fill_i32(c, (int *)ctr, 0, 12);
   a.status = wsT<int>(c, "cx_status", M);
   a.norm = wsT<double>(c, "cx_norm", 3 * M);
   int *nodeCap = wsT<int>(c, "cx_nodeCap", M), *compCap = wsT<int>(c, "cx_compCap", M);
@@ -833,23 +1253,23 @@ void clip_complex(Context &c, const JoinInputs &in, const int *parts, long M,
   a.recOff = wsT<long long>(c, "cx_recOff", M + 1);
   a.ringOff = wsT<long long>(c, "cx_ringOff", M + 1);
   a.edgeOff = wsT<long long>(c, "cx_edgeOff", M + 1);
-  hipLaunchKernelGGL(k_complex_setup, dim3((unsigned)M), dim3(kComplexW), 0, c.stream, M, a,
-                     nodeCap, compCap, rings, edgesP);
-  HIP_CHECK(hipGetLastError());
+  res.swapped = wsT<int>(c, "cx_swapped", M);
+  int2 *hits = wsT<int2>(c, "cx_hits", (long long)kCxHits * M);
   {
     LaunchTimer t(c, "gh_complex_count");
-    hipLaunchKernelGGL(k_complex_count, dim3((unsigned)M), dim3(kComplexW), 0, c.stream, M, a,
-                       recCnt, nodeCap, compCap);
+    hipLaunchKernelGGL(k_complex_setup, dim3((unsigned)M), dim3(kCxSetup), 0, c.stream, M, a,
+                       nodeCap, compCap, rings, edgesP, recCnt, res.swapped, ctr + 1,
+                       kComplexLds, hits);
     HIP_CHECK(hipGetLastError());
   }
-  scan_i32_to_i64(c, nodeCap, a.nodeOff, M);
-  scan_i32_to_i64(c, compCap, a.compOff, M);
-  scan_i32_to_i64(c, recCnt, a.recOff, M);
-  scan_i32_to_i64(c, rings, a.ringOff, M);
-  scan_i32_to_i64(c, edgesP, a.edgeOff, M);
-  long long tot[6];
+  scan_i32_to_i64_multi(c, {{nodeCap, a.nodeOff, M},
+                            {compCap, a.compOff, M},
+                            {recCnt, a.recOff, M},
+                            {rings, a.ringOff, M},
+                            {edgesP, a.edgeOff, M}});
+  long long tot[7];
   read_scalars(c, {a.nodeOff + M, a.compOff + M, a.recOff + M, a.ringOff + M, a.edgeOff + M,
-                   (const long long *)a.bad},
+                   (const long long *)a.bad, (const long long *)ctr + 1},
                tot);
   if (tot[5] != 0)
     throw Error{GCMF_ERR_ARG, "complex clip: a pair's rings lie outside its layer"};
@@ -873,6 +1293,7 @@ void clip_complex(Context &c, const JoinInputs &in, const int *parts, long M,
   w.oprev = wsT<int>(c, "cx_oprev", nodes);
   w.ocompRoot = wsT<int>(c, "cx_ocompRoot", comps);
   w.roots = wsT<int>(c, "cx_roots", nrings);
+  w.recP = wsT<int>(c, "cx_recP", recs);
   w.recQ = wsT<int>(c, "cx_recQ", recs);
   w.recT = wsT<int>(c, "cx_recT", recs);
   w.recA = wsT<double>(c, "cx_recA", recs);
@@ -885,14 +1306,14 @@ void clip_complex(Context &c, const JoinInputs &in, const int *parts, long M,
   w.cleanup = opt.cleanup;
   {
     LaunchTimer t(c, "gh_complex_clip");
-    hipLaunchKernelGGL(k_complex_clip, dim3((unsigned)M), dim3(kComplexW), 0, c.stream, M, a,
-                       w);
+    const int lds = (int)((tot[6] + 15) & ~15LL);
+    hipLaunchKernelGGL(k_complex_clip, dim3((unsigned)M), dim3(kComplexW), (size_t)lds, c.stream,
+                       M, a, w, (const int2 *)hits, lds);
     HIP_CHECK(hipGetLastError());
   }
   res.vertOff = wsT<long long>(c, "cx_vOff", M + 1);
   res.compOff = wsT<long long>(c, "cx_cOff", M + 1);
-  scan_i32_to_i64(c, w.outNVerts, res.vertOff, M);
-  scan_i32_to_i64(c, w.outNComp, res.compOff, M);
+  scan_i32_to_i64_multi(c, {{w.outNVerts, res.vertOff, M}, {w.outNComp, res.compOff, M}});
   res.xy = wsT<double>(c, "cx_out_xy", 2 * nodes);
   res.compSizes = wsT<int>(c, "cx_out_comp", comps);
   hipLaunchKernelGGL(k_gather_out<64>, dim3(pgrp_grid(M, 64)), dim3(pgrp_block(64)), 0, c.stream,
@@ -901,12 +1322,9 @@ void clip_complex(Context &c, const JoinInputs &in, const int *parts, long M,
                      w.compLen, res.xy, res.compSizes);
   HIP_CHECK(hipGetLastError());
   res.status = a.status;
-  res.swapped = wsT<int>(c, "cx_swapped", M);
-  fill_i32(c, res.swapped, 0, M);
   res.ncomp = w.outNComp;
   res.nverts = w.outNVerts;
-  unsigned long long *sc = wsT<unsigned long long>(c, "cx_status_counts", 4);
-  fill_i32(c, (int *)sc, 0, 8);
+  unsigned long long *sc = ctr + 2;
   hipLaunchKernelGGL(k_status_counts, dim3(std::min<unsigned>(kStatBlocks, grid_for(M, 256))),
                      dim3(256), 0, c.stream, M, (const int *)a.status, sc);
   HIP_CHECK(hipGetLastError());

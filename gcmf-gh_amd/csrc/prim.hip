@@ -603,7 +603,7 @@ __global__ void k_lb_clear_all(unsigned long long *desc) {
 // up to kLbSegs arrays scanned by one launch: segment j takes the tiles
 // [t0[j], t0[j + 1]) (at least one, so that out[0] = 0 of an empty array
 // is written too)
-constexpr int kLbSegs = 4;
+constexpr int kLbSegs = 5;
 struct LbSegs {
   const int *in[kLbSegs];
   long long *out[kLbSegs];

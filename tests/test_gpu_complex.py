@@ -102,3 +102,35 @@ def test_complex_rejects_bad_parts(gctx):
     finally:
         db.free()
         do.free()
+
+
+@pytest.mark.parametrize("union", [False, True])
+@pytest.mark.parametrize("sizes", [(3, 3), (63, 65), (64, 128), (700, 650), (900, 850)])
+def test_complex_wave_path_edges(gctx, sizes, union):
+    """The whole-wave path (pairs whose arrays fit in LDS, up to about 1600
+    vertices) and lane 0's replay (larger pairs, and pairs on a coordinate
+    grid, with shared vertices and collinear edges) at wave and LDS edges:
+    bit for bit the oracle's, a hole and its island crossed by the other
+    side or not."""
+    cases = []
+    for s in range(6):
+        P, Q = G.gen_single_pair(0, 40 + s, *sizes)
+        h = 0.35 * P[::-1] + np.array([0.05 * s, -0.02])
+        cases.append(([P, h, 0.2 * h], [Q]))
+        cases.append(([P], [Q, 0.4 * Q[::-1]]))
+        g = 0.05
+        cases.append(([np.round(P / g) * g], [np.round(Q / g) * g]))
+    for P, Q in cases:  # the grid leaves repeated vertices: drop them
+        for side in (P, Q):
+            for i, r in enumerate(side):
+                side[i] = r[(r != np.roll(r, 1, 0)).any(1)]
+    cases = [(P, Q) for P, Q in cases if min(len(r) for r in P + Q) >= 3]
+    flags = G.CLIP_NORMALIZE | (G.CLIP_UNION if union else 0)
+    st, (status, res) = run_complex(gctx, cases, flags)
+    mode = 5 | (8 if union else 0)
+    # a trace that does not close fails in the oracle (-1) and here (-1, or
+    # -5 when the replay's output region fills before its step limit)
+    failed = [k for k in range(len(cases)) if O.clip_multi(*cases[k], mode)[0] < 0]
+    assert all(status[k] in (-1, -5) and res[k] == [] for k in failed)
+    rest = [k for k in range(len(cases)) if k not in failed]
+    check([cases[k] for k in rest], [status[k] for k in rest], [res[k] for k in rest], mode)
