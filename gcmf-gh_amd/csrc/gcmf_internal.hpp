@@ -69,7 +69,7 @@ struct Tuning {
                             // LDS); 0: a wave's lanes of one pair walk it together by runs
   int countBlock = 128;     // threads per block of the count kernel (64, 128, 256)
   int labelLds = 20480;     // LDS bytes per labelling wave for a pair's arrays (0: none)
-  int ldsMaxQ = 1024;       // pairs with Q rings above cullMin and up to this size are
+  int ldsMaxQ = 0;          // pairs with Q rings above cullMin and up to this size are
                             // counted with Q binned in LDS (at most 1024; 0: none)
 };
 

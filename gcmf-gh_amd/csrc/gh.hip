@@ -1810,21 +1810,30 @@ __device__ __forceinline__ double wave_uniform(double v) {
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-// The next group of a wave's lanes for the wave walk: the pending lanes
-// (P edges walked over their whole Q ring, not yet counted) of the pair of
-// the first pending lane, with that ring's first global edge e0 and length
-// n, and U, the union of the group's widened boxes over the lanes that walk
-// (all of the plane when one of them may form a tiny pair).  False when no
-// lane is pending.  Every lane of the wave calls it.
-__device__ __forceinline__ bool wave_group(const CountLane &L, bool pending, bool &group,
-                                           EdgeBox &U, long long &e0, int &n) {
+// A group of a wave's lanes that walk one Q ring together: the ring's first
+// global edge e0 and length n, and what the runs of the ring are tested
+// against first: U, the union of the walking
+// lanes' widened boxes, and la, the shortest of the walking lanes' edges that
+// may form a tiny pair (infinite without one), with the pair's threshold T.
+struct WaveGroup {
+  bool mine;   // this lane is of the group
+  bool walks;  // ... and its edge is walked
+  EdgeBox U;
+  double la, T;
+  long long e0;
+  int n;
+};
+
+// The next group: the pending lanes (P edges not yet counted) of the pair of
+// the first pending lane.  False when no lane is pending.  Every lane of the
+// wave calls it.
+__device__ __forceinline__ bool wave_group(const CountLane &L, bool pending, WaveGroup &G) {
   const unsigned long long pm = __ballot(pending);
   if (!pm) return false;
   const int first = __ffsll((long long)pm) - 1;
   const int k0 = __shfl(L.k, first, 64);
-  group = pending && L.k == k0;
-  const bool walks = group && L.flag;
-  const bool anyTiny = __ballot(walks && L.f.tiny) != 0;
+  G.mine = pending && L.k == k0;
+  const bool walks = G.walks = G.mine && L.flag;
   double x0 = walks ? L.f.wide.x0 : INFINITY, y0 = walks ? L.f.wide.y0 : INFINITY;
   double x1 = walks ? L.f.wide.x1 : -INFINITY, y1 = walks ? L.f.wide.y1 : -INFINITY;
   for (int off = 32; off > 0; off >>= 1) {
@@ -1833,17 +1842,21 @@ __device__ __forceinline__ bool wave_group(const CountLane &L, bool pending, boo
     x1 = fmax(x1, __shfl_xor(x1, off, 64));
     y1 = fmax(y1, __shfl_xor(y1, off, 64));
   }
-  if (anyTiny) {
-    x0 = y0 = -INFINITY;
-    x1 = y1 = INFINITY;
+  double la = INFINITY;
+  if (__ballot(walks && L.f.tiny)) {
+    if (walks && L.f.tiny) la = L.f.la;
+    for (int off = 32; off > 0; off >>= 1) la = fmin(la, __shfl_xor(la, off, 64));
   }
   // the same in every lane: held in scalar registers
-  U = EdgeBox{wave_uniform(x0), wave_uniform(y0), wave_uniform(x1), wave_uniform(y1)};
+  G.U = EdgeBox{wave_uniform(x0), wave_uniform(y0), wave_uniform(x1), wave_uniform(y1)};
+  G.la = wave_uniform(la);
+  G.T = wave_uniform(__shfl(L.f.T, first, 64));
   const long long b0 = __shfl(L.bBase, first, 64);
   const int n0 = (int)__shfl(L.bN, first, 64);
-  e0 = (long long)__builtin_amdgcn_readfirstlane((unsigned)b0) |
-       ((long long)__builtin_amdgcn_readfirstlane((unsigned)((unsigned long long)b0 >> 32)) << 32);
-  n = __builtin_amdgcn_readfirstlane(n0);
+  G.e0 = (long long)__builtin_amdgcn_readfirstlane((unsigned)b0) |
+         ((long long)__builtin_amdgcn_readfirstlane((unsigned)((unsigned long long)b0 >> 32))
+          << 32);
+  G.n = __builtin_amdgcn_readfirstlane(n0);
   return true;
 }
 
@@ -1855,34 +1868,86 @@ __device__ __forceinline__ double lane_d(double v, int l) {
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-// The count pass of a group of a wave's lanes that share one Q ring (global
-// edges [e0, e0 + n)), walked by every lane of the wave in step: the ring's
-// runs of kRun1 edges (boxes b1, global edge order) whose box misses U are
-// left out, since U holds the widened boxes of every walking lane of the
-// group, none with a possible tiny pair (U is the whole plane otherwise), so
-// each walking lane's filter skips every edge of such a run (its endpoints
-// lie beyond one side of the lane's widened box); of each other run, lanes
-// 0..kRun1 load its vertices once and every lane reads them from there (in
-// scalar registers), in index order.  Lanes that do not walk take part
-// without visiting.
+// The walk of a group of a wave's lanes over their Q ring, in index order,
+// by its runs of kRun1 edges (boxes in global edge order).  64 runs at a time,
+// lane r tests run r against the group's box and tiny bound; on rings above
+// the culling threshold each lane then tests the runs that pass against its
+// own widened box and tiny bound (run_hit, the test of the lane-by-lane
+// culled walk), and a run that no lane's edge can pair with is left out.  Of
+// each other run, lanes 0..kRun1 load its vertices once
+// and every lane reads them from there (in scalar registers); f(hit, q, B_q,
+// B_q+1) is called with whether the lane itself has to visit.  Rings of more
+// than kWaveRun2 edges find their runs through the kRun2-edge runs first
+// where those boxes exist.  Returns the edges this lane visited.
+//
+// What bounds it is the visited runs (17 loads' latency and 16 x 8 readlanes
+// each) and the lanes' classifications, one after another.  Rings above the
+// culling threshold used to be walked by each lane by itself through all
+// three levels of runs; in this walk the count of the 10^6 x 10^5 pair takes
+// 0.66 instead of 0.82 ms and that of 20 000 pairs of log-normal sizes 0.42
+// instead of 0.52 ms.  Rings up to the threshold skip the lanes' own tests:
+// with them the join workload's pass took 0.40 instead of 0.37 ms.
+constexpr int kWaveRun2 = 1024;
+
 template <class F>
-__device__ __forceinline__ int wave_ring_edges(const double *V, long long e0, int n,
-                                               const double *b1, const EdgeBox &U, F &&f) {
-  // run r covers the ring's edges [r kRun1 - o, (r + 1) kRun1 - o)
-  const double *b = b1 + 4 * (e0 / kRun1);
-  const int o = (int)(e0 % kRun1);
-  const int lane = (int)__lane_id();
+__device__ __forceinline__ int wave_ring_edges(const double *V, const WaveGroup &G,
+                                               const CountLane &L, const RunBoxes &rb, F &&f) {
+  const long long e0 = G.e0;
+  const int n = G.n, lane = (int)__lane_id();
   int visited = 0;
-  for (int qa = 0, qz = kRun1 - o; qa < n; qa = qz, qz += kRun1, b += 4) {
-    if (U.x0 > b[2] || U.x1 < b[0] || U.y0 > b[3] || U.y1 < b[1]) continue;
-    const int z = min(qz, n);
-    visited += z - qa;
-    // vertices qa .. z (the last one wraps to 0 at the ring's end)
-    pt v{0.0, 0.0};
-    if (lane <= z - qa) v = ld(V, qa + lane == n ? 0 : qa + lane);
-    for (int q = qa; q < z; q++) {
-      const int j = q - qa;
-      f(q, pt{lane_d(v.x, j), lane_d(v.y, j)}, pt{lane_d(v.x, j + 1), lane_d(v.y, j + 1)});
+  // whether the group may pair with edges of run r
+  auto group_hits = [&](const double *box, const double *len, long long r, long long z,
+                        double b[4], double &lmin) {
+    if (r >= z) return false;
+    b[0] = box[4 * r];
+    b[1] = box[4 * r + 1];
+    b[2] = box[4 * r + 2];
+    b[3] = box[4 * r + 3];
+    lmin = len[r];
+    return box_hit(b, G.U) || G.la * lmin < G.T;
+  };
+  auto runs = [&](long long a, long long z) {
+    for (long long g = a; g < z; g += 64) {
+      double b[4] = {0.0, 0.0, 0.0, 0.0}, lmin = 0.0;
+      unsigned long long m = __ballot(group_hits(rb.b1, rb.l1, g + lane, z, b, lmin));
+      while (m) {
+        const int l = __ffsll((long long)m) - 1;
+        m &= m - 1;
+        bool hit = G.walks;
+        if (n > rb.cullMin) {
+          const double bl[4] = {lane_d(b[0], l), lane_d(b[1], l), lane_d(b[2], l),
+                                lane_d(b[3], l)};
+          hit = hit && (box_hit(bl, L.f.wide) || (L.f.tiny && L.f.la * lane_d(lmin, l) < L.f.T));
+          if (!__ballot(hit)) continue;
+        }
+        const long long q0 = (g + l) * kRun1 - e0;  // the run's edges [qa, qz)
+        const int qa = (int)max(q0, 0LL), qz = (int)min(q0 + kRun1, (long long)n);
+        if (hit) visited += qz - qa;
+        // vertices qa .. qz (the last one wraps to 0 at the ring's end)
+        pt v{0.0, 0.0};
+        if (lane <= qz - qa) v = ld(V, qa + lane == n ? 0 : qa + lane);
+        for (int q = qa; q < qz; q++) {
+          const int j = q - qa;
+          f(hit, q, pt{lane_d(v.x, j), lane_d(v.y, j)},
+            pt{lane_d(v.x, j + 1), lane_d(v.y, j + 1)});
+        }
+      }
+    }
+  };
+  const long long a1 = e0 / kRun1, z1 = (e0 + n - 1) / kRun1 + 1;
+  if (rb.b2 == nullptr || n <= kWaveRun2) {
+    runs(a1, z1);
+    return visited;
+  }
+  constexpr int kUp = kRun2 / kRun1;
+  const long long z2 = (z1 - 1) / kUp + 1;
+  for (long long g = a1 / kUp; g < z2; g += 64) {
+    double b[4], lmin;
+    unsigned long long m = __ballot(group_hits(rb.b2, rb.l2, g + lane, z2, b, lmin));
+    while (m) {
+      const int l = __ffsll((long long)m) - 1;
+      m &= m - 1;
+      runs(max((g + l) * kUp, a1), min((g + l) * kUp + kUp, z1));
     }
   }
   return visited;
@@ -1942,18 +2007,16 @@ __device__ __forceinline__ void count_edge_cpu(const CountLane &L, const double 
 
 // count_edge_cpu for a group of a wave's lanes that walks one Q ring
 // together (wave_ring_edges); every lane of the wave calls it
-__device__ __forceinline__ void count_edge_wave(const CountLane &L, bool group,
+__device__ __forceinline__ void count_edge_wave(const CountLane &L, const WaveGroup &G,
                                                 const double *ringQ, int *cnt1P, int *cnt2P,
-                                                int *boolP, int *lstP, long long e0, int n,
-                                                const double *b1, const EdgeBox &U,
+                                                int *boolP, int *lstP, const RunBoxes &rb,
                                                 unsigned long long &ev, unsigned long long &tv) {
-  const bool walks = group && L.flag;
   const pt A1 = L.A1, A2 = L.A2;
   const CpuFilter &f = L.f;
   int c1 = 0, c2 = 0;
   int *lst = lstP + (long long)L.ga * kPartners;
-  auto visit = [&](int q, pt B1, pt B2) {
-    if (!walks || f.skip(q, A1, A2, B1, B2)) return;
+  auto visit = [&](bool hit, int q, pt B1, pt B2) {
+    if (!hit || f.skip(q, A1, A2, B1, B2)) return;
     double al, be;
     ev++;
     const int t = itype(A1, A2, B1, B2, al, be);
@@ -1963,11 +2026,8 @@ __device__ __forceinline__ void count_edge_wave(const CountLane &L, bool group,
     }
     c2 += ins_on_p(t) ? 1 : 0;
   };
-  if (__ballot(walks)) {
-    const int vis = wave_ring_edges(ringQ + 2 * e0, e0, n, b1, U, visit);
-    if (walks) tv = vis;
-  }
-  if (group) {
+  if (__ballot(G.walks)) tv += wave_ring_edges(ringQ + 2 * G.e0, G, L, rb, visit);
+  if (G.mine) {
     cnt1P[L.ga] = c1;
     cnt2P[L.ga] = c2 + 1;
     boolP[L.ga] = L.flag;
@@ -1977,21 +2037,18 @@ __device__ __forceinline__ void count_edge_wave(const CountLane &L, bool group,
 // five waves per SIMD for the plain walk (at most 102 VGPRs, no spills): it
 // is bound by latency, and 5 waves run it 6 % faster than the 4 that its
 // register count would otherwise allow (0.42 vs 0.45 ms on the join
-// workload); the culled walk keeps the registers it needs to run without spills
-// skipQ (optional): the Q edges' kRun1-edge run boxes, with which the P
-// edges of a wave walked over their whole Q ring walk it together, one
-// group per pair, leaving out the runs no lane of the group can pair with
-// (count_edge_wave).  WAVE: skipQ is given and every edge is a P edge
-// (edgesQ = 0), so that without culling no lane walks on its own and the
-// lane walk is left out of the kernel.
+// workload); the culled lane walk keeps the registers it needs to run without
+// spills.  WAVE (Tuning::countStage 0): the P edges of a wave walk their Q
+// rings together, one group per pair (count_edge_wave; boxQ holds the Q
+// edges' run boxes); otherwise every lane walks on its own, rings above the
+// culling threshold through the run boxes when CULL.
 template <bool CULL, bool WAVE>
 __global__ void __launch_bounds__(256, CULL ? 1 : 5)
     k_count_cpu(long edgesP, long edgesQ, const int *mapP, const int *mapQ,
                 const long long *offP, const long long *offQ, const double *ringP,
                 const double *ringQ, const double *cf, int *cnt1P, int *cnt2P, int *cnt1Q,
                 int *cnt2Q, int *boolP, int *boolQ, unsigned long long *wstat, int *lstP,
-                int *lstQ, RunBoxes boxP, RunBoxes boxQ, int ldsQ, int stageOk,
-                const double *skipQ) {
+                int *lstQ, RunBoxes boxP, RunBoxes boxQ, int ldsQ, int stageOk) {
   const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
   unsigned long long ev = 0, tv = 0;
   // stage the wave's Q ring when every P edge of the wave is of one pair
@@ -2021,26 +2078,118 @@ __global__ void __launch_bounds__(256, CULL ? 1 : 5)
   }
   const CountLane L = count_prep(g, edgesP, edgesQ, mapP, mapQ, offP, offQ, ringP, ringQ, cf,
                                  boxP.cullMin, ldsQ);
-  // P edges walked over their whole Q ring: one group per pair of the wave
-  bool pending = WAVE && L.live && L.sideP && !(CULL && L.bN > boxP.cullMin);
   if (WAVE) {
-    EdgeBox U;
-    long long e0;
-    int n;
-    bool group;
-    while (wave_group(L, pending, group, U, e0, n)) {
-      count_edge_wave(L, group, ringQ, cnt1P, cnt2P, boolP, lstP, e0, n, skipQ, U, ev, tv);
-      if (group) pending = false;
+    bool pending = L.live;
+    WaveGroup G;
+    while (wave_group(L, pending, G)) {
+      count_edge_wave(L, G, ringQ, cnt1P, cnt2P, boolP, lstP, boxQ, ev, tv);
+      if (G.mine) pending = false;
     }
-  }
-  if ((CULL || !WAVE) && L.live && !(WAVE && L.sideP && !(CULL && L.bN > boxP.cullMin)))
+  } else if (L.live) {
     count_edge_cpu<CULL>(L, ringP, ringQ, cnt1P, cnt2P, cnt1Q, cnt2Q, boolP, boolQ, lstP, lstQ,
                          boxP, boxQ, stage, ev, tv);
+  }
   // every lane of every wave reaches the statistics
   wave_stats(wstat, g, ev, tv);
 }
 
+// The count pass of a call with few P edges: one wave per P edge.  64 runs at
+// a time, lane r tests run r as the lane-by-lane culled walk does (run_hit);
+// the edges of the runs that pass are then taken four runs at a time, one
+// edge per lane, and ballots put the partners in index order.  Counts, flags,
+// lists and classified pairs are the other walks'.
+//
+// The walks with one lane per P edge visit and classify a wave's edges one
+// after another, which hides behind other waves only where there are
+// thousands of them; here an edge waits for about four dependent loads, but a
+// launch spends a wave on it.  Measured on one MI355X, this form against the
+// wave walk, in us: 64 P edges 7 / 25, 2 000 12 / 111, 7 500 (37 pairs) 12 /
+// 50, 47 000 (200 pairs) 41 / 49, 107 000 (400 pairs) 82 / 52; 32 000 of
+// joined pairs 26 / 127, 316 000 204 / 217, 688 000 437 / 254.  The line lies
+// where the batches' two sides meet.
+constexpr long kCountEdgeMax = 65536;
+
+__global__ void __launch_bounds__(256)
+    k_count_edge(long edgesP, const int *mapP, const long long *offP, const long long *offQ,
+                 const double *ringP, const double *ringQ, const double *cf, int *cnt1P,
+                 int *cnt2P, int *boolP, unsigned long long *wstat, int *lstP, RunBoxes rb) {
+  const long g = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (g >= edgesP) return;
+  const int lane = (int)__lane_id();
+  const CountLane L = count_prep(g, edgesP, 0, mapP, nullptr, offP, offQ, ringP, ringQ, cf, 0, 0);
+  const long long e0 = L.bBase, n = L.bN;
+  const double *V = ringQ + 2 * e0;
+  int c1 = 0, c2 = 0, ev = 0, tv = 0;
+  int *lst = lstP + g * kPartners;
+  auto hits = [&](const double *box, const double *len, long long r, long long z) {
+    return r < z && run_hit(box + 4 * r, len + r, L.f.wide, L.f.la, L.f.T);
+  };
+  auto runs = [&](long long a, long long z) {
+    for (long long r0 = a; r0 < z; r0 += 64) {
+      unsigned long long m = __ballot(hits(rb.b1, rb.l1, r0 + lane, z));
+      while (m) {
+        long long run = -1;  // this lane's of the next four runs
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          if (!m) break;
+          if ((lane >> 4) == u) run = r0 + __ffsll((long long)m) - 1;
+          m &= m - 1;
+        }
+        const long long q = run * kRun1 + (lane & 15) - e0;
+        const bool in = run >= 0 && q >= 0 && q < n;
+        int t = 0;
+        bool seen = false;
+        if (in) {
+          const pt B1 = ld(V, q), B2 = ld(V, q + 1 == n ? 0 : q + 1);
+          if (!L.f.skip((int)q, L.A1, L.A2, B1, B2)) {
+            double al, be;
+            seen = true;
+            t = itype(L.A1, L.A2, B1, B2, al, be);
+          }
+        }
+        const unsigned long long h = __ballot(t != 0);
+        const int k = c1 + rank_lt(h);
+        if (t != 0 && k < kPartners) lst[k] = (int)q;
+        c1 += __popcll(h);
+        c2 += __popcll(__ballot(ins_on_p(t)));
+        ev += __popcll(__ballot(seen));
+        tv += __popcll(__ballot(in));
+      }
+    }
+  };
+  static_assert(kRun1 == 16, "a run is 16 lanes");
+  if (L.flag && n > 0) {
+    const long long a1 = e0 / kRun1, z1 = (e0 + n - 1) / kRun1 + 1;
+    if (rb.b2 == nullptr || n <= kWaveRun2) {
+      runs(a1, z1);
+    } else {
+      constexpr int kUp = kRun2 / kRun1;
+      const long long z2 = (z1 - 1) / kUp + 1;
+      for (long long r0 = a1 / kUp; r0 < z2; r0 += 64) {
+        unsigned long long m = __ballot(hits(rb.b2, rb.l2, r0 + lane, z2));
+        while (m) {
+          const long long r = r0 + __ffsll((long long)m) - 1;
+          m &= m - 1;
+          runs(max(r * kUp, a1), min(r * kUp + kUp, z1));
+        }
+      }
+    }
+  }
+  if (lane == 0) {
+    cnt1P[g] = c1;
+    cnt2P[g] = c2 + 1;
+    boolP[g] = L.flag;
+    wstat[2 * g] = ev;
+    wstat[2 * g + 1] = tv;
+  }
+}
+
 // ---------------------------------------- count pass, Q binned in LDS ----
+// Off by default (Tuning::ldsMaxQ 0): it gives a pair one block, and the wave
+// walk, whose waves share a long P ring, has become the faster form (20 000
+// pairs of log-normal sizes: 6.3 ms in this pass for the pairs it took, 0.05
+// ms more in the walk without it).  gcmf_tune_clip still tries both.
+//
 // The CPU route's count pass for the pairs whose Q ring is longer than the
 // culling threshold and fits in LDS (Tuning::cullMin < nQ <= Tuning::ldsMaxQ
 // <= kLdsQ): one block per pair.  (Shorter rings keep the lockstep walk of
@@ -5420,11 +5569,10 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
         sum_wave_stats(c, bstat, M, stats);
       }
       {  // the ring walk: every pair the LDS pass does not take
-        const bool cull = boxQ.b1 != nullptr;
-        // the Q edges' kRun1-edge run boxes for the waves' walks (the
-        // staged walk, Tuning::countStage, walks lane by lane instead)
-        const double *skipQ = c.tune.countStage ? nullptr : boxQ.b1;
-        if (!skipQ && !c.tune.countStage && edgesQ > 0) {
+        const bool cull = boxQ.b1 != nullptr, wave = c.tune.countStage == 0;
+        // the wave walk needs the Q edges' kRun1-edge run boxes
+        RunBoxes walkQ = boxQ;
+        if (wave && !cull && edgesQ > 0) {
           const long r1 = (edgesQ + kRun1 - 1) / kRun1;
           double *b1 = wsT<double>(c, "gh_rb1Q", 4 * r1);
           double *l1 = wsT<double>(c, "gh_rl1Q", r1);
@@ -5432,25 +5580,33 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
                              edgesQ, mapQ, (const long long *)offQ, (const double *)ringQ, b1,
                              l1);
           HIP_CHECK(hipGetLastError());
-          skipQ = b1;
+          walkQ.b1 = b1;
+          walkQ.l1 = l1;
         }
         const int cb = c.tune.countBlock;
-        const unsigned grid = grid_for(edgesP, cb);
-        const long waves = (long)grid * cb / 64;
+        const bool perEdge = wave && capQ <= minQ && edgesP <= kCountEdgeMax;
+        const unsigned grid = perEdge ? grid_for(edgesP, 4) : grid_for(edgesP, cb);
+        const long waves = perEdge ? edgesP : (long)grid * cb / 64;
         unsigned long long *wstat = wsT<unsigned long long>(c, "gh_wave_stats", 2 * waves);
-        {
+        if (perEdge) {
+          LaunchTimer t(c, "gh_count");
+          hipLaunchKernelGGL(k_count_edge, dim3(grid), dim3(256), 0, c.stream, edgesP, mapP,
+                             (const long long *)offP, (const long long *)offQ,
+                             (const double *)ringP, (const double *)ringQ, (const double *)cf,
+                             cnt1P, cnt2P, boolP, wstat, lstP, walkQ);
+          HIP_CHECK(hipGetLastError());
+        } else {
           LaunchTimer t(c, "gh_count");
           // the Q-ring staging slices: kStageQ points per wave
           const size_t stageBytes = c.tune.countStage ? (size_t)(cb / 64) * kStageQ * 16 : 0;
-          // (P edges only, so the wave walk's form applies whenever skipQ is given)
-          auto kern = cull ? (skipQ ? k_count_cpu<true, true> : k_count_cpu<true, false>)
-                           : (skipQ ? k_count_cpu<false, true> : k_count_cpu<false, false>);
+          auto kern = wave ? k_count_cpu<false, true>
+                           : (cull ? k_count_cpu<true, false> : k_count_cpu<false, false>);
           hipLaunchKernelGGL(kern, dim3(grid), dim3(cb),
                              stageBytes, c.stream, edgesP, 0L, mapP, mapQ,
                              (const long long *)offP, (const long long *)offQ, ringP, ringQ,
                              (const double *)cf,
                              cnt1P, cnt2P, cnt1Q, cnt2Q, boolP, boolQ, wstat, lstP, lstQ, boxP,
-                             boxQ, capQ > minQ ? capQ : 0, c.tune.countStage, skipQ);
+                             walkQ, capQ > minQ ? capQ : 0, c.tune.countStage);
           HIP_CHECK(hipGetLastError());
         }
         sum_wave_stats(c, wstat, waves, stats);

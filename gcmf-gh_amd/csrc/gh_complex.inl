@@ -459,20 +459,6 @@ __device__ __forceinline__ ComplexSide complex_side(const ComplexArgs &a, const 
                      side ? cp.on : cp.bn};
 }
 
-// Whether one parameter of the edge pair lies well outside [-eps, 1 - eps),
-// so that itype() is 0: with the ends of one edge strictly on one side of the
-// other's line, a = A1 / (A1 - A2) is at least 1 - 2^-53 when |A1| >
-// |A1 - A2| and below -1e-6 (1 - 2^-50) when it is negative and |A1| > 1e-6
-// |A1 - A2|, and no type takes such a parameter.
-__device__ __forceinline__ bool edges_apart(pt P1, pt P2, pt Q1, pt Q2) {
-  const double AP1 = triA(P1, Q1, Q2), AP2 = triA(P2, Q1, Q2), dP = AP1 - AP2;
-  const double AQ1 = triA(Q1, P1, P2), AQ2 = triA(Q2, P1, P2), dQ = AQ1 - AQ2;
-  const bool sP = (AP1 > 0 && AP2 > 0) || (AP1 < 0 && AP2 < 0);
-  const bool sQ = (AQ1 > 0 && AQ2 > 0) || (AQ1 < 0 && AQ2 < 0);
-  return fabs(dP) > kGhEps &&
-         ((sP && fabs(AP1) > 1e-6 * fabs(dP)) || (sQ && fabs(AQ1) > 1e-6 * fabs(dQ)));
-}
-
 // edge v of a side in the frame nrm
 __device__ __forceinline__ void complex_edge(const ComplexSide &S, int v, const double nrm[3],
                                              pt &A, pt &B) {

@@ -216,7 +216,7 @@ typedef struct {
   int lds_max_q;       /* pairs whose Q ring is longer than cull_min and has at
                           most this many vertices are counted with Q binned in
                           LDS, one block per pair; the others walk Q's ring
-                          (0..1024, 1024; 0 or <= cull_min: no LDS pass) */
+                          (0..1024, 0; 0 or <= cull_min: no LDS pass) */
   int label_lds;       /* bytes of LDS each labelling wave keeps a pair's node
                           arrays and scratch in; what does not fit stays in
                           HBM (0..65536, a multiple of 16; 20480) */

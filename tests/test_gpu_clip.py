@@ -724,3 +724,36 @@ def test_clip_grid_labelling_batch(gctx):
             for x, y in zip(a, b):
                 np.testing.assert_array_equal(x, y)
         check_results(gctx, st, cases, NORM)
+
+
+@pytest.mark.parametrize("n_p, n_q, kind, snap", [
+    (5, 3, 0, 0.0), (64, 16, 0, 0.0), (65, 17, 0, 0.0), (700, 1024, 0, 0.0),
+    (1200, 1025, 0, 0.0), (6000, 2500, 1, 0.0), (2500, 2300, 1, 1e-2), (40, 1500, 1, 1e-2)])
+def test_count_one_wave_per_edge(gctx, n_p, n_q, kind, snap):
+    """A call with few P edges is counted by one wave per P edge: its arrays
+    equal the lane-by-lane walk's (count_stage 1) bit for bit, at the edges of
+    the 16-edge runs and of the walk through the 256-edge runs, tiny and
+    collinear edges included."""
+    cases = [("p%d" % s,) + tuple(G.gen_single_pair(kind, 70 + s, n_p, n_q, snap=snap))
+             for s in range(3)]
+    default = gctx.tuning()
+    out = []
+    try:
+        for stage in (0, 1):
+            for cull in (64, 1 << 40):
+                gctx.set_tuning(cull, default["big_nodes"], default["count_block"], 0,
+                                count_stage=stage)
+                st = run_batch(gctx, cases, G.CLIP_NORMALIZE)
+                assert st["edges_p"] <= 65536
+                n = {"psP1": st["edges_p"] + 1, "psP2": st["edges_p"] + 1,
+                     "psQ1": st["edges_q"] + 1, "psQ2": st["edges_q"] + 1,
+                     "boolP": st["edges_p"], "iP": 2 * st["slots_p"], "iQ": 2 * st["slots_q"],
+                     "nbP": st["slots_p"], "nbQ": st["slots_q"], "status": len(cases),
+                     "comp_sizes": st["total_comps"], "xy": 2 * st["total_verts"]}
+                out.append((st, {f: gctx.clip_get(f, c) for f, c in n.items()}))
+    finally:
+        gctx.set_tuning(**default)
+    for st, arrays in out[1:]:
+        assert st["n_eval"] == out[0][0]["n_eval"]
+        for f in arrays:
+            np.testing.assert_array_equal(arrays[f], out[0][1][f], err_msg=f)
