@@ -4742,6 +4742,288 @@ enum {
   LP_FAILED = 5        // overflow or failed trace
 };
 
+// Steps 2 to 6 of labelIntersections and createResult for a pair with
+// degenerate labels or one-sided links, by lane 0 over the intersection
+// vertices alone: they are the only ones those steps change or stop at, and a
+// ring of ten thousand vertices has a few hundred of them.  The group lists
+// them (positions ascending on each ring) and, after lane 0 has noted the
+// result as runs of consecutive ring positions, writes the vertices.  The
+// statements are label_and_trace's; what the list of intersection vertices
+// alone does not decide returns false with nothing changed, and
+// label_and_trace then takes the pair: a ring without a crossing or without
+// an ordinary vertex, a chain (step 2) that leaves the intersection vertices,
+// a walk that starts without a status, does not close, or outgrows its room.
+//
+// What bounds it: lane 0's chain of dependent accesses, so the list lies in
+// LDS where it fits.  Measured on one MI355X, a pair of 8001 x 2003 vertices
+// snapped to a grid (about 400 intersection vertices): 10.1 -> 0.53 ms by one
+// block; 4849 x 1833 (160): 5.8 -> 0.51 ms by one wave.
+template <int W>
+__device__ __forceinline__ bool contracted_trace(const Nodes &N, OutBuf &O, double *xy, int *clen, int *rg,
+                                 int nP, int nQ, int Dc, int *omap, const int pinHint[4],
+                                 char *lds, int ldsBytes) {
+  const int lane = grp_rank<W>();
+  const int n = nP + nQ, nE = even_up(n);
+  if (pinHint[0] < 0 || pinHint[2] < 0 || Dc < 8) return false;
+  int *rk = rg, *base = rg + nE;
+  if (20LL * Dc <= ldsBytes) base = (int *)lds;  // (one block's LDS: never for kGrid)
+  int *pos = base, *nxt = base + Dc, *prv = base + 2 * Dc, *nb = base + 3 * Dc;
+  int *st = base + 4 * Dc;  // label, enex and flags
+  enum { LAB = 15, EN = 4, FL = 6 };
+  // the result's runs in the global scratch: [0, 4) what lane 0 found, then
+  // (first output position, first ring position, ring and direction) each
+  int *seg = rg + nE + 5 * Dc;
+  const int maxSeg = (4 * Dc - 4) / 3;
+  int X[2];
+  for (int ring = 0; ring < 2; ring++) {
+    const int r0 = ring ? nP : 0, c0 = ring ? X[0] : 0;
+    X[ring] = grp_scan_range<W, int>(
+        ring ? nQ : nP, [&](int j) { return isint(N, r0 + j) ? 1 : 0; },
+        [&](int j, int pre, int f) {
+          if (f && c0 + pre < Dc) {
+            rk[r0 + j] = c0 + pre;
+            pos[c0 + pre] = r0 + j;
+          }
+        });
+  }
+  const int C = X[0] + X[1];
+  if (X[0] < 1 || X[1] < 1 || C > Dc) return false;
+  grp_sync<W>();
+  for (int c = lane; c < C; c += grp_size<W>()) {
+    const int c0 = c < X[0] ? 0 : X[0], z = c < X[0] ? X[0] : C, u = pos[c], q = N.nb[u];
+    nxt[c] = c + 1 == z ? c0 : c + 1;
+    prv[c] = c == c0 ? z - 1 : c - 1;
+    nb[c] = q >= 0 && isint(N, q) ? rk[q] : -1;
+    st[c] = N.lab[u] | (NEITHER << EN) | (F_INT << FL);
+  }
+  grp_sync<W>();
+  if (lane == 0) {
+    auto lab = [&](int c) { return st[c] & LAB; };
+    auto enex = [&](int c) { return (st[c] >> EN) & 3; };
+    auto set_lab = [&](int c, int l) { st[c] = (st[c] & ~LAB) | l; };
+    auto set_enex = [&](int c, int e) { st[c] = (st[c] & ~(3 << EN)) | (e << EN); };
+    auto has = [&](int c, int f) { return (st[c] & (f << FL)) != 0; };
+    bool ok = true;
+    // step 2: intersection chains
+    for (int it = 0; it < X[0] && ok; it++) {
+      if (lab(it) != L_LEFT_ON && lab(it) != L_RIGHT_ON) continue;
+      int I = it;
+      const int x = lab(I) == L_LEFT_ON ? 0 : 1;
+      do {
+        set_lab(I, L_NONE);
+        if (nb[I] >= 0) set_lab(nb[I], L_NONE);
+        const int J = nxt[I];
+        if (pos[J] != (pos[I] + 1 == nP ? 0 : pos[I] + 1)) ok = false;
+        I = J;
+      } while (ok && lab(I) == L_ON_ON);
+      const int y = lab(I) == L_ON_LEFT ? 0 : 1;
+      const int ct = x != y ? L_DELAYED_CROSSING : L_DELAYED_BOUNCING;
+      set_lab(it, ct);
+      set_lab(I, ct);
+      if (nb[it] >= 0) set_lab(nb[it], ct);
+      if (nb[I] >= 0) set_lab(nb[I], ct);
+    }
+    // step 3.5: both rings have a crossing; step 4 from each ring's first
+    // ordinary vertex on
+    for (int ring = 0; ring < 2 && ok; ring++) {
+      const int c0 = ring ? X[0] : 0, z = ring ? C : X[0];
+      bool any = false;
+      int start = c0;
+      for (int c = c0; c < z; c++) {
+        any |= lab(c) == L_CROSSING || lab(c) == L_DELAYED_CROSSING;
+        if (pos[c] < pinHint[2 * ring]) start = c + 1;
+      }
+      if (!any) ok = false;
+      int status = pinHint[2 * ring + 1] ? EXIT : ENTRY;
+      bool first = true;
+      for (int i = 0; i < z - c0 && ok; i++) {
+        const int I = start + i < z ? start + i : start + i - (z - c0);
+        const int l = lab(I);
+        if (l == L_CROSSING) {
+          set_enex(I, status);
+          toggle(status);
+        }
+        if (l == L_BOUNCING && status == EXIT) st[I] |= F_SPLIT << FL;
+        if (l == L_DELAYED_CROSSING) {
+          set_enex(I, status);
+          if (first) {
+            if (status == EXIT) set_lab(I, L_CROSSING);
+            first = false;
+          } else {
+            if (status == ENTRY) set_lab(I, L_CROSSING);
+            first = true;
+            toggle(status);
+          }
+        }
+        if (l == L_DELAYED_BOUNCING) {
+          set_enex(I, status);
+          if (first) {
+            if (status == EXIT) st[I] |= F_CROSS << FL;
+            first = false;
+          } else {
+            if (status == ENTRY) st[I] |= F_CROSS << FL;
+            first = true;
+          }
+          toggle(status);
+        }
+      }
+    }
+    // step 5: split pairs; a copy has its vertex's position
+    int T = C;
+    auto put_after = [&](int v, int c) {
+      nxt[v] = nxt[c];
+      prv[v] = c;
+      prv[nxt[c]] = v;
+      nxt[c] = v;
+    };
+    auto turn = [&](int u) {
+      const int r0 = u < nP ? 0 : nP, z = u < nP ? nP : n;
+      return triA(P_(N, u == r0 ? z - 1 : u - 1), P_(N, u), P_(N, u + 1 == z ? r0 : u + 1));
+    };
+    for (int I = 0; I < X[0] && ok; I++) {
+      const int IQ = nb[I];
+      if (!has(I, F_SPLIT) || IQ < 0 || !has(IQ, F_SPLIT)) continue;
+      if (T + 2 > Dc) {
+        ok = false;
+        break;
+      }
+      const int VP = T++, VQ = T++;
+      pos[VP] = pos[I];
+      pos[VQ] = pos[IQ];
+      if (turn(pos[I]) * turn(pos[IQ]) > 0) {
+        nb[I] = VQ;
+        nb[VQ] = I;
+        nb[IQ] = VP;
+        nb[VP] = IQ;
+      } else {
+        nb[VP] = VQ;
+        nb[VQ] = VP;
+      }
+      put_after(VP, I);
+      put_after(VQ, IQ);
+      const int keep = (st[IQ] >> FL) & ~F_INT;  // IQ stays flagged, I does not
+      st[I] = L_CROSSING | (EXIT << EN) | ((((st[I] >> FL) & ~F_SPLIT) | F_INT) << FL);
+      st[IQ] = L_CROSSING | (EXIT << EN) | ((keep | F_INT) << FL);
+      st[VP] = st[VQ] = L_CROSSING | (ENTRY << EN) | (F_INT << FL);
+    }
+    // step 6
+    for (int I = 0; I < X[0] && ok; I++)
+      if (has(I, F_CROSS) && nb[I] >= 0 && has(nb[I], F_CROSS)) {
+        set_lab(I, L_CROSSING);
+        set_lab(nb[I], L_CROSSING);
+      }
+    // createResult
+    int ns = 0, nc = 0, tot = 0, lastEnd = -1, lastKey = -1;
+    auto emit = [&](int p, int len, int ringdir) {
+      // len vertices from ring position p on, joined to the run before when
+      // they continue it
+      if (lastKey != ringdir || lastEnd != p) {
+        if (ns >= maxSeg) {
+          ok = false;
+          return;
+        }
+        seg[4 + 3 * ns] = tot;
+        seg[4 + 3 * ns + 1] = p;
+        seg[4 + 3 * ns + 2] = ringdir;
+        ns++;
+      }
+      tot += len;
+      const int r0 = ringdir & 2 ? nP : 0, nR = ringdir & 2 ? nQ : nP;
+      const int o = (ringdir & 1) ? (p - r0 + len) % nR : (p - r0 + nR - len % nR) % nR;
+      lastEnd = r0 + o;
+      lastKey = ringdir;
+    };
+    const long long guard = 4LL * T + 64;
+    int I = 0;
+    do {
+      if (ok && has(I, F_INT) && lab(I) == L_CROSSING) {
+        if (nc >= O.capComp) ok = false;
+        const int start = tot;
+        lastKey = -1;
+        int V = I;
+        long long hops = 0;
+        st[V] &= ~(F_INT << FL);
+        do {
+          int status = enex(V);
+          toggle(status);
+          if (status == NEITHER) ok = false;
+          const bool fwd = status == EXIT;
+          do {
+            const int d = fwd ? nxt[V] : prv[V];
+            const bool onQ = pos[d] >= nP;
+            const int r0 = onQ ? nP : 0, nR = onQ ? nQ : nP;
+            // from V's position (excluded) to d's; a copy follows its vertex
+            // at once (index >= C: a copy)
+            int len = fwd ? pos[d] - pos[V] : pos[V] - pos[d];
+            int p = fwd ? pos[V] + 1 : pos[V] - 1;
+            if (len == 0 && (fwd ? d >= C && V < C : V >= C && d < C)) {
+              len = 1;
+              p = pos[d];
+            } else if (len <= 0) {
+              len += nR;
+            }
+            if (p >= r0 + nR) p -= nR;
+            if (p < r0) p += nR;
+            emit(p, len, (onQ ? 2 : 0) | (fwd ? 1 : 0));
+            V = d;
+            st[V] &= ~(F_INT << FL);
+            if (++hops > guard || tot > n) ok = false;
+          } while (ok && enex(V) != status && V != I);
+          if (ok && V != I) {
+            V = nb[V];
+            if (V < 0) {
+              ok = false;
+            } else {
+              st[V] &= ~(F_INT << FL);
+            }
+          }
+        } while (ok && V != I);
+        if (ok) {
+          O.compRoot[nc] = start;
+          clen[nc] = tot - start;
+          nc++;
+        }
+      }
+      I = nxt[I];
+    } while (ok && I != 0);
+    if (tot > O.cap) ok = false;
+    seg[0] = ok ? 1 : 0;
+    seg[1] = ns;
+    seg[2] = nc;
+    seg[3] = tot;
+  }
+  grp_sync<W>();
+  const bool ok = seg[0] != 0;
+  const int ns = seg[1], nc = seg[2], tot = seg[3];
+  if (!ok) return false;
+  O.n = tot;
+  O.ncomp = nc;
+  int *cw = rk;
+  grp_sync<W>();  // rk is dead
+  for (int w = lane; w < tot; w += grp_size<W>()) {
+    int a = 0, z = ns;  // the run that holds position w
+    while (z - a > 1) {
+      const int m = (a + z) >> 1;
+      if (seg[4 + 3 * m] <= w) a = m;
+      else z = m;
+    }
+    const int rd = seg[4 + 3 * a + 2], r0 = rd & 2 ? nP : 0, nR = rd & 2 ? nQ : nP;
+    const int o = w - seg[4 + 3 * a], p = seg[4 + 3 * a + 1] - r0;
+    const int u = r0 + ((rd & 1) ? (p + o) % nR : (p + nR - o % nR) % nR);
+    omap[w] = u;
+    gcmf::st(xy, w, P_orig(N, u));
+    int c = 0, e = nc;  // its component
+    while (e - c > 1) {
+      const int m = (c + e) >> 1;
+      if (O.compRoot[m] <= w) c = m;
+      else e = m;
+    }
+    cw[w] = c;
+  }
+  grp_sync<W>();
+  return true;
+}
+
 // gives the sequential steps, which insert nodes, the pair's nodes in its
 // global region G: copies the arrays of N that lie in the LDS arena there,
 // writes the ring links and the original coordinates (which the parallel
@@ -4769,9 +5051,11 @@ __device__ void spill_nodes(Nodes &N, const Nodes &G, int nP, int nQ) {
 }
 
 // arena / arenaBytes: the group's LDS for the pair's arrays (null: none)
+// (contracted_trace takes the LDS the arena has left, at least `spare` bytes
+// of it where the later arrays leave room for that)
 template <int W>
-__device__ int label_pair(long k, int *status, const SlotArrays &s, const TraceArgs &a,
-                          int *aux, char *arena, int arenaBytes) {
+__device__ __forceinline__ int label_pair(long k, int *status, const SlotArrays &s, const TraceArgs &a,
+                          int *aux, char *arena, int arenaBytes, int spare = 0) {
   const int lane = grp_rank<W>();
   if (status[k] != GH_OK) {
     if (lane == 0) {
@@ -4806,11 +5090,11 @@ __device__ int label_pair(long k, int *status, const SlotArrays &s, const TraceA
   // ring) and the original coordinates stay in the slots, so neither is
   // materialised here.
   Nodes N = G;
-  N.pn = ar.take<double>(2 * n, G.pn);
-  N.nb = ar.take<int>(n, G.nb);
-  N.fl = ar.take<unsigned char>(n, G.fl);
-  N.lab = ar.take<signed char>(n, G.lab);
-  N.enex = ar.take<signed char>(n, G.enex);
+  N.pn = ar.take<double>(2 * n, G.pn, spare);
+  N.nb = ar.take<int>(n, G.nb, spare);
+  N.fl = ar.take<unsigned char>(n, G.fl, spare);
+  N.lab = ar.take<signed char>(n, G.lab, spare);
+  N.enex = ar.take<signed char>(n, G.enex, spare);
   N.next = N.prev = nullptr;
   N.po = nullptr;
   N.oP = s.oP + 2 * sbP;
@@ -4997,9 +5281,9 @@ __device__ int label_pair(long k, int *status, const SlotArrays &s, const TraceA
   nCrossP = grp_sum<W>(nCrossP);
   nInt = grp_sum<W>(nInt);
   const int Dc = even_up(min(2 * nInt, n));
-  rg = ar.take<int>(seg_scratch_ints(n, Dc), rg);
+  rg = ar.take<int>(seg_scratch_ints(n, Dc), rg, spare);
   // output position -> node (the clean-up reads the node's normalised point)
-  int *omap = ar.take<int>(n, (int *)O.pn);
+  int *omap = ar.take<int>(n, (int *)O.pn, spare);
   int VP = -1, VQ = -1;
   if (!slow) {
     VP = grp_first_nonint<W>(N, 0, nP);
@@ -5056,6 +5340,7 @@ __device__ int label_pair(long k, int *status, const SlotArrays &s, const TraceA
       if (rc == SEG_SLOW) slow = true;
     }
   }
+  int pinHint[4] = {-1, 0, -1, 0};
   if (slow) {
     // sequential path for degenerate pairs, from step 2 on.  Step 1's P
     // labels above are the sequential step 1's (the same function of the
@@ -5063,8 +5348,6 @@ __device__ int label_pair(long k, int *status, const SlotArrays &s, const TraceA
     // P intersection vertex's label to its neighbour in ring order, so a Q
     // vertex linked from several P vertices ends with the last one's label:
     // the largest such P index, found by an atomic maximum.
-    spill_nodes<W>(N, G, nP, nQ);
-    O.pn = a.opn + 2 * nb0;
     int *owner = rg;  // nQ entries of the segment scratch
     for (int j = lane; j < nQ; j += grp_size<W>()) owner[j] = -1;
     grp_sync<W>();
@@ -5079,7 +5362,6 @@ __device__ int label_pair(long k, int *status, const SlotArrays &s, const TraceA
     // step 4's point-in-polygon tests of each ring's first non-intersection
     // vertex (the rings are still in index order; the flags do not change
     // before step 4), in parallel
-    int pinHint[4] = {-1, 0, -1, 0};
     {
       const int vp = grp_first_nonint<W>(N, 0, nP), vq = grp_first_nonint<W>(N, nP, nQ);
       if (vp >= 0 && vq >= 0) {
@@ -5089,6 +5371,15 @@ __device__ int label_pair(long k, int *status, const SlotArrays &s, const TraceA
         pinHint[3] = grp_pip<W>(N, 0, nP, P_(N, vq)) ? 1 : 0;
       }
     }
+    grp_sync<W>();
+    // (the clean-up below takes its result too)
+    slow = !contracted_trace<W>(N, O, xy, clen, rg, nP, nQ, Dc, omap, pinHint, ar.p,
+                                ar.p ? ar.left : 0);
+    path = LP_SEQUENTIAL;
+  }
+  if (slow) {
+    spill_nodes<W>(N, G, nP, nQ);
+    O.pn = a.opn + 2 * nb0;
     if (lane != 0) return LP_SEQUENTIAL;
     O.n = 0;
     O.ncomp = 0;
@@ -5256,13 +5547,16 @@ __global__ void __launch_bounds__(kGridBlock)
 }
 
 // One block of kBigGroup threads per listed pair, the blocks taking the list
-// in turn
+// in turn; the block's LDS is kept for contracted_trace (up to 1600
+// intersection vertices)
+constexpr int kBlockLds = 32768;
 __global__ void __launch_bounds__(kBigGroup)
     k_label_block(const int *list, const unsigned long long *cnt, unsigned long long *next,
                   int *status, SlotArrays s, TraceArgs a, int *aux, int *lpath,
                   long long *lticks) {
   const long n = (long)*cnt;
   __shared__ long s_i;
+  __shared__ __align__(16) char block_lds[kBlockLds];
   for (;;) {
     // the next listed pair from a device counter: a block held up by a slow
     // pair (a sequential fallback) takes no further pairs meanwhile
@@ -5272,12 +5566,42 @@ __global__ void __launch_bounds__(kBigGroup)
     if (i >= n) return;
     const long k = list[i];
     const long long t0 = wall_clock64();
-    const int path = label_pair<kBigGroup>(k, status, s, a, aux, nullptr, 0);
+    const int path = label_pair<kBigGroup>(k, status, s, a, aux, block_lds, kBlockLds, kBlockLds);
     if (threadIdx.x == 0 && lpath) {
       lpath[k] = path;
       lticks[k] = wall_clock64() - t0;
     }
     __syncthreads();
+  }
+}
+
+// The pairs of a call with at most one per CU, one kBigGroup-thread block
+// each: a pair of kFewNodes nodes or more is labelled by the block, a smaller
+// one by its first wave.  Such a call waits for its slowest pair, so a wave
+// gets only what it finishes sooner: on one MI355X a wave takes 23, 28, 58,
+// 158 and 404 us for pairs of 144, 240, 514, 1300 and 3200 nodes, a block 40,
+// 42, 51, 80 and 123 us; and one launch serves both, where the blocks of
+// larger calls run beside the waves on a second stream, which costs 33 us of
+// events.  Each block has a CU's LDS to itself.
+constexpr int kFewNodes = 512;
+constexpr int kFewLds = 131072;
+
+__global__ void __launch_bounds__(kBigGroup)
+    k_label_few(int *status, SlotArrays s, TraceArgs a, int *aux, int *lpath, long long *lticks,
+                long long bigNodes, long long gridNodes, int waveBytes) {
+  const long k = blockIdx.x;
+  const long long n = pair_nodes(a, k);
+  if (n >= gridNodes) return;  // k_label_grid's
+  const bool wave = n < min(bigNodes, (long long)kFewNodes);
+  if (wave && threadIdx.x >= 64) return;
+  const long long t0 = wall_clock64();
+  extern __shared__ __align__(16) char label_lds[];
+  const int path =
+      wave ? label_pair<64>(k, status, s, a, aux, waveBytes > 0 ? label_lds : nullptr, waveBytes)
+           : label_pair<kBigGroup>(k, status, s, a, aux, label_lds, kFewLds, kBlockLds);
+  if (threadIdx.x == 0 && lpath) {
+    lpath[k] = path;
+    lticks[k] = wall_clock64() - t0;
   }
 }
 
@@ -6127,7 +6451,8 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
     int *aux = wsT<int>(c, "gh_aux", 5 * nodes);
     res.labelPath = wsT<int>(c, "gh_lpath", M);
     res.labelTicks = wsT<long long>(c, "gh_lticks", M);
-    if (nBig > 0 && !c.side) {
+    const bool few = M <= c.cu_count && !c.tune.labelSteal;
+    if (nBig > 0 && !few && !c.side) {
       HIP_CHECK(hipStreamCreate(&c.side));
       HIP_CHECK(hipEventCreateWithFlags(&c.ev_fork, hipEventDisableTiming));
       HIP_CHECK(hipEventCreateWithFlags(&c.ev_join, hipEventDisableTiming));
@@ -6135,7 +6460,7 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
     // batches of many pairs are labelled largest first; the sorted order's
     // first nBig entries are then the block path's pairs, largest first
     int *order = nullptr;
-    if (M >= kLptMinPairs) {
+    if (M >= kLptMinPairs && !few) {
       LaunchTimer t(c, "gh_label_order");
       uint64_t *ok = wsT<uint64_t>(c, "gh_lpt_keys", M), *ok2 = wsT<uint64_t>(c, "gh_lpt_keys2", M);
       int *ov = wsT<int>(c, "gh_lpt_vals", M);
@@ -6150,7 +6475,7 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
     LaunchTimer t(c, "gh_label_trace");
     // the large pairs on the side stream, concurrently with one wave per
     // remaining pair on the main one (disjoint pairs, disjoint regions)
-    if (nBig > 0) {
+    if (nBig > 0 && !few) {
       unsigned long long *bigNext = ctr + 26;
       HIP_CHECK(hipEventRecord(c.ev_fork, c.stream));
       HIP_CHECK(hipStreamWaitEvent(c.side, c.ev_fork, 0));
@@ -6162,7 +6487,12 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
       HIP_CHECK(hipGetLastError());
       HIP_CHECK(hipEventRecord(c.ev_join, c.side));
     }
-    if (c.tune.labelSteal) {
+    if (few) {
+      hipLaunchKernelGGL(k_label_few, dim3((unsigned)M), dim3(kBigGroup), (size_t)kFewLds,
+                         c.stream, pm.status, s, ta, aux, res.labelPath, res.labelTicks,
+                         (long long)c.tune.bigNodes, (long long)c.tune.gridNodes,
+                         c.tune.labelLds);
+    } else if (c.tune.labelSteal) {
       // persistent waves taking the pairs in turn
       if (c.label_steal_blocks <= 0) {
         int perCu = 0;
@@ -6189,7 +6519,7 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
                          res.labelTicks, c.tune.labelLds);
     }
     HIP_CHECK(hipGetLastError());
-    if (nBig > 0) HIP_CHECK(hipStreamWaitEvent(c.stream, c.ev_join, 0));
+    if (nBig > 0 && !few) HIP_CHECK(hipStreamWaitEvent(c.stream, c.ev_join, 0));
     if (nGrid > 0) {
       // the pairs of gridNodes nodes or more, one cooperative launch each over
       // as many blocks as the GPU holds at once, after the other labelling

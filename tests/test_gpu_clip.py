@@ -757,3 +757,52 @@ def test_count_one_wave_per_edge(gctx, n_p, n_q, kind, snap):
         assert st["n_eval"] == out[0][0]["n_eval"]
         for f in arrays:
             np.testing.assert_array_equal(arrays[f], out[0][1][f], err_msg=f)
+
+
+@pytest.mark.parametrize("n_p, n_q, snap", [
+    (120, 60, 5e-2), (260, 250, 2e-2), (900, 400, 1e-2), (4000, 900, 1e-3), (2600, 2600, 5e-3)])
+@pytest.mark.parametrize("cleanup", [True, False])
+def test_clip_degenerate_over_intersections(gctx, n_p, n_q, snap, cleanup):
+    """Grid-snapped pairs (chains, bouncing and shared vertices, one-sided
+    links), whose sequential steps run over the intersection vertices alone:
+    the oracle's results bit for bit, by a block and (big_nodes above every
+    pair, and more pairs than CUs) by one wave each."""
+    cases = [("g%d" % s,) + tuple(G.gen_single_pair(1, 300 + s, n_p, n_q, snap=snap))
+             for s in range(8)]
+    flags = G.CLIP_NORMALIZE | (0 if cleanup else G.CLIP_NO_CLEANUP)
+    mode = 5 | (0 if cleanup else 2)
+    st = run_batch(gctx, cases, flags)
+    check_results(gctx, st, cases, mode)
+    few = gctx.clip_get("xy", 2 * st["total_verts"])
+    many = cases * 40  # 320 pairs: one wave each
+    default = gctx.tuning()
+    try:
+        gctx.set_tuning(default["cull_min"], 1 << 30, default["count_block"])
+        st = run_batch(gctx, many, flags)
+        np.testing.assert_array_equal(gctx.clip_get("xy", 2 * st["total_verts"]),
+                                      np.tile(few, 40))
+    finally:
+        gctx.set_tuning(**default)
+
+
+@pytest.mark.parametrize("pairs", [1, 255, 256, 257])
+def test_clip_few_pairs_label_alike(gctx, pairs):
+    """Calls of at most one pair per CU are labelled by blocks and their first
+    waves in one launch: the results of the first pairs do not depend on how
+    many others the call has, with pairs around the 512 nodes between."""
+    P, Q = G.gen_pair_layers(300, seed=21, median=150.0, sigma=1.0, nmax=3000)
+    db, do = G.DeviceLayer(gctx, P), G.DeviceLayer(gctx, Q)
+    try:
+        idx = np.repeat(np.arange(300, dtype=np.int32), 2).reshape(-1, 2)
+        st = gctx.clip(db, do, idx)
+        s0, r0 = gctx.clip_results(st)
+        st = gctx.clip(db, do, idx[:pairs])
+        s1, r1 = gctx.clip_results(st)
+    finally:
+        db.free()
+        do.free()
+    np.testing.assert_array_equal(s1, s0[:pairs])
+    for a, b in zip(r1, r0):
+        assert len(a) == len(b)
+        for x, y in zip(a, b):
+            np.testing.assert_array_equal(x, y)
