@@ -167,6 +167,13 @@ __device__ __forceinline__ int pgrp_split_part(int split) {
   return W == 64 ? 0 : (int)(blockIdx.x % (unsigned)split);
 }
 
+// Loads a lane of the per-pair kernels issues before it uses the first: the
+// longest ring of a batch, tens of thousands of vertices on one wave, sets
+// their time, one round trip to memory per step (20 000 pairs of log-normal
+// sizes, the largest ring 50 000: set-up 343 -> @SU@ us, fill and filter
+// constants 283 + 356 in two launches -> @FI@, gather 224 -> @GA@).
+constexpr int kSetStage = 8;
+
 // one group per pair: sizes, swap (|P| >= |Q|, ghcuda.cpp:64-91), ring MBRs
 // (readShapefile.h:304-334), CMBR and disjointness (ghcuda.cpp:94-125)
 // out[0] = max of bm[2b], out[1] = max of bm[2b + 1] over b < n (out zeroed
@@ -306,12 +313,17 @@ __global__ void __launch_bounds__(W == 64 ? 256 : W)
         mxy = fmax(mxy, d[3]);
       }
     } else {
-      for (int i = lane; i < n; i += W) {
-        double x = c[2 * i], y = c[2 * i + 1];
-        mnx = fmin(mnx, x);
-        mny = fmin(mny, y);
-        mxx = fmax(mxx, x);
-        mxy = fmax(mxy, y);
+      for (int i = lane; i < n; i += kSetStage * W) {
+        pt v[kSetStage];  // (past the end: the last vertex again)
+#pragma unroll
+        for (int u = 0; u < kSetStage; u++) v[u] = ld(c, min(i + u * W, n - 1));
+#pragma unroll
+        for (int u = 0; u < kSetStage; u++) {
+          mnx = fmin(mnx, v[u].x);
+          mny = fmin(mny, v[u].y);
+          mxx = fmax(mxx, v[u].x);
+          mxy = fmax(mxy, v[u].y);
+        }
       }
     }
     pgrp_minmax<W>(mnx, mxx);
@@ -362,35 +374,6 @@ __global__ void __launch_bounds__(W == 64 ? 256 : W)
   pm.cmbrN[4 * k + 3] = (cm[3] - cy) * s;
   eP[k] = status == GH_OK ? nP : 0;
   eQ[k] = status == GH_OK ? nQ : 0;
-}
-
-// one group per pair (split over several blocks at width 1024): edge ->
-// pair maps and normalised rings
-template <int W>
-__global__ void __launch_bounds__(W == 64 ? 256 : W)
-    k_pair_fill(long M, int split, const int *pairs, const double *bCoords,
-                const double *oCoords, PairMeta pm, const long long *offP, const long long *offQ,
-                int *mapP, int *mapQ, double *nP_, double *nQ_) {
-  const long k = pgrp_split_pair<W>(split);
-  if (k >= M) return;
-  const int lane = pgrp_lane<W>() + W * pgrp_split_part<W>(split);
-  const long long stride = (long long)W * split;
-  const int sw = pm.swapped[k];
-  const double cx = pm.norm[3 * k], cy = pm.norm[3 * k + 1], s = pm.norm[3 * k + 2];
-  for (int side = 0; side < 2; side++) {
-    const long long base = side == 0 ? offP[k] : offQ[k];
-    const long long n = (side == 0 ? offP[k + 1] : offQ[k + 1]) - base;
-    const double *c = (side == 0) == (sw == 0) ? bCoords : oCoords;
-    const long start = side == 0 ? pm.startP[k] : pm.startQ[k];
-    int *map = side == 0 ? mapP : mapQ;
-    double *dst = side == 0 ? nP_ : nQ_;
-    for (long long i = lane; i < n; i += stride) {
-      double x = c[2 * (start + i)], y = c[2 * (start + i) + 1];
-      dst[2 * (base + i)] = (x - cx) * s;
-      dst[2 * (base + i) + 1] = (y - cy) * s;
-      map[base + i] = (int)k;
-    }
-  }
 }
 
 // ------------------------------------------------- edge-pair prefilter ----
@@ -445,48 +428,6 @@ struct RunBoxes {
   const double *l1, *l2, *l3;  // [runs] shortest edge of the run
   long cullMin;                // rings longer than this are walked through the runs
 };
-
-// one thread per edge; the kRun1 = 16 lanes of a run combine their boxes
-__global__ void __launch_bounds__(256)
-    k_run_boxes(long edges, const int *map, const long long *off, const double *ring,
-                double *box1, double *len1) {
-  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  double x0 = INFINITY, y0 = INFINITY, x1 = -INFINITY, y1 = -INFINITY, lmin = INFINITY;
-  bool nan = false;
-  if (e < edges) {
-    const int k = map[e];
-    const long long b = off[k], n = off[k + 1] - b;
-    const pt p = ld(ring, e), q = ld(ring, e - b == n - 1 ? b : e + 1);
-    nan = (p.x != p.x) | (p.y != p.y) | (q.x != q.x) | (q.y != q.y);
-    x0 = fmin(p.x, q.x);
-    y0 = fmin(p.y, q.y);
-    x1 = fmax(p.x, q.x);
-    y1 = fmax(p.y, q.y);
-    const double dx = q.x - p.x, dy = q.y - p.y;
-    lmin = sqrt(dx * dx + dy * dy);
-  }
-  for (int off2 = 1; off2 < kRun1; off2 <<= 1) {
-    x0 = fmin(x0, __shfl_xor(x0, off2, 64));
-    y0 = fmin(y0, __shfl_xor(y0, off2, 64));
-    x1 = fmax(x1, __shfl_xor(x1, off2, 64));
-    y1 = fmax(y1, __shfl_xor(y1, off2, 64));
-    lmin = fmin(lmin, __shfl_xor(lmin, off2, 64));
-    nan |= __shfl_xor((int)nan, off2, 64) != 0;
-  }
-  const long G = e / kRun1;
-  if ((e & (kRun1 - 1)) != 0 || e >= edges) return;
-  if (nan) {
-    // a run with a NaN coordinate is never left out
-    x0 = y0 = -INFINITY;
-    x1 = y1 = INFINITY;
-    lmin = 0.0;
-  }
-  box1[4 * G] = x0;
-  box1[4 * G + 1] = y0;
-  box1[4 * G + 2] = x1;
-  box1[4 * G + 3] = y1;
-  len1[G] = lmin;
-}
 
 // boxes of the next level: 16 boxes merged
 __global__ void k_run_boxes_merge(long runsIn, const double *in, const double *lenIn,
@@ -1498,46 +1439,84 @@ __device__ __forceinline__ void write_cf(double *c, const double bx[2][4], const
   c[CF_C0] = K.c0;
 }
 
-// one group per pair: ring boxes, then the shortest edge and the largest
-// margin of each ring (the edges' own lengths and margins are recomputed
-// where they are needed)
+// One group per pair (split over several blocks at width 1024): edge -> pair
+// maps and normalised rings; with cf (split 1), the pair's filter constants
+// too: the ring boxes, then the shortest edge and the largest margin of each
+// ring (the edges' own lengths and margins are recomputed where they are
+// needed), the vertices normalised again from the layer with the same
+// operations.
 template <int W>
 __global__ void __launch_bounds__(W == 64 ? 256 : W)
-    k_cpu_filter_setup(long M, const int *status, const long long *offP, const long long *offQ,
-                       const double *ringP, const double *ringQ, double *cf) {
-  const long k = pgrp_pair<W>();
-  if (k >= M || status[k] != GH_OK) return;
-  const int lane = pgrp_lane<W>();
+    k_pair_fill(long M, int split, const int *pairs, const double *bCoords,
+                const double *oCoords, PairMeta pm, const long long *offP, const long long *offQ,
+                int *mapP, int *mapQ, double *nP_, double *nQ_, double *cf) {
+  const long k = pgrp_split_pair<W>(split);
+  if (k >= M) return;
+  const int lane = pgrp_lane<W>() + W * pgrp_split_part<W>(split);
+  const long long stride = (long long)W * split;
+  const int sw = pm.swapped[k];
+  const double cx = pm.norm[3 * k], cy = pm.norm[3 * k + 1], s = pm.norm[3 * k + 2];
+  auto norm = [&](pt v) { return pt{(v.x - cx) * s, (v.y - cy) * s}; };
   double bx[2][4];
   for (int side = 0; side < 2; side++) {
-    const long long b = side ? offQ[k] : offP[k], n = (side ? offQ[k + 1] : offP[k + 1]) - b;
-    const double *V = side ? ringQ : ringP;
+    const long long base = side == 0 ? offP[k] : offQ[k];
+    const long long n = (side == 0 ? offP[k + 1] : offQ[k + 1]) - base;
+    const double *c = ((side == 0) == (sw == 0) ? bCoords : oCoords) +
+                      2 * (side == 0 ? pm.startP[k] : pm.startQ[k]);
+    int *map = side == 0 ? mapP : mapQ;
+    double *dst = side == 0 ? nP_ : nQ_;
     double x0 = INFINITY, y0 = INFINITY, x1 = -INFINITY, y1 = -INFINITY;
-    for (long long i = lane; i < n; i += W) {
-      const pt p = ld(V, b + i);
-      x0 = fmin(x0, p.x);
-      y0 = fmin(y0, p.y);
-      x1 = fmax(x1, p.x);
-      y1 = fmax(y1, p.y);
+    for (long long i = lane; i < n; i += kSetStage * stride) {
+      pt v[kSetStage];
+#pragma unroll
+      for (int u = 0; u < kSetStage; u++)
+        v[u] = norm(ld(c, min(i + u * stride, n - 1)));
+#pragma unroll
+      for (int u = 0; u < kSetStage; u++) {
+        const long long j = i + u * stride;
+        if (j < n) {
+          st(dst, base + j, v[u]);
+          map[base + j] = (int)k;
+        }
+        x0 = fmin(x0, v[u].x);
+        y0 = fmin(y0, v[u].y);
+        x1 = fmax(x1, v[u].x);
+        y1 = fmax(y1, v[u].y);
+      }
     }
-    pgrp_minmax<W>(x0, x1);
-    pgrp_minmax<W>(y0, y1);
+    if (cf) {
+      pgrp_minmax<W>(x0, x1);
+      pgrp_minmax<W>(y0, y1);
+    }
     bx[side][0] = x0;
     bx[side][1] = y0;
     bx[side][2] = x1;
     bx[side][3] = y1;
   }
+  if (!cf || pm.status[k] != GH_OK) return;  // the same in every thread of the group
   const FilterK K = filter_consts(bx);
   double minL[2], maxM[2];
+  constexpr int kS = kSetStage / 2;
   for (int side = 0; side < 2; side++) {
-    const long long b = side ? offQ[k] : offP[k], n = (side ? offQ[k + 1] : offP[k + 1]) - b;
-    const double *V = side ? ringQ : ringP;
+    const long long n = side == 0 ? offP[k + 1] - offP[k] : offQ[k + 1] - offQ[k];
+    const double *c = ((side == 0) == (sw == 0) ? bCoords : oCoords) +
+                      2 * (side == 0 ? pm.startP[k] : pm.startQ[k]);
     double mn = INFINITY, mx = 0.0;
-    for (long long i = lane; i < n; i += W) {
-      double L, m;
-      edge_margin(K, ld(V, b + i), ld(V, b + (i + 1 == n ? 0 : i + 1)), side != 0, L, m);
-      mn = fmin(mn, L);
-      mx = fmax(mx, m);
+    for (long long i = lane; i < n; i += kS * W) {
+      pt p[kS], q[kS];
+#pragma unroll
+      for (int u = 0; u < kS; u++) {
+        const long long j = min(i + u * W, n - 1);
+        p[u] = ld(c, j);
+        q[u] = ld(c, j + 1 == n ? 0 : j + 1);
+      }
+#pragma unroll
+      for (int u = 0; u < kS; u++) {
+        double L, m;
+        edge_margin(K, norm(p[u]), norm(q[u]), side != 0, L, m);
+        mn = fmin(mn, L);
+        mx = fmax(mx, m);
+      }
     }
     pgrp_minmax<W>(mn, mx);
     minL[side] = mn;
@@ -1546,13 +1525,16 @@ __global__ void __launch_bounds__(W == 64 ? 256 : W)
   if (lane == 0) write_cf(cf + (long long)CF_N * k, bx, minL, maxM, K);
 }
 
-// The same over `split` 1024-thread blocks per pair, for a few large pairs:
+// The filter constants over `split` 1024-thread blocks per pair, for a few
+// large pairs (rings above kFillRing vertices):
 // the ring boxes' parts (k_filter_box_parts), combined into the constants'
 // box fields (k_filter_box_combine); then each block takes its share of
 // the edges' lengths and margins to parts of their minimum and maximum
 // (k_filter_edge_parts), which k_filter_finish combines into the remaining
 // constants.  Minima and maxima are exact in any order, so the constants
-// are those of k_cpu_filter_setup.
+// are those of k_pair_fill, whose one block per pair takes one launch for
+// five (64 x 48 vertices: 34 us of these four and the fill -> @FF@).
+constexpr long kFillRing = 131072;
 __global__ void __launch_bounds__(1024)
     k_filter_box_parts(long M, int split, const int *status, const long long *offP,
                        const long long *offQ, const double *ringP, const double *ringQ,
@@ -1721,6 +1703,90 @@ __device__ __forceinline__ CpuFilter cpu_filter(const double *cf, int k, bool si
   f.wide = EdgeBox{0.0, 0.0, 0.0, 0.0};
   f.c = c;
   return f;
+}
+
+// One thread per edge; the kRun1 = 16 lanes of a run combine their boxes, and
+// the block's 16 runs are one run of kRun2.  With flag (the Q edges of the
+// CPU route; off2 are then P's offsets): the edges' prefilter flags too (the
+// flag the count kernel records for a P edge: a possible tiny pair, or the
+// edge's box within G of the other ring's box), and the transposition's
+// counters start here, count1 at 0 and count2 at 1 (the parent).
+static_assert(kRun2 == 256, "a block's edges are one run of kRun2");
+__global__ void __launch_bounds__(256)
+    k_run_boxes(long edges, const int *map, const long long *off, const double *ring,
+                double *box1, double *len1, double *box2, double *len2, const double *cf,
+                int *flag, int *cnt1, int *cnt2) {
+  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  double x0 = INFINITY, y0 = INFINITY, x1 = -INFINITY, y1 = -INFINITY, lmin = INFINITY;
+  bool nan = false;
+  if (e < edges) {
+    const int k = map[e];
+    const long long b = off[k], n = off[k + 1] - b;
+    const pt p = ld(ring, e), q = ld(ring, e - b == n - 1 ? b : e + 1);
+    nan = (p.x != p.x) | (p.y != p.y) | (q.x != q.x) | (q.y != q.y);
+    x0 = fmin(p.x, q.x);
+    y0 = fmin(p.y, q.y);
+    x1 = fmax(p.x, q.x);
+    y1 = fmax(p.y, q.y);
+    const double dx = q.x - p.x, dy = q.y - p.y;
+    lmin = sqrt(dx * dx + dy * dy);
+    if (flag) {
+      const CpuFilter f = cpu_filter(cf, k, false, p, q);
+      const double *ob = cf + (long long)CF_N * k + CF_BOXP;
+      const EdgeBox ab = edge_box(p, q);
+      const double ogap =
+          fmax(fmax(ob[0] - ab.x1, ab.x0 - ob[2]), fmax(ob[1] - ab.y1, ab.y0 - ob[3]));
+      flag[e] = (f.tiny || !(ogap > f.G)) ? 1 : 0;
+      cnt1[e] = 0;
+      cnt2[e] = 1;
+    }
+  }
+  auto combine = [&](int o) {
+    x0 = fmin(x0, __shfl_xor(x0, o, 64));
+    y0 = fmin(y0, __shfl_xor(y0, o, 64));
+    x1 = fmax(x1, __shfl_xor(x1, o, 64));
+    y1 = fmax(y1, __shfl_xor(y1, o, 64));
+    lmin = fmin(lmin, __shfl_xor(lmin, o, 64));
+  };
+  for (int o = 1; o < kRun1; o <<= 1) {
+    combine(o);
+    nan |= __shfl_xor((int)nan, o, 64) != 0;
+  }
+  if (nan) {
+    // a run with a NaN coordinate is never left out
+    x0 = y0 = -INFINITY;
+    x1 = y1 = INFINITY;
+    lmin = 0.0;
+  }
+  auto put = [&](double *box, double *len, long r) {
+    box[4 * r] = x0;
+    box[4 * r + 1] = y0;
+    box[4 * r + 2] = x1;
+    box[4 * r + 3] = y1;
+    len[r] = lmin;
+  };
+  if ((e & (kRun1 - 1)) == 0 && e < edges) put(box1, len1, e / kRun1);
+  if (!box2) return;  // the same in every thread
+  for (int o = kRun1; o < 64; o <<= 1) combine(o);
+  __shared__ double part[4][5];
+  const int w = threadIdx.x >> 6;
+  if (__lane_id() == 0) {
+    part[w][0] = x0;
+    part[w][1] = y0;
+    part[w][2] = x1;
+    part[w][3] = y1;
+    part[w][4] = lmin;
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  for (int i = 1; i < 4; i++) {
+    x0 = fmin(x0, part[i][0]);
+    y0 = fmin(y0, part[i][1]);
+    x1 = fmax(x1, part[i][2]);
+    y1 = fmax(y1, part[i][3]);
+    lmin = fmin(lmin, part[i][4]);
+  }
+  put(box2, len2, blockIdx.x);
 }
 
 __device__ __forceinline__ bool ins_on_p(int t) { return t == 1 || t == 3 || t == 5 || t == 7; }
@@ -2453,20 +2519,23 @@ __global__ void __launch_bounds__(64)
         n += __popcll(m);
       }
     };
-    if (rb.b1 == nullptr || bN <= rb.cullMin) {
+    if (rb.b2 == nullptr || bN <= rb.cullMin) {
       scan(0, bN);
     } else {
       const double G = f.G * (1.0 + 1e-12) + 1e-300;
       const EdgeBox ab0 = edge_box(A1, A2);
       const EdgeBox ab{ab0.x0 - G, ab0.y0 - G, ab0.x1 + G, ab0.y1 + G};
-      const long long e0 = bBase, e1 = bBase + bN;
-      for (long long S3 = e0 / kRun3; S3 * kRun3 < e1; S3++) {
-        if (!run_hit(rb.b3 + 4 * S3, rb.l3 + S3, ab, f.la, f.T)) continue;
-        const long long a2 = max(S3 * 16, e0 / kRun2),
-                        z2 = min(S3 * 16 + 16, (e1 - 1) / kRun2 + 1);
-        for (long long S2 = a2; S2 < z2; S2++)
-          if (run_hit(rb.b2 + 4 * S2, rb.l2 + S2, ab, f.la, f.T))
-            scan(max(S2 * kRun2, e0) - e0, min(S2 * kRun2 + kRun2, e1) - e0);
+      // 64 runs of kRun2 edges at a time, one per lane
+      const long long e0 = bBase, e1 = bBase + bN, z2 = (e1 - 1) / kRun2 + 1;
+      for (long long S = e0 / kRun2; S < z2; S += 64) {
+        const long long r = S + __lane_id();
+        unsigned long long m =
+            __ballot(r < z2 && run_hit(rb.b2 + 4 * r, rb.l2 + r, ab, f.la, f.T));
+        while (m) {
+          const long long S2 = S + __ffsll((long long)m) - 1;
+          m &= m - 1;
+          scan(max(S2 * kRun2, e0) - e0, min(S2 * kRun2 + kRun2, e1) - e0);
+        }
       }
     }
     for (long long r = n + __lane_id(); r < c1; r += 64) dst[r] = 0;
@@ -2506,27 +2575,6 @@ __global__ void __launch_bounds__(256)
     j++;
   };
   listed_edges(ringQ + 2 * qBase, (int)qN, lstAllP + j0, (int)(psP1[g + 1] - j0), visit);
-}
-
-// The Q edges' prefilter flags of the CPU route (the flag the count kernel
-// records for a P edge: a possible tiny pair, or the edge's box within G of
-// the P ring's box), for a batch whose Q side is built by transposition.
-__global__ void __launch_bounds__(256)
-    k_cpu_flags_q(long edgesQ, const int *mapQ, const long long *offP, const long long *offQ,
-                  const double *ringQ, const double *cf, int *boolQ, int *cnt1Q, int *cnt2Q) {
-  const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= edgesQ) return;
-  // the transposition's counters start here: count1 0, count2 1 (the parent)
-  cnt1Q[g] = 0;
-  cnt2Q[g] = 1;
-  const int k = mapQ[g];
-  const long long aBase = offQ[k], aN = offQ[k + 1] - aBase;
-  const pt A1 = ld(ringQ, g), A2 = ld(ringQ, g - aBase == aN - 1 ? aBase : g + 1);
-  const CpuFilter f = cpu_filter(cf, k, false, A1, A2);
-  const double *ob = cf + (long long)CF_N * k + CF_BOXP;
-  const EdgeBox ab = edge_box(A1, A2);
-  const double ogap = fmax(fmax(ob[0] - ab.x1, ab.x0 - ob[2]), fmax(ob[1] - ab.y1, ab.y0 - ob[3]));
-  boolQ[g] = (f.tiny || !(ogap > f.G)) ? 1 : 0;
 }
 
 // CPU-route slot records
@@ -5661,12 +5709,24 @@ __global__ void __launch_bounds__(W == 64 ? 256 : W)
   const int lane = pgrp_lane<W>() + W * pgrp_split_part<W>(split);
   const long long stride = (long long)W * split;
   const long long nv = vOff[k + 1] - vOff[k], nc = cOff[k + 1] - cOff[k];
-  for (long long i = lane; i < nv; i += stride) {
-    xy[2 * (vOff[k] + i)] = xyTmp[2 * (nodeOff[k] + i)];
-    xy[2 * (vOff[k] + i) + 1] = xyTmp[2 * (nodeOff[k] + i) + 1];
+  const double *src = xyTmp + 2 * nodeOff[k];
+  for (long long i = lane; i < nv; i += kSetStage * stride) {
+    pt v[kSetStage];
+#pragma unroll
+    for (int u = 0; u < kSetStage; u++) v[u] = ld(src, min(i + u * stride, nv - 1));
+#pragma unroll
+    for (int u = 0; u < kSetStage; u++)
+      if (i + u * stride < nv) st(xy, vOff[k] + i + u * stride, v[u]);
   }
-  for (long long i = lane; i < nc; i += stride)
-    compSizes[cOff[k] + i] = compLen[compCapOff[k] + i];
+  const int *len = compLen + compCapOff[k];
+  for (long long i = lane; i < nc; i += kSetStage * stride) {
+    int v[kSetStage];
+#pragma unroll
+    for (int u = 0; u < kSetStage; u++) v[u] = len[min(i + u * stride, nc - 1)];
+#pragma unroll
+    for (int u = 0; u < kSetStage; u++)
+      if (i + u * stride < nc) compSizes[cOff[k] + i + u * stride] = v[u];
+  }
 }
 
 template <typename T>
@@ -5771,26 +5831,30 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
   int *mapP = wsT<int>(c, "gh_mapP", edgesP), *mapQ = wsT<int>(c, "gh_mapQ", edgesQ);
   double *ringP = wsT<double>(c, "gh_ringP", 2 * edgesP);
   double *ringQ = wsT<double>(c, "gh_ringQ", 2 * edgesQ);
-  {
-    LaunchTimer t(c, "gh_pair_fill");
-    const int split = pgrp_split(M, pw);
-    hipLaunchKernelGGL(pw == 64 ? k_pair_fill<64> : k_pair_fill<1024>,
-                       dim3(pgrp_grid(M, pw) * (unsigned)split), dim3(pgrp_block(pw)), 0,
-                       c.stream, M, split, pairs,
-                       in.bCoords, in.oCoords, pm, (const long long *)offP,
-                       (const long long *)offQ, mapP, mapQ, ringP, ringQ);
-    HIP_CHECK(hipGetLastError());
-  }
   // phase 1 of the CPU route (computeIntersections) or of the GPU route
   // (calculateIntersections, whose phase-1 arrays the view then holds)
   const bool cpuRoute = opt.route != 0;
   double *cf = nullptr;
+  // one launch fills the rings and finds the filter constants, except for a
+  // few large pairs, which split both over several blocks
+  const bool splitFill = pw == 1024 && std::max(maxRingP, maxRingQ) > kFillRing;
+  if (cpuRoute) cf = wsT<double>(c, "gh_cf", (long long)CF_N * M);
+  {
+    LaunchTimer t(c, "gh_pair_fill");
+    const int split = splitFill ? pgrp_split(M, pw) : 1;
+    hipLaunchKernelGGL(pw == 64 ? k_pair_fill<64> : k_pair_fill<1024>,
+                       dim3(pgrp_grid(M, pw) * (unsigned)split), dim3(pgrp_block(pw)), 0,
+                       c.stream, M, split, pairs,
+                       in.bCoords, in.oCoords, pm, (const long long *)offP,
+                       (const long long *)offQ, mapP, mapQ, ringP, ringQ,
+                       splitFill ? nullptr : cf);
+    HIP_CHECK(hipGetLastError());
+  }
   if (cpuRoute) {
     if (maxRingP >= (1L << 27) || maxRingQ >= (1L << 27))
       throw Error{GCMF_ERR_OVERFLOW, "CPU-route clip takes rings of fewer than 2^27 vertices"};
-    cf = wsT<double>(c, "gh_cf", (long long)CF_N * M);
-    const int split = pgrp_split(M, pw);
-    if (split > 1) {
+    if (splitFill) {
+      const int split = pgrp_split(M, pw);
       // few large pairs: over several blocks per pair
       double *boxPart = wsT<double>(c, "gh_filter_box_parts", 8 * M * (long)split);
       double *lenPart = wsT<double>(c, "gh_filter_len_parts", 4 * M * (long)split);
@@ -5809,12 +5873,6 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
       HIP_CHECK(hipGetLastError());
       hipLaunchKernelGGL(k_filter_finish, dim3((unsigned)M), dim3(256), 0, c.stream, M, split,
                          (const int *)pm.status, (const double *)lenPart, cf);
-    } else {
-      hipLaunchKernelGGL(pw == 64 ? k_cpu_filter_setup<64> : k_cpu_filter_setup<1024>,
-                         dim3(pgrp_grid(M, pw)), dim3(pgrp_block(pw)), 0, c.stream, M,
-                         (const int *)pm.status, (const long long *)offP,
-                         (const long long *)offQ, (const double *)ringP, (const double *)ringQ,
-                         cf);
     }
     HIP_CHECK(hipGetLastError());
   }
@@ -5825,38 +5883,46 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
   int *lstQ = wsT<int>(c, "gh_lstQ", (long)kPartners * edgesQ);
   // [0] edge pairs classified, [1] intersection records, [2] edge pairs tested
   unsigned long long *stats = ctr + 2;
-  // run boxes of a side, when some ring of it is long enough to be culled
-  auto run_boxes = [&](bool qside, long edges, const int *map, const long long *off,
-                       const double *ring) {
+  // run boxes of a side: the 16-edge runs', with `up` the two levels above
+  // (the third only where lanes walk on their own), and the Q flags and
+  // counters of the CPU route in the same launch
+  auto run_boxes = [&](bool qside, bool up, bool up3, bool flags) {
     RunBoxes r{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, c.tune.cullMin};
+    const long edges = qside ? edgesQ : edgesP;
     const long r1 = (edges + kRun1 - 1) / kRun1, r2 = (r1 + 15) / 16, r3 = (r2 + 15) / 16;
     double *b1 = wsT<double>(c, qside ? "gh_rb1Q" : "gh_rb1P", 4 * r1);
-    double *b2 = wsT<double>(c, qside ? "gh_rb2Q" : "gh_rb2P", 4 * r2);
-    double *b3 = wsT<double>(c, qside ? "gh_rb3Q" : "gh_rb3P", 4 * r3);
     double *l1 = wsT<double>(c, qside ? "gh_rl1Q" : "gh_rl1P", r1);
-    double *l2 = wsT<double>(c, qside ? "gh_rl2Q" : "gh_rl2P", r2);
-    double *l3 = wsT<double>(c, qside ? "gh_rl3Q" : "gh_rl3P", r3);
+    double *b2 = nullptr, *l2 = nullptr;
+    if (up) {
+      b2 = wsT<double>(c, qside ? "gh_rb2Q" : "gh_rb2P", 4 * r2);
+      l2 = wsT<double>(c, qside ? "gh_rl2Q" : "gh_rl2P", r2);
+    }
     hipLaunchKernelGGL(k_run_boxes, dim3(grid_for(edges, 256)), dim3(256), 0, c.stream, edges,
-                       map, off, ring, b1, l1);
-    hipLaunchKernelGGL(k_run_boxes_merge, dim3(grid_for(r2, 256)), dim3(256), 0, c.stream, r1,
-                       (const double *)b1, (const double *)l1, b2, l2);
-    hipLaunchKernelGGL(k_run_boxes_merge, dim3(grid_for(r3, 256)), dim3(256), 0, c.stream, r2,
-                       (const double *)b2, (const double *)l2, b3, l3);
+                       qside ? mapQ : mapP, (const long long *)(qside ? offQ : offP),
+                       (const double *)(qside ? ringQ : ringP), b1, l1, b2, l2,
+                       (const double *)cf, flags ? boolQ : nullptr, cnt1Q, cnt2Q);
+    if (up && up3) {
+      double *b3 = wsT<double>(c, qside ? "gh_rb3Q" : "gh_rb3P", 4 * r3);
+      double *l3 = wsT<double>(c, qside ? "gh_rl3Q" : "gh_rl3P", r3);
+      hipLaunchKernelGGL(k_run_boxes_merge, dim3(grid_for(r3, 256)), dim3(256), 0, c.stream, r2,
+                         (const double *)b2, (const double *)l2, b3, l3);
+      r.b3 = b3;
+      r.l3 = l3;
+    }
     HIP_CHECK(hipGetLastError());
     r.b1 = b1;
     r.b2 = b2;
-    r.b3 = b3;
     r.l1 = l1;
     r.l2 = l2;
-    r.l3 = l3;
     return r;
   };
   RunBoxes boxP{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, c.tune.cullMin};
   RunBoxes boxQ{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, c.tune.cullMin};
-  if (maxRingP > c.tune.cullMin && edgesP > 0)
-    boxP = run_boxes(false, edgesP, mapP, (const long long *)offP, (const double *)ringP);
-  if (maxRingQ > c.tune.cullMin && edgesQ > 0)
-    boxQ = run_boxes(true, edgesQ, mapQ, (const long long *)offQ, (const double *)ringQ);
+  const bool cullQ = maxRingQ > c.tune.cullMin;
+  if (!cpuRoute && maxRingP > c.tune.cullMin && edgesP > 0)
+    boxP = run_boxes(false, true, true, false);
+  if (edgesQ > 0 && (cpuRoute || cullQ))
+    boxQ = run_boxes(true, cullQ, !cpuRoute || c.tune.countStage != 0, cpuRoute);
   long long *psP1 = wsT<long long>(c, "gh_psP1", edgesP + 1);
   long long *psP2 = wsT<long long>(c, "gh_psP2", edgesP + 1);
   long long *psQ1 = wsT<long long>(c, "gh_psQ1", edgesQ + 1);
@@ -5893,20 +5959,7 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
         sum_wave_stats(c, bstat, M, stats);
       }
       {  // the ring walk: every pair the LDS pass does not take
-        const bool cull = boxQ.b1 != nullptr, wave = c.tune.countStage == 0;
-        // the wave walk needs the Q edges' kRun1-edge run boxes
-        RunBoxes walkQ = boxQ;
-        if (wave && !cull && edgesQ > 0) {
-          const long r1 = (edgesQ + kRun1 - 1) / kRun1;
-          double *b1 = wsT<double>(c, "gh_rb1Q", 4 * r1);
-          double *l1 = wsT<double>(c, "gh_rl1Q", r1);
-          hipLaunchKernelGGL(k_run_boxes, dim3(grid_for(edgesQ, 256)), dim3(256), 0, c.stream,
-                             edgesQ, mapQ, (const long long *)offQ, (const double *)ringQ, b1,
-                             l1);
-          HIP_CHECK(hipGetLastError());
-          walkQ.b1 = b1;
-          walkQ.l1 = l1;
-        }
+        const bool cull = cullQ, wave = c.tune.countStage == 0;
         const int cb = c.tune.countBlock;
         const bool perEdge = wave && capQ <= minQ && edgesP <= kCountEdgeMax;
         const unsigned grid = perEdge ? grid_for(edgesP, 4) : grid_for(edgesP, cb);
@@ -5917,7 +5970,7 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
           hipLaunchKernelGGL(k_count_edge, dim3(grid), dim3(256), 0, c.stream, edgesP, mapP,
                              (const long long *)offP, (const long long *)offQ,
                              (const double *)ringP, (const double *)ringQ, (const double *)cf,
-                             cnt1P, cnt2P, boolP, wstat, lstP, walkQ);
+                             cnt1P, cnt2P, boolP, wstat, lstP, boxQ);
           HIP_CHECK(hipGetLastError());
         } else {
           LaunchTimer t(c, "gh_count");
@@ -5930,7 +5983,7 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
                              (const long long *)offP, (const long long *)offQ, ringP, ringQ,
                              (const double *)cf,
                              cnt1P, cnt2P, cnt1Q, cnt2Q, boolP, boolQ, wstat, lstP, lstQ, boxP,
-                             walkQ, capQ > minQ ? capQ : 0, c.tune.countStage);
+                             boxQ, capQ > minQ ? capQ : 0, c.tune.countStage);
           HIP_CHECK(hipGetLastError());
         }
         sum_wave_stats(c, wstat, waves, stats);
@@ -5977,10 +6030,6 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
                          boxQ);
     HIP_CHECK(hipGetLastError());
     // -- the Q side by transposition
-    if (edgesQ > 0)
-      hipLaunchKernelGGL(k_cpu_flags_q, dim3(grid_for(edgesQ, 256)), dim3(256), 0, c.stream,
-                         edgesQ, mapQ, (const long long *)offP, (const long long *)offQ,
-                         (const double *)ringQ, (const double *)cf, boolQ, cnt1Q, cnt2Q);
     uint64_t *tk = wsT<uint64_t>(c, "gh_trK", H), *tk2 = wsT<uint64_t>(c, "gh_trK2", H);
     int *tv = wsT<int>(c, "gh_trV", H);
     lstAllQ = wsT<int>(c, "gh_lstAllQ", H);
