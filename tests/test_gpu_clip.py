@@ -806,3 +806,50 @@ def test_clip_few_pairs_label_alike(gctx, pairs):
         assert len(a) == len(b)
         for x, y in zip(a, b):
             np.testing.assert_array_equal(x, y)
+
+
+@pytest.mark.parametrize("pairs, n_p, n_q", [
+    (1, 5, 3), (1, 4096, 4), (1, 4097, 30), (3, 8192, 16), (1, 16384, 9), (1, 16385, 9),
+    (33, 500, 120), (300, 50, 40)])
+def test_clip_small_call_glue(gctx, pairs, n_p, n_q):
+    """Calls around the sizes at which one block does the scans, lists and
+    checks between the passes (4096 edges a round, 16384 in all): phase-1
+    offsets are the exclusive scans of the counts they hold and the results
+    the oracle's, disjoint and nested pairs among them."""
+    cases = []
+    for s in range(pairs):
+        P, Q = G.gen_single_pair(0, 900 + s, n_p, n_q)
+        Q = Q + 5.0 if s % 7 == 3 else 0.1 * Q if s % 7 == 5 else Q
+        cases.append(("c%d" % s, P, Q))
+    st = run_batch(gctx, cases, G.CLIP_NORMALIZE)
+    off = gctx.clip_get("offP", pairs + 1)
+    assert off[0] == 0 and off[-1] == st["edges_p"] and (np.diff(off) >= 0).all()
+    for f, n in (("psP1", st["edges_p"]), ("psP2", st["edges_p"]), ("psQ1", st["edges_q"]),
+                 ("psQ2", st["edges_q"])):
+        ps = gctx.clip_get(f, n + 1)
+        assert ps[0] == 0 and (np.diff(ps) >= (1 if f.endswith("2") else 0)).all()
+    assert gctx.clip_get("psP2", st["edges_p"] + 1)[-1] == st["slots_p"]
+    assert gctx.clip_get("psQ2", st["edges_q"] + 1)[-1] == st["slots_q"]
+    check_results(gctx, st, cases, 5)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 1023, 1025, 4097, 8191, 8192, 8193])
+@pytest.mark.parametrize("bits", [1, 8, 13, 64])
+def test_radix_sort_one_block(gctx, n, bits):
+    """Sorts of up to 8192 keys run in one block: stable, every pass count."""
+    rs = np.random.RandomState(n + bits)
+    mask = np.uint64((1 << bits) - 1)
+    keys = rs.randint(0, 1 << 62, n).astype(np.uint64) * np.uint64(5) & mask
+    keys[::3] = keys[0]
+    vals = np.arange(n, dtype=np.int32)[::-1].copy()
+    bufs = [gctx.upload(keys), gctx.upload(vals), gctx.upload(keys), gctx.upload(vals)]
+    try:
+        gctx.radix_sort(*bufs, n, bits)
+        k = gctx.download(bufs[2], np.uint64, n)
+        v = gctx.download(bufs[3], np.int32, n)
+    finally:
+        for b in bufs:
+            b.free()
+    order = np.argsort(keys, kind="stable")
+    np.testing.assert_array_equal(k, keys[order])
+    np.testing.assert_array_equal(v, vals[order])
