@@ -332,8 +332,7 @@ def main():
 
     kernels = ["mbr_endpoints", "sort_hist", "sort_scatter", "scan_tile", "scan_reduce",
                "scan_downsweep", "scan_lookback", "compact_lookback", "mbr_sweep_prep",
-               "mbr_sweep_count", "mbr_sweep_write", "get_cmbr", "pip", "cmf_count", "cmf_apply",
-               "segment_join", "gh_pair_setup", "gh_pair_fill", "gh_count", "gh_transpose",
+               "mbr_sweep_count", "mbr_sweep_write", "refine_count", "refine_apply", "gh_pair_setup", "gh_pair_fill", "gh_count", "gh_transpose",
                "gh_nmap", "gh_calc_own", "gh_calc", "gh_sort_p", "gh_sort_runs", "gh_sort_q",
                "gh_init_label", "gh_cpu_fill", "gh_cpu_sort", "gh_cpu_link", "gh_label_trace",
                "gh_gather_out", "fill_i32"]
@@ -639,10 +638,11 @@ def prims(args):
         out.append({"prim": "mbr_filter", "keys": 4 * npoly, "candidates": K,
                     "ms": round(ms, 4), "sweep_ms": round(sweep_ms, 4), "GB/s": round(gb, 1),
                     "frac": round(gb / HBM_PEAK_GBS, 4)})
-        # CMF edge filter (count + apply) over the same join's candidates that
-        # the PiP test did not settle: every vertex of both polygons read
-        # (16 B) and every surviving edge index written (4 B)
-        cmf_ms = ctx.timer("cmf_count")[0] + ctx.timer("cmf_apply")[0]
+        # the two refine passes (PiP, CMF edge filter, segment test) over the
+        # same join's candidates, priced by the filter over those that the PiP
+        # test did not settle: every vertex of both polygons read (16 B) and
+        # every surviving edge index written (4 B)
+        cmf_ms = ctx.timer("refine_count")[0] + ctx.timer("refine_apply")[0]
         pairs = ctx.join_get("pairs", 2 * K).reshape(-1, 2)
         pip = ctx.join_get("pip_flag", K)
         todo = pairs[pip != 1]

@@ -59,9 +59,7 @@ void run_join(gcmf_ctx *ctx, const gcmf_dlayer *base, const gcmf_dlayer *over,
   if (ctx->c.replay == 0) no_graph(ctx);
   ctx->join_valid = false;
   ctx->jin = to_inputs(base, over);
-  ctx->K = gcmf::mbr_filter(ctx->c, base->npoly, over->npoly, base->d_mbr, over->d_mbr,
-                            &ctx->counts, &ctx->pairs, &ctx->sv, base->d_vnum, over->d_vnum);
-  gcmf::join_refine(ctx->c, ctx->jin, ctx->K, ctx->pairs, ctx->jr);
+  ctx->K = gcmf::join_run(ctx->c, ctx->jin, &ctx->counts, &ctx->pairs, &ctx->sv, ctx->jr);
   ctx->c.flush_timers();
   ctx->join_valid = true;
   if (st) {

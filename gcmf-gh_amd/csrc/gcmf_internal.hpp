@@ -113,8 +113,6 @@ struct Context {
   std::vector<std::vector<char>> rec_bytes;
   size_t rec_bytes_pos = 0;
   int *graph_flag = nullptr;
-  // mean vertex count per polygon of the last join's layers (-1: unknown)
-  double avgVerts = -1.0;
   // the persistent labelling launch's grid (waves the GPU holds at once) for
   // the LDS arena size it was measured with
   long label_steal_blocks = 0;

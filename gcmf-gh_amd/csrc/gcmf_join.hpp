@@ -21,25 +21,23 @@ struct MbrSortView {
 };
 
 // Stage 1.  Returns K; *pairs_out = workspace array of 2K int32 (b, o).
-// With the vertex counts, their mean per polygon is kept in c.avgVerts.
 long mbr_filter(Context &c, long B, long O, const uint64_t *bMBR, const uint64_t *oMBR,
-                int **counts_out, int **pairs_out, MbrSortView *sv,
-                const int *bVNum = nullptr, const int *oVNum = nullptr);
+                int **counts_out, int **pairs_out);
 
 // Stages 2-5, all device arrays in the context workspace.
 struct JoinRefine {
   long K = 0, pipNum = 0, within = 0, cmfCand = 0, E = 0, hits = 0, nJoined = 0;
   long nbEdges = 0, noEdges = 0;
   double *cmbr = nullptr;
-  int *pipFlag = nullptr, *joinFlag = nullptr, *pipCand = nullptr;
+  int *pipFlag = nullptr, *joinFlag = nullptr;
   signed char *pipType = nullptr;
   int *bCount = nullptr, *oCount = nullptr;
-  long long *bOff = nullptr, *oOff = nullptr;
   int *bEdge = nullptr, *oEdge = nullptr;
-  int *segFlag = nullptr, *list = nullptr, *joined = nullptr;
-  int *joinedIdx = nullptr, *joinedPairs = nullptr;
+  int *segFlag = nullptr, *joinedPairs = nullptr;
 };
-void join_refine(Context &c, const JoinInputs &in, long K, const int *pairs, JoinRefine &r);
+// All stages; returns K, with *pairs_out as from mbr_filter.
+long join_run(Context &c, const JoinInputs &in, int **counts_out, int **pairs_out,
+              MbrSortView *sv, JoinRefine &r);
 
 // single-stage launchers used by the reference-surface entry points
 void launch_get_cmbr(Context &c, long K, const int *pairs, const double *bMBR2,

@@ -24,6 +24,7 @@
 #include <hip/hip_cooperative_groups.h>
 
 #include "gcmf_device.hpp"
+#include "gcmf_block.hpp"
 #include "gcmf_internal.hpp"
 #include "gcmf_join.hpp"
 
@@ -5764,14 +5765,6 @@ __device__ __forceinline__ long long glue_scan(long long v, long long &total) {
   const long long r = block_scan_ll(v, total);
   __syncthreads();
   return r;
-}
-
-// value j of a read-back (the last one the look-back error word)
-__device__ __forceinline__ void put_slots(long long *slots, const long long *v, int n,
-                                          const long long *lbErr) {
-  if (!slots) return;
-  for (int j = 0; j < n; j++) slots[j] = v[j];
-  slots[n] = lbErr ? *lbErr : 0;
 }
 
 // in[i], in[i + 1].. of a 16-byte aligned workspace array, 0 past n

@@ -8,16 +8,19 @@
 //      its own two endpoints in a structure-of-arrays record stream
 //      (endpoint id, partner y-interval), one wave64 per polygon, ballots
 //      for counting and ordered output.
-//   2. CMBR + PiP candidate flags [Join.h:397-432, GPU_Join.h:461-508].
-//   3. PiP "within" refine, one wave per candidate, crossing parity from
-//      ballot popcounts [Join.h:437-467, GPU_Join.h:839-943].
-//   4. CMF edge filter count + apply, one wave per surviving pair, ordered
-//      edge lists from ballot ranks [Join.h:157-287, GPU_Join.h:511-735].
-//   5. Segment-intersection refine, one wave per CMF survivor, wave-uniform
-//      early exit [Join.h:356-393, GPU_Join.h:326-456].
+//   2. CMBR + PiP candidate flags [Join.h:397-432, GPU_Join.h:461-508],
+//   3. PiP "within" refine, crossing parity from ballot popcounts
+//      [Join.h:437-467, GPU_Join.h:839-943],
+//   4. CMF edge filter, ordered edge lists from ballot ranks
+//      [Join.h:157-287, GPU_Join.h:511-735],
+//   5. Segment-intersection refine with a uniform early exit
+//      [Join.h:356-393, GPU_Join.h:326-456]: two fused passes over the
+//      candidates, one group of 8, 16 or 64 lanes each; as kernels of their
+//      own for the entry points that run one stage.
 #include <algorithm>
 #include <vector>
 
+#include "gcmf_block.hpp"
 #include "gcmf_device.hpp"
 #include "gcmf_internal.hpp"
 #include "gcmf_join.hpp"
@@ -27,17 +30,48 @@ namespace gcmf {
 constexpr uint64_t kKeyMod = 10000000000000000ULL;  // 16 decimal digits
 
 // ------------------------------------------------------------ stage 1 ----
-// mm: x key min, x key max, y key min, y key max (over both corners) and,
-// when the vertex counts are given, their sum; a grid of at most
-// kEndpointBlocks blocks striding over the polygons
+// mm: x key min, x key max, y key min, y key max (over both corners), when
+// the vertex counts are given their sum, and the height class of the y strips
+constexpr int kMmVals = 6;
 constexpr unsigned kEndpointBlocks = 1024;
-__global__ void k_endpoints(long B, long O, const uint64_t *bMBR, const uint64_t *oMBR,
-                            const int *bVNum, const int *oVNum, uint64_t *keys, int *idx,
-                            uint64_t *Y, unsigned long long *mm) {
-  uint64_t lo = ~0ULL, hi = 0, ylo = ~0ULL, yhi = 0, vs = 0;
+constexpr int kStripSample = 1024;
+
+struct MinMax {
+  uint64_t v[5];
+};
+__device__ __forceinline__ MinMax mm_none() { return MinMax{{~0ULL, 0, ~0ULL, 0, 0}}; }
+__device__ __forceinline__ void mm_merge(MinMax &a, const MinMax &b) {
+  a.v[0] = min(a.v[0], b.v[0]);
+  a.v[1] = max(a.v[1], b.v[1]);
+  a.v[2] = min(a.v[2], b.v[2]);
+  a.v[3] = max(a.v[3], b.v[3]);
+  a.v[4] += b.v[4];
+}
+// of the whole block, in thread 0 (lds: one per wave)
+__device__ __forceinline__ void mm_block(MinMax &a, MinMax *lds) {
+  for (int off = 32; off > 0; off >>= 1) {
+    MinMax o;
+#pragma unroll
+    for (int j = 0; j < 5; j++) o.v[j] = __shfl_xor(a.v[j], off, 64);
+    mm_merge(a, o);
+  }
+  if (__lane_id() == 0) lds[threadIdx.x >> 6] = a;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    for (int w = 1; w < (int)(blockDim.x >> 6); w++) mm_merge(a, lds[w]);
+}
+
+// Keys, ids and y values of every endpoint; each block's minima and maxima
+// go to part (bound by that reduction when it was five atomics per block on
+// one cache line: 66 us for 550 000 polygons on one MI355X, against 8 us of
+// loads and stores; 13 us this way).
+__global__ void __launch_bounds__(256)
+    k_endpoints(long B, long O, const uint64_t *bMBR, const uint64_t *oMBR, const int *bVNum,
+                const int *oVNum, uint64_t *keys, int *idx, uint64_t *Y, MinMax *part) {
+  __shared__ MinMax lds[4];
+  MinMax a = mm_none();
   for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < B + O;
        e += (long)gridDim.x * blockDim.x) {
-    if (bVNum) vs += (uint64_t)(e < B ? bVNum[e] : oVNum[e - B]);
     const uint64_t *m = e < B ? bMBR + 4 * e : oMBR + 4 * (e - B);
     const uint64_t x1 = m[0] % kKeyMod, x2 = m[2] % kKeyMod, y1 = m[1], y2 = m[3];
     keys[2 * e] = x1;
@@ -46,114 +80,209 @@ __global__ void k_endpoints(long B, long O, const uint64_t *bMBR, const uint64_t
     idx[2 * e + 1] = (int)(2 * e + 1);
     Y[2 * e] = y1;
     Y[2 * e + 1] = y2;
-    lo = min(lo, min(x1, x2));
-    hi = max(hi, max(x1, x2));
-    ylo = min(ylo, min(y1, y2));
-    yhi = max(yhi, max(y1, y2));
+    mm_merge(a, MinMax{{min(x1, x2), max(x1, x2), min(y1, y2), max(y1, y2),
+                        bVNum ? (uint64_t)(e < B ? bVNum[e] : oVNum[e - B]) : 0}});
   }
-  // wave min/max, block min/max, then one atomic per block and value
-  // (atomics on one cache line serialise across the chip, so the grid is
-  // capped)
-  __shared__ uint64_t slo[4], shi[4], sylo[4], syhi[4], svs[4];
-  for (int off = 32; off > 0; off >>= 1) {
-    uint64_t l2 = __shfl_xor(lo, off, 64), h2 = __shfl_xor(hi, off, 64);
-    uint64_t yl2 = __shfl_xor(ylo, off, 64), yh2 = __shfl_xor(yhi, off, 64);
-    lo = l2 < lo ? l2 : lo;
-    hi = h2 > hi ? h2 : hi;
-    ylo = yl2 < ylo ? yl2 : ylo;
-    yhi = yh2 > yhi ? yh2 : yhi;
-    vs += __shfl_xor(vs, off, 64);
-  }
-  if (__lane_id() == 0) {
-    slo[threadIdx.x >> 6] = lo;
-    shi[threadIdx.x >> 6] = hi;
-    sylo[threadIdx.x >> 6] = ylo;
-    syhi[threadIdx.x >> 6] = yhi;
-    svs[threadIdx.x >> 6] = vs;
-  }
+  mm_block(a, lds);
+  if (threadIdx.x == 0) part[blockIdx.x] = a;
+}
+
+// The blocks' minima and maxima combined, and the class of the median MBR
+// height of ns sampled polygons (j N / ns, j < ns): the power of two at or
+// above twice a height.  The class never decreases with the height, so the
+// median's class is the classes' median, found from their histogram.  One
+// block of kStripSample threads; the values also go to slots.
+__global__ void __launch_bounds__(kStripSample)
+    k_minmax_final(const MinMax *part, int nPart, long N, const uint64_t *Y, int ns,
+                   long long *mm, long long *slots, const long long *lbErr) {
+  __shared__ MinMax lds[kStripSample / 64];
+  __shared__ int hist[66];
+  if (threadIdx.x < 66) hist[threadIdx.x] = 0;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < (int)(blockDim.x >> 6); w++) {
-      lo = slo[w] < lo ? slo[w] : lo;
-      hi = shi[w] > hi ? shi[w] : hi;
-      ylo = sylo[w] < ylo ? sylo[w] : ylo;
-      yhi = syhi[w] > yhi ? syhi[w] : yhi;
-      vs += svs[w];
-    }
-    atomicMin(mm, (unsigned long long)lo);
-    atomicMax(mm + 1, (unsigned long long)hi);
-    atomicMin(mm + 2, (unsigned long long)ylo);
-    atomicMax(mm + 3, (unsigned long long)yhi);
-    if (vs) atomicAdd(mm + 4, (unsigned long long)vs);
+  const int j = threadIdx.x;
+  if (j < ns) {
+    const long e = (long)((long long)j * N / ns);
+    const uint64_t a = Y[2 * e], b = Y[2 * e + 1], h = a > b ? a - b : b - a;
+    atomicAdd(&hist[h == 0 ? 0 : h == 1 ? 1 : 65 - __clzll(h - 1)], 1);
   }
+  MinMax a = mm_none();
+  for (int i = j; i < nPart; i += kStripSample) mm_merge(a, part[i]);
+  mm_block(a, lds);
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  int cls = 0;
+  for (int c = hist[0]; cls < 65 && c <= ns / 2; c += hist[cls]) cls++;
+  long long v[kMmVals];
+  for (int k = 0; k < 5; k++) v[k] = (long long)a.v[k];
+  v[5] = cls;
+  for (int k = 0; k < kMmVals; k++) mm[k] = v[k];
+  put_slots(slots, v, kMmVals, lbErr);
 }
 
-__global__ void k_init_minmax(unsigned long long *mm) {
-  if (threadIdx.x < 5) mm[threadIdx.x] = threadIdx.x == 4 || (threadIdx.x & 1) ? 0ULL : ~0ULL;
-}
-
-__global__ void k_sub_key(uint64_t *keys, long n, const unsigned long long *mn) {
+__global__ void k_sub_key(uint64_t *keys, long n, const long long *mn) {
   long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) keys[i] -= *mn;
+  if (i < n) keys[i] -= (uint64_t)*mn;
 }
 
-// rank[perm[i]] = i; sweep records in sorted order
-__global__ void k_sweep_prep(const int *perm, long n, const uint64_t *Y, int *rank, int *rec_id,
-                             uint64_t *rec_ylo, uint64_t *rec_yhi) {
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  int e = perm[i];
-  rank[e] = (int)i;
-  rec_id[i] = e;
-  int m = e & ~1;
-  rec_ylo[i] = Y[m];
-  rec_yhi[i] = Y[m + 1];
+// The sorted endpoint stream: endpoint ids and, for left endpoints (the only
+// ones a polygon takes as a candidate), the polygon's y interval; as arrays
+// for the sweep, whose lanes read consecutive ranks, or as one record a rank
+// for the strips, whose lanes read ranks far apart.
+struct SweepRec {
+  int id;
+  uint64_t y1, y2;
+};
+struct SweepRecs {
+  int *id = nullptr;
+  uint64_t *ylo = nullptr, *yhi = nullptr;
+  SweepRec *aos = nullptr;
+};
+
+struct Strips {
+  uint64_t y0;
+  int shift, S;
+};
+__device__ __forceinline__ int strip_of(const Strips &g, uint64_t y) {
+  const uint64_t s = (y - g.y0) >> g.shift;
+  return s >= (uint64_t)g.S ? g.S - 1 : (int)s;
 }
 
-// one wave per polygon element (or per polygon of list[0, nList)); pairs ==
-// nullptr -> count only
+// rank[perm[i]] = i and the stream's record at rank i; with strips also
+// cnt[i], the number of strips the record is listed in
 __global__ void __launch_bounds__(256)
-    k_sweep(long B, long O, const int *rank, const int *rec_id, const uint64_t *rec_ylo,
-            const uint64_t *rec_yhi, const uint64_t *Y, int *counts, const long long *offs,
-            int *pairs, const int *list, long nList) {
-  long e = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (list) {
-    if (e >= nList) return;
-    e = list[e];
-  } else if (e >= B + O) {
+    k_sweep_prep(const int *perm, long n, const uint64_t *Y, int *rank, SweepRecs r, Strips g,
+                 int *cnt) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int e = perm[i];
+  rank[e] = (int)i;
+  const bool left = !(e & 1);
+  const uint64_t a = left ? Y[e] : 0, b = left ? Y[e + 1] : 0;
+  if (r.aos) {
+    r.aos[i] = SweepRec{e, a, b};
+    cnt[i] = left ? strip_of(g, a < b ? b : a) - strip_of(g, a < b ? a : b) + 1 : 0;
     return;
   }
+  r.id[i] = e;
+  if (left) {
+    r.ylo[i] = a;
+    r.yhi[i] = b;
+  }
+}
+
+// The order of at most kRankSort endpoints: their places among all keys, and
+// with them the ranks and records, in one launch and without the read-back
+// of the keys' range that the radix passes need.  Every block makes all keys
+// itself (a few per thread).
+__global__ void __launch_bounds__(kRankThreads)
+    k_order_few(int B, int O, const uint64_t *bMBR, const uint64_t *oMBR, uint64_t *Y, int *perm,
+                int *rank, SweepRecs rec) {
+  __shared__ RankLds lds;
+  const int n = 2 * (B + O);
+  auto mbr_of = [&](int e) { return e < B ? bMBR + 4L * e : oMBR + 4L * (e - B); };
+  const int i = rank_among(n, lds, [&](int j) { return mbr_of(j >> 1)[2 * (j & 1)] % kKeyMod; });
+  const int e = (int)blockIdx.x * kRankKeys + (int)threadIdx.x;
+  if (threadIdx.x >= kRankKeys || e >= n) return;
+  const uint64_t *m = mbr_of(e >> 1);
+  perm[i] = e;
+  rank[e] = i;
+  rec.id[i] = e;
+  Y[e] = m[2 * (e & 1) + 1];
+  if (e & 1) return;
+  rec.ylo[i] = m[1];
+  rec.yhi[i] = m[3];
+}
+
+// One wave walks polygon e's rank range: the number of candidates, which go
+// to pairs[pos..] (those below cap) when pairs is given.
+template <bool AOS>
+__device__ __forceinline__ int sweep_polygon(long e, long B, const int *rank, const SweepRecs &r,
+                                             const uint64_t *Y, long long pos, int *pairs,
+                                             long long cap) {
   const int lane = __lane_id();
   const int lo = rank[2 * e], hi = rank[2 * e + 1];
   const uint64_t ey1 = Y[2 * e], ey2 = Y[2 * e + 1];
   const bool overlay = e >= B;
   const int lim = (int)(2 * B);
-  long long pos = pairs ? offs[e] : 0;
   int cnt = 0;
   for (int i0 = lo + 1; i0 < hi; i0 += 64) {
     int i = i0 + lane;
     bool ok = false;
     int m = 0;
     if (i < hi) {
-      m = rec_id[i];
+      m = AOS ? r.aos[i].id : r.id[i];
       bool other = overlay ? (m < lim) : (m >= lim);
-      ok = other && !(m & 1) && !(ey1 > rec_yhi[i]) && !(rec_ylo[i] > ey2);
+      ok = other && !(m & 1) && !(ey1 > (AOS ? r.aos[i].y2 : r.yhi[i])) &&
+           !((AOS ? r.aos[i].y1 : r.ylo[i]) > ey2);
     }
     unsigned long long msk = __ballot(ok);
     if (pairs && ok) {
       long long p = pos + __popcll(msk & ((1ULL << lane) - 1ULL));
-      if (!overlay) {
-        pairs[2 * p] = (int)e;
-        pairs[2 * p + 1] = m / 2 - (int)B;
-      } else {
-        pairs[2 * p] = m / 2;
-        pairs[2 * p + 1] = (int)(e - B);
+      if (p < cap) {
+        pairs[2 * p] = overlay ? m / 2 : (int)e;
+        pairs[2 * p + 1] = overlay ? (int)(e - B) : m / 2 - (int)B;
       }
     }
     pos += __popcll(msk);
     cnt += __popcll(msk);
   }
-  if (!pairs && lane == 0) counts[e] = cnt;
+  return cnt;
+}
+
+// one wave per polygon; pairs == nullptr -> count only
+__global__ void __launch_bounds__(256)
+    k_sweep(long B, long O, const int *rank, SweepRecs r, const uint64_t *Y, int *counts,
+            const long long *offs, int *pairs, long long cap) {
+  const long e = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (e >= B + O) return;
+  const int cnt = sweep_polygon<false>(e, B, rank, r, Y, pairs ? offs[e] : 0, pairs, cap);
+  if (!pairs && __lane_id() == 0) counts[e] = cnt;
+}
+
+// the same over the *nList polygons of list, on a fixed grid (an empty list
+// costs one launch and no read-back of its length)
+constexpr unsigned kHeavyBlocks = 512;
+__global__ void __launch_bounds__(256)
+    k_sweep_heavy(long B, const int *rank, SweepRecs r, const uint64_t *Y, int *counts,
+                  const long long *offs, int *pairs, long long cap, const int *list,
+                  const int *nList) {
+  const int n = *nList;
+  for (int w = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6); w < n; w += (int)gridDim.x * 4) {
+    const long e = list[w];
+    const int cnt = sweep_polygon<true>(e, B, rank, r, Y, pairs ? offs[e] : 0, pairs, cap);
+    if (!pairs && __lane_id() == 0) counts[e] = cnt;
+  }
+}
+
+// sum of v over a block of 256 threads
+__device__ __forceinline__ long long block_sum256(long long v, long long *lds) {
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  __syncthreads();
+  if (__lane_id() == 0) lds[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return lds[0] + lds[1] + lds[2] + lds[3];
+}
+
+// The write pass of a small call: each block sums the counts before its four
+// polygons itself, in place of a scan launch (at most kFewPolys counts, from
+// L2); the last block stores their total in *total.
+__global__ void __launch_bounds__(256)
+    k_sweep_write_few(long B, long O, const int *rank, SweepRecs r, const uint64_t *Y,
+                      const int *counts, int *pairs, long long cap, long long *total) {
+  __shared__ long long lds[4];
+  const int e0 = (int)blockIdx.x * 4, N = (int)(B + O);
+  long long s = 0;
+  for (int i = threadIdx.x; i < e0; i += 256) s += counts[i];
+  s = block_sum256(s, lds);
+  if (threadIdx.x == 0 && e0 + 4 >= N) {
+    long long t = s;
+    for (int i = e0; i < N; i++) t += counts[i];
+    *total = t;
+  }
+  const int e = e0 + (int)(threadIdx.x >> 6);
+  if (e >= N) return;
+  for (int i = e0; i < e; i++) s += counts[i];
+  sweep_polygon<false>(e, B, rank, r, Y, s, pairs, cap);
 }
 
 // ------------------------------------------------ stage 1, y strips ----
@@ -175,50 +304,19 @@ __global__ void __launch_bounds__(256)
 // (one wave each), so the candidate list is the sweep's, entry for entry.
 constexpr int kStripSpan = 4;
 constexpr int kStripScan = 256;
-constexpr int kStripSample = 1024;
 constexpr long kStripMax = 1L << 22;
-
-struct Strips {
-  uint64_t y0;
-  int shift, S;
-};
-__device__ __forceinline__ int strip_of(const Strips &g, uint64_t y) {
-  const uint64_t s = (y - g.y0) >> g.shift;
-  return s >= (uint64_t)g.S ? g.S - 1 : (int)s;
-}
-
-// |ymax - ymin| of polygons j N / ns, j < ns
-__global__ void k_height_sample(long N, const uint64_t *Y, int ns, uint64_t *out) {
-  const int j = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (j >= ns) return;
-  const long e = (long)((long long)j * N / ns);
-  const uint64_t a = Y[2 * e], b = Y[2 * e + 1];
-  out[j] = a > b ? a - b : b - a;
-}
-
-// the number of strips each record (left endpoint at rank i) is listed in
-__global__ void k_strip_rec_count(long n, const int *rec_id, const uint64_t *rec_ylo,
-                                  const uint64_t *rec_yhi, Strips g, int *cnt) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  int c = 0;
-  if (!(rec_id[i] & 1)) {
-    const uint64_t a = rec_ylo[i], b = rec_yhi[i];
-    c = strip_of(g, a < b ? b : a) - strip_of(g, a < b ? a : b) + 1;
-  }
-  cnt[i] = c;
-}
 
 // (layer * S + strip, rank) for every listing, in rank order; layer 1 is
 // the overlay (endpoint ids from 2B)
-__global__ void k_strip_rec_emit(long n, long B, const int *rec_id, const uint64_t *rec_ylo,
-                                 const uint64_t *rec_yhi, Strips g, const long long *off,
-                                 uint64_t *keys, int *vals) {
+__global__ void k_strip_rec_emit(long n, long B, const SweepRec *rec, Strips g,
+                                 const long long *off, uint64_t *keys, int *vals) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n || (rec_id[i] & 1)) return;
-  const uint64_t a = rec_ylo[i], b = rec_yhi[i];
-  const int s0 = strip_of(g, a < b ? a : b), s1 = strip_of(g, a < b ? b : a);
-  const uint64_t side = rec_id[i] < 2 * B ? 0 : 1;
+  if (i >= n) return;
+  const SweepRec x = rec[i];
+  if (x.id & 1) return;
+  const int s0 = strip_of(g, x.y1 < x.y2 ? x.y1 : x.y2),
+            s1 = strip_of(g, x.y1 < x.y2 ? x.y2 : x.y1);
+  const uint64_t side = x.id < 2 * B ? 0 : 1;
   long long o = off[i];
   for (int s = s0; s <= s1; s++, o++) {
     keys[o] = side * (uint64_t)g.S + (uint64_t)s;
@@ -227,28 +325,16 @@ __global__ void k_strip_rec_emit(long n, long B, const int *rec_id, const uint64
 }
 
 // sOff[k] = the first listing of key k in the sorted keys, k <= 2S (each
-// entry written once: the keys in (key[i - 1], key[i]] start at i)
-__global__ void k_strip_bounds(long R, const uint64_t *skeys, long nk, long long *sOff) {
+// entry written once: the keys in (key[i - 1], key[i]] start at i); also
+// clears the length of the list of polygons left to the sweep
+__global__ void k_strip_bounds(long R, const uint64_t *skeys, long nk, long long *sOff,
+                               int *heavy) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0) heavy[0] = 0;
   if (i > R) return;
   const long cur = i < R ? (long)skeys[i] : nk;
   const long prev = i > 0 ? (long)skeys[i - 1] : -1;
   for (long k = prev + 1; k <= cur; k++) sOff[k] = i;
-}
-
-// what a search needs of the left-endpoint record at rank r: its endpoint id
-// (2 e), the rank of polygon e's right endpoint and the y interval, in one
-// record so that a random visit touches one cache line
-struct StripRec {
-  int id, hi;
-  uint64_t y1, y2;
-};
-__global__ void k_strip_recs(long n, const int *rec_id, const uint64_t *rec_ylo,
-                             const uint64_t *rec_yhi, const int *rank, StripRec *qrec) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int m = rec_id[i];
-  if (!(m & 1)) qrec[i] = StripRec{m, rank[m + 1], rec_ylo[i], rec_yhi[i]};
 }
 
 // first index of [l, r) whose rank is above v
@@ -312,7 +398,7 @@ __device__ __forceinline__ bool strip_hit(const Strips &g, int s, uint64_t ey1, 
 constexpr int kStripInline = 8;
 __global__ void __launch_bounds__(256)
     k_strip_query(long B, long O, Strips g, const long long *sOff, const int *list,
-                  const uint64_t *skeys, long R, const int *rank, const StripRec *qrec,
+                  const uint64_t *skeys, long R, const int *rank, const SweepRec *qrec,
                   const uint64_t *Y, int *counts, const long long *offs, int *pairs,
                   int *heavy, int *inl) {
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -328,13 +414,13 @@ __global__ void __launch_bounds__(256)
   } else {
     if (t >= R) return;
     lo = list[t];
-    const StripRec me = qrec[lo];
+    const SweepRec me = qrec[lo];
     e = me.id / 2;
-    hi = me.hi;
     ey1 = me.y1;
     ey2 = me.y2;
     const long key = (long)skeys[t];
     if ((key >= g.S ? key - g.S : key) != strip_of(g, ey1 < ey2 ? ey1 : ey2)) return;
+    hi = rank[me.id + 1];
   }
   const bool overlay = e >= B;
   int *mine = inl + (long long)kStripInline * e;
@@ -378,7 +464,7 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
     for (int u = 0; u < kStripSpan; u++)
       if (u == best) q.p0[u]++;
-    const StripRec x = qrec[br];
+    const SweepRec x = qrec[br];
     if (!strip_hit(g, q.sa + best, ey1, ey2, ya, x.y1, x.y2)) continue;
     const int m = x.id;
     if (pairs) {
@@ -393,40 +479,99 @@ __global__ void __launch_bounds__(256)
   if (!pairs) counts[e] = cnt;
 }
 
+// The order of the endpoints and the stream of records (mbr_order).
+constexpr long kFewPolys = kRankSort / 2;
+struct MbrOrder {
+  long B = 0, O = 0;
+  bool few = false;     // made by k_order_few
+  bool strips = false;  // y strips: records as SweepRec, with their listings
+  double avg = -1.0;    // mean vertex count per polygon (-1: unknown)
+  int *perm = nullptr, *rank = nullptr;
+  uint64_t *Y = nullptr;
+  SweepRecs rec;
+  Strips g{0, 0, 1};
+  int *cnt = nullptr;  // listings per rank
+};
+
+static void mbr_order(Context &c, long B, long O, const uint64_t *bMBR, const uint64_t *oMBR,
+                      const int *bVNum, const int *oVNum, MbrOrder &m) {
+  const long N = B + O, n = 2 * N;
+  m.B = B;
+  m.O = O;
+  m.strips = N >= c.tune.stripMin;
+  m.few = N <= kFewPolys && !m.strips;
+  m.Y = (uint64_t *)c.ws.get("mbr_Y", 8 * (size_t)n);
+  m.perm = (int *)c.ws.get("mbr_perm", 4 * (size_t)n);
+  m.rank = (int *)c.ws.get("mbr_rank", 4 * (size_t)n);
+  if (m.strips) {
+    m.rec.aos = (SweepRec *)c.ws.get("mbr_recs", sizeof(SweepRec) * (size_t)n);
+    m.cnt = (int *)c.ws.get("strip_cnt", 4 * (size_t)n);
+  } else {
+    m.rec.id = (int *)c.ws.get("mbr_rec_id", 4 * (size_t)n);
+    m.rec.ylo = (uint64_t *)c.ws.get("mbr_rec_ylo", 8 * (size_t)n);
+    m.rec.yhi = (uint64_t *)c.ws.get("mbr_rec_yhi", 8 * (size_t)n);
+  }
+  if (m.few) {
+    LaunchTimer t(c, "mbr_endpoints");
+    hipLaunchKernelGGL(k_order_few, dim3(grid_for(n, kRankKeys)), dim3(kRankThreads), 0, c.stream,
+                       (int)B, (int)O, bMBR, oMBR, m.Y, m.perm, m.rank, m.rec);
+    HIP_CHECK(hipGetLastError());
+    return;
+  }
+  uint64_t *keys = (uint64_t *)c.ws.get("mbr_keys", 8 * (size_t)n);
+  int *idx = (int *)c.ws.get("mbr_idx", 4 * (size_t)n);
+  uint64_t *skeys = (uint64_t *)c.ws.get("mbr_skeys", 8 * (size_t)n);
+  MinMax *part = (MinMax *)c.ws.get("mbr_minmax_part", sizeof(MinMax) * kEndpointBlocks);
+  long long *mm = (long long *)c.ws.get("mbr_minmax", 8 * kMmVals);
+  const unsigned eb = std::min(grid_for(N, 256), kEndpointBlocks);
+  const bool verts = bVNum && oVNum;
+  {
+    LaunchTimer t(c, "mbr_endpoints");
+    hipLaunchKernelGGL(k_endpoints, dim3(eb), dim3(256), 0, c.stream, B, O, bMBR, oMBR,
+                       verts ? bVNum : nullptr, oVNum, keys, idx, m.Y, part);
+    HIP_CHECK(hipGetLastError());
+    hipLaunchKernelGGL(k_minmax_final, dim3(1), dim3(kStripSample), 0, c.stream,
+                       (const MinMax *)part, (int)eb, N, (const uint64_t *)m.Y,
+                       (int)std::min<long>(kStripSample, N), mm, slots_begin(c),
+                       (const long long *)c.lb_err);
+    HIP_CHECK(hipGetLastError());
+  }
+  long long h[kHostSlots];
+  slots_end(c, {mm, mm + 1, mm + 2, mm + 3, mm + 4, mm + 5}, h);
+  m.avg = verts ? (double)h[4] / (double)N : -1.0;
+  const uint64_t range = (uint64_t)h[1] - (uint64_t)h[0];
+  int bits = 0;
+  while (bits < 64 && (range >> bits) != 0) bits++;
+  hipLaunchKernelGGL(k_sub_key, dim3(grid_for(n, 256)), dim3(256), 0, c.stream, keys, n,
+                     (const long long *)mm);
+  HIP_CHECK(hipGetLastError());
+  radix_sort_u64(c, keys, idx, skeys, m.perm, n, bits);
+  if (m.strips) {
+    // at most kStripMax strips
+    const uint64_t yr = (uint64_t)h[3] - (uint64_t)h[2];
+    int shift = std::min((int)h[5], 63);
+    while (shift < 63 && (yr >> shift) + 1 > (uint64_t)kStripMax) shift++;
+    m.g = Strips{(uint64_t)h[2], shift, (int)((yr >> shift) + 1)};
+  }
+  LaunchTimer t(c, "mbr_sweep_prep");
+  hipLaunchKernelGGL(k_sweep_prep, dim3(grid_for(n, 256)), dim3(256), 0, c.stream,
+                     (const int *)m.perm, n, (const uint64_t *)m.Y, m.rank, m.rec, m.g, m.cnt);
+  HIP_CHECK(hipGetLastError());
+}
+
 // The strip form of the sweep: fills counts[N] and offs[N + 1] and returns
 // the candidate count, with the pairs written to *pairs_out; returns -1
 // (nothing written) when the records would be listed more than four times
-// each on average, where the plain sweep is used instead.
-static long strip_sweep(Context &c, long B, long O, const int *rank, const int *rec_id,
-                        const uint64_t *rec_ylo, const uint64_t *rec_yhi, const uint64_t *Y,
-                        uint64_t y0, uint64_t y1, int *counts, long long *offs,
+// each on average, where the polygons are swept instead.
+static long strip_sweep(Context &c, const MbrOrder &m, int *counts, long long *offs,
                         int **pairs_out) {
-  const long N = B + O, n = 2 * N;
-  // strip height: the power of two at or above twice the median sampled MBR
-  // height, at most kStripMax strips
-  const int ns = (int)std::min<long>(kStripSample, N);
-  uint64_t *samp = (uint64_t *)c.ws.get("strip_sample", 8 * (size_t)ns);
-  hipLaunchKernelGGL(k_height_sample, dim3(grid_for(ns, 256)), dim3(256), 0, c.stream, N, Y, ns,
-                     samp);
-  HIP_CHECK(hipGetLastError());
-  std::vector<uint64_t> hs((size_t)ns);
-  host_read(c, hs.data(), samp, 8 * (size_t)ns);
-  std::nth_element(hs.begin(), hs.begin() + ns / 2, hs.end());
-  const uint64_t range = y1 - y0, h2 = 2 * hs[(size_t)ns / 2];
-  int shift = 0;
-  while (shift < 63 && ((1ULL << shift) < h2 || (range >> shift) + 1 > (uint64_t)kStripMax))
-    shift++;
-  Strips g{y0, shift, (int)((range >> shift) + 1)};
+  const long B = m.B, O = m.O, N = B + O, n = 2 * N;
+  const Strips g = m.g;
+  int *heavy = (int *)c.ws.get("strip_heavy", 4 * (size_t)(N + 1));
+  const int *hlist = heavy + 1;
   // listings, in rank order, then stably sorted by (layer, strip)
-  int *cnt = (int *)c.ws.get("strip_cnt", 4 * (size_t)n);
   long long *off = (long long *)c.ws.get("strip_off", 8 * (size_t)(n + 1));
-  {
-    LaunchTimer t(c, "mbr_strip_build");
-    hipLaunchKernelGGL(k_strip_rec_count, dim3(grid_for(n, 256)), dim3(256), 0, c.stream, n,
-                       rec_id, rec_ylo, rec_yhi, g, cnt);
-    HIP_CHECK(hipGetLastError());
-  }
-  scan_i32_to_i64(c, cnt, off, n);
+  scan_i32_to_i64(c, m.cnt, off, n);
   const long R = (long)read_scalar(c, off + n);
   if (R > 4 * N) return -1;
   const long nk = 2L * g.S;
@@ -436,11 +581,10 @@ static long strip_sweep(Context &c, long B, long O, const int *rank, const int *
   uint64_t *skeys = (uint64_t *)c.ws.get("strip_skeys", 8 * R1);
   int *list = (int *)c.ws.get("strip_list", 4 * R1);
   long long *sOff = (long long *)c.ws.get("strip_soff", 8 * (size_t)(nk + 1));
-  StripRec *qrec = (StripRec *)c.ws.get("strip_recs", sizeof(StripRec) * (size_t)n);
   {
     LaunchTimer t(c, "mbr_strip_build");
     hipLaunchKernelGGL(k_strip_rec_emit, dim3(grid_for(n, 256)), dim3(256), 0, c.stream, n, B,
-                       rec_id, rec_ylo, rec_yhi, g, (const long long *)off, keys, vals);
+                       (const SweepRec *)m.rec.aos, g, (const long long *)off, keys, vals);
     HIP_CHECK(hipGetLastError());
   }
   int kbits = 0;
@@ -449,30 +593,25 @@ static long strip_sweep(Context &c, long B, long O, const int *rank, const int *
   {
     LaunchTimer t(c, "mbr_strip_build");
     hipLaunchKernelGGL(k_strip_bounds, dim3(grid_for(R + 1, 256)), dim3(256), 0, c.stream, R,
-                       (const uint64_t *)skeys, nk, sOff);
-    HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(k_strip_recs, dim3(grid_for(n, 256)), dim3(256), 0, c.stream, n, rec_id,
-                       rec_ylo, rec_yhi, rank, qrec);
+                       (const uint64_t *)skeys, nk, sOff, heavy);
     HIP_CHECK(hipGetLastError());
   }
   // counts; the polygons the strips leave to the sweep
-  int *heavy = (int *)c.ws.get("strip_heavy", 4 * (size_t)(N + 1));
   int *inl = (int *)c.ws.get("strip_inline", 4 * (size_t)kStripInline * (size_t)N);
-  fill_i32(c, heavy, 0, 1);
   {
     LaunchTimer t(c, "mbr_strip_count");
     hipLaunchKernelGGL(k_strip_query, dim3(grid_for(R, 256)), dim3(256), 0, c.stream, B, O, g,
                        (const long long *)sOff, (const int *)list, (const uint64_t *)skeys, R,
-                       rank, (const StripRec *)qrec, Y, counts, (const long long *)nullptr,
-                       (int *)nullptr, heavy, inl);
+                       (const int *)m.rank, (const SweepRec *)m.rec.aos, (const uint64_t *)m.Y,
+                       counts, (const long long *)nullptr, (int *)nullptr, heavy, inl);
     HIP_CHECK(hipGetLastError());
   }
-  const int nHeavy = read_scalar(c, (const int *)heavy);
-  if (nHeavy > 0) {
+  {
     LaunchTimer t(c, "mbr_sweep_count");
-    hipLaunchKernelGGL(k_sweep, dim3(grid_for(nHeavy, 4)), dim3(256), 0, c.stream, B, O, rank,
-                       rec_id, rec_ylo, rec_yhi, Y, counts, (const long long *)nullptr,
-                       (int *)nullptr, (const int *)(heavy + 1), (long)nHeavy);
+    hipLaunchKernelGGL(k_sweep_heavy, dim3(kHeavyBlocks), dim3(256), 0, c.stream, B,
+                       (const int *)m.rank, m.rec, (const uint64_t *)m.Y, counts,
+                       (const long long *)nullptr, (int *)nullptr, 0LL, hlist,
+                       (const int *)heavy);
     HIP_CHECK(hipGetLastError());
   }
   scan_i32_to_i64(c, counts, offs, N);
@@ -483,167 +622,165 @@ static long strip_sweep(Context &c, long B, long O, const int *rank, const int *
       LaunchTimer t(c, "mbr_strip_write");
       hipLaunchKernelGGL(k_strip_query, dim3(grid_for(N, 256)), dim3(256), 0, c.stream, B, O, g,
                          (const long long *)sOff, (const int *)list, (const uint64_t *)skeys, R,
-                         rank, (const StripRec *)qrec, Y, counts, (const long long *)offs,
-                         pairs, heavy, inl);
+                         (const int *)m.rank, (const SweepRec *)m.rec.aos,
+                         (const uint64_t *)m.Y, counts, (const long long *)offs, pairs, heavy,
+                         inl);
       HIP_CHECK(hipGetLastError());
     }
-    if (nHeavy > 0) {
-      LaunchTimer t(c, "mbr_sweep_write");
-      hipLaunchKernelGGL(k_sweep, dim3(grid_for(nHeavy, 4)), dim3(256), 0, c.stream, B, O, rank,
-                         rec_id, rec_ylo, rec_yhi, Y, counts, (const long long *)offs, pairs,
-                         (const int *)(heavy + 1), (long)nHeavy);
-      HIP_CHECK(hipGetLastError());
-    }
+    LaunchTimer t(c, "mbr_sweep_write");
+    hipLaunchKernelGGL(k_sweep_heavy, dim3(kHeavyBlocks), dim3(256), 0, c.stream, B,
+                       (const int *)m.rank, m.rec, (const uint64_t *)m.Y, counts,
+                       (const long long *)offs, pairs, (long long)K, hlist,
+                       (const int *)heavy);
+    HIP_CHECK(hipGetLastError());
   }
   *pairs_out = pairs;
   return K;
 }
 
-long mbr_filter(Context &c, long B, long O, const uint64_t *bMBR, const uint64_t *oMBR,
-                int **counts_out, int **pairs_out, MbrSortView *sv, const int *bVNum,
-                const int *oVNum) {
-  const long N = B + O, n = 2 * N;
-  if (N <= 0) return 0;
-  uint64_t *keys = (uint64_t *)c.ws.get("mbr_keys", 8 * (size_t)n);
-  int *idx = (int *)c.ws.get("mbr_idx", 4 * (size_t)n);
-  uint64_t *Y = (uint64_t *)c.ws.get("mbr_Y", 8 * (size_t)n);
-  unsigned long long *mm = (unsigned long long *)c.ws.get("mbr_minmax", 40);
-  uint64_t *skeys = (uint64_t *)c.ws.get("mbr_skeys", 8 * (size_t)n);
-  int *perm = (int *)c.ws.get("mbr_perm", 4 * (size_t)n);
-  int *rank = (int *)c.ws.get("mbr_rank", 4 * (size_t)n);
-  int *rec_id = (int *)c.ws.get("mbr_rec_id", 4 * (size_t)n);
-  uint64_t *rec_ylo = (uint64_t *)c.ws.get("mbr_rec_ylo", 8 * (size_t)n);
-  uint64_t *rec_yhi = (uint64_t *)c.ws.get("mbr_rec_yhi", 8 * (size_t)n);
-  int *counts = (int *)c.ws.get("mbr_counts", 4 * (size_t)N);
-  long long *offs = (long long *)c.ws.get("mbr_offs", 8 * (size_t)(N + 1));
-  hipLaunchKernelGGL(k_init_minmax, dim3(1), dim3(64), 0, c.stream, mm);
-  {
-    LaunchTimer t(c, "mbr_endpoints");
-    hipLaunchKernelGGL(k_endpoints, dim3(std::min(grid_for(N, 256), kEndpointBlocks)), dim3(256),
-                       0, c.stream, B, O, bMBR, oMBR, bVNum && oVNum ? bVNum : nullptr, oVNum,
-                       keys, idx, Y, mm);
-    HIP_CHECK(hipGetLastError());
-  }
-  unsigned long long h[5];
-  host_read(c, h, mm, 40);
-  c.avgVerts = bVNum && oVNum ? (double)h[4] / (double)N : -1.0;
-  unsigned long long range = h[1] - h[0];
-  int bits = 0;
-  while (bits < 64 && (range >> bits) != 0) bits++;
-  hipLaunchKernelGGL(k_sub_key, dim3(grid_for(n, 256)), dim3(256), 0, c.stream, keys, n, mm);
-  HIP_CHECK(hipGetLastError());
-  radix_sort_u64(c, keys, idx, skeys, perm, n, bits);
-  {
+// Counts per polygon, their offsets, and the candidate pairs.  With cap <= 0
+// the count is read back and the pairs are sized to it; with cap > 0 the
+// pairs below cap are written without a read-back and the count stays at
+// *kDev, which the caller compares with cap when it reads it.
+static long mbr_candidates(Context &c, MbrOrder &m, long cap, int *counts, long long *offs,
+                           int **pairs_out, const long long **kDev) {
+  const long B = m.B, O = m.O, N = B + O;
+  if (m.strips) {
+    const long K = strip_sweep(c, m, counts, offs, pairs_out);
+    if (K >= 0) return K;
+    // records as arrays for the sweep of every polygon
+    const long n = 2 * N;
+    m.strips = false;
+    m.rec.aos = nullptr;
+    m.rec.id = (int *)c.ws.get("mbr_rec_id", 4 * (size_t)n);
+    m.rec.ylo = (uint64_t *)c.ws.get("mbr_rec_ylo", 8 * (size_t)n);
+    m.rec.yhi = (uint64_t *)c.ws.get("mbr_rec_yhi", 8 * (size_t)n);
     LaunchTimer t(c, "mbr_sweep_prep");
-    hipLaunchKernelGGL(k_sweep_prep, dim3(grid_for(n, 256)), dim3(256), 0, c.stream, perm, n, Y,
-                       rank, rec_id, rec_ylo, rec_yhi);
+    hipLaunchKernelGGL(k_sweep_prep, dim3(grid_for(n, 256)), dim3(256), 0, c.stream,
+                       (const int *)m.perm, n, (const uint64_t *)m.Y, m.rank, m.rec, m.g,
+                       (int *)nullptr);
     HIP_CHECK(hipGetLastError());
   }
-  long K = -1;
-  int *pairs = nullptr;
-  if (N >= c.tune.stripMin)
-    K = strip_sweep(c, B, O, rank, rec_id, rec_ylo, rec_yhi, Y, h[2], h[3], counts, offs, &pairs);
-  if (K < 0) {
-    {
-      LaunchTimer t(c, "mbr_sweep_count");
-      hipLaunchKernelGGL(k_sweep, dim3(grid_for(N, 4)), dim3(256), 0, c.stream, B, O, rank,
-                         rec_id, rec_ylo, rec_yhi, Y, counts, (const long long *)nullptr,
-                         (int *)nullptr, (const int *)nullptr, 0L);
-      HIP_CHECK(hipGetLastError());
-    }
-    scan_i32_to_i64(c, counts, offs, N);
-    K = (long)read_scalar(c, offs + N);
-    pairs = (int *)c.ws.get("mbr_pairs", 8 * (size_t)(K > 0 ? K : 1));
-    if (K > 0) {
-      LaunchTimer t(c, "mbr_sweep_write");
-      hipLaunchKernelGGL(k_sweep, dim3(grid_for(N, 4)), dim3(256), 0, c.stream, B, O, rank,
-                         rec_id, rec_ylo, rec_yhi, Y, counts, (const long long *)offs, pairs,
-                         (const int *)nullptr, 0L);
-      HIP_CHECK(hipGetLastError());
-    }
+  {
+    LaunchTimer t(c, "mbr_sweep_count");
+    hipLaunchKernelGGL(k_sweep, dim3(grid_for(N, 4)), dim3(256), 0, c.stream, B, O,
+                       (const int *)m.rank, m.rec, (const uint64_t *)m.Y, counts,
+                       (const long long *)nullptr, (int *)nullptr, 0LL);
+    HIP_CHECK(hipGetLastError());
   }
-  if (counts_out) *counts_out = counts;
-  if (pairs_out) *pairs_out = pairs;
-  if (sv) {
-    sv->perm = perm;
-    sv->rank = rank;
-    sv->n = n;
-  }
+  const bool fold = m.few && cap > 0;
+  long K = cap;
+  if (!fold) scan_i32_to_i64(c, counts, offs, N);
+  if (cap <= 0) K = (long)read_scalar(c, offs + N);
+  int *pairs = (int *)c.ws.get("mbr_pairs", 8 * (size_t)(K > 0 ? K : 1));
+  *pairs_out = pairs;
+  if (kDev) *kDev = offs + N;
+  if (K <= 0) return K;
+  LaunchTimer t(c, "mbr_sweep_write");
+  if (fold)
+    hipLaunchKernelGGL(k_sweep_write_few, dim3(grid_for(N, 4)), dim3(256), 0, c.stream, B, O,
+                       (const int *)m.rank, m.rec, (const uint64_t *)m.Y, (const int *)counts,
+                       pairs, (long long)K, offs + N);
+  else
+    hipLaunchKernelGGL(k_sweep, dim3(grid_for(N, 4)), dim3(256), 0, c.stream, B, O,
+                       (const int *)m.rank, m.rec, (const uint64_t *)m.Y, counts,
+                       (const long long *)offs, pairs, (long long)K);
+  HIP_CHECK(hipGetLastError());
   return K;
 }
 
-// ------------------------------------------------------------ stage 2 ----
-// zero0..zero2 (optional): per-candidate arrays of the later passes,
-// cleared here rather than by fills of their own
+long mbr_filter(Context &c, long B, long O, const uint64_t *bMBR, const uint64_t *oMBR,
+                int **counts_out, int **pairs_out) {
+  const long N = B + O;
+  if (N <= 0) return 0;
+  MbrOrder m;
+  mbr_order(c, B, O, bMBR, oMBR, nullptr, nullptr, m);
+  *counts_out = (int *)c.ws.get("mbr_counts", 4 * (size_t)N);
+  long long *offs = (long long *)c.ws.get("mbr_offs", 8 * (size_t)(N + 1));
+  return mbr_candidates(c, m, 0, *counts_out, offs, pairs_out, nullptr);
+}
+
+// -------------------------------------------------------- stages 2 to 5 ----
+__device__ __forceinline__ void cmbr_of(const double *bm, const double *om, double *box,
+                                        int &type) {
+  const double x1 = bm[0], x2 = bm[2], y1 = bm[1], y2 = bm[3];
+  const double a1 = om[0], a2 = om[2], b1 = om[1], b2 = om[3];
+  box[0] = a1 > x1 ? a1 : x1;
+  box[1] = b1 > y1 ? b1 : y1;
+  box[2] = a2 < x2 ? a2 : x2;
+  box[3] = b2 < y2 ? b2 : y2;
+  type = x1 == box[0] && x2 == box[2] && y1 == box[1] && y2 == box[3]   ? 1
+         : a1 == box[0] && a2 == box[2] && b1 == box[1] && b2 == box[3] ? 2
+                                                                        : 0;
+}
+
 __global__ void k_get_cmbr(long K, const int *pairs, const double *bMBR2, const double *oMBR2,
-                           double *cmbr, int *pipFlag, signed char *pipType, int *joinFlag,
-                           int *zero0, int *zero1, int *zero2) {
+                           double *cmbr, int *pipFlag, signed char *pipType, int *joinFlag) {
   long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= K) return;
-  if (zero0) {
-    zero0[k] = 0;
-    zero1[k] = 0;
-    zero2[k] = 0;
-  }
-  int b = pairs[2 * k], o = pairs[2 * k + 1];
-  double x1 = bMBR2[4 * b], x2 = bMBR2[4 * b + 2], y1 = bMBR2[4 * b + 1], y2 = bMBR2[4 * b + 3];
-  double a1 = oMBR2[4 * o], a2 = oMBR2[4 * o + 2], b1 = oMBR2[4 * o + 1], b2 = oMBR2[4 * o + 3];
-  double cX1 = a1 > x1 ? a1 : x1, cX2 = a2 < x2 ? a2 : x2;
-  double cY1 = b1 > y1 ? b1 : y1, cY2 = b2 < y2 ? b2 : y2;
-  cmbr[4 * k] = cX1;
-  cmbr[4 * k + 1] = cY1;
-  cmbr[4 * k + 2] = cX2;
-  cmbr[4 * k + 3] = cY2;
+  double box[4];
+  int t;
+  cmbr_of(bMBR2 + 4L * pairs[2 * k], oMBR2 + 4L * pairs[2 * k + 1], box, t);
+  for (int j = 0; j < 4; j++) cmbr[4 * k + j] = box[j];
   joinFlag[k] = 1;
-  int f = 0, t = 0;
-  if (x1 == cX1 && x2 == cX2 && y1 == cY1 && y2 == cY2) {
-    f = 1;
-    t = 1;
-  } else if (a1 == cX1 && a2 == cX2 && b1 == cY1 && b2 == cY2) {
-    f = 1;
-    t = 2;
-  }
-  pipFlag[k] = f;
+  pipFlag[k] = t != 0;
   pipType[k] = (signed char)t;
 }
 
-// ------------------------------------------------------------ stage 3 ----
-__global__ void __launch_bounds__(256)
-    k_pip(long nCand, const int *cand, const int *pairs, const signed char *pipType,
-          const double *bCoords, const long *bVPSNum, const double *oCoords, const long *oVPSNum,
-          int *pipFlag, int *joinFlag, const long long *nDev) {
-  const long w = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (w >= (nDev ? (long)*nDev : nCand)) return;
-  const int lane = __lane_id();
-  const int k = cand[w];
-  const int b = pairs[2 * k], o = pairs[2 * k + 1];
-  const long bS = b > 0 ? bVPSNum[b - 1] : 0, oS = o > 0 ? oVPSNum[o - 1] : 0;
-  double pX, pY;
-  const double *poly;
-  long vNum;
-  if (pipType[k] == 1) {
-    pX = bCoords[2 * bS];
-    pY = bCoords[2 * bS + 1];
-    vNum = oVPSNum[o] - oS;
-    poly = oCoords + 2 * oS;
-  } else {
-    pX = oCoords[2 * oS];
-    pY = oCoords[2 * oS + 1];
-    vNum = bVPSNum[b] - bS;
-    poly = bCoords + 2 * bS;
-  }
+// Groups of G lanes (8, 16 or 64, a wave's aligned parts) take one candidate
+// each; their ballots are masked to the group, so groups of one wave may be
+// at different loop counts.
+template <int G>
+__device__ __forceinline__ unsigned long long group_ballot(bool v) {
+  const unsigned long long m = __ballot(v);
+  if (G == 64) return m;
+  return m & (((1ULL << (G & 63)) - 1ULL) << ((int)__lane_id() & ~(G - 1)));
+}
+
+// crossing parity of the point over the ring, one edge per lane
+template <int G>
+__device__ __forceinline__ int pip_parity(double pX, double pY, const double *poly, long vNum) {
+  const int g = (int)__lane_id() & (G - 1);
   int parity = 0;
-  for (long i0 = 0; i0 < vNum; i0 += 64) {
-    long i = i0 + lane;
+  for (long i0 = 0; i0 < vNum; i0 += G) {
+    long i = i0 + g;
     bool tog = false;
     if (i < vNum) {
       long j = i == 0 ? vNum - 1 : i - 1;
       double X1 = poly[2 * i], Y1 = poly[2 * i + 1], X2 = poly[2 * j], Y2 = poly[2 * j + 1];
       if ((Y1 > pY) != (Y2 > pY)) tog = pX < (X2 - X1) * (pY - Y1) / (Y2 - Y1) + X1;
     }
-    parity ^= __popcll(__ballot(tog)) & 1;
+    parity ^= __popcll(group_ballot<G>(tog)) & 1;
   }
-  if (lane == 0) {
+  return parity;
+}
+
+struct PolyRefs {
+  const double *bCoords, *oCoords;
+  const int *bVNum, *oVNum;
+  const long *bVPSNum, *oVPSNum;
+};
+static PolyRefs poly_refs(const JoinInputs &in) {
+  return PolyRefs{in.bCoords, in.oCoords, in.bVNum, in.oVNum, in.bVPSNum, in.oVPSNum};
+}
+
+// the PiP test of a candidate of type 1 (base in overlay) or 2
+template <int G>
+__device__ __forceinline__ int pip_within(const PolyRefs &p, int b, int o, int type) {
+  const long bS = b > 0 ? p.bVPSNum[b - 1] : 0, oS = o > 0 ? p.oVPSNum[o - 1] : 0;
+  const double *pt = type == 1 ? p.bCoords + 2 * bS : p.oCoords + 2 * oS;
+  return type == 1 ? pip_parity<G>(pt[0], pt[1], p.oCoords + 2 * oS, p.oVPSNum[o] - oS)
+                   : pip_parity<G>(pt[0], pt[1], p.bCoords + 2 * bS, p.bVPSNum[b] - bS);
+}
+
+__global__ void __launch_bounds__(256)
+    k_pip(long nCand, const int *cand, const int *pairs, const signed char *pipType, PolyRefs p,
+          int *pipFlag, int *joinFlag) {
+  const long w = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (w >= nCand) return;
+  const int k = cand[w];
+  const int parity = pip_within<64>(p, pairs[2 * k], pairs[2 * k + 1], pipType[k]);
+  if (__lane_id() == 0) {
     pipFlag[k] = parity;
     if (parity == 1) joinFlag[k] = 0;
   }
@@ -665,61 +802,66 @@ __device__ __forceinline__ bool cmf_edge(const double *c, int vNum, int i, doubl
   return true;
 }
 
-__device__ __forceinline__ long long list_base(const long long *off, int k, bool inclusive) {
-  return inclusive ? (k > 0 ? off[k - 1] : 0) : off[k];
+// The edges of one ring that the box keeps, counted and, when asked for,
+// listed in ring order: out[0..] in global memory and the first kSegList of
+// them in lds.
+constexpr int kSegList = 64;
+template <typename EdgeT, int G>
+__device__ __forceinline__ int cmf_ring(const double *c, int vNum, const double *box, EdgeT *out,
+                                        int *lds) {
+  const int lane = __lane_id(), g = lane & (G - 1);
+  int n = 0;
+  for (int i0 = 0; i0 < vNum; i0 += G) {
+    const int i = i0 + g;
+    const bool ok = i < vNum && cmf_edge(c, vNum, i, box[0], box[1], box[2], box[3]);
+    const unsigned long long m = group_ballot<G>(ok);
+    if (out && ok) {
+      const int p = n + __popcll(m & ((1ULL << lane) - 1ULL));
+      out[p] = (EdgeT)i;
+      if (lds && p < kSegList) lds[p] = i;
+    }
+    n += __popcll(m);
+  }
+  return n;
 }
 
-// polygons of at most this many vertices on average take the 16-lane CMF
-constexpr double kCmfSmall = 32.0;
+__device__ __forceinline__ const double *ring_of(const double *c, const long *vps, int k) {
+  return c + 2 * (k > 0 ? vps[k - 1] : 0);
+}
 
-// count mode (bEdge == nullptr): counts and clears joinFlag when a side has
-// no edge; apply mode: writes the ordered edge lists at the pair offsets
-// (exclusive offsets, or the reference's inclusive prefix when inclusive).
-// One group of G lanes per pair (G = 16: four pairs per wave, for layers of
-// small polygons; G = 64: one wave per pair); ballots are masked to the
-// group, whose edges are ranked in ring order.
-template <typename EdgeT, int G>
+// the reference's two passes, one wave per listed pair: counts (and clears
+// joinFlag when a side has no edge) ...
 __global__ void __launch_bounds__(256)
-    k_cmf(long nList, const int *list, const int *pairs, const double *cmbr,
-          const double *bCoords, const int *bVNum, const long *bVPSNum, const double *oCoords,
-          const int *oVNum, const long *oVPSNum, int *joinFlag, int *bCount, int *oCount,
-          const long long *bOff, const long long *oOff, EdgeT *bEdge, EdgeT *oEdge,
-          bool inclusive, const long long *nDev) {
-  const long w = (long)blockIdx.x * (256 / G) + (threadIdx.x / G);
-  if (w >= (nDev ? (long)*nDev : nList)) return;
-  const int lane = __lane_id(), g = lane & (G - 1);
-  const unsigned long long gm = G == 64 ? ~0ULL : (((1ULL << G) - 1ULL) << (lane & ~(G - 1)));
-  const int k = list[w];
-  const int b = pairs[2 * k], o = pairs[2 * k + 1];
-  const double cX1 = cmbr[4 * k], cY1 = cmbr[4 * k + 1], cX2 = cmbr[4 * k + 2],
-               cY2 = cmbr[4 * k + 3];
-  int cnt[2];
-  for (int side = 0; side < 2; side++) {
-    const double *c = side == 0 ? bCoords + 2 * (b > 0 ? bVPSNum[b - 1] : 0)
-                                : oCoords + 2 * (o > 0 ? oVPSNum[o - 1] : 0);
-    const int vNum = side == 0 ? bVNum[b] : oVNum[o];
-    EdgeT *outE = side == 0 ? bEdge : oEdge;
-    long long pos = bEdge ? list_base(side == 0 ? bOff : oOff, k, inclusive) : 0;
-    int n = 0;
-    for (int i0 = 0; i0 < vNum; i0 += G) {
-      int i = i0 + g;
-      bool ok = i < vNum && cmf_edge(c, vNum, i, cX1, cY1, cX2, cY2);
-      unsigned long long m = __ballot(ok) & gm;
-      if (outE && ok) outE[pos + n + __popcll(m & ((1ULL << lane) - 1ULL))] = (EdgeT)i;
-      n += __popcll(m);
-    }
-    cnt[side] = n;
-  }
-  if (!bEdge && g == 0) {
-    if (cnt[0] == 0 || cnt[1] == 0) {
-      joinFlag[k] = 0;
-      bCount[k] = 0;
-      oCount[k] = 0;
-    } else {
-      bCount[k] = cnt[0];
-      oCount[k] = cnt[1];
-    }
-  }
+    k_cmf_count(long nList, const int *list, const int *pairs, const double *cmbr, PolyRefs p,
+                int *joinFlag, int *bCount, int *oCount) {
+  const long w = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (w >= nList) return;
+  const int k = list[w], b = pairs[2 * k], o = pairs[2 * k + 1];
+  const int nb = cmf_ring<int, 64>(ring_of(p.bCoords, p.bVPSNum, b), p.bVNum[b], cmbr + 4L * k,
+                                   nullptr, nullptr);
+  const int no = cmf_ring<int, 64>(ring_of(p.oCoords, p.oVPSNum, o), p.oVNum[o], cmbr + 4L * k,
+                                   nullptr, nullptr);
+  if (__lane_id() != 0) return;
+  const bool keep = nb && no;
+  if (!keep) joinFlag[k] = 0;
+  bCount[k] = keep ? nb : 0;
+  oCount[k] = keep ? no : 0;
+}
+
+// ... and writes the 16-bit edge lists at its inclusive prefix
+__device__ __forceinline__ long long incl_base(const long long *off, int k) {
+  return k > 0 ? off[k - 1] : 0;
+}
+__global__ void __launch_bounds__(256)
+    k_cmf_apply(long nList, const int *list, const int *pairs, const double *cmbr, PolyRefs p,
+                const long long *bIncl, const long long *oIncl, short *bEdge, short *oEdge) {
+  const long w = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (w >= nList) return;
+  const int k = list[w], b = pairs[2 * k], o = pairs[2 * k + 1];
+  cmf_ring<short, 64>(ring_of(p.bCoords, p.bVPSNum, b), p.bVNum[b], cmbr + 4L * k,
+                      bEdge + incl_base(bIncl, k), nullptr);
+  cmf_ring<short, 64>(ring_of(p.oCoords, p.oVPSNum, o), p.oVNum[o], cmbr + 4L * k,
+                      oEdge + incl_base(oIncl, k), nullptr);
 }
 
 // ------------------------------------------------------------ stage 5 ----
@@ -775,67 +917,52 @@ __device__ __forceinline__ int seg_stride(int bE) {
   return S;
 }
 
-// counts come from bCount/oCount, or (when null) from the offsets; the flag
-// goes to segFlag[k] or, with flagByList, to segFlag[w] (the reference's
-// per-survivor layout).
-template <typename EdgeT>
-__global__ void __launch_bounds__(256)
-    k_segjoin(long nList, const int *list, const int *pairs, const double *bCoords,
-              const long *bVPSNum, const double *oCoords, const long *oVPSNum, const int *bCount,
-              const int *oCount, const long long *bOff, const long long *oOff,
-              const EdgeT *bEdge, const EdgeT *oEdge, int *segFlag, bool inclusive,
-              bool flagByList, const long long *nDev) {
-  const long w = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (w >= (nDev ? (long)*nDev : nList)) return;
-  const int lane = __lane_id();
-  const int k = list[w];
-  const int b = pairs[2 * k], o = pairs[2 * k + 1];
-  const long bBase = b > 0 ? bVPSNum[b - 1] : 0, oBase = o > 0 ? oVPSNum[o - 1] : 0;
-  const int bV = (int)(bVPSNum[b] - bBase), oV = (int)(oVPSNum[o] - oBase);
-  const long long b0 = list_base(bOff, k, inclusive), o0 = list_base(oOff, k, inclusive);
-  const int bE = bCount ? bCount[k] : (int)(bOff[k] - b0);
-  const int oE = oCount ? oCount[k] : (int)(oOff[k] - o0);
-  const EdgeT *be = bEdge + b0, *oe = oEdge + o0;
-  const double *bc = bCoords + 2 * bBase, *oc = oCoords + 2 * oBase;
+// Whether some pair of the two edge lists (bAt(i), oAt(j): ring positions)
+// hits, over a group of G lanes.
+template <int G, typename FB, typename FO>
+__device__ __forceinline__ int seg_any(const double *bc, int bV, const double *oc, int oV, int bE,
+                                       int oE, FB bAt, FO oAt) {
+  const int lane = (int)__lane_id() & (G - 1);
+  // pairs per lane a round: a small group's few pairs fill one
+  constexpr int U = G == 64 ? kSegStage : 1;
   const long long total = (long long)bE * oE;
   int flag = 0;
-  // edge pair t's four vertices; false when the base edge is degenerate
-  auto pair_at = [&](long long t, double *v) {
-    const int bi = be[t / oE], oi = oe[t % oE];
-    const int b2 = bi < bV - 1 ? bi + 1 : 0, o2 = oi < oV - 1 ? oi + 1 : 0;
-    v[0] = bc[2 * bi], v[1] = bc[2 * bi + 1], v[2] = bc[2 * b2], v[3] = bc[2 * b2 + 1];
-    v[4] = oc[2 * oi], v[5] = oc[2 * oi + 1], v[6] = oc[2 * o2], v[7] = oc[2 * o2 + 1];
-    return !(v[0] == v[2] && v[1] == v[3]);
-  };
   if (total >= 0x7fffffffLL) {
     // lists of 2^31 pairs or more (rings of tens of thousands of listed
     // edges): one pair per lane a round, 64-bit indices
-    for (long long t0 = 0; t0 < total && !flag; t0 += 64) {
+    for (long long t0 = 0; t0 < total && !flag; t0 += G) {
       const long long t = t0 + lane;
-      double v[8];
-      const bool hit = t < total && pair_at(t, v) &&
-                       seg_hit(v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]);
-      flag = __ballot(hit) != 0ULL;
+      bool hit = false;
+      if (t < total) {
+        const int bi = bAt((int)(t / oE)), oi = oAt((int)(t % oE));
+        const int b2 = bi < bV - 1 ? bi + 1 : 0, o2 = oi < oV - 1 ? oi + 1 : 0;
+        const double v0 = bc[2 * bi], v1 = bc[2 * bi + 1], v2 = bc[2 * b2], v3 = bc[2 * b2 + 1];
+        hit = !(v0 == v2 && v1 == v3) && seg_hit(v0, v1, v2, v3, oc[2 * oi], oc[2 * oi + 1],
+                                                 oc[2 * o2], oc[2 * o2 + 1]);
+      }
+      flag = group_ballot<G>(hit) != 0ULL;
     }
-    if (lane == 0) segFlag[flagByList ? w : k] = flag;
-    return;
+    return flag;
   }
-  // kSegStage edge pairs per lane a round, all their loads issued before
+  // U edge pairs per lane a round, all their loads issued before
   // the tests; the flag is "some pair hits", which testing pairs past the
   // first hit cannot change
   const unsigned tot = (unsigned)total, uoE = (unsigned)(oE > 0 ? oE : 1);
-  const unsigned long long S = (unsigned long long)seg_stride(bE);
-  for (unsigned t0 = 0; t0 < tot && !flag; t0 += 64 * kSegStage) {
-    int bi[kSegStage], oi[kSegStage];
+  const unsigned long long S = (unsigned long long)(tot > G * U ? seg_stride(bE) : 1);
+  for (unsigned t0 = 0; t0 < tot && !flag; t0 += G * U) {
+    int bi[U], oi[U];
 #pragma unroll
-    for (int u = 0; u < kSegStage; u++) {
-      const unsigned t = t0 + 64 * u + lane;
-      bi[u] = t < tot ? (int)be[(unsigned)((t / uoE) * S % (unsigned long long)bE)] : -1;
-      oi[u] = t < tot ? (int)oe[t % uoE] : -1;
+    for (int u = 0; u < U; u++) {
+      const unsigned t = t0 + G * u + lane;
+      bi[u] = oi[u] = -1;
+      if (t >= tot) continue;
+      const unsigned q = t / uoE;
+      bi[u] = bAt(S == 1 ? (int)q : (int)(q * S % (unsigned long long)bE));
+      oi[u] = oAt((int)(t - q * uoE));
     }
-    double s[kSegStage][8];
+    double s[U][8];
 #pragma unroll
-    for (int u = 0; u < kSegStage; u++) {
+    for (int u = 0; u < U; u++) {
       if (bi[u] < 0) continue;
       const int b2 = bi[u] < bV - 1 ? bi[u] + 1 : 0, o2 = oi[u] < oV - 1 ? oi[u] + 1 : 0;
       s[u][0] = bc[2 * bi[u]];
@@ -849,129 +976,428 @@ __global__ void __launch_bounds__(256)
     }
     bool hit = false;
 #pragma unroll
-    for (int u = 0; u < kSegStage; u++) {
+    for (int u = 0; u < U; u++) {
       if (bi[u] < 0) continue;
       if (!(s[u][0] == s[u][2] && s[u][1] == s[u][3]))
         hit |= seg_hit(s[u][0], s[u][1], s[u][2], s[u][3], s[u][4], s[u][5], s[u][6], s[u][7]);
     }
-    flag = __ballot(hit) != 0ULL;
+    flag = group_ballot<G>(hit) != 0ULL;
   }
-  if (lane == 0) segFlag[flagByList ? w : k] = flag;
+  return flag;
 }
 
-__global__ void k_join_final(long K, const int *pipFlag, const int *segFlag, int *joined) {
-  long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < K) joined[k] = (pipFlag[k] == 1 || segFlag[k] == 1) ? 1 : 0;
+// the reference's refine: one wave per listed pair over 16-bit lists at the
+// inclusive prefixes, the flag by list position
+__global__ void __launch_bounds__(256)
+    k_segjoin(long nList, const int *list, const int *pairs, PolyRefs p, const long long *bIncl,
+              const long long *oIncl, const short *bEdge, const short *oEdge, int *flagByList) {
+  const long w = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (w >= nList) return;
+  const int k = list[w], b = pairs[2 * k], o = pairs[2 * k + 1];
+  const long bS = b > 0 ? p.bVPSNum[b - 1] : 0, oS = o > 0 ? p.oVPSNum[o - 1] : 0;
+  const long long b0 = incl_base(bIncl, k), o0 = incl_base(oIncl, k);
+  const short *be = bEdge + b0, *oe = oEdge + o0;
+  const int flag = seg_any<64>(
+      p.bCoords + 2 * bS, (int)(p.bVPSNum[b] - bS), p.oCoords + 2 * oS, (int)(p.oVPSNum[o] - oS),
+      (int)(bIncl[k] - b0), (int)(oIncl[k] - o0), [&](int i) { return (int)be[i]; },
+      [&](int i) { return (int)oe[i]; });
+  if (__lane_id() == 0) flagByList[w] = flag;
 }
 
-__global__ void k_gather_pairs(long n, const int *idx, const int *pairs, int *out) {
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  int k = idx[i];
-  out[2 * i] = pairs[2 * k];
-  out[2 * i + 1] = pairs[2 * k + 1];
+// ------------------------------------------------- stages 2 to 5, fused ----
+// A candidate goes through CMBR, PiP and the CMF count in one pass by one
+// group of lanes (k_refine_count) and, once the edge lists have their places,
+// through the CMF lists and the segment test in a second one
+// (k_refine_apply), its short edge lists in LDS between the two.  For 550 000
+// polygons of 8 vertices on one MI355X the stages as passes of their own over
+// compacted lists, one wave per pair in the segment test, took 600 us of
+// kernel time in 13 launches: that test alone 331 us with 64 lanes on about
+// nine edge pairs.  The two passes take 88 and 131 us, and 110 and 170 with 16
+// lanes per candidate instead of 8.  What bounds both now is the chain of
+// dependent loads (pair, ring bounds, vertices); groups of 8 lanes keep eight
+// chains per wave in flight.
+//
+// n is the length of the per-candidate arrays; the candidates are *kDev of
+// them (all n without it), and none is touched when *kDev exceeds n.
+struct RefineOut {
+  double *cmbr;
+  int *pipFlag, *joinFlag, *bCount, *oCount, *segFlag, *joined;
+  signed char *pipType;
+};
+
+template <int G>
+__global__ void __launch_bounds__(256)
+    k_refine_count(long n, const long long *kDev, const int *pairs, PolyRefs p,
+                   const double *bMBR2, const double *oMBR2, RefineOut r) {
+  const long K = kDev ? (long)*kDev : n;
+  if (K > n) return;
+  const int g = (int)__lane_id() & (G - 1);
+  const long step = (long)gridDim.x * (256 / G);
+  for (long k = (long)blockIdx.x * (256 / G) + threadIdx.x / G; k < n; k += step) {
+    if (k >= K) {  // past the candidates: the scans' inputs
+      if (g == 0) r.bCount[k] = r.oCount[k] = r.joined[k] = 0;
+      continue;
+    }
+    const int b = pairs[2 * k], o = pairs[2 * k + 1];
+    double box[4];
+    int type;
+    cmbr_of(bMBR2 + 4L * b, oMBR2 + 4L * o, box, type);
+    const int within = type ? pip_within<G>(p, b, o, type) : 0;
+    int nb = 0, no = 0;
+    if (!within) {
+      nb = cmf_ring<int, G>(ring_of(p.bCoords, p.bVPSNum, b), p.bVNum[b], box, nullptr, nullptr);
+      if (nb)
+        no = cmf_ring<int, G>(ring_of(p.oCoords, p.oVPSNum, o), p.oVNum[o], box, nullptr,
+                              nullptr);
+    }
+    const bool keep = nb && no;
+    if (g < 4) r.cmbr[4 * k + g] = g == 0 ? box[0] : g == 1 ? box[1] : g == 2 ? box[2] : box[3];
+    if (g == 0) {
+      r.pipFlag[k] = within;
+      r.pipType[k] = (signed char)type;
+      r.joinFlag[k] = keep;
+      r.bCount[k] = keep ? nb : 0;
+      r.oCount[k] = keep ? no : 0;
+      r.segFlag[k] = 0;
+      r.joined[k] = within;
+    }
+  }
 }
 
-void join_refine(Context &c, const JoinInputs &in, long K, const int *pairs, JoinRefine &r) {
-  r.K = K;
-  long Kc = K > 0 ? K : 1;
-  r.cmbr = (double *)c.ws.get("jr_cmbr", 32 * (size_t)Kc);
-  r.pipFlag = (int *)c.ws.get("jr_pipFlag", 4 * (size_t)Kc);
-  r.pipType = (signed char *)c.ws.get("jr_pipType", (size_t)Kc);
-  r.joinFlag = (int *)c.ws.get("jr_joinFlag", 4 * (size_t)Kc);
-  r.pipCand = (int *)c.ws.get("jr_pipCand", 4 * (size_t)Kc);
-  r.bCount = (int *)c.ws.get("jr_bCount", 4 * (size_t)Kc);
-  r.oCount = (int *)c.ws.get("jr_oCount", 4 * (size_t)Kc);
-  r.bOff = (long long *)c.ws.get("jr_bOff", 8 * (size_t)(Kc + 1));
-  r.oOff = (long long *)c.ws.get("jr_oOff", 8 * (size_t)(Kc + 1));
-  r.segFlag = (int *)c.ws.get("jr_segFlag", 4 * (size_t)Kc);
-  r.list = (int *)c.ws.get("jr_list", 4 * (size_t)Kc);
-  r.joined = (int *)c.ws.get("jr_joined", 4 * (size_t)Kc);
-  if (K <= 0) {
-    r.pipNum = r.within = r.cmfCand = r.E = r.hits = r.nJoined = 0;
-    r.joinedPairs = (int *)c.ws.get("jr_joinedPairs", 8);
-    return;
+// FOLD (small calls): each block takes a run of candidates and sums the
+// counts before it itself, in place of a scan launch, and writes the offsets.
+// A list that would end beyond capB or capO is not written: the totals tell.
+template <int G, bool FOLD>
+__global__ void __launch_bounds__(256)
+    k_refine_apply(long n, const long long *kDev, const int *pairs, PolyRefs p, RefineOut r,
+                   long long *bOff, long long *oOff, int *bEdge, int *oEdge, long long capB,
+                   long long capO) {
+  constexpr int per = 256 / G;
+  __shared__ int lists[per][2][kSegList];
+  __shared__ long long lds[4];
+  const long K = kDev ? (long)*kDev : n;
+  if (K > n) return;
+  const int g = (int)__lane_id() & (G - 1), grp = threadIdx.x / G;
+  int *lb = lists[grp][0], *lo = lists[grp][1];
+  long k0 = (long)blockIdx.x * per, k1 = K, step = (long)gridDim.x * per, run = 0;
+  long long sb = 0, so = 0;
+  if (FOLD) {
+    run = (K + (long)gridDim.x * per - 1) / ((long)gridDim.x * per) * per;
+    k0 = (long)blockIdx.x * run;
+    k1 = k0 + run < K ? k0 + run : K;
+    step = per;
+    if (k0 >= K && !(blockIdx.x == 0 && K == 0)) return;
+    for (long j = threadIdx.x; j < k0; j += 256) {
+      sb += r.bCount[j];
+      so += r.oCount[j];
+    }
+    sb = block_sum256(sb, lds);
+    so = block_sum256(so, lds);
+    if (threadIdx.x == 0 && k1 == K) {
+      long long tb = sb, to = so;
+      for (long j = k0; j < K; j++) {
+        tb += r.bCount[j];
+        to += r.oCount[j];
+      }
+      bOff[K] = tb;
+      oOff[K] = to;
+    }
   }
+  for (long k = k0 + grp, prev = k0; k < k1; k += step) {
+    long long pb, po;
+    if (FOLD) {
+      for (; prev < k; prev++) {
+        sb += r.bCount[prev];
+        so += r.oCount[prev];
+      }
+      pb = sb;
+      po = so;
+      if (g == 0) {
+        bOff[k] = pb;
+        oOff[k] = po;
+      }
+    } else {
+      pb = bOff[k];
+      po = oOff[k];
+    }
+    if (!r.joinFlag[k]) continue;
+    const int bE = r.bCount[k], oE = r.oCount[k];
+    if (pb + bE > capB || po + oE > capO) continue;
+    const int b = pairs[2 * k], o = pairs[2 * k + 1];
+    const double *bc = ring_of(p.bCoords, p.bVPSNum, b), *oc = ring_of(p.oCoords, p.oVPSNum, o);
+    const int bV = (int)(p.bVPSNum[b] - (b > 0 ? p.bVPSNum[b - 1] : 0)),
+              oV = (int)(p.oVPSNum[o] - (o > 0 ? p.oVPSNum[o - 1] : 0));
+    double box[4];
+    for (int j = 0; j < 4; j++) box[j] = r.cmbr[4 * k + j];
+    int *be = bEdge + pb, *oe = oEdge + po;
+    __threadfence_block();  // the last candidate's list reads, before the writes
+    cmf_ring<int, G>(bc, p.bVNum[b], box, be, lb);
+    cmf_ring<int, G>(oc, p.oVNum[o], box, oe, lo);
+    __threadfence_block();  // the lists, before other lanes read them
+    const int flag =
+        bE <= kSegList && oE <= kSegList
+            ? seg_any<G>(bc, bV, oc, oV, bE, oE, [&](int i) { return lb[i]; },
+                         [&](int i) { return lo[i]; })
+            : seg_any<G>(bc, bV, oc, oV, bE, oE, [&](int i) { return be[i]; },
+                         [&](int i) { return oe[i]; });
+    if (g == 0 && flag) {
+      r.segFlag[k] = 1;
+      r.joined[k] = 1;
+    }
+  }
+}
+
+// What a join reads back: candidates, edges listed on either side, PiP
+// candidates, within, CMF survivors and intersecting pairs.
+constexpr int kJoinStats = 7;
+
+// The end of a small call in one block: the joined pairs in order and the
+// read-back values.  Rounds of four candidates per thread.
+__global__ void __launch_bounds__(1024)
+    k_refine_out_few(long n, const long long *kDev, const int *pairs, RefineOut r,
+                     const long long *bOff, const long long *oOff, long long capB, long long capO,
+                     int *jidx, int *jpairs, long long *st, long long *slots,
+                     const long long *lbErr) {
+  __shared__ int lds[16];
+  __shared__ long long lds64[16];
+  const long K = (long)*kDev;
+  long long acc = 0;  // PiP candidates, within, survivors, hits: 16 bits each (n <= 2^15)
+  const bool fits = K <= n && bOff[K] <= capB && oOff[K] <= capO;
+  int base = 0;
+  for (long k0 = 0; fits && k0 < K; k0 += 4096) {
+    int f[4], c = 0;
+    for (int u = 0; u < 4; u++) {
+      const long k = k0 + 4 * threadIdx.x + u;
+      f[u] = k < K ? r.joined[k] : 0;
+      c += f[u];
+      if (k < K)
+        acc += (r.pipType[k] != 0) + ((long long)(r.pipFlag[k] == 1) << 16) +
+               ((long long)(r.joinFlag[k] != 0) << 32) + ((long long)(r.segFlag[k] != 0) << 48);
+    }
+    int tot;
+    int at = base + block_excl_scan<int>(c, lds, tot);
+    for (int u = 0; u < 4; u++) {
+      if (!f[u]) continue;
+      const long k = k0 + 4 * threadIdx.x + u;
+      jidx[at] = (int)k;
+      jpairs[2 * at] = pairs[2 * k];
+      jpairs[2 * at + 1] = pairs[2 * k + 1];
+      at++;
+    }
+    base += tot;
+  }
+  long long all;
+  block_excl_scan<long long>(acc, lds64, all);
+  if (threadIdx.x != 0) return;
+  long long v[kJoinStats] = {K, K <= n ? bOff[K] : 0, K <= n ? oOff[K] : 0};
+  for (int i = 0; i < 4; i++) v[3 + i] = (all >> (16 * i)) & 0xffff;
+  for (int i = 0; i < kJoinStats; i++) st[i] = v[i];
+  put_slots(slots, v, kJoinStats, lbErr);
+}
+
+// The same end in two launches: the pairs of the compacted list and each
+// block's counts, then their sums.
+constexpr unsigned kOutBlocks = 512;
+__global__ void __launch_bounds__(256)
+    k_refine_out(long n, const long long *kDev, const int *pairs, RefineOut r, const int *jidx,
+                 const long long *nJoined, int *jpairs, long long *part) {
+  __shared__ long long lds[4];
+  const long K = kDev ? (long)*kDev : n;
+  long long c[4] = {0, 0, 0, 0};
+  if (K <= n) {
+    const long nj = (long)*nJoined, step = (long)gridDim.x * 256;
+    for (long k = (long)blockIdx.x * 256 + threadIdx.x; k < K; k += step) {
+      if (k < nj) {
+        const int j = jidx[k];
+        jpairs[2 * k] = pairs[2 * j];
+        jpairs[2 * k + 1] = pairs[2 * j + 1];
+      }
+      c[0] += r.pipType[k] != 0;
+      c[1] += r.pipFlag[k] == 1;
+      c[2] += r.joinFlag[k] != 0;
+      c[3] += r.segFlag[k] != 0;
+    }
+  }
+  for (int i = 0; i < 4; i++) {
+    const long long s = block_sum256(c[i], lds);
+    if (threadIdx.x == 0) part[4 * blockIdx.x + i] = s;
+  }
+}
+__global__ void __launch_bounds__(256)
+    k_refine_stats(long n, const long long *kDev, const long long *bOff, const long long *oOff,
+                   const long long *part, int nPart, long long *st, long long *slots,
+                   const long long *lbErr) {
+  __shared__ long long lds[4];
+  long long v[kJoinStats];
+  for (int i = 0; i < 4; i++) {
+    long long s = 0;
+    for (int j = threadIdx.x; j < nPart; j += 256) s += part[4 * j + i];
+    v[3 + i] = block_sum256(s, lds);
+  }
+  if (threadIdx.x != 0) return;
+  v[0] = kDev ? *kDev : n;
+  v[1] = bOff[n];
+  v[2] = oOff[n];
+  for (int i = 0; i < kJoinStats; i++) st[i] = v[i];
+  put_slots(slots, v, kJoinStats, lbErr);
+}
+
+// polygons of at most this many vertices on average take groups of 16 lanes
+// (one group per candidate, eight per wave, of at most kCmfTiny)
+constexpr double kCmfSmall = 32.0, kCmfTiny = 12.0;
+constexpr long long kEdgeGuess = 1LL << 26;
+
+// Stages 2 to 5 over n candidate places, *kDev of them candidates (null: all
+// n).  Returns false, nothing else valid, when there are more than n.
+static bool refine(Context &c, const JoinInputs &in, long n, const long long *kDev, bool few,
+                   double avg, const int *pairs, JoinRefine &r) {
+  const size_t n1 = (size_t)std::max(n, 1L);
+  r.cmbr = (double *)c.ws.get("jr_cmbr", 32 * n1);
+  r.pipFlag = (int *)c.ws.get("jr_pipFlag", 4 * n1);
+  r.pipType = (signed char *)c.ws.get("jr_pipType", n1);
+  r.joinFlag = (int *)c.ws.get("jr_joinFlag", 4 * n1);
+  r.bCount = (int *)c.ws.get("jr_bCount", 4 * n1);
+  r.oCount = (int *)c.ws.get("jr_oCount", 4 * n1);
+  long long *bOff = (long long *)c.ws.get("jr_bOff", 8 * (n1 + 1));
+  long long *oOff = (long long *)c.ws.get("jr_oOff", 8 * (n1 + 1));
+  r.segFlag = (int *)c.ws.get("jr_segFlag", 4 * n1);
+  int *joined = (int *)c.ws.get("jr_joined", 4 * n1);
+  int *jidx = (int *)c.ws.get("jr_joined_idx", 4 * n1);
+  r.joinedPairs = (int *)c.ws.get("jr_joinedPairs", 8 * n1);
+  r.K = r.pipNum = r.within = r.cmfCand = r.E = r.hits = r.nJoined = 0;
+  r.nbEdges = r.noEdges = 0;
+  if (n <= 0) return true;
+  const PolyRefs p = poly_refs(in);
+  const RefineOut o{r.cmbr,   r.pipFlag, r.joinFlag, r.bCount,
+                    r.oCount, r.segFlag, joined,     r.pipType};
+  long long *st = (long long *)c.ws.get("jr_stats", 8 * kJoinStats);
+  // Edge lists are given a place before their lengths are known: the polygons'
+  // mean vertex count per candidate, within 8 to 32.  Totals beyond that (or
+  // beyond what an earlier call left) cost the second pass again; above
+  // kEdgeGuess places the totals are read first.
+  const long long est = n * (avg < 0 ? 32 : (long long)std::min(std::max(avg, 8.0), 32.0));
+  auto cap_of = [&](const char *name) {
+    const long long have = c.replay ? 0 : (long long)(c.ws.slots[name].bytes / 4);
+    return std::max(est, have);
+  };
+  long long capB = cap_of("jr_bEdge"), capO = cap_of("jr_oEdge");
+  // four candidates per wave where the layers' polygons are small on average;
+  // a small call has waves to spare
+  const int G = c.tune.cmfGroup         ? c.tune.cmfGroup
+                : few || avg < 0        ? 64
+                : avg <= kCmfTiny       ? 8
+                : avg <= kCmfSmall      ? 16
+                                        : 64;
+  const int per = 256 / G;
+  // known counts: a group per candidate; else at most four times the waves
+  // that the GPU holds, as most places are empty
+  const unsigned full = 32u * (unsigned)c.cu_count;
+  const unsigned grid = kDev ? std::min(grid_for(n, per), full) : grid_for(n, per);
   {
-    LaunchTimer t(c, "get_cmbr");
-    hipLaunchKernelGGL(k_get_cmbr, dim3(grid_for(K, 256)), dim3(256), 0, c.stream, K, pairs,
-                       in.bMBR2, in.oMBR2, r.cmbr, r.pipFlag, r.pipType, r.joinFlag, r.bCount,
-                       r.oCount, r.segFlag);
+    LaunchTimer t(c, "refine_count");
+    auto kern = G == 8 ? k_refine_count<8> : G == 16 ? k_refine_count<16> : k_refine_count<64>;
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, c.stream, n, kDev, pairs, p, in.bMBR2,
+                       in.oMBR2, o);
     HIP_CHECK(hipGetLastError());
   }
-  // list sizes stay on the device (grids are sized by K); they come back in
-  // one read at the end
-  const long long *pipN = compact_flags_dev(c, r.pipFlag, K, r.pipCand, "pip");
-  {
-    LaunchTimer t(c, "pip");
-    hipLaunchKernelGGL(k_pip, dim3(grid_for(K, 4)), dim3(256), 0, c.stream, K, r.pipCand, pairs,
-                       r.pipType, in.bCoords, in.bVPSNum, in.oCoords, in.oVPSNum, r.pipFlag,
-                       r.joinFlag, pipN);
-    HIP_CHECK(hipGetLastError());
+  if (!few) scan_i32_to_i64_multi(c, {{r.bCount, bOff, n}, {r.oCount, oOff, n}});
+  if (!kDev && est > kEdgeGuess) {
+    long long tot[kHostSlots];
+    read_scalars(c, {bOff + n, oOff + n}, tot);
+    capB = std::max(tot[0], 1LL);
+    capO = std::max(tot[1], 1LL);
   }
-  // within count = number of pipFlag==1 after the test (bCount, oCount and
-  // segFlag were cleared by k_get_cmbr)
-  const long long *withinN = compact_flags_dev(c, r.pipFlag, K, r.list, "within");
-  const long long *cmfN = compact_flags_dev(c, r.joinFlag, K, r.list, "cmf");
-  // four pairs per wave where the layers' polygons are small on average
-  const bool cmf16 = c.tune.cmfGroup == 16 ||
-                     (c.tune.cmfGroup == 0 && c.avgVerts >= 0 && c.avgVerts <= kCmfSmall);
-  const int cmfPer = cmf16 ? 16 : 4;
-  {
-    LaunchTimer t(c, "cmf_count");
-    hipLaunchKernelGGL((cmf16 ? k_cmf<int, 16> : k_cmf<int, 64>), dim3(grid_for(K, cmfPer)),
-                       dim3(256), 0, c.stream, K, r.list,
-                       pairs, r.cmbr, in.bCoords, in.bVNum, in.bVPSNum, in.oCoords, in.oVNum,
-                       in.oVPSNum, r.joinFlag, r.bCount, r.oCount, (const long long *)nullptr,
-                       (const long long *)nullptr, (int *)nullptr, (int *)nullptr, false, cmfN);
-    HIP_CHECK(hipGetLastError());
+  for (;;) {
+    r.bEdge = (int *)c.ws.get("jr_bEdge", 4 * (size_t)capB);
+    r.oEdge = (int *)c.ws.get("jr_oEdge", 4 * (size_t)capO);
+    {
+      LaunchTimer t(c, "refine_apply");
+      auto kern = few       ? (G == 16 ? k_refine_apply<16, true> : k_refine_apply<64, true>)
+                  : G == 8  ? k_refine_apply<8, false>
+                  : G == 16 ? k_refine_apply<16, false>
+                            : k_refine_apply<64, false>;
+      hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, c.stream, n, kDev, pairs, p, o, bOff,
+                         oOff, r.bEdge, r.oEdge, capB, capO);
+      HIP_CHECK(hipGetLastError());
+    }
+    if (few) {
+      hipLaunchKernelGGL(k_refine_out_few, dim3(1), dim3(1024), 0, c.stream, n, kDev, pairs, o,
+                         (const long long *)bOff, (const long long *)oOff, capB, capO, jidx,
+                         r.joinedPairs, st, slots_begin(c), (const long long *)c.lb_err);
+      HIP_CHECK(hipGetLastError());
+    } else {
+      const long long *nj = compact_flags_dev(c, joined, n, jidx, "joined");
+      long long *part = (long long *)c.ws.get("jr_stats_part", 32 * (size_t)kOutBlocks);
+      const unsigned ob = std::min(grid_for(n, 256), kOutBlocks);
+      hipLaunchKernelGGL(k_refine_out, dim3(ob), dim3(256), 0, c.stream, n, kDev, pairs, o,
+                         (const int *)jidx, nj, r.joinedPairs, part);
+      HIP_CHECK(hipGetLastError());
+      hipLaunchKernelGGL(k_refine_stats, dim3(1), dim3(256), 0, c.stream, n, kDev,
+                         (const long long *)bOff, (const long long *)oOff,
+                         (const long long *)part, (int)ob, st, slots_begin(c),
+                         (const long long *)c.lb_err);
+      HIP_CHECK(hipGetLastError());
+    }
+    long long v[kHostSlots];
+    slots_end(c, {st, st + 1, st + 2, st + 3, st + 4, st + 5, st + 6}, v);
+    if (v[0] > n) return false;
+    if (v[1] <= capB && v[2] <= capO) {
+      r.K = (long)v[0];
+      r.nbEdges = (long)v[1];
+      r.noEdges = (long)v[2];
+      r.pipNum = (long)v[3];
+      r.within = (long)v[4];
+      r.E = (long)v[5];
+      r.hits = (long)v[6];
+      break;
+    }
+    capB = std::max(capB, v[1]);
+    capO = std::max(capO, v[2]);
   }
-  scan_i32_to_i64_multi(c, {{r.bCount, r.bOff, K}, {r.oCount, r.oOff, K}});
-  long long rb[kHostSlots];
-  read_scalars(c, {r.bOff + K, r.oOff + K}, rb);
-  r.nbEdges = (long)rb[0];
-  r.noEdges = (long)rb[1];
-  r.bEdge = (int *)c.ws.get("jr_bEdge", 4 * (size_t)(r.nbEdges + 1));
-  r.oEdge = (int *)c.ws.get("jr_oEdge", 4 * (size_t)(r.noEdges + 1));
-  const long long *EN = compact_flags_dev(c, r.joinFlag, K, r.list, "cmf2");
-  {
-    LaunchTimer t(c, "cmf_apply");
-    hipLaunchKernelGGL((cmf16 ? k_cmf<int, 16> : k_cmf<int, 64>), dim3(grid_for(K, cmfPer)),
-                       dim3(256), 0, c.stream, K, r.list,
-                       pairs, r.cmbr, in.bCoords, in.bVNum, in.bVPSNum, in.oCoords, in.oVNum,
-                       in.oVPSNum, r.joinFlag, r.bCount, r.oCount, (const long long *)r.bOff,
-                       (const long long *)r.oOff, r.bEdge, r.oEdge, false, EN);
-    HIP_CHECK(hipGetLastError());
+  // a candidate within the other polygon goes no further, so the CMF takes
+  // the rest and the joined pairs are the within and the intersecting ones
+  r.cmfCand = r.K - r.within;
+  r.nJoined = r.within + r.hits;
+  return true;
+}
+
+// Layers of at most this many polygons are joined without reading the
+// candidate count back in between: the candidates get kOptFew (when the order
+// takes one block) or kOptMid places per polygon.  More candidates than that
+// cost the attempt's nearly empty launches; the polygons of larger layers,
+// whose idle places would cost more than the 12 us of a read-back, are counted
+// first.
+constexpr long kOptPolys = 1L << 16;
+constexpr long kOptFew = 8, kOptMid = 4;
+static_assert(kOptFew * kFewPolys <= 1L << 15, "16-bit sums of k_refine_out_few");
+
+long join_run(Context &c, const JoinInputs &in, int **counts_out, int **pairs_out,
+              MbrSortView *sv, JoinRefine &r) {
+  const long N = in.B + in.O;
+  if (N <= 0) {
+    refine(c, in, 0, nullptr, false, -1.0, nullptr, r);
+    return 0;
   }
-  {
-    LaunchTimer t(c, "segment_join");
-    hipLaunchKernelGGL(k_segjoin<int>, dim3(grid_for(K, 4)), dim3(256), 0, c.stream, K, r.list,
-                       pairs, in.bCoords, in.bVPSNum, in.oCoords, in.oVPSNum, r.bCount, r.oCount,
-                       (const long long *)r.bOff, (const long long *)r.oOff, r.bEdge, r.oEdge,
-                       r.segFlag, false, false, EN);
-    HIP_CHECK(hipGetLastError());
+  MbrOrder m;
+  mbr_order(c, in.B, in.O, in.bMBR, in.oMBR, in.bVNum, in.oVNum, m);
+  int *counts = (int *)c.ws.get("mbr_counts", 4 * (size_t)N);
+  long long *offs = (long long *)c.ws.get("mbr_offs", 8 * (size_t)(N + 1));
+  bool done = false;
+  if (!m.strips && N <= kOptPolys) {
+    const long cap = (m.few ? kOptFew : kOptMid) * N;
+    const long long *kDev = nullptr;
+    mbr_candidates(c, m, cap, counts, offs, pairs_out, &kDev);
+    done = refine(c, in, cap, kDev, m.few, m.avg, *pairs_out, r);
   }
-  int *tmp = (int *)c.ws.get("jr_hits_idx", 4 * (size_t)Kc);
-  const long long *hitsN = compact_flags_dev(c, r.segFlag, K, tmp, "hits");
-  hipLaunchKernelGGL(k_join_final, dim3(grid_for(K, 256)), dim3(256), 0, c.stream, K, r.pipFlag,
-                     r.segFlag, r.joined);
-  HIP_CHECK(hipGetLastError());
-  int *jidx = (int *)c.ws.get("jr_joined_idx", 4 * (size_t)Kc);
-  const long long *joinedN = compact_flags_dev(c, r.joined, K, jidx, "joined");
-  read_scalars(c, {pipN, withinN, cmfN, EN, hitsN, joinedN}, rb);
-  r.pipNum = (long)rb[0];
-  r.within = (long)rb[1];
-  r.cmfCand = (long)rb[2];
-  r.E = (long)rb[3];
-  r.hits = (long)rb[4];
-  r.nJoined = (long)rb[5];
-  r.joinedIdx = jidx;
-  r.joinedPairs = (int *)c.ws.get("jr_joinedPairs", 8 * (size_t)(r.nJoined > 0 ? r.nJoined : 1));
-  if (r.nJoined > 0) {
-    hipLaunchKernelGGL(k_gather_pairs, dim3(grid_for(r.nJoined, 256)), dim3(256), 0, c.stream,
-                       r.nJoined, jidx, pairs, r.joinedPairs);
-    HIP_CHECK(hipGetLastError());
+  if (!done) {
+    const long K = mbr_candidates(c, m, 0, counts, offs, pairs_out, nullptr);
+    refine(c, in, K, nullptr, false, m.avg, *pairs_out, r);
   }
+  *counts_out = counts;
+  sv->perm = m.perm;
+  sv->rank = m.rank;
+  sv->n = 2 * N;
+  return r.K;
 }
 
 // ------------------------------------------- single-stage launchers ----
@@ -981,8 +1407,7 @@ void launch_get_cmbr(Context &c, long K, const int *pairs, const double *bMBR2,
   if (K <= 0) return;
   LaunchTimer t(c, "get_cmbr");
   hipLaunchKernelGGL(k_get_cmbr, dim3(grid_for(K, 256)), dim3(256), 0, c.stream, K, pairs, bMBR2,
-                     oMBR2, cmbr, pipFlag, pipType, joinFlag, (int *)nullptr, (int *)nullptr,
-                     (int *)nullptr);
+                     oMBR2, cmbr, pipFlag, pipType, joinFlag);
   HIP_CHECK(hipGetLastError());
 }
 
@@ -992,8 +1417,8 @@ void launch_pip(Context &c, long nCand, const int *cand, const int *pairs,
   if (nCand <= 0) return;
   LaunchTimer t(c, "pip");
   hipLaunchKernelGGL(k_pip, dim3(grid_for(nCand, 4)), dim3(256), 0, c.stream, nCand, cand, pairs,
-                     pipType, bCoords, bVPSNum, oCoords, oVPSNum, pipFlag, joinFlag,
-                     (const long long *)nullptr);
+                     pipType, (PolyRefs{bCoords, oCoords, nullptr, nullptr, bVPSNum, oVPSNum}),
+                     pipFlag, joinFlag);
   HIP_CHECK(hipGetLastError());
 }
 
@@ -1002,12 +1427,8 @@ void launch_cmf_count(Context &c, long nList, const int *list, const int *pairs,
                       int *oCount) {
   if (nList <= 0) return;
   LaunchTimer t(c, "cmf_count");
-  hipLaunchKernelGGL((k_cmf<int, 64>), dim3(grid_for(nList, 4)), dim3(256), 0, c.stream, nList,
-                     list,
-                     pairs, cmbr, in.bCoords, in.bVNum, in.bVPSNum, in.oCoords, in.oVNum,
-                     in.oVPSNum, joinFlag, bCount, oCount, (const long long *)nullptr,
-                     (const long long *)nullptr, (int *)nullptr, (int *)nullptr, false,
-                     (const long long *)nullptr);
+  hipLaunchKernelGGL(k_cmf_count, dim3(grid_for(nList, 4)), dim3(256), 0, c.stream, nList, list,
+                     pairs, cmbr, poly_refs(in), joinFlag, bCount, oCount);
   HIP_CHECK(hipGetLastError());
 }
 
@@ -1016,11 +1437,8 @@ void launch_cmf_apply_short(Context &c, long nList, const int *list, const int *
                             const long long *oIncl, short *bEdge, short *oEdge) {
   if (nList <= 0) return;
   LaunchTimer t(c, "cmf_apply");
-  hipLaunchKernelGGL((k_cmf<short, 64>), dim3(grid_for(nList, 4)), dim3(256), 0, c.stream,
-                     nList, list,
-                     pairs, cmbr, in.bCoords, in.bVNum, in.bVPSNum, in.oCoords, in.oVNum,
-                     in.oVPSNum, (int *)nullptr, (int *)nullptr, (int *)nullptr, bIncl, oIncl,
-                     bEdge, oEdge, true, (const long long *)nullptr);
+  hipLaunchKernelGGL(k_cmf_apply, dim3(grid_for(nList, 4)), dim3(256), 0, c.stream, nList, list,
+                     pairs, cmbr, poly_refs(in), bIncl, oIncl, bEdge, oEdge);
   HIP_CHECK(hipGetLastError());
 }
 
@@ -1029,10 +1447,8 @@ void launch_segjoin_short(Context &c, long nList, const int *list, const int *pa
                           const short *bEdge, const short *oEdge, int *flagByList) {
   if (nList <= 0) return;
   LaunchTimer t(c, "segment_join");
-  hipLaunchKernelGGL(k_segjoin<short>, dim3(grid_for(nList, 4)), dim3(256), 0, c.stream, nList,
-                     list, pairs, in.bCoords, in.bVPSNum, in.oCoords, in.oVPSNum,
-                     (const int *)nullptr, (const int *)nullptr, bIncl, oIncl, bEdge, oEdge,
-                     flagByList, true, true, (const long long *)nullptr);
+  hipLaunchKernelGGL(k_segjoin, dim3(grid_for(nList, 4)), dim3(256), 0, c.stream, nList, list,
+                     pairs, poly_refs(in), bIncl, oIncl, bEdge, oEdge, flagByList);
   HIP_CHECK(hipGetLastError());
 }
 

@@ -19,6 +19,7 @@
 #include <mutex>
 
 #include "../../include/gcmf_hip.h"
+#include "gcmf_block.hpp"
 #include "gcmf_internal.hpp"
 
 namespace gcmf {
@@ -248,36 +249,6 @@ constexpr int kScanItems = 16;
 constexpr int kScanTile = kScanThreads * kScanItems;
 // up to this many tiles every tile sums its predecessors' partials itself
 constexpr long kScanPrefixTiles = 2048;
-
-template <typename T>
-__device__ __forceinline__ T wave_incl_scan(T v) {
-  const int lane = __lane_id();
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    T u = __shfl_up(v, off, 64);
-    if (lane >= off) v += u;
-  }
-  return v;
-}
-
-// Block-wide exclusive scan of one value per thread; returns the block total.
-template <typename T>
-__device__ __forceinline__ T block_excl_scan(T v, T *lds_waves, T &total) {
-  const int lane = __lane_id(), wave = threadIdx.x >> 6;
-  T inc = wave_incl_scan(v);
-  if (lane == 63) lds_waves[wave] = inc;
-  __syncthreads();
-  T wbase = 0, tot = 0;
-  const int nw = blockDim.x >> 6;
-  for (int w = 0; w < nw; w++) {
-    T s = lds_waves[w];
-    if (w < wave) wbase += s;
-    tot += s;
-  }
-  __syncthreads();
-  total = tot;
-  return wbase + inc - v;
-}
 
 template <typename TI, typename TA>
 __global__ void __launch_bounds__(kScanThreads) k_tile_reduce(const TI *in, long n, TA *partials) {
@@ -1190,93 +1161,17 @@ __global__ void __launch_bounds__(kSortThreads)
   }
 }
 
-// All passes of a sort of at most kOneSort keys in one launch of one block,
-// the keys in LDS between the passes; the rounds are k_sort_scatter's.  Such a
-// sort is bound by launches: 4000 keys of 64 bits took 67 us of kernel time in
-// 16 launches on one MI355X and take 27 in this one.
-constexpr int kOneThreads = 1024;
-constexpr int kOneItems = 8;
-constexpr int kOneSort = kOneThreads * kOneItems;
-constexpr int kOneWaves = kOneThreads / 64;
-
-__global__ void __launch_bounds__(kOneThreads)
-    k_sort_one(const uint64_t *keys, const int *vals, int n, int passes, uint64_t *keys_out,
-               int *vals_out) {
-  __shared__ uint64_t sk[kOneSort];
-  __shared__ int sv[kOneSort];
-  __shared__ int wcnt[kOneWaves][256];
-  __shared__ int dstart[256];
-  __shared__ int lds_scan[kOneWaves];
-  const int lane = __lane_id(), wave = threadIdx.x >> 6;
-  // a wave's keys are contiguous; the waves share the n keys evenly
-  const int rounds = (n + kOneThreads - 1) / kOneThreads, wbase = wave * 64 * rounds;
-  uint64_t kk[kOneItems];
-  int vv[kOneItems], pos[kOneItems];
-#pragma unroll
-  for (int r = 0; r < kOneItems; r++) {
-    const int i = wbase + r * 64 + lane;
-    kk[r] = r < rounds && i < n ? keys[i] : 0;
-    vv[r] = r < rounds && i < n ? vals[i] : 0;
-  }
-  for (int p = 0; p < passes; p++) {
-    const int shift = 8 * p;
-    for (int d = threadIdx.x; d < 256 * kOneWaves; d += kOneThreads) (&wcnt[0][0])[d] = 0;
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < kOneItems; r++) {
-      if (r >= rounds) break;
-      const bool valid = wbase + r * 64 + lane < n;
-      const int d = (int)((kk[r] >> shift) & 255);
-      unsigned long long peers = __ballot(valid);
-#pragma unroll
-      for (int b = 0; b < 8; b++) {
-        const unsigned long long m = __ballot((d >> b) & 1);
-        peers &= ((d >> b) & 1) ? m : ~m;
-      }
-      const int before = valid ? wcnt[wave][d] : 0;
-      const int rk = __popcll(peers & ((1ULL << lane) - 1ULL));
-      pos[r] = valid ? before + rk : -1;
-      __builtin_amdgcn_wave_barrier();
-      if (valid && rk == 0) wcnt[wave][d] = before + __popcll(peers);
-      __builtin_amdgcn_wave_barrier();
-    }
-    __syncthreads();
-    int s = 0;
-    if (threadIdx.x < 256) {
-      for (int w = 0; w < kOneWaves; w++) {
-        const int v = wcnt[w][threadIdx.x];
-        wcnt[w][threadIdx.x] = s;
-        s += v;
-      }
-    }
-    int tot;
-    const int st = block_excl_scan<int>(s, lds_scan, tot);
-    if (threadIdx.x < 256) dstart[threadIdx.x] = st;
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < kOneItems; r++) {
-      if (r >= rounds || pos[r] < 0) continue;
-      const int d = (int)((kk[r] >> shift) & 255);
-      const int lp = dstart[d] + wcnt[wave][d] + pos[r];
-      sk[lp] = kk[r];
-      sv[lp] = vv[r];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < kOneItems; r++) {
-      const int i = wbase + r * 64 + lane;
-      if (r >= rounds || i >= n) continue;
-      kk[r] = sk[i];
-      vv[r] = sv[i];
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < kOneItems; r++) {
-    const int i = wbase + r * 64 + lane;
-    if (r >= rounds || i >= n) continue;
-    keys_out[i] = kk[r];
-    vals_out[i] = vv[r];
-  }
+// A sort of at most kRankSort keys (by the bits that mask keeps): every key
+// straight to its place, one launch (rank_among).
+__global__ void __launch_bounds__(kRankThreads)
+    k_sort_rank(const uint64_t *__restrict__ keys, const int *__restrict__ vals, int n,
+                uint64_t mask, uint64_t *__restrict__ keys_out, int *__restrict__ vals_out) {
+  __shared__ RankLds lds;
+  const int i = (int)blockIdx.x * kRankKeys + (int)threadIdx.x;
+  const int at = rank_among(n, lds, [&](int j) { return keys[j] & mask; });
+  if (threadIdx.x >= kRankKeys || i >= n) return;
+  keys_out[at] = keys[i];
+  vals_out[at] = vals[i];
 }
 
 void radix_sort_u64(Context &c, const uint64_t *keys_in, const int *vals_in, uint64_t *keys_out,
@@ -1290,10 +1185,11 @@ void radix_sort_u64(Context &c, const uint64_t *keys_in, const int *vals_in, uin
                              c.stream));
     return;
   }
-  if (n <= kOneSort) {
+  if (n <= kRankSort) {
     LaunchTimer t(c, "sort_scatter");
-    hipLaunchKernelGGL(k_sort_one, dim3(1), dim3(kOneThreads), 0, c.stream, keys_in, vals_in,
-                       (int)n, passes, keys_out, vals_out);
+    hipLaunchKernelGGL(k_sort_rank, dim3(grid_for(n, kRankKeys)), dim3(kRankThreads), 0, c.stream,
+                       keys_in, vals_in, (int)n, passes < 8 ? (1ULL << (8 * passes)) - 1 : ~0ULL,
+                       keys_out, vals_out);
     HIP_CHECK(hipGetLastError());
     return;
   }

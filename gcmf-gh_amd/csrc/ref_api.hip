@@ -171,9 +171,7 @@ gcmf::JoinRefine &st_intersect(gcmf_ctx &x, long bPolNum, long oPolNum, coord_t 
   in.oMBR2 = (const double *)up("om2", seqOMBR2, 32 * (size_t)oPolNum);
   x.join_valid = false;
   x.jin = in;
-  x.K = gcmf::mbr_filter(c, bPolNum, oPolNum, in.bMBR, in.oMBR, &x.counts, &x.pairs, &x.sv,
-                         in.bVNum, in.oVNum);
-  gcmf::join_refine(c, in, x.K, x.pairs, x.jr);
+  x.K = gcmf::join_run(c, in, &x.counts, &x.pairs, &x.sv, x.jr);
   x.join_valid = true;
   return x.jr;
 }
@@ -203,7 +201,7 @@ long SortBaseMBROverlap(long bPolNum, long oPolNum, mbr_t *dbMBR, mbr_t *doMBR, 
       o = so;
     }
     int *counts = nullptr, *pairs = nullptr;
-    long k = gcmf::mbr_filter(c, bPolNum, oPolNum, b, o, &counts, &pairs, nullptr);
+    long k = gcmf::mbr_filter(c, bPolNum, oPolNum, b, o, &counts, &pairs);
     int *dc = dalloc<int>(bPolNum + oPolNum), *dv = dalloc<int>(2 * k);
     HIP_CHECK(hipMemcpyAsync(dc, counts, 4 * (size_t)(bPolNum + oPolNum), hipMemcpyDeviceToDevice,
                              c.stream));
@@ -597,9 +595,7 @@ int spatialJoin(int argc, char *argv[], int **pIDList, int **qIDList, long *tota
     in.oMBR = dk[1];
     x.join_valid = false;
     x.jin = in;
-    x.K = gcmf::mbr_filter(c, B, O, in.bMBR, in.oMBR, &x.counts, &x.pairs, &x.sv, in.bVNum,
-                           in.oVNum);
-    gcmf::join_refine(c, in, x.K, x.pairs, x.jr);
+    x.K = gcmf::join_run(c, in, &x.counts, &x.pairs, &x.sv, x.jr);
     x.join_valid = true;
     // the joined pairs (within U intersecting; the reference hands over the
     // within pairs only, spatialJoin3.cu:407)

@@ -116,6 +116,36 @@ def test_join_c2_strip_sweep(gctx):
     assert st["candidates"] > 10000
 
 
+@pytest.mark.parametrize("case", [
+    # (polygons per layer, vertices, radius): the small call's one-launch order
+    # (4096 polygons in all) and the first that takes the radix sort, the
+    # smallest calls, groups of 8 lanes, more candidates than the places given
+    # before the count is known in either form, more listed edges than places
+    (1, 1, 8, 8, 0.4), (1, 63, 5, 40, 0.2), (2049, 2047, 8, 16, 0.02), (2049, 2048, 8, 16, 0.02),
+    (3000, 2500, 3, 8, 0.02), (200, 180, 8, 12, 0.5), (2400, 2400, 8, 10, 0.12),
+    (40, 50, 600, 900, 0.3), (40, 50, 600, 900, 0.15), (2500, 2500, 200, 300, 0.02),
+    (2500, 2500, 200, 300, 0.013)])
+def test_join_places_given_before_the_count(case):
+    """Candidate and edge places sized before the counts are known, on a
+    context of its own so that no earlier call has left larger ones: every
+    stage's output equals the oracle's, on the second call too."""
+    nb, no, nmin, nmax, r = case
+    base, over = G.gen_join_layers(nb, no, seed=17, rmin=0.5 * r, rmax=r, nmin=nmin, nmax=nmax)
+    ctx = G.Context()
+    try:
+        for _ in range(2):
+            check_join(ctx, base, over)
+    finally:
+        ctx.close()
+
+
+def test_join_no_candidates(gctx):
+    """Layers apart from each other: no candidate in the small call's form."""
+    base, over = G.gen_join_layers(30, 40, seed=2, rmin=1e-6, rmax=2e-6, nmin=8, nmax=8)
+    st = check_join(gctx, base, over)
+    assert st["candidates"] == 0 and st["joined"] == 0
+
+
 def test_join_then_clip_pipeline(gctx):
     base, over = G.gen_join_layers(3000, 3000, seed=5, rmin=2e-3, rmax=2e-2, nmin=16, nmax=128)
     db, do = G.DeviceLayer(gctx, base), G.DeviceLayer(gctx, over)
