@@ -330,9 +330,10 @@ def main():
     ctx.synchronize()
     ctx.set_timing(False)
 
-    kernels = ["mbr_endpoints", "sort_hist", "sort_scatter", "scan_tile", "scan_reduce",
-               "scan_downsweep", "scan_lookback", "compact_lookback", "mbr_sweep_prep",
-               "mbr_sweep_count", "mbr_sweep_write", "refine_count", "refine_apply", "gh_pair_setup", "gh_pair_fill", "gh_count", "gh_transpose",
+    kernels = ["mbr_endpoints", "sort_hist", "sort_starts", "sort_scatter", "scan_tile",
+               "scan_reduce", "scan_downsweep", "scan_lookback", "compact_lookback",
+               "mbr_sweep_prep", "mbr_sweep_count", "mbr_sweep_write", "refine_count",
+               "refine_apply", "gh_pair_setup", "gh_pair_fill", "gh_count", "gh_transpose",
                "gh_nmap", "gh_calc_own", "gh_calc", "gh_sort_p", "gh_sort_runs", "gh_sort_q",
                "gh_init_label", "gh_cpu_fill", "gh_cpu_sort", "gh_cpu_link", "gh_label_trace",
                "gh_gather_out", "fill_i32"]
@@ -626,9 +627,10 @@ def prims(args):
         ctx.join(db, do)
         ctx.synchronize()
         ctx.set_timing(False)
-        names = ["mbr_endpoints", "sort_hist", "sort_scatter", "scan_tile", "scan_reduce",
-                 "scan_downsweep", "scan_lookback", "mbr_sweep_prep", "mbr_sweep_count",
-                 "mbr_sweep_write", "mbr_strip_build", "mbr_strip_count", "mbr_strip_write"]
+        names = ["mbr_endpoints", "sort_hist", "sort_starts", "sort_scatter", "scan_tile",
+                 "scan_reduce", "scan_downsweep", "scan_lookback", "mbr_sweep_prep",
+                 "mbr_sweep_count", "mbr_sweep_write", "mbr_strip_build", "mbr_strip_count",
+                 "mbr_strip_write"]
         ms = sum(ctx.timer(k)[0] for k in names)
         sweep_ms = sum(ctx.timer(k)[0] for k in ("mbr_sweep_prep", "mbr_sweep_count",
                                                   "mbr_sweep_write", "mbr_strip_build",

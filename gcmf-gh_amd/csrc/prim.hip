@@ -449,18 +449,18 @@ __global__ void __launch_bounds__(256)
 // Each poll is a device-scope load that bypasses the XCD's L2, and tile t
 // reaches the nearest published inclusive prefix only after the tiles
 // before it have published theirs, so the chain of look-backs, not HBM,
-// bounds this path on long arrays: measured on MI355X, 0.67 ms for 2^27
-// elements against 0.44 ms for the reduce-then-scan path.  It is used up
-// to 2^22 elements (1024 tiles), where it replaces that path's four or more
-// launches by one.  One launch may scan several arrays (segments, up to
-// kLbSegs): each segment's first tile publishes an inclusive prefix, so no
-// look-back crosses into the segment before it.
+// bounds this path on long arrays: measured on MI355X, 23 us for 733 tiles,
+// of which the loads and stores are 7.  It is used up to kLbMaxTiles tiles a
+// launch, where one launch beats the two of k_seg_reduce and k_seg_down.  One
+// launch may scan several arrays (segments, up to kLbSegs): each segment's
+// first tile publishes an inclusive prefix, so no look-back crosses into the
+// segment before it.
 constexpr unsigned long long kLbAgg = 1, kLbIncl = 2;
-constexpr long kLbMaxN = 1L << 22;
+constexpr long kLbMaxTiles = 192;
 constexpr int kLbSpinLimit = 1 << 22;
 // descriptors per half: the tiles of one launch and the tile counter
-constexpr long kLbSlots = 4096;
-static_assert(kLbMaxN / 4096 + 1 <= kLbSlots, "descriptor half too small");
+constexpr long kLbSlots = 256;
+static_assert(kLbMaxTiles + 1 <= kLbSlots, "descriptor half too small");
 
 // every launch clears the other half, which the next launch uses
 __device__ __forceinline__ void lb_clear_next(unsigned long long *next) {
@@ -596,6 +596,12 @@ struct LbSegs {
   int k;
 };
 
+__device__ __forceinline__ int seg_of(const LbSegs &S, long t) {
+  int j = 0;
+  while (j + 1 < S.k && t >= S.t0[j + 1]) j++;
+  return j;
+}
+
 // desc[tiles] holds the tile counter
 __global__ void __launch_bounds__(256)
     k_lb_scan(LbSegs S, unsigned long long *desc, unsigned long long *next, long tiles,
@@ -607,8 +613,7 @@ __global__ void __launch_bounds__(256)
   if (threadIdx.x == 0) s_tile = (long)atomicAdd(desc + tiles, 1ULL);
   __syncthreads();
   const long t = s_tile;
-  int j = 0;
-  while (j + 1 < S.k && t >= S.t0[j + 1]) j++;
+  const int j = seg_of(S, t);
   const int *in = S.in[j];
   long long *out = S.out[j];
   const long n = S.n[j], lt = t - S.t0[j];
@@ -621,6 +626,70 @@ __global__ void __launch_bounds__(256)
   for (int k = 0; k < 4; k++) s[k] = (long long)v[k].x + v[k].y + v[k].z + v[k].w;
   block_excl_scan4(s, e, tot, lds);
   const long long pre = lb_tile_prefix(desc, t, tot, err, &s_pre, lt == 0);
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const long long o0 = pre + e[k], o1 = o0 + v[k].x, o2 = o1 + v[k].y, o3 = o2 + v[k].z;
+    const long long i = base + k * 1024 + 4 * threadIdx.x;
+    if (full) {
+      longlong2 *d = (longlong2 *)(out + i);
+      d[0] = make_longlong2(o0, o1);
+      d[1] = make_longlong2(o2, o3);
+    } else {
+      if (i < n) out[i] = o0;
+      if (i + 1 < n) out[i + 1] = o1;
+      if (i + 2 < n) out[i + 2] = o2;
+      if (i + 3 < n) out[i + 3] = o3;
+    }
+  }
+  if (t == S.t0[j + 1] - 1 && threadIdx.x == 0) out[n] = pre + tot;
+}
+
+// The same segments in two launches, for more tiles: every tile's sum, then
+// every tile adds up the sums before its own (at most kSumTiles, from L2) and
+// scans.  3 000 000 values on one MI355X: a scan call takes
+// 27 us, and 35 with the look-back; 1 000 000 values (245 tiles) 22.6 either way.
+constexpr long kSumTiles = 4096;
+__global__ void __launch_bounds__(256) k_seg_reduce(LbSegs S, long long *part) {
+  __shared__ long long lds[4];
+  const long t = blockIdx.x;
+  const int j = seg_of(S, t);
+  const long long base = (long long)(t - S.t0[j]) * kVecTile;
+  int4 v[4];
+  ld_tile4(S.in[j], S.n[j], base, base + kVecTile <= S.n[j], v);
+  long long s = 0;
+#pragma unroll
+  for (int k = 0; k < 4; k++) s += (long long)v[k].x + v[k].y + v[k].z + v[k].w;
+  long long tot;
+  block_excl_scan<long long>(s, lds, tot);
+  if (threadIdx.x == 0) part[t] = tot;
+}
+
+// the sum of part[t0, t), over a block of 256 threads
+__device__ __forceinline__ long long sum_before(const long long *part, long t0, long t,
+                                                long long *lds) {
+  long long c = 0, tot;
+#pragma unroll 4
+  for (long i = t0 + threadIdx.x; i < t; i += 256) c += part[i];
+  block_excl_scan<long long>(c, lds, tot);
+  return tot;
+}
+
+__global__ void __launch_bounds__(256) k_seg_down(LbSegs S, const long long *part) {
+  __shared__ long long lds4[4][4];
+  __shared__ long long lds[4];
+  const long t = blockIdx.x;
+  const int j = seg_of(S, t);
+  const long n = S.n[j];
+  long long *out = S.out[j];
+  const long long base = (long long)(t - S.t0[j]) * kVecTile;
+  const bool full = base + kVecTile <= n;
+  int4 v[4];
+  ld_tile4(S.in[j], n, base, full, v);
+  const long long pre = sum_before(part, S.t0[j], t, lds);
+  long long s[4], e[4], tot;
+#pragma unroll
+  for (int k = 0; k < 4; k++) s[k] = (long long)v[k].x + v[k].y + v[k].z + v[k].w;
+  block_excl_scan4(s, e, tot, lds4);
 #pragma unroll
   for (int k = 0; k < 4; k++) {
     const long long o0 = pre + e[k], o1 = o0 + v[k].x, o2 = o1 + v[k].y, o3 = o2 + v[k].z;
@@ -704,19 +773,14 @@ void lb_reset(Context &c) {
   if (c.lb_err) fill_i32(c, (int *)c.lb_err, 0, 2);
 }
 
-static bool lb_fits(const void *a, const void *b, long n) {
-  return n > 0 && n <= kLbMaxN && !((uintptr_t)a & 15) && !((uintptr_t)b & 15);
-}
-
-// one look-back launch over the given arrays, when every one suits it and
-// their tiles fit one descriptor half
-static bool lb_scan_segs(Context &c, std::initializer_list<ScanJob> jobs) {
+// one look-back launch, or two launches, over the given arrays, when every one
+// suits them and their tiles are not too many
+static bool scan_segs(Context &c, std::initializer_list<ScanJob> jobs) {
   LbSegs S{};
   long tiles = 0;
   if (jobs.size() == 0 || jobs.size() > (size_t)kLbSegs) return false;
   for (const ScanJob &j : jobs) {
-    if (j.n < 0 || j.n > kLbMaxN || ((uintptr_t)j.in & 15) || ((uintptr_t)j.out & 15))
-      return false;
+    if (j.n < 0 || ((uintptr_t)j.in & 15) || ((uintptr_t)j.out & 15)) return false;
     S.in[S.k] = j.in;
     S.out[S.k] = j.out;
     S.n[S.k] = j.n;
@@ -725,7 +789,20 @@ static bool lb_scan_segs(Context &c, std::initializer_list<ScanJob> jobs) {
     S.k++;
   }
   S.t0[S.k] = tiles;
-  if (tiles + 1 > kLbSlots) return false;
+  if (tiles > kSumTiles) return false;
+  if (tiles > kLbMaxTiles) {
+    long long *part = (long long *)c.ws.get("scan_seg_parts", sizeof(long long) * (size_t)tiles);
+    {
+      LaunchTimer t(c, "scan_reduce");
+      hipLaunchKernelGGL(k_seg_reduce, dim3((unsigned)tiles), dim3(256), 0, c.stream, S, part);
+      HIP_CHECK(hipGetLastError());
+    }
+    LaunchTimer t(c, "scan_downsweep");
+    hipLaunchKernelGGL(k_seg_down, dim3((unsigned)tiles), dim3(256), 0, c.stream, S,
+                       (const long long *)part);
+    HIP_CHECK(hipGetLastError());
+    return true;
+  }
   long long *err = lb_err_word(c);
   unsigned long long *next;
   unsigned long long *desc = lb_halves(c, &next);
@@ -737,16 +814,12 @@ static bool lb_scan_segs(Context &c, std::initializer_list<ScanJob> jobs) {
   return true;
 }
 
-static bool lb_scan(Context &c, const int *in, long long *out, long n) {
-  return n > 0 && lb_scan_segs(c, {ScanJob{in, out, n}});
-}
-
 // returns the device address of the count, or nullptr when the arrays do
 // not suit the single-pass path
 static const long long *lb_compact(Context &c, const int *flag, long n, int *out_idx,
                                    const std::string &t) {
-  if (!lb_fits(flag, flag, n)) return nullptr;
   const long tiles = (n + kVecTile - 1) / kVecTile;
+  if (n <= 0 || tiles > kLbMaxTiles || ((uintptr_t)flag & 15)) return nullptr;
   long long *count = (long long *)c.ws.get(t + "_n", sizeof(long long));
   long long *err = lb_err_word(c);
   unsigned long long *next;
@@ -844,13 +917,13 @@ void scan_i32_to_i64(Context &c, const int *in, long long *out, long n) {
     HIP_CHECK(hipGetLastError());
     return;
   }
-  if (lb_scan(c, in, out, n)) return;
+  if (scan_segs(c, {ScanJob{in, out, n}})) return;
   if (vscan(c, in, out, n)) return;
   scan_impl<int, long long>(c, in, out, n, 0);
 }
 
 void scan_i32_to_i64_multi(Context &c, std::initializer_list<ScanJob> jobs) {
-  if (lb_scan_segs(c, jobs)) return;
+  if (scan_segs(c, jobs)) return;
   for (const ScanJob &j : jobs) scan_i32_to_i64(c, j.in, j.out, j.n);
 }
 
@@ -904,26 +977,18 @@ __global__ void __launch_bounds__(256) k_vcompact_count(const int *flag, long n,
 }
 
 __global__ void __launch_bounds__(256)
-    k_vcompact_write(const int *flag, long n, const long long *offsets, long tiles, int *out) {
+    k_vcompact_write(const int *flag, long n, const long long *offsets, long tiles, int *out,
+                     long long *total) {
   __shared__ long long lds[4];
   __shared__ int stage[kVecTile];
   const long T = xcd_tile(blockIdx.x, tiles);
   const long long base = (long long)T * kVecTile;
-  const long long carry = offsets[T];
   const bool full = base + kVecTile <= n;
   int4 v[4];
-#pragma unroll
-  for (int k = 0; k < 4; k++) {
-    if (full) {
-      v[k] = ld_i4(flag, base, k);
-    } else {
-      const long long i = base + k * 1024 + 4 * threadIdx.x;
-      v[k].x = i < n ? flag[i] : 0;
-      v[k].y = i + 1 < n ? flag[i + 1] : 0;
-      v[k].z = i + 2 < n ? flag[i + 2] : 0;
-      v[k].w = i + 3 < n ? flag[i + 3] : 0;
-    }
-  }
+  ld_tile4(flag, n, base, full, v);
+  // the tiles' counts (total given: the tiles before are added up here), or
+  // their scan
+  const long long carry = total ? sum_before(offsets, 0, T, lds) : offsets[T];
   long long packed = 0;
 #pragma unroll
   for (int k = 0; k < 4; k++)
@@ -944,6 +1009,7 @@ __global__ void __launch_bounds__(256)
   }
   __syncthreads();
   for (int j = threadIdx.x; j < start; j += 256) out[carry + j] = (int)base + stage[j];
+  if (total && T == tiles - 1 && threadIdx.x == 0) *total = carry + start;
 }
 
 // the vector path of compaction; returns the device address of the count, or
@@ -956,9 +1022,10 @@ static const long long *vcompact(Context &c, const int *flag, long n, int *out_i
   hipLaunchKernelGGL(k_vcompact_count, dim3((unsigned)tiles), dim3(256), 0, c.stream, flag, n,
                      cnt);
   HIP_CHECK(hipGetLastError());
-  scan_impl<long long, long long>(c, cnt, cnt, tiles, 1);
+  const bool sum = tiles <= kSumTiles;
+  if (!sum) scan_impl<long long, long long>(c, cnt, cnt, tiles, 1);
   hipLaunchKernelGGL(k_vcompact_write, dim3((unsigned)tiles), dim3(256), 0, c.stream, flag, n,
-                     (const long long *)cnt, tiles, out_idx);
+                     (const long long *)cnt, tiles, out_idx, sum ? cnt + tiles : nullptr);
   HIP_CHECK(hipGetLastError());
   return cnt + tiles;
 }
@@ -1003,97 +1070,160 @@ const long long *compact_flags_dev(Context &c, const int *flag, long n, int *out
 }
 
 // --------------------------------------------------------- radix sort ----
+// A pass is a digit histogram per tile (k_sort_hist), the tiles' starts inside
+// each digit (k_sort_starts) and the scatter.  The histograms and starts are
+// tile-major, so a block's 256 counters are one coalesced row; the digits'
+// own starts follow from the last tile's row, in the scatter.
 constexpr int kSortThreads = 256;
-constexpr int kSortItems = 16;  // per lane
-constexpr int kSortTile = kSortThreads * kSortItems;
-constexpr int kWaveKeys = 64 * kSortItems;
 
-// Per-tile digit histogram, written digit-major: hist[d * tiles + tile].
+// The 256 rows [tile][digit] of a sort: item counts of 4, 8 and 16 per lane
+// make tiles of 1024, 2048 and 4096 keys.
+template <int I>
+constexpr int kSortTileOf = kSortThreads *I;
+
+template <int I>
 __global__ void __launch_bounds__(kSortThreads)
     k_sort_hist(const uint64_t *keys, long n, int shift, int *hist, long tiles) {
   __shared__ int h[256];
   h[threadIdx.x] = 0;
   __syncthreads();
-  // tiles in XCD order, so that the neighbouring tiles whose counts share a
-  // cache line of every digit's row are counted under one L2
+  // tiles in XCD order, as the scatter reads them
   const long T = xcd_tile(blockIdx.x, tiles);
-  const long base = T * kSortTile;
+  const long base = T * kSortTileOf<I>;
   // every load issued before the first LDS update; a full tile of 16-byte
   // aligned keys is read as 16-byte pairs (the counts do not depend on which
   // thread holds which key)
-  uint64_t kk[kSortItems];
-  const bool vec = base + kSortTile <= n && ((uintptr_t)keys & 15) == 0;
+  uint64_t kk[I];
+  const bool vec = base + kSortTileOf<I> <= n && ((uintptr_t)keys & 15) == 0;
   if (vec) {
     const ulonglong2 *k2 = (const ulonglong2 *)(keys + base);
 #pragma unroll
-    for (int k = 0; k < kSortItems / 2; k++) {
+    for (int k = 0; k < I / 2; k++) {
       const ulonglong2 v = k2[k * kSortThreads + threadIdx.x];
       kk[2 * k] = v.x;
       kk[2 * k + 1] = v.y;
     }
   } else {
 #pragma unroll
-    for (int k = 0; k < kSortItems; k++) {
+    for (int k = 0; k < I; k++) {
       const long i = base + (long)k * kSortThreads + threadIdx.x;
       kk[k] = i < n ? keys[i] : 0;
     }
   }
 #pragma unroll
-  for (int k = 0; k < kSortItems; k++) {
+  for (int k = 0; k < I; k++) {
     const long i = base + (long)k * kSortThreads + threadIdx.x;
     if (vec || i < n) atomicAdd(&h[(int)((kk[k] >> shift) & 255)], 1);
   }
   __syncthreads();
-  hist[(long)threadIdx.x * tiles + T] = h[threadIdx.x];
+  hist[T * 256 + threadIdx.x] = h[threadIdx.x];
 }
 
-// Stable scatter: wave w ranks its 1024 keys in 16 rounds of 64 in order;
+// off[tile][d] = the keys of digit d in earlier tiles.  A block takes
+// kStartDigits digits, its groups of as many lanes a run of tiles each: summed
+// (kept in registers up to kStartKeep tiles a run, else read twice), the runs'
+// starts scanned over the block, then written.  It replaces a general scan
+// over the digit-major counts: 8.6 us a pass for 3 000 000 keys on one MI355X,
+// 4.9 this way, bound by its chain of load, scan and store.
+constexpr int kStartThreads = 1024;
+constexpr int kStartDigits = 8;
+constexpr int kStartKeep = 8;
+__global__ void __launch_bounds__(kStartThreads)
+    k_sort_starts(const int *hist, long tiles, long long *off) {
+  constexpr int D = kStartDigits, R = kStartThreads / D, W = kStartThreads / 64;
+  __shared__ long long sum[W][D];
+  const int lane = __lane_id(), w = threadIdx.x >> 6;
+  const int d = threadIdx.x % D, s = threadIdx.x / D;
+  const long per = (tiles + R - 1) / R, t0 = s * per, t1 = min(tiles, t0 + per);
+  const int *h = hist + blockIdx.x * D + d;
+  long long *o = off + blockIdx.x * D + d;
+  int v[kStartKeep];
+  long long c = 0;
+  if (per <= kStartKeep) {
+#pragma unroll
+    for (int u = 0; u < kStartKeep; u++) {
+      v[u] = t0 + u < t1 ? h[256 * (t0 + u)] : 0;
+      c += v[u];
+    }
+  } else {
+#pragma unroll 8
+    for (long t = t0; t < t1; t++) c += h[256 * t];
+  }
+  // over the wave's runs of this digit, then over the waves
+  long long inc = c;
+#pragma unroll
+  for (int q = D; q < 64; q <<= 1) {
+    const long long u = __shfl_up(inc, q, 64);
+    if (lane >= q) inc += u;
+  }
+  if (lane >= 64 - D) sum[w][d] = inc;
+  __syncthreads();
+  c = inc - c;
+#pragma unroll
+  for (int x = 0; x < W; x++) c += x < w ? sum[x][d] : 0;
+  if (per <= kStartKeep) {
+#pragma unroll
+    for (int u = 0; u < kStartKeep; u++) {
+      if (t0 + u < t1) o[256 * (t0 + u)] = c;
+      c += v[u];
+    }
+  } else {
+#pragma unroll 8
+    for (long t = t0; t < t1; t++) {
+      const int x = h[256 * t];
+      o[256 * t] = c;
+      c += x;
+    }
+  }
+}
+
+// Stable scatter: wave w ranks its 64 I keys in I rounds of 64 in order;
 // position = tile digit offset + earlier waves' counts + rank within wave.
-// The tile digit offsets come from off (the exclusive scan of the
-// digit-major histograms) or, for sorts of at most kSortFuseTiles tiles,
-// from the histograms themselves (hist): every block adds up its digit's
-// row and scans the digits' totals, which saves the scan's launch.
+// The tile digit offsets come from k_sort_starts (off) or, for sorts of at
+// most kSortFuseTiles tiles (off null), from the histograms themselves: every
+// block adds up the rows, which saves a launch.
 constexpr long kSortFuseTiles = 64;
+template <int I>
 __global__ void __launch_bounds__(kSortThreads)
     k_sort_scatter(const uint64_t *keys, const int *vals, long n, int shift,
                    const long long *off, const int *hist, long tiles, uint64_t *keys_out,
                    int *vals_out) {
+  constexpr int tile = kSortTileOf<I>;
   __shared__ int wcnt[kSortThreads / 64][256];
   __shared__ long long lds_hist[kSortThreads / 64];
   const int lane = __lane_id(), wave = threadIdx.x >> 6;
   const long T = xcd_tile(blockIdx.x, tiles);
-  // this tile's output start for digit threadIdx.x (256 threads, 256
-  // digits), fetched now so that its latency hides behind the ranking
-  long long dOff;
-  if (hist) {
-    const int *row = hist + (long)threadIdx.x * tiles;
-    long long tot = 0, pre = 0;
-    for (long t = 0; t < tiles; t++) {
-      const int h = row[t];
-      tot += h;
-      pre += t < T ? h : 0;
-    }
-    long long all;
-    dOff = block_excl_scan<long long>(tot, lds_hist, all) + pre;
-  } else {
-    dOff = off[(long)threadIdx.x * tiles + T];
-  }
-  for (int d = threadIdx.x; d < 256 * (kSortThreads / 64); d += kSortThreads)
-    (&wcnt[0][0])[d] = 0;
-  const long wbase = T * kSortTile + (long)wave * kWaveKeys;
-  uint64_t kk[kSortItems];
-  int vv[kSortItems];
-  int pos[kSortItems];
+  const long wbase = T * tile + (long)wave * 64 * I;
+  uint64_t kk[I];
+  int vv[I];
+  int pos[I];
   // all of the wave's loads in flight at once, before the ranking rounds
 #pragma unroll
-  for (int r = 0; r < kSortItems; r++) {
+  for (int r = 0; r < I; r++) {
     const long i = wbase + (long)r * 64 + lane;
     kk[r] = i < n ? keys[i] : 0;
     vv[r] = i < n ? vals[i] : 0;
   }
-  __syncthreads();
+  // this tile's output start for digit threadIdx.x (256 threads, 256 digits)
+  const int *hrow = hist + threadIdx.x;
+  long long pre = 0, dtot = 0;
+  if (off) {
+    pre = off[T * 256 + threadIdx.x];
+    dtot = off[(tiles - 1) * 256 + threadIdx.x] + hrow[(tiles - 1) * 256];
+  } else {
+#pragma unroll 16
+    for (int t = 0; t < (int)tiles; t++) {
+      const int h = hrow[256 * t];
+      dtot += h;
+      pre += t < T ? h : 0;
+    }
+  }
+  for (int d = threadIdx.x; d < 256 * (kSortThreads / 64); d += kSortThreads)
+    (&wcnt[0][0])[d] = 0;
+  long long all;
+  const long long dOff = block_excl_scan<long long>(dtot, lds_hist, all) + pre;
 #pragma unroll
-  for (int r = 0; r < kSortItems; r++) {
+  for (int r = 0; r < I; r++) {
     long i = wbase + (long)r * 64 + lane;
     bool valid = i < n;
     uint64_t key = kk[r];
@@ -1131,10 +1261,10 @@ __global__ void __launch_bounds__(kSortThreads)
   }
   __syncthreads();
   // the tile sorted by digit in LDS, stably ...
-  __shared__ uint64_t sk[kSortTile];
-  __shared__ int sv[kSortTile];
+  __shared__ uint64_t sk[tile];
+  __shared__ int sv[tile];
 #pragma unroll
-  for (int r = 0; r < kSortItems; r++) {
+  for (int r = 0; r < I; r++) {
     if (pos[r] < 0) continue;
     const int d = (int)((kk[r] >> shift) & 255);
     const int lp = dstart[d] + wcnt[wave][d] + pos[r];
@@ -1150,8 +1280,7 @@ __global__ void __launch_bounds__(kSortThreads)
   __syncthreads();
   // ... then written out in that order: consecutive threads store
   // consecutive addresses inside each digit's run
-  const long tbase = T * kSortTile;
-  const int tn = (int)min((long)kSortTile, n - tbase);
+  const int tn = (int)min((long)tile, n - T * tile);
   for (int i = threadIdx.x; i < tn; i += kSortThreads) {
     const uint64_t key = sk[i];
     const int d = (int)((key >> shift) & 255);
@@ -1174,6 +1303,65 @@ __global__ void __launch_bounds__(kRankThreads)
   vals_out[at] = vals[i];
 }
 
+// One pass over the tiles of I items per lane; hist and off hold 256 counters
+// per tile.
+template <int I>
+static void sort_pass(Context &c, const uint64_t *k, const int *v, long n, int shift, int *hist,
+                      long long *off, bool fuse, uint64_t *dk, int *dv) {
+  const long tiles = (n + kSortTileOf<I> - 1) / kSortTileOf<I>;
+  {
+    LaunchTimer t(c, "sort_hist");
+    hipLaunchKernelGGL(k_sort_hist<I>, dim3((unsigned)tiles), dim3(kSortThreads), 0, c.stream, k,
+                       n, shift, hist, tiles);
+    HIP_CHECK(hipGetLastError());
+  }
+  if (!fuse) {
+    LaunchTimer t(c, "sort_starts");
+    hipLaunchKernelGGL(k_sort_starts, dim3(256 / kStartDigits), dim3(kStartThreads), 0, c.stream,
+                       (const int *)hist, tiles, off);
+    HIP_CHECK(hipGetLastError());
+  }
+  LaunchTimer t(c, "sort_scatter");
+  hipLaunchKernelGGL(k_sort_scatter<I>, dim3((unsigned)tiles), dim3(kSortThreads), 0, c.stream, k,
+                     v, n, shift, fuse ? (const long long *)nullptr : (const long long *)off,
+                     (const int *)hist, tiles, dk, dv);
+  HIP_CHECK(hipGetLastError());
+}
+
+// Items per lane: a block per CU before longer runs per digit.  64-bit keys on
+// one MI355X, us with 4 / 8 / 16 items: 131 072 keys 104 / - / 158, 1 000 000
+// 182 / 177 / 198, 16 000 000 - / 1383 / 1101.
+constexpr long kSortSmall4 = 1L << 18, kSortSmall8 = 1L << 20;
+static int sort_items(long n) { return n <= kSortSmall4 ? 4 : n <= kSortSmall8 ? 8 : 16; }
+
+static void sort_passes(Context &c, const uint64_t *keys_in, const int *vals_in,
+                        uint64_t *keys_out, int *vals_out, long n, int passes, uint64_t *kb,
+                        int *vb, int *hist, long long *off) {
+  if (n <= kRankSort) {
+    LaunchTimer t(c, "sort_scatter");
+    hipLaunchKernelGGL(k_sort_rank, dim3(grid_for(n, kRankKeys)), dim3(kRankThreads), 0, c.stream,
+                       keys_in, vals_in, (int)n, passes < 8 ? (1ULL << (8 * passes)) - 1 : ~0ULL,
+                       keys_out, vals_out);
+    HIP_CHECK(hipGetLastError());
+    return;
+  }
+  const int I = sort_items(n);
+  const bool fuse = (n + kSortThreads * I - 1) / (kSortThreads * I) <= kSortFuseTiles;
+  // ping-pong so that the last pass lands in *_out
+  const uint64_t *src_k = keys_in;
+  const int *src_v = vals_in;
+  for (int p = 0; p < passes; p++) {
+    const bool to_out = ((passes - 1 - p) % 2) == 0;
+    uint64_t *dk = to_out ? keys_out : kb;
+    int *dv = to_out ? vals_out : vb;
+    (I == 4   ? sort_pass<4>
+     : I == 8 ? sort_pass<8>
+              : sort_pass<16>)(c, src_k, src_v, n, 8 * p, hist, off, fuse, dk, dv);
+    src_k = dk;
+    src_v = dv;
+  }
+}
+
 void radix_sort_u64(Context &c, const uint64_t *keys_in, const int *vals_in, uint64_t *keys_out,
                     int *vals_out, long n, int bits) {
   if (n <= 0) return;
@@ -1185,73 +1373,39 @@ void radix_sort_u64(Context &c, const uint64_t *keys_in, const int *vals_in, uin
                              c.stream));
     return;
   }
-  if (n <= kRankSort) {
-    LaunchTimer t(c, "sort_scatter");
-    hipLaunchKernelGGL(k_sort_rank, dim3(grid_for(n, kRankKeys)), dim3(kRankThreads), 0, c.stream,
-                       keys_in, vals_in, (int)n, passes < 8 ? (1ULL << (8 * passes)) - 1 : ~0ULL,
-                       keys_out, vals_out);
-    HIP_CHECK(hipGetLastError());
-    return;
-  }
-  long tiles = (n + kSortTile - 1) / kSortTile;
+  const int per = kSortThreads * sort_items(n);
+  const size_t rows = n <= kRankSort ? 0 : 256 * (size_t)((n + per - 1) / per);
   uint64_t *kb = (uint64_t *)c.ws.get("sort_kb", sizeof(uint64_t) * (size_t)n);
   int *vb = (int *)c.ws.get("sort_vb", sizeof(int) * (size_t)n);
-  int *hist = (int *)c.ws.get("sort_hist", sizeof(int) * (size_t)(256 * tiles));
-  long long *off = (long long *)c.ws.get("sort_off", sizeof(long long) * (size_t)(256 * tiles + 1));
-  // ping-pong so that the last pass lands in *_out
-  const uint64_t *src_k = keys_in;
-  const int *src_v = vals_in;
-  for (int p = 0; p < passes; p++) {
-    bool to_out = ((passes - 1 - p) % 2) == 0;
-    uint64_t *dk = to_out ? keys_out : kb;
-    int *dv = to_out ? vals_out : vb;
-    {
-      LaunchTimer t(c, "sort_hist");
-      hipLaunchKernelGGL(k_sort_hist, dim3((unsigned)tiles), dim3(kSortThreads), 0, c.stream,
-                         src_k, n, 8 * p, hist, tiles);
-      HIP_CHECK(hipGetLastError());
-    }
-    const bool fuse = tiles <= kSortFuseTiles;
-    if (!fuse) scan_i32_to_i64(c, hist, off, 256 * tiles);
-    {
-      LaunchTimer t(c, "sort_scatter");
-      hipLaunchKernelGGL(k_sort_scatter, dim3((unsigned)tiles), dim3(kSortThreads), 0, c.stream,
-                         src_k, src_v, n, 8 * p, (const long long *)off,
-                         fuse ? (const int *)hist : nullptr, tiles, dk, dv);
-      HIP_CHECK(hipGetLastError());
-    }
-    src_k = dk;
-    src_v = dv;
-  }
+  int *hist = (int *)c.ws.get("sort_hist", sizeof(int) * rows);
+  long long *off = (long long *)c.ws.get("sort_off", sizeof(long long) * rows);
+  sort_passes(c, keys_in, vals_in, keys_out, vals_out, n, passes, kb, vb, hist, off);
 }
 
 // ---------------------------------------------- sort without allocation ----
 // gcmf_radix_sort_u64_noalloc keeps its scratch -- the ping-pong key and value
-// buffers, the per-tile digit histograms, their scanned offsets and the
-// scan's tile partials -- in one static device array per GPU, so that the
-// call allocates nothing.  Every region is fully written before it is read
+// buffers, the per-tile digit histograms and the tiles' starts -- in one static
+// device array per GPU, so that the call allocates nothing.  Every region is fully written before it is read
 // in every pass, so no clearing is needed; calls that overlap on one GPU
 // race on it.
 constexpr long kNoAllocSortMax = 1L << 21;                    // keys per call
-constexpr long kNoAllocTiles = kNoAllocSortMax / kSortTile;  // 512
-constexpr long kNoAllocHist = 256 * kNoAllocTiles;
-constexpr long kNoAllocParts = kNoAllocHist / kScanTile + 1;
+constexpr long kNoAllocRows = 256 * (kNoAllocSortMax / kSortTileOf<16>);  // no sort has more
+static_assert(kSortSmall4 / kSortTileOf<4> <= kNoAllocRows / 256 &&
+                  kSortSmall8 / kSortTileOf<8> <= kNoAllocRows / 256,
+              "more tiles than rows");
 constexpr size_t noalloc_round(size_t b) { return (b + 255) & ~(size_t)255; }
 constexpr size_t kNoAllocKeys = 0;
 constexpr size_t kNoAllocVals = kNoAllocKeys + noalloc_round(8 * kNoAllocSortMax);
 constexpr size_t kNoAllocHistAt = kNoAllocVals + noalloc_round(4 * kNoAllocSortMax);
-constexpr size_t kNoAllocOffAt = kNoAllocHistAt + noalloc_round(4 * kNoAllocHist);
-constexpr size_t kNoAllocPartAt = kNoAllocOffAt + noalloc_round(8 * (kNoAllocHist + 1));
-constexpr size_t kNoAllocBytes = kNoAllocPartAt + noalloc_round(8 * kNoAllocParts);
-static_assert(kNoAllocHist / kScanTile + 1 <= kScanPrefixTiles, "histogram scan too long");
-
-static_assert(kNoAllocBytes == (size_t)GCMF_NOALLOC_SCRATCH_BYTES, "header disagrees");
+constexpr size_t kNoAllocOffAt = kNoAllocHistAt + noalloc_round(4 * kNoAllocRows);
+static_assert(kNoAllocOffAt + 8 * kNoAllocRows <= (size_t)GCMF_NOALLOC_SCRATCH_BYTES,
+              "scratch too small");
 static_assert(kNoAllocSortMax == GCMF_NOALLOC_SORT_MAX, "header disagrees");
 
-static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
+static __device__ __align__(256) unsigned char scratch[GCMF_NOALLOC_SCRATCH_BYTES];
 
 long noalloc_sort_max() { return kNoAllocSortMax; }
-size_t noalloc_scratch_bytes() { return kNoAllocBytes; }
+size_t noalloc_scratch_bytes() { return GCMF_NOALLOC_SCRATCH_BYTES; }
 
 // The device address of `scratch` on the current device, looked up once per
 // device (the array's host-side name is no device address).
@@ -1285,40 +1439,9 @@ void radix_sort_u64_noalloc(Context &c, const uint64_t *keys_in, const int *vals
     return;
   }
   unsigned char *s = (unsigned char *)c.scratch;
-  uint64_t *kb = (uint64_t *)(s + kNoAllocKeys);
-  int *vb = (int *)(s + kNoAllocVals);
-  int *hist = (int *)(s + kNoAllocHistAt);
-  long long *off = (long long *)(s + kNoAllocOffAt);
-  long long *parts = (long long *)(s + kNoAllocPartAt);
-  const long tiles = (n + kSortTile - 1) / kSortTile;
-  const long nh = 256 * tiles, st = (nh + kScanTile - 1) / kScanTile;
-  const uint64_t *src_k = keys_in;
-  const int *src_v = vals_in;
-  for (int p = 0; p < passes; p++) {
-    const bool to_out = ((passes - 1 - p) % 2) == 0;
-    uint64_t *dk = to_out ? keys_out : kb;
-    int *dv = to_out ? vals_out : vb;
-    hipLaunchKernelGGL(k_sort_hist, dim3((unsigned)tiles), dim3(kSortThreads), 0, c.stream,
-                       src_k, n, 8 * p, hist, tiles);
-    // exclusive scan of the histograms into off (the total at off[nh])
-    if (st == 1) {
-      hipLaunchKernelGGL((k_tile_scan<int, long long, long long>), dim3(1), dim3(kScanThreads),
-                         0, c.stream, (const int *)hist, nh, off, (const long long *)nullptr,
-                         off + nh);
-    } else {
-      hipLaunchKernelGGL((k_tile_reduce<int, long long>), dim3((unsigned)st), dim3(kScanThreads),
-                         0, c.stream, (const int *)hist, nh, parts);
-      hipLaunchKernelGGL((k_tile_scan_prefix<int, long long>), dim3((unsigned)st),
-                         dim3(kScanThreads), 0, c.stream, (const int *)hist, nh, off,
-                         (const long long *)parts, st);
-    }
-    hipLaunchKernelGGL(k_sort_scatter, dim3((unsigned)tiles), dim3(kSortThreads), 0, c.stream,
-                       src_k, src_v, n, 8 * p, (const long long *)off, (const int *)nullptr,
-                       tiles, dk, dv);
-    HIP_CHECK(hipGetLastError());
-    src_k = dk;
-    src_v = dv;
-  }
+  sort_passes(c, keys_in, vals_in, keys_out, vals_out, n, passes, (uint64_t *)(s + kNoAllocKeys),
+              (int *)(s + kNoAllocVals), (int *)(s + kNoAllocHistAt),
+              (long long *)(s + kNoAllocOffAt));
 }
 
 }  // namespace gcmf

@@ -835,8 +835,8 @@ def test_clip_small_call_glue(gctx, pairs, n_p, n_q):
 
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 1023, 1025, 4097, 8191, 8192, 8193])
 @pytest.mark.parametrize("bits", [1, 8, 13, 64])
-def test_radix_sort_one_block(gctx, n, bits):
-    """Sorts of up to 8192 keys run in one block: stable, every pass count."""
+def test_radix_sort_few_keys(gctx, n, bits):
+    """Sorts of up to 8192 keys take one launch: stable, every pass count."""
     rs = np.random.RandomState(n + bits)
     mask = np.uint64((1 << bits) - 1)
     keys = rs.randint(0, 1 << 62, n).astype(np.uint64) * np.uint64(5) & mask

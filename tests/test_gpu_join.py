@@ -243,6 +243,24 @@ def test_scan_and_compact_entry_points(gctx, n):
         b.free()
 
 
+# the last tile counts of the one-launch forms and of the two-launch forms
+@pytest.mark.parametrize("tiles", [191, 192, 193, 4096, 4097])
+@pytest.mark.parametrize("extra", [0, 1])
+def test_scan_and_compact_tile_limits(gctx, tiles, extra):
+    """Scan and compaction at the tile counts where their form changes."""
+    test_scan_and_compact_entry_points(gctx, 4096 * tiles + extra)
+
+
+# around the sizes where the tile of a sort changes (1024, 2048, 4096 keys), the
+# fused form ends (64 tiles) and a run of tiles is read twice (above 1024 tiles)
+@pytest.mark.parametrize("n", [8193, 64 * 1024, 64 * 1024 + 1, (1 << 18) - 1, (1 << 18) + 1,
+                               1 << 20, (1 << 20) + 1, 1024 * 4096 + 4097])
+@pytest.mark.parametrize("bits", [8, 22])
+def test_radix_sort_tile_forms(gctx, n, bits):
+    """Stable at every tile size and form of the passes, few and many ties."""
+    test_radix_sort_entry_point(gctx, n, bits)
+
+
 @pytest.mark.parametrize("n", [(1 << 20) - 3, (1 << 21) + 4099])
 def test_compact_dense_and_empty_tiles(gctx, n):
     """Compaction over tiles of 4096 flags that are all set (every group of
