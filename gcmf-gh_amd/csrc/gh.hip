@@ -4049,6 +4049,7 @@ __device__ __forceinline__ Departure departure(const Nodes &N, const int *dn, in
   return r;
 }
 
+constexpr int kShortCycle = 8;
 enum { SEG_DONE = 0, SEG_SLOW = 2, SEG_OVERFLOW = 3 };
 
 __host__ __device__ constexpr int even_up(int v) { return (v + 1) & ~1; }
@@ -4153,9 +4154,7 @@ __device__ int segment_trace(const Nodes &N, OutBuf &O, double *xy, int *clen, i
   while ((1 << rounds) < D) rounds++;
   int cur = 0;
   for (int t = 0; t < rounds; t++) {
-    // for the whole grid, the grid barrier of the grp_any before orders the
-    // last round's stores
-    if constexpr (W != kGrid) grp_sync<W>();
+    grp_sync<W>();
     const int2 *__restrict__ vs = vc[cur];
     const int *__restrict__ ns = nx[cur];
     int2 *__restrict__ vd = vc[cur ^ 1];
@@ -4219,7 +4218,7 @@ __device__ int segment_trace(const Nodes &N, OutBuf &O, double *xy, int *clen, i
   // once no element still points anywhere
   cur = 0;
   for (int t = 0; t < rounds; t++) {
-    if constexpr (W != kGrid) grp_sync<W>();
+    grp_sync<W>();
     const int *__restrict__ ss = S[cur];
     const int *__restrict__ ns = nx[cur];
     int *__restrict__ sd = S[cur ^ 1];
@@ -4296,35 +4295,6 @@ __device__ int segment_trace(const Nodes &N, OutBuf &O, double *xy, int *clen, i
   // departures' statuses, components and the vertices' coordinates, is
   // issued for all the chunks before it is used; the stores come last)
   int *cw = rk;  // output position -> component
-  if constexpr (W == kGrid) {
-    // the whole grid: one vertex per thread at a time, in block tiles
-    for (int ring = 0; ring < 2; ring++) {
-      const int rb = ring ? nP : 0, nR = ring ? nQ : nP, base = ring ? XP : 0;
-      const int XR = ring ? XQ : XP;
-      grp_scan_range<W, int>(
-          nR, [&](int j) { return dmult(N, rb + j); },
-          [&](int j, int r, int mu) {
-            const int u = rb + j, ri = r + mu;
-            const pt ou = P_orig(N, u);
-            for (int side = 0; side < 2; side++) {
-              const int dd = base + (side ? (ri == XR ? 0 : ri) : (r == 0 ? XR - 1 : r - 1));
-              const int of = off[dd], cd = dn[dd];
-              if (of < 0 || dep_enex(N, cd) != (side ? EXIT : ENTRY)) continue;
-              const int ud = cd >> 1;
-              int dist = side ? ud - u : u - ud;
-              if (dist <= 0) dist += nR;
-              const int w = of + dist - 1;
-              if (w >= 0 && w < O.n) {
-                st(xy, w, ou);
-                cw[w] = ciD[dd];
-                omap[w] = u;
-              }
-            }
-          });
-    }
-    grp_sync<W>();
-    return SEG_DONE;
-  }
   constexpr int kRS = W == 64 ? kRingStageWave : kRingStage;
   for (int ring = 0; ring < 2; ring++) {
     const int rb = ring ? nP : 0, nR = ring ? nQ : nP, base = ring ? XP : 0;
@@ -4388,6 +4358,331 @@ __device__ int segment_trace(const Nodes &N, OutBuf &O, double *xy, int *clen, i
         }
       }
     }
+  }
+  grp_sync<W>();
+  return SEG_DONE;
+}
+
+// The same for the whole grid, where a grid barrier (about 25 us) follows every
+// step and every round.
+__device__ int grid_segment_trace(const Nodes &N, OutBuf &O, double *xy, int *clen, int *rg,
+                                  int nP, int nQ, int Dc, int *omap) {
+  constexpr int W = kGrid;
+  const int lane = grp_rank<W>();
+  const int n = nP + nQ, nE = even_up(n);
+  // rk: per node; the rest per departure.  fs: the P departure that starts the
+  // departure's list (-1: not traced, kLong: not known yet), fp: its output
+  // offset there (a start: its list's length)
+  int *rk = rg, *dn = rg + nE, *fs = rg + nE + 3 * Dc, *fp = rg + nE + 4 * Dc;
+  int2 *vc[2] = {(int2 *)(rg + nE + Dc), (int2 *)(rg + nE + 7 * Dc)};
+  int *nx[2] = {rg + nE + 5 * Dc, rg + nE + 6 * Dc};
+  int *cbase = rg + nE + 7 * Dc, *off = rg + nE + 8 * Dc;  // (vc[1]'s, once that is dead)
+  constexpr int kLong = -2;
+  // departures by ring order
+  int XP = 0, XQ = 0;
+  for (int ring = 0; ring < 2; ring++) {
+    const int rb = ring ? nP : 0, nR = ring ? nQ : nP, r0 = ring ? XP : 0;
+    const int tot = grp_scan_range<W, int>(
+        nR, [&](int j) { return dmult(N, rb + j); },
+        [&](int j, int pre, int mu) {
+          const int u = rb + j, r = r0 + pre;
+          if (mu > 0 && r + mu <= Dc) {
+            rk[u] = r;
+            dn[r] = 2 * u;
+            if (mu == 2) dn[r + 1] = 2 * u + 1;
+          }
+        });
+    if (ring == 0) XP = tot;
+    else XQ = tot;
+  }
+  const int D = XP + XQ;
+  if (XP != XQ || XP == 0 || D > Dc) return SEG_SLOW;
+  grp_sync<W>();
+  // successor of each departure: the departure from the neighbour of its
+  // arrival; the arrival must carry the status the inner loop stops on.
+  // Key .x: the P departure of the departure's intersection point.
+  bool bad = false;
+  for (int d = lane; d < D; d += grp_size<W>()) {
+    const Departure p = departure(N, dn, d, nP, nQ, XP, XQ);
+    const bool onP = d < XP;
+    const int ua = dn[p.arr] >> 1, u = p.code >> 1;
+    const int q = N.nb[ua], pn = N.nb[u];
+    if (dep_enex(N, dn[p.arr]) != (p.fwd ? EXIT : ENTRY) || q < 0 || pn < 0 ||
+        (q < nP) == onP || (pn < nP) == onP || dmult(N, q) == 0 || dmult(N, pn) == 0) {
+      bad = true;
+      continue;
+    }
+    const int s = dep_partner(N, rk, dn[p.arr], nP, nQ);
+    const int key = onP ? d : dep_partner(N, rk, p.code, nP, nQ);
+    if (s < 0 || s >= D || key < 0 || key >= XP) {
+      bad = true;
+      continue;
+    }
+    nx[0][d] = s;
+    vc[0][d] = make_int2(key, p.dist);
+  }
+  if (grp_any<W>(bad)) return SEG_SLOW;
+  // A cycle of at most kShortCycle departures is walked from each of them: its
+  // smallest key, whether that P departure is on it (then it is traced, from
+  // there), and the lengths.  Most cycles of rings that cross often are that
+  // short: of the 2 700 000 departures of the wavy 1e6 x 1e5 pair 99 % are, of
+  // the 12 500 of the 2000 x 1500 pair 85 %.  Only the others take the rounds
+  // of pointer jumping below: 2130 us of rounds for the large pair on one
+  // MI355X when all took them in 512 blocks, 1200 with the walks (70) in 256;
+  // the rounds are left with their grid barriers.  (A wave or a block, whose
+  // barriers are cheap, keeps to the rounds: the walk's registers slowed its
+  // other passes by as much as it saved.)
+  for (int d0 = lane; d0 < D; d0 += 4 * grp_size<W>()) {
+    int2 a[4];
+    int mk[4], at[4], sum[4], x[4];
+    bool hit[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const int d = d0 + grp_size<W>() * k;
+      a[k] = d < D ? vc[0][d] : make_int2(0, 0);
+      x[k] = d < D ? nx[0][d] : d;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      mk[k] = a[k].x;
+      at[k] = 0;
+      sum[k] = a[k].y;
+      hit[k] = a[k].x == d0 + grp_size<W>() * k;
+    }
+    for (int h = 1; h < kShortCycle; h++) {
+      int2 b[4];
+      int y[4];
+      bool more = false;
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const bool go = x[k] != d0 + grp_size<W>() * k;
+        more |= go;
+        b[k] = go ? vc[0][x[k]] : make_int2(0x7fffffff, 0);
+        y[k] = go ? nx[0][x[k]] : x[k];
+      }
+      if (__ballot(more) == 0ULL) break;
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        if (b[k].x < mk[k] || (b[k].x == mk[k] && x[k] == mk[k])) {
+          mk[k] = b[k].x;
+          hit[k] = x[k] == b[k].x;
+          at[k] = sum[k];
+        }
+        sum[k] += b[k].y;
+        x[k] = y[k];
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const int d = d0 + grp_size<W>() * k;
+      if (d >= D) continue;
+      if (x[k] != d) {
+        fs[d] = kLong;
+      } else {
+        fs[d] = hit[k] ? mk[k] : -1;
+        fp[d] = mk[k] == d ? sum[k] : sum[k] - at[k];
+        // (the successors are a permutation, so no longer cycle leads here;
+        // were it otherwise, the rounds would still find indices in range)
+        vc[1][d] = a[k];
+        nx[1][d] = d;
+      }
+    }
+  }
+  // the departures of the longer cycles, in an array that only the sequential
+  // steps use
+  int *lg = O.next;
+  grp_sync<W>();
+  const int L = grp_scan_range<W, int>(
+      D, [&](int d) { return fs[d] == kLong ? 1 : 0; },
+      [&](int d, int pre, int x) {
+        if (x) lg[pre] = d;
+      });
+  grp_sync<W>();
+  if (L > 0) {
+    // the longer cycles, by pointer jumping: smallest P key (.x) and smallest
+    // departure (.y, in the first round the index itself) of every cycle; four
+    // independent chains per lane in flight.  After round t every value is the
+    // minimum over the next 2^t departures of its cycle; a round that changes
+    // no value means every window already spans its cycle's minimum, so the
+    // loop ends there instead of after ceil(log2 D) rounds.
+    int rounds = 0;
+    while ((1 << rounds) < L) rounds++;
+    int cur = 0;
+    for (int t = 0; t < rounds; t++) {
+      // (the grid barrier of the grp_any before orders the last round's stores)
+      const int2 *__restrict__ vs = vc[cur];
+      const int *__restrict__ ns = nx[cur];
+      int2 *__restrict__ vd = vc[cur ^ 1];
+      int *__restrict__ nd = nx[cur ^ 1];
+      bool changed = false;
+      for (int i0 = lane; i0 < L; i0 += 4 * grp_size<W>()) {
+        int d[4], x[4];
+        int2 a[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          const int i = i0 + grp_size<W>() * k;
+          d[k] = i < L ? lg[i] : -1;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          x[k] = d[k] >= 0 ? ns[d[k]] : -1;
+          a[k] = d[k] >= 0 ? vs[d[k]] : make_int2(0, 0);
+        }
+        int2 b[4];
+        int y[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          b[k] = x[k] >= 0 ? vs[x[k]] : make_int2(0, 0);
+          y[k] = x[k] >= 0 ? ns[x[k]] : 0;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          if (x[k] >= 0) {
+            if (t == 0) {
+              a[k].y = d[k];
+              b[k].y = x[k];
+            }
+            const int2 m = make_int2(min(a[k].x, b[k].x), min(a[k].y, b[k].y));
+            changed |= m.x != a[k].x || m.y != a[k].y;
+            vd[d[k]] = m;
+            nd[d[k]] = y[k];
+          }
+        }
+      }
+      cur ^= 1;
+      if (!grp_any<W>(changed)) break;
+    }
+    grp_sync<W>();
+    const int2 *mc = vc[cur];
+    // a cycle is traced when it holds the departure of its smallest P key; its
+    // list starts there.  S: segment lengths, then suffix sums
+    int *S[2] = {(int *)vc[cur ^ 1], (int *)vc[cur ^ 1] + Dc};
+    for (int i = lane; i < L; i += grp_size<W>()) {
+      const int d = lg[i];
+      const int2 c = mc[d];
+      const int sd = c.x;
+      int nxt = -1, dist = 0;
+      const bool sel = fs[sd] == kLong && mc[sd].y == c.y;
+      if (sel) {
+        const Departure p = departure(N, dn, d, nP, nQ, XP, XQ);
+        const int s = dep_partner(N, rk, dn[p.arr], nP, nQ);
+        nxt = s == sd ? -1 : s;
+        dist = p.dist;
+      }
+      fp[d] = sel ? sd : -1;
+      S[0][d] = dist;
+      nx[0][d] = nxt;
+    }
+    grp_sync<W>();
+    // list ranking of the traced lists (nxt = -1 ends a list): the loop ends
+    // once no element still points anywhere
+    cur = 0;
+    for (int t = 0; t < rounds; t++) {
+      const int *__restrict__ ss = S[cur];
+      const int *__restrict__ ns = nx[cur];
+      int *__restrict__ sd = S[cur ^ 1];
+      int *__restrict__ nd = nx[cur ^ 1];
+      bool live = false;
+      for (int i0 = lane; i0 < L; i0 += 4 * grp_size<W>()) {
+        int d[4], x[4], a[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          const int i = i0 + grp_size<W>() * k;
+          d[k] = i < L ? lg[i] : -1;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          x[k] = d[k] >= 0 ? ns[d[k]] : -1;
+          a[k] = d[k] >= 0 ? ss[d[k]] : 0;
+        }
+        int b[4], y[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          b[k] = x[k] >= 0 ? ss[x[k]] : 0;
+          y[k] = x[k] >= 0 ? ns[x[k]] : -1;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          if (d[k] >= 0) {
+            sd[d[k]] = a[k] + b[k];
+            nd[d[k]] = y[k];
+            live |= y[k] >= 0;
+          }
+        }
+      }
+      cur ^= 1;
+      if (!grp_any<W>(live)) break;
+    }
+    grp_sync<W>();
+    const int *Sf = S[cur];
+    for (int i = lane; i < L; i += grp_size<W>()) {
+      const int d = lg[i], sd = fp[d];
+      fs[d] = sd;
+      if (sd >= 0) fp[d] = sd == d ? Sf[d] : Sf[sd] - Sf[d];
+    }
+    grp_sync<W>();
+  }
+  // each intersection point departs exactly once over the traced cycles
+  for (int d = lane; d < XP; d += grp_size<W>())
+    if ((fs[d] >= 0) == (fs[dep_partner(N, rk, dn[d], nP, nQ)] >= 0)) bad = true;
+  if (grp_any<W>(bad)) return SEG_SLOW;
+  // components in order of their start departure
+  int *cix = nx[0], *ciD = nx[1];
+  // one scan of (components << 32) + vertices
+  const long long vc_all = grp_scan_range<W, long long>(
+      XP, [&](int d) { return fs[d] == d ? (1LL << 32) + fp[d] : 0LL; },
+      [&](int d, long long pre, long long x) {
+        if (x == 0) return;
+        const int ci = (int)(pre >> 32), base = (int)(pre & 0xffffffffLL);
+        cbase[d] = base;
+        cix[d] = ci;
+        if (ci < O.capComp) {
+          O.compRoot[ci] = base;
+          clen[ci] = (int)(x & 0xffffffffLL);
+        }
+      });
+  const int vcarry = (int)(vc_all & 0xffffffffLL), ccarry = (int)(vc_all >> 32);
+  if (vcarry > O.cap || ccarry > O.capComp) return SEG_OVERFLOW;
+  // the output position map holds n entries
+  if (vcarry > n) return SEG_SLOW;
+  O.n = vcarry;
+  O.ncomp = ccarry;
+  grp_sync<W>();
+  for (int d = lane; d < D; d += grp_size<W>()) {
+    const int sd = fs[d];
+    if (sd >= 0) {
+      off[d] = cbase[sd] + (sd == d ? 0 : fp[d]);
+      ciD[d] = cix[sd];
+    } else {
+      off[d] = -1;
+    }
+  }
+  grp_sync<W>();
+  // as segment_trace's, one vertex per thread at a time, in block tiles
+  int *cw = rk;  // output position -> component
+  for (int ring = 0; ring < 2; ring++) {
+    const int rb = ring ? nP : 0, nR = ring ? nQ : nP, base = ring ? XP : 0;
+    const int XR = ring ? XQ : XP;
+    grp_scan_range<W, int>(
+        nR, [&](int j) { return dmult(N, rb + j); },
+        [&](int j, int r, int mu) {
+          const int u = rb + j, ri = r + mu;
+          const pt ou = P_orig(N, u);
+          for (int side = 0; side < 2; side++) {
+            const int dd = base + (side ? (ri == XR ? 0 : ri) : (r == 0 ? XR - 1 : r - 1));
+            const int of = off[dd], cd = dn[dd];
+            if (of < 0 || dep_enex(N, cd) != (side ? EXIT : ENTRY)) continue;
+            const int ud = cd >> 1;
+            int dist = side ? ud - u : u - ud;
+            if (dist <= 0) dist += nR;
+            const int w = of + dist - 1;
+            if (w >= 0 && w < O.n) {
+              st(xy, w, ou);
+              cw[w] = ciD[dd];
+              omap[w] = u;
+            }
+          }
+        });
   }
   grp_sync<W>();
   return SEG_DONE;
@@ -4808,22 +5103,24 @@ enum {
 // them (positions ascending on each ring) and, after lane 0 has noted the
 // result as runs of consecutive ring positions, writes the vertices.  The
 // statements are label_and_trace's; what the list of intersection vertices
-// alone does not decide returns false with nothing changed, and
+// alone does not decide returns CT_SLOW with nothing changed, and
 // label_and_trace then takes the pair: a ring without a crossing or without
 // an ordinary vertex, a chain (step 2) that leaves the intersection vertices,
-// a walk that starts without a status, does not close, or outgrows its room.
+// a walk that starts without a status or closes after outgrowing its room.  A
+// walk that cannot close fails here as it would there (CT_FAILED).
 //
 // What bounds it: lane 0's chain of dependent accesses, so the list lies in
 // LDS where it fits.  Measured on one MI355X, a pair of 8001 x 2003 vertices
 // snapped to a grid (about 400 intersection vertices): 10.1 -> 0.53 ms by one
 // block; 4849 x 1833 (160): 5.8 -> 0.51 ms by one wave.
+enum { CT_SLOW = 0, CT_DONE = 1, CT_FAILED = 2 };
 template <int W>
-__device__ __forceinline__ bool contracted_trace(const Nodes &N, OutBuf &O, double *xy, int *clen, int *rg,
+__device__ __forceinline__ int contracted_trace(const Nodes &N, OutBuf &O, double *xy, int *clen, int *rg,
                                  int nP, int nQ, int Dc, int *omap, const int pinHint[4],
                                  char *lds, int ldsBytes) {
   const int lane = grp_rank<W>();
   const int n = nP + nQ, nE = even_up(n);
-  if (pinHint[0] < 0 || pinHint[2] < 0 || Dc < 8) return false;
+  if (pinHint[0] < 0 || pinHint[2] < 0 || Dc < 8) return CT_SLOW;
   int *rk = rg, *base = rg + nE;
   if (20LL * Dc <= ldsBytes) base = (int *)lds;  // (one block's LDS: never for kGrid)
   int *pos = base, *nxt = base + Dc, *prv = base + 2 * Dc, *nb = base + 3 * Dc;
@@ -4846,7 +5143,7 @@ __device__ __forceinline__ bool contracted_trace(const Nodes &N, OutBuf &O, doub
         });
   }
   const int C = X[0] + X[1];
-  if (X[0] < 1 || X[1] < 1 || C > Dc) return false;
+  if (X[0] < 1 || X[1] < 1 || C > Dc) return CT_SLOW;
   grp_sync<W>();
   for (int c = lane; c < C; c += grp_size<W>()) {
     const int c0 = c < X[0] ? 0 : X[0], z = c < X[0] ? X[0] : C, u = pos[c], q = N.nb[u];
@@ -4973,14 +5270,16 @@ __device__ __forceinline__ bool contracted_trace(const Nodes &N, OutBuf &O, doub
       }
     // createResult
     int ns = 0, nc = 0, tot = 0, lastEnd = -1, lastKey = -1;
+    // full: the walk is longer than what can be noted here; it goes on without
+    // notes, as label_and_trace does.  failed: it will never return to its
+    // start (a state met twice: Brent's cycle detection, as there) or meets a
+    // vertex without a link, where label_and_trace fails too
+    bool full = false, failed = false;
     auto emit = [&](int p, int len, int ringdir) {
       // len vertices from ring position p on, joined to the run before when
       // they continue it
       if (lastKey != ringdir || lastEnd != p) {
-        if (ns >= maxSeg) {
-          ok = false;
-          return;
-        }
+        if (ns >= maxSeg) return false;
         seg[4 + 3 * ns] = tot;
         seg[4 + 3 * ns + 1] = p;
         seg[4 + 3 * ns + 2] = ringdir;
@@ -4991,6 +5290,7 @@ __device__ __forceinline__ bool contracted_trace(const Nodes &N, OutBuf &O, doub
       const int o = (ringdir & 1) ? (p - r0 + len) % nR : (p - r0 + nR - len % nR) % nR;
       lastEnd = r0 + o;
       lastKey = ringdir;
+      return tot <= n;
     };
     const long long guard = 4LL * T + 64;
     int I = 0;
@@ -4999,8 +5299,9 @@ __device__ __forceinline__ bool contracted_trace(const Nodes &N, OutBuf &O, doub
         if (nc >= O.capComp) ok = false;
         const int start = tot;
         lastKey = -1;
-        int V = I;
+        int V = I, savedV = -1, savedS = -1;
         long long hops = 0;
+        unsigned power = 1, lam = 0;
         st[V] &= ~(F_INT << FL);
         do {
           int status = enex(V);
@@ -5023,20 +5324,29 @@ __device__ __forceinline__ bool contracted_trace(const Nodes &N, OutBuf &O, doub
             }
             if (p >= r0 + nR) p -= nR;
             if (p < r0) p += nR;
-            emit(p, len, (onQ ? 2 : 0) | (fwd ? 1 : 0));
+            if (!full) full = !emit(p, len, (onQ ? 2 : 0) | (fwd ? 1 : 0));
             V = d;
             st[V] &= ~(F_INT << FL);
-            if (++hops > guard || tot > n) ok = false;
+            if (ok && V == savedV && status == savedS) failed = true;
+            if (lam++ == power) {
+              savedV = V;
+              savedS = status;
+              power <<= 1;
+              lam = 0;
+            }
+            if (++hops > guard || failed) ok = false;
           } while (ok && enex(V) != status && V != I);
           if (ok && V != I) {
             V = nb[V];
             if (V < 0) {
+              failed = true;
               ok = false;
             } else {
               st[V] &= ~(F_INT << FL);
             }
           }
         } while (ok && V != I);
+        if (full && !failed) ok = false;
         if (ok) {
           O.compRoot[nc] = start;
           clen[nc] = tot - start;
@@ -5046,15 +5356,14 @@ __device__ __forceinline__ bool contracted_trace(const Nodes &N, OutBuf &O, doub
       I = nxt[I];
     } while (ok && I != 0);
     if (tot > O.cap) ok = false;
-    seg[0] = ok ? 1 : 0;
+    seg[0] = ok ? CT_DONE : failed ? CT_FAILED : CT_SLOW;
     seg[1] = ns;
     seg[2] = nc;
     seg[3] = tot;
   }
   grp_sync<W>();
-  const bool ok = seg[0] != 0;
-  const int ns = seg[1], nc = seg[2], tot = seg[3];
-  if (!ok) return false;
+  const int rc = seg[0], ns = seg[1], nc = seg[2], tot = seg[3];
+  if (rc != CT_DONE) return rc;
   O.n = tot;
   O.ncomp = nc;
   int *cw = rk;
@@ -5080,7 +5389,7 @@ __device__ __forceinline__ bool contracted_trace(const Nodes &N, OutBuf &O, doub
     cw[w] = c;
   }
   grp_sync<W>();
-  return true;
+  return CT_DONE;
 }
 
 // gives the sequential steps, which insert nodes, the pair's nodes in its
@@ -5387,7 +5696,9 @@ __device__ __forceinline__ int label_pair(long k, int *status, const SlotArrays 
       const bool pinQ = grp_pip<W>(N, 0, nP, P_(N, VQ));
       grp_enex<W>(N, nP, nQ, VQ, pinQ ? EXIT : ENTRY);
       grp_sync<W>();
-      const int rc = segment_trace<W>(N, O, xy, clen, rg, nP, nQ, Dc, omap);
+      int rc;
+      if constexpr (W == kGrid) rc = grid_segment_trace(N, O, xy, clen, rg, nP, nQ, Dc, omap);
+      else rc = segment_trace<W>(N, O, xy, clen, rg, nP, nQ, Dc, omap);
       if (rc == SEG_OVERFLOW) {
         if (lane == 0) {
           status[k] = GH_OVERFLOW;
@@ -5432,8 +5743,17 @@ __device__ __forceinline__ int label_pair(long k, int *status, const SlotArrays 
     }
     grp_sync<W>();
     // (the clean-up below takes its result too)
-    slow = !contracted_trace<W>(N, O, xy, clen, rg, nP, nQ, Dc, omap, pinHint, ar.p,
-                                ar.p ? ar.left : 0);
+    const int rc = contracted_trace<W>(N, O, xy, clen, rg, nP, nQ, Dc, omap, pinHint, ar.p,
+                                       ar.p ? ar.left : 0);
+    if (rc == CT_FAILED) {
+      if (lane == 0) {
+        status[k] = GH_TRACE_FAIL;
+        a.outNComp[k] = 0;
+        a.outNVerts[k] = 0;
+      }
+      return LP_FAILED;
+    }
+    slow = rc != CT_DONE;
     path = LP_SEQUENTIAL;
   }
   if (slow) {
@@ -5487,7 +5807,7 @@ __device__ __forceinline__ int label_pair(long k, int *status, const SlotArrays 
 constexpr int kBigGroup = 1024;
 // Pairs with at least Tuning::gridNodes nodes are labelled by the whole GPU,
 // one cooperative launch of kGridBlock-thread blocks each (k_label_grid).
-constexpr int kGridBlock = 256;
+constexpr int kGridBlock = 512;
 // batches of at least this many pairs are labelled largest first
 constexpr long kLptMinPairs = 1024;
 
@@ -6937,7 +7257,11 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
       int perCu = 0;
       HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCu, k_label_grid, kGridBlock,
                                                              0));
-      const int blocks = (perCu > 0 ? perCu : 1) * c.cu_count;
+      // (a block on every other CU: the grid barriers, which every block
+      // writes its caches back for, cost more than the idle CUs would save.  The
+      // wavy 1e6 x 1e5 pair: 7.9 ms in 512 blocks of 256 threads, 5.6 in 256 of
+      // 512, 5.15 in 128, 5.9 in 64)
+      const int blocks = std::max(1, std::min(perCu * c.cu_count, c.cu_count / 2));
       long long *part = wsT<long long>(c, "gh_grid_part", 2L * blocks);
       for (int kp : gl) {
         long kk = kp;

@@ -833,6 +833,30 @@ def test_clip_small_call_glue(gctx, pairs, n_p, n_q):
     check_results(gctx, st, cases, 5)
 
 
+@pytest.mark.parametrize("kind,nP,nQ,snap", [(0, 300, 200, 0.0), (1, 3000, 2000, 0.0),
+                                             (1, 20000, 2000, 0.0), (0, 4000, 3000, 0.0),
+                                             (0, 4001, 1003, 1e-3)])
+def test_clip_whole_gpu_labels_alike(gctx, kind, nP, nQ, snap):
+    """Pairs with cycles of few and of many departures, with and without
+    degenerate vertices, labelled by the whole GPU and by one block: the same
+    status and result, bit for bit."""
+    P, Q = G.gen_single_pair(kind, 5, nP, nQ, snap)
+    default = gctx.tuning()
+    got = []
+    try:
+        for nodes in (64, 1 << 40):
+            gctx.set_tuning(**dict(default, grid_nodes=nodes, big_nodes=64))
+            st = run_batch(gctx, [("p", P, Q)], G.CLIP_NORMALIZE)
+            got.append(gctx.clip_results(st))
+    finally:
+        gctx.set_tuning(**default)
+    (sa, ra), (sb, rb) = got
+    np.testing.assert_array_equal(sa, sb)
+    assert [len(c) for c in ra[0]] == [len(c) for c in rb[0]]
+    for a, b in zip(ra[0], rb[0]):
+        np.testing.assert_array_equal(a, b)
+
+
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 1023, 1025, 4097, 8191, 8192, 8193])
 @pytest.mark.parametrize("bits", [1, 8, 13, 64])
 def test_radix_sort_few_keys(gctx, n, bits):
