@@ -5232,8 +5232,12 @@ __device__ __forceinline__ int contracted_trace(const Nodes &N, OutBuf &O, doubl
       prv[nxt[c]] = v;
       nxt[c] = v;
     };
-    auto turn = [&](int u) {
-      const int r0 = u < nP ? 0 : nP, z = u < nP ? nP : n;
+    // the area at c on the list: a vertex that has a copy already (a Q vertex
+    // that a second P vertex links to, where P touches itself) is followed by
+    // that copy, which lies on it
+    auto turn = [&](int c) {
+      if (nxt[c] >= C) return 0.0;
+      const int u = pos[c], r0 = u < nP ? 0 : nP, z = u < nP ? nP : n;
       return triA(P_(N, u == r0 ? z - 1 : u - 1), P_(N, u), P_(N, u + 1 == z ? r0 : u + 1));
     };
     for (int I = 0; I < X[0] && ok; I++) {
@@ -5246,7 +5250,7 @@ __device__ __forceinline__ int contracted_trace(const Nodes &N, OutBuf &O, doubl
       const int VP = T++, VQ = T++;
       pos[VP] = pos[I];
       pos[VQ] = pos[IQ];
-      if (turn(pos[I]) * turn(pos[IQ]) > 0) {
+      if (turn(I) * turn(IQ) > 0) {
         nb[I] = VQ;
         nb[VQ] = I;
         nb[IQ] = VP;
@@ -5312,11 +5316,12 @@ __device__ __forceinline__ int contracted_trace(const Nodes &N, OutBuf &O, doubl
             const int d = fwd ? nxt[V] : prv[V];
             const bool onQ = pos[d] >= nP;
             const int r0 = onQ ? nP : 0, nR = onQ ? nQ : nP;
-            // from V's position (excluded) to d's; a copy follows its vertex
-            // at once (index >= C: a copy)
+            // from V's position (excluded) to d's; copies (index >= C)
+            // follow their vertex at once, so a step onto one, or back from
+            // one, stays at its position
             int len = fwd ? pos[d] - pos[V] : pos[V] - pos[d];
             int p = fwd ? pos[V] + 1 : pos[V] - 1;
-            if (len == 0 && (fwd ? d >= C && V < C : V >= C && d < C)) {
+            if (fwd ? d >= C : V >= C) {
               len = 1;
               p = pos[d];
             } else if (len <= 0) {

@@ -877,3 +877,60 @@ def test_radix_sort_few_keys(gctx, n, bits):
     order = np.argsort(keys, kind="stable")
     np.testing.assert_array_equal(k, keys[order])
     np.testing.assert_array_equal(v, vals[order])
+
+
+def petals(rs, n, tips, first):
+    """n whole-number vertices around the origin with the origin itself
+    before `tips` of them; a tip is vertex 0, or (first False) is not."""
+    th = 2 * np.pi * (np.arange(n) + rs.uniform(0, 0.8, n)) / n
+    r = rs.uniform(2.0, 6.0, n)
+    xy = np.rint(np.stack([r * np.cos(th), r * np.sin(th)], 1))
+    at = rs.choice(n, tips, replace=False)
+    ring = []
+    for i in np.roll(np.arange(n), -at[0] if first else -at[0] - 1):
+        ring += [(0.0, 0.0), tuple(xy[i])] if i in at else [tuple(xy[i])]
+    ring = np.array(ring)
+    return ring[(ring != np.roll(ring, 1, 0)).any(1)]
+
+
+def petal_cases(n, first):
+    """Pairs whose P touches itself two to four times at a vertex of Q, so
+    that several P vertices link to one Q vertex and step 5 may split that
+    vertex more than once.  Walks that never close are among them."""
+    cases = []
+    for s in range(n):
+        rs = np.random.RandomState(s)
+        m = rs.randint(6, 16)
+        cases.append(("petals%d" % s, petals(rs, m, rs.randint(2, 5), first),
+                      petals(rs, rs.randint(4, m - 1), rs.randint(1, 3), False)))
+    return cases
+
+
+# two notches of P that meet in a vertex of Q
+NOTCHES = ("notches",
+           np.array([(-4, -4), (4, -4), (4, 4), (1, 4), (0, 0), (-1, 4), (-4, 4), (-4, 1),
+                     (0, 0), (-4, -1)], float),
+           np.array([(-3, -5), (5, -5), (5, -1), (0, 0), (5, 1), (5, 3), (-3, 3)], float))
+
+
+@pytest.mark.parametrize("form", ["waves", "blocks", "few_waves", "few_blocks", "grid"])
+@pytest.mark.parametrize("cleanup", [True, False])
+@pytest.mark.parametrize("first", [False])
+def test_clip_q_vertex_split_twice(gctx, form, cleanup, first):
+    """The oracle's status and vertices, bit for bit, by every labelling
+    launch: one wave or one block per pair, the same in calls of at most one
+    pair per CU, and the whole GPU."""
+    cases = [NOTCHES] + petal_cases(599, first)
+    flags = G.CLIP_NORMALIZE | (0 if cleanup else G.CLIP_NO_CLEANUP)
+    per = {"few_waves": 200, "few_blocks": 200}.get(form, len(cases))
+    if form == "grid":
+        cases, per = cases[:200], 200
+    default = gctx.tuning()
+    try:
+        gctx.set_tuning(**dict(default, big_nodes=1 if "blocks" in form else 1 << 40,
+                               grid_nodes=1 if form == "grid" else 1 << 40))
+        for i in range(0, len(cases), per):
+            st = run_batch(gctx, cases[i:i + per], flags)
+            check_results(gctx, st, cases[i:i + per], NORM | (0 if cleanup else 2))
+    finally:
+        gctx.set_tuning(**default)
