@@ -3276,6 +3276,7 @@ __device__ int label_and_trace(Nodes &N, int rootP, int rootQ, OutBuf &O, bool l
     if (found && !out_copy_ring(O, N, rootP)) return GH_OVERFLOW;
   }
   // step 4: entry/exit (:549-655)
+  int splitFrom = rootP;
   for (int i = 0; i < 2; i++) {
     if (noInter[i]) continue;
     int Pr = i == 0 ? rootP : rootQ, Qr = i == 0 ? rootQ : rootP;
@@ -3307,6 +3308,7 @@ __device__ int label_and_trace(Nodes &N, int rootP, int rootQ, OutBuf &O, bool l
       }
       if (V < 0) return GH_TRACE_FAIL;
     }
+    if (i == 0) splitFrom = V;
     int status = ENTRY;
     const bool pin = (pinHint && pinHint[2 * i] == V) ? pinHint[2 * i + 1] != 0
                                                       : node_pip(N, Qr, P_(N, V));
@@ -3361,10 +3363,11 @@ __device__ int label_and_trace(Nodes &N, int rootP, int rootQ, OutBuf &O, bool l
       }
     }
   }
-  // step 5: split bouncing vertex pairs (:661-714); step 6 (:722-734)
+  // step 5: split bouncing vertex pairs, in the order in which step 4 met
+  // them (:661-714: where P touches itself at a vertex of Q, that vertex is
+  // split more than once, and the order decides the links); step 6 (:722-734)
   {
-    const int nNodes = N.n;
-    int I = rootP;
+    int I = splitFrom;
     do {
       int nextI = N.next[I];
       if ((N.fl[I] & F_SPLIT) && N.nb[I] >= 0 && (N.fl[N.nb[I]] & F_SPLIT)) {
@@ -3390,8 +3393,7 @@ __device__ int label_and_trace(Nodes &N, int rootP, int rootQ, OutBuf &O, bool l
         N.fl[I] &= ~F_SPLIT;  // handled
       }
       I = nextI;
-    } while (I != rootP);
-    (void)nNodes;
+    } while (I != splitFrom);
     I = rootP;
     do {
       const int In = N.next[I];  // labels only change below
@@ -5160,6 +5162,7 @@ __device__ __forceinline__ int contracted_trace(const Nodes &N, OutBuf &O, doubl
     auto set_enex = [&](int c, int e) { st[c] = (st[c] & ~(3 << EN)) | (e << EN); };
     auto has = [&](int c, int f) { return (st[c] & (f << FL)) != 0; };
     bool ok = true;
+    int splitFrom = 0;
     // step 2: intersection chains
     for (int it = 0; it < X[0] && ok; it++) {
       if (lab(it) != L_LEFT_ON && lab(it) != L_RIGHT_ON) continue;
@@ -5190,6 +5193,7 @@ __device__ __forceinline__ int contracted_trace(const Nodes &N, OutBuf &O, doubl
         if (pos[c] < pinHint[2 * ring]) start = c + 1;
       }
       if (!any) ok = false;
+      if (ring == 0) splitFrom = start;
       int status = pinHint[2 * ring + 1] ? EXIT : ENTRY;
       bool first = true;
       for (int i = 0; i < z - c0 && ok; i++) {
@@ -5224,7 +5228,7 @@ __device__ __forceinline__ int contracted_trace(const Nodes &N, OutBuf &O, doubl
         }
       }
     }
-    // step 5: split pairs; a copy has its vertex's position
+    // step 5: split pairs, in step 4's order; a copy has its vertex's position
     int T = C;
     auto put_after = [&](int v, int c) {
       nxt[v] = nxt[c];
@@ -5240,7 +5244,8 @@ __device__ __forceinline__ int contracted_trace(const Nodes &N, OutBuf &O, doubl
       const int u = pos[c], r0 = u < nP ? 0 : nP, z = u < nP ? nP : n;
       return triA(P_(N, u == r0 ? z - 1 : u - 1), P_(N, u), P_(N, u + 1 == z ? r0 : u + 1));
     };
-    for (int I = 0; I < X[0] && ok; I++) {
+    for (int i = 0; i < X[0] && ok; i++) {
+      const int I = splitFrom + i < X[0] ? splitFrom + i : splitFrom + i - X[0];
       const int IQ = nb[I];
       if (!has(I, F_SPLIT) || IQ < 0 || !has(IQ, F_SPLIT)) continue;
       if (T + 2 > Dc) {

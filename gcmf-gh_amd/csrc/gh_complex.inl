@@ -272,10 +272,13 @@ __device__ int label_trace_multi(Nodes &N, const int *const *roots, const int *n
       }
     }
   }
-  // step 5: split bouncing vertex pairs (:661-714), P's candidates in list
-  // order (each pair is handled on its own); step 6 (:722-734)
+  // step 5: split bouncing vertex pairs (:661-714), P's candidates in the
+  // order in which step 4 met them (a vertex of Q that several vertices of P
+  // link to is split more than once, and the order decides the links); step 6
+  // (:722-734)
   for (int c = 0; c < nr[0]; c++) {
-    const int r = roots[0][c];
+    if (skip[0][c]) continue;
+    const int r = node_nonint_vertex(N, roots[0][c]);  // step 4's start
     int I = r;
     do {
       const int nextI = N.next[I];

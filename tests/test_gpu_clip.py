@@ -912,15 +912,23 @@ NOTCHES = ("notches",
                      (0, 0), (-4, -1)], float),
            np.array([(-3, -5), (5, -5), (5, -1), (0, 0), (5, 1), (5, 3), (-3, 3)], float))
 
+# P touches itself in its vertex 0, a vertex of Q: the splits are taken from
+# P's first ordinary vertex on, not from vertex 0
+TOUCHES_0 = ("touches0",
+             np.array([(0, 0), (1, 2), (0, 2), (0, 1), (0, 0), (-1, 2), (-2, 1), (-2, 0),
+                       (-3, 0), (-2, -1), (0, -1), (3, -3), (1, 0)], float),
+             np.array([(2, 1), (2, 2), (-1, 1), (0, 0), (1, 0), (1, -1), (1, 0), (2, 0)],
+                      float))
+
 
 @pytest.mark.parametrize("form", ["waves", "blocks", "few_waves", "few_blocks", "grid"])
 @pytest.mark.parametrize("cleanup", [True, False])
-@pytest.mark.parametrize("first", [False])
+@pytest.mark.parametrize("first", [False, True])
 def test_clip_q_vertex_split_twice(gctx, form, cleanup, first):
     """The oracle's status and vertices, bit for bit, by every labelling
     launch: one wave or one block per pair, the same in calls of at most one
     pair per CU, and the whole GPU."""
-    cases = [NOTCHES] + petal_cases(599, first)
+    cases = [NOTCHES, TOUCHES_0] + petal_cases(598, first)
     flags = G.CLIP_NORMALIZE | (0 if cleanup else G.CLIP_NO_CLEANUP)
     per = {"few_waves": 200, "few_blocks": 200}.get(form, len(cases))
     if form == "grid":

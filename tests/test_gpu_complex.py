@@ -10,6 +10,7 @@ import pytest
 import gcmf_amd as G
 import oracle_py as O
 from conftest import REFDATA, load_poly_text, printed
+from test_gpu_clip import NOTCHES, TOUCHES_0, petal_cases
 from test_oracle_multi import random_complex_pairs
 
 pytestmark = pytest.mark.gpu
@@ -133,4 +134,19 @@ def test_complex_wave_path_edges(gctx, sizes, union):
     failed = [k for k in range(len(cases)) if O.clip_multi(*cases[k], mode)[0] < 0]
     assert all(status[k] in (-1, -5) and res[k] == [] for k in failed)
     rest = [k for k in range(len(cases)) if k not in failed]
+    check([cases[k] for k in rest], [status[k] for k in rest], [res[k] for k in rest], mode)
+
+
+@pytest.mark.parametrize("union", [False, True])
+def test_complex_q_vertex_split_twice(gctx, union):
+    """P touching itself in a vertex of Q, its vertex 0 among them: the
+    vertex is split more than once, in the order of step 4's walk."""
+    cases = [([P], [Q]) for _, P, Q in [NOTCHES, TOUCHES_0] + petal_cases(400, True)]
+    mode = 5 | (8 if union else 0)
+    st, (status, res) = run_complex(gctx, cases,
+                                    G.CLIP_NORMALIZE | (G.CLIP_UNION if union else 0))
+    failed = [k for k in range(len(cases)) if O.clip_multi(*cases[k], mode)[0] < 0]
+    assert all(status[k] in (-1, -5) and res[k] == [] for k in failed)
+    rest = [k for k in range(len(cases)) if k not in failed]
+    assert len(rest) > 150
     check([cases[k] for k in rest], [status[k] for k in rest], [res[k] for k in rest], mode)
