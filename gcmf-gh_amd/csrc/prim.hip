@@ -1334,9 +1334,25 @@ static void sort_pass(Context &c, const uint64_t *k, const int *v, long n, int s
 constexpr long kSortSmall4 = 1L << 18, kSortSmall8 = 1L << 20;
 static int sort_items(long n) { return n <= kSortSmall4 ? 4 : n <= kSortSmall8 ? 8 : 16; }
 
+// The outputs may be the inputs' buffers (a sort in place).  An even number of
+// passes reads the inputs in its first pass alone, which writes to kb and vb;
+// the one launch of a small sort and the first of an odd number of passes
+// read while they write the outputs, so they take copies then.
 static void sort_passes(Context &c, const uint64_t *keys_in, const int *vals_in,
                         uint64_t *keys_out, int *vals_out, long n, int passes, uint64_t *kb,
                         int *vb, int *hist, long long *off) {
+  const size_t kBytes = sizeof(uint64_t) * (size_t)n, vBytes = sizeof(int) * (size_t)n;
+  auto meet = [](const void *a, size_t an, const void *b, size_t bn) {
+    return (uintptr_t)a < (uintptr_t)b + bn && (uintptr_t)b < (uintptr_t)a + an;
+  };
+  if ((n <= kRankSort || passes % 2 != 0) &&
+      (meet(keys_in, kBytes, keys_out, kBytes) || meet(keys_in, kBytes, vals_out, vBytes) ||
+       meet(vals_in, vBytes, keys_out, kBytes) || meet(vals_in, vBytes, vals_out, vBytes))) {
+    HIP_CHECK(hipMemcpyAsync(kb, keys_in, kBytes, hipMemcpyDeviceToDevice, c.stream));
+    HIP_CHECK(hipMemcpyAsync(vb, vals_in, vBytes, hipMemcpyDeviceToDevice, c.stream));
+    keys_in = kb;
+    vals_in = vb;
+  }
   if (n <= kRankSort) {
     LaunchTimer t(c, "sort_scatter");
     hipLaunchKernelGGL(k_sort_rank, dim3(grid_for(n, kRankKeys)), dim3(kRankThreads), 0, c.stream,

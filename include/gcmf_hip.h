@@ -76,7 +76,8 @@ int gcmf_timer_get(gcmf_ctx *ctx, const char *kernel, double *total_ms, long *la
 /* Stable LSD radix sort of n u64 keys carrying i32 values over their low
  * `bits` bits (8 bits per pass, bits <= 64); replaces RadixSort
  * (GPU_Utility.h:242-289) with its digit-bucket kernels
- * (GPU_RadixSort.h:27-146, 16 decimal-digit passes there). */
+ * (GPU_RadixSort.h:27-146, 16 decimal-digit passes there).  The outputs may
+ * be the inputs' own buffers. */
 int gcmf_radix_sort_u64(gcmf_ctx *ctx, const uint64_t *d_keys_in, const int *d_vals_in,
                         uint64_t *d_keys_out, int *d_vals_out, long n, int bits);
 /* No reference counterpart.  gcmf_radix_sort_u64 for callers that cannot

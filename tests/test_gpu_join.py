@@ -261,6 +261,36 @@ def test_radix_sort_tile_forms(gctx, n, bits):
     test_radix_sort_entry_point(gctx, n, bits)
 
 
+# either side of the one-launch sort's limit and of the fused passes' one, odd
+# and even numbers of passes
+@pytest.mark.parametrize("n", [17, 5000, 8192, 8193, 70001])
+@pytest.mark.parametrize("bits", [8, 16, 24, 64])
+@pytest.mark.parametrize("shift", [0, 3])
+@pytest.mark.parametrize("noalloc", [False, True])
+def test_radix_sort_in_place(gctx, n, bits, shift, noalloc):
+    """Outputs that are the inputs' own buffers, or begin `shift` elements into
+    them: the stable argsort all the same."""
+    rs = np.random.RandomState(n + bits)
+    mask = np.uint64((1 << bits) - 1)
+    keys = rs.randint(0, 1 << 62, size=n, dtype=np.int64).astype(np.uint64) * np.uint64(5) & mask
+    keys[::3] = keys[0]
+    vals = np.arange(n, dtype=np.int32)
+    bk = gctx.upload(np.concatenate([keys, np.zeros(shift, np.uint64)]))
+    bv = gctx.upload(np.concatenate([vals, np.zeros(shift, np.int32)]))
+    sort = gctx.radix_sort_noalloc if noalloc else gctx.radix_sort
+    try:
+        sort(bk, bv, _At(bk, 8 * shift), _At(bv, 4 * shift), n, bits)
+        gctx.synchronize()
+        k = gctx.download(bk, np.uint64, n + shift)[shift:]
+        v = gctx.download(bv, np.int32, n + shift)[shift:]
+    finally:
+        bk.free()
+        bv.free()
+    order = np.argsort(keys, kind="stable")
+    np.testing.assert_array_equal(k, keys[order])
+    np.testing.assert_array_equal(v, order)
+
+
 @pytest.mark.parametrize("n", [(1 << 20) - 3, (1 << 21) + 4099])
 def test_compact_dense_and_empty_tiles(gctx, n):
     """Compaction over tiles of 4096 flags that are all set (every group of
