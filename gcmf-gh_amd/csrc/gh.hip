@@ -6145,9 +6145,12 @@ __global__ void __launch_bounds__(kGlueThreads)
     const int sw = noswap ? 0 : (nb < no);
     double m[2][4];
     for (int side = 0; side < 2; side++) {
-      double x0 = INFINITY, y0 = INFINITY, x1 = -INFINITY, y1 = -INFINITY;
+      // (the first part seeds every lane: a coordinate that is NaN in every
+      // vertex stays NaN, as in k_pair_setup)
+      const double *parts = part + 8 * (long)k * split + 4 * side;
+      double x0 = parts[0], y0 = parts[1], x1 = parts[2], y1 = parts[3];
       for (int j = lane; j < split; j += 64) {
-        const double *d = part + 8 * ((long)k * split + j) + 4 * side;
+        const double *d = parts + 8 * j;
         x0 = fmin(x0, d[0]);
         y0 = fmin(y0, d[1]);
         x1 = fmax(x1, d[2]);

@@ -942,3 +942,18 @@ def test_clip_q_vertex_split_twice(gctx, form, cleanup, first):
             check_results(gctx, st, cases[i:i + per], NORM | (0 if cleanup else 2))
     finally:
         gctx.set_tuning(**default)
+
+
+@pytest.mark.parametrize("copies", [1, 32, 33])
+@pytest.mark.parametrize("cols", [[0], [1], [0, 1]])
+@pytest.mark.parametrize("side", [0, 1])
+def test_clip_nan_coordinate(gctx, copies, cols, side):
+    """A ring whose x or y is NaN in every vertex has a NaN box, which is apart
+    from nothing: the oracle's status, in calls set up by blocks per pair and
+    by waves."""
+    P = np.array([(0, 0), (4, 0), (4, 4), (0, 4), (-1, 2)], float)
+    Q = np.array([(1, 1), (5, 1), (5, 3), (1, 3)], float)
+    (P, Q)[side][:, cols] = np.nan
+    cases = [("nan", P, Q)] * copies
+    st = run_batch(gctx, cases, G.CLIP_NORMALIZE)
+    check_results(gctx, st, cases, NORM)
