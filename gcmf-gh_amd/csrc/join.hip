@@ -233,13 +233,14 @@ __device__ __forceinline__ int sweep_polygon(long e, long B, const int *rank, co
   return cnt;
 }
 
-// one wave per polygon: the counts, or with WRITE the pairs
+// one wave per polygon: the counts, or with WRITE the pairs (none when there
+// are more than cap in all)
 template <bool WRITE>
 __global__ void __launch_bounds__(256)
     k_sweep(long B, long O, const int *rank, SweepRecs r, const uint64_t *Y, int *counts,
             const long long *offs, int *pairs, long long cap) {
   const long e = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (e >= B + O) return;
+  if (e >= B + O || (WRITE && offs[B + O] > cap)) return;
   const int cnt = sweep_polygon<false, WRITE>(e, B, rank, r, Y, WRITE ? offs[e] : 0, pairs, cap);
   if (!WRITE && __lane_id() == 0) counts[e] = cnt;
 }
@@ -287,7 +288,7 @@ __global__ void __launch_bounds__(256)
     *total = t;
   }
   const int e = e0 + (int)(threadIdx.x >> 6);
-  if (e >= N) return;
+  if (e >= N || s >= cap) return;
   for (int i = e0; i < e; i++) s += counts[i];
   sweep_polygon<false, true>(e, B, rank, r, Y, s, pairs, cap);
 }
@@ -645,10 +646,30 @@ static long strip_sweep(Context &c, const MbrOrder &m, int *counts, long long *o
   return K;
 }
 
+// The pairs of the counted candidates (fold: from the counts alone), into
+// places for K of them.
+static void mbr_write(Context &c, const MbrOrder &m, long K, bool fold, int *counts,
+                      long long *offs, int **pairs_out) {
+  const long B = m.B, O = m.O, N = B + O;
+  int *pairs = (int *)c.ws.get("mbr_pairs", 8 * (size_t)(K > 0 ? K : 1));
+  *pairs_out = pairs;
+  if (K <= 0) return;
+  LaunchTimer t(c, "mbr_sweep_write");
+  if (fold)
+    hipLaunchKernelGGL(k_sweep_write_few, dim3(grid_for(N, 4)), dim3(256), 0, c.stream, B, O,
+                       (const int *)m.rank, m.rec, (const uint64_t *)m.Y, (const int *)counts,
+                       pairs, (long long)K, offs + N);
+  else
+    hipLaunchKernelGGL(k_sweep<true>, dim3(grid_for(N, 4)), dim3(256), 0, c.stream, B, O,
+                       (const int *)m.rank, m.rec, (const uint64_t *)m.Y, counts,
+                       (const long long *)offs, pairs, (long long)K);
+  HIP_CHECK(hipGetLastError());
+}
+
 // Counts per polygon, their offsets, and the candidate pairs.  With cap <= 0
-// the count is read back and the pairs are sized to it; with cap > 0 the
-// pairs below cap are written without a read-back and the count stays at
-// *kDev, which the caller compares with cap when it reads it.
+// the count is read back and the pairs are sized to it; with cap > 0 they are
+// given cap places without a read-back and the count stays at *kDev, which
+// the caller compares with cap when it reads it.
 static long mbr_candidates(Context &c, MbrOrder &m, long cap, int *counts, long long *offs,
                            int **pairs_out, const long long **kDev) {
   const long B = m.B, O = m.O, N = B + O;
@@ -679,20 +700,8 @@ static long mbr_candidates(Context &c, MbrOrder &m, long cap, int *counts, long 
   long K = cap;
   if (!fold) scan_i32_to_i64(c, counts, offs, N);
   if (cap <= 0) K = (long)read_scalar(c, offs + N);
-  int *pairs = (int *)c.ws.get("mbr_pairs", 8 * (size_t)(K > 0 ? K : 1));
-  *pairs_out = pairs;
   if (kDev) *kDev = offs + N;
-  if (K <= 0) return K;
-  LaunchTimer t(c, "mbr_sweep_write");
-  if (fold)
-    hipLaunchKernelGGL(k_sweep_write_few, dim3(grid_for(N, 4)), dim3(256), 0, c.stream, B, O,
-                       (const int *)m.rank, m.rec, (const uint64_t *)m.Y, (const int *)counts,
-                       pairs, (long long)K, offs + N);
-  else
-    hipLaunchKernelGGL(k_sweep<true>, dim3(grid_for(N, 4)), dim3(256), 0, c.stream, B, O,
-                       (const int *)m.rank, m.rec, (const uint64_t *)m.Y, counts,
-                       (const long long *)offs, pairs, (long long)K);
-  HIP_CHECK(hipGetLastError());
+  mbr_write(c, m, K, fold, counts, offs, pairs_out);
   return K;
 }
 
@@ -1155,15 +1164,16 @@ __global__ void __launch_bounds__(256)
 }
 
 // What a join reads back: candidates, edges listed on either side, PiP
-// candidates, within, CMF survivors and intersecting pairs.
+// candidates, within, CMF survivors and intersecting pairs; of a small call
+// also the layers' vertices, which it has not summed before.
 constexpr int kJoinStats = 7;
 
 // The end of a small call in one block: the joined pairs in order and the
 // read-back values.  Rounds of four candidates per thread.
 __global__ void __launch_bounds__(1024)
-    k_refine_out_few(long n, const long long *kDev, const int *pairs, RefineOut r,
-                     const long long *bOff, const long long *oOff, long long capB, long long capO,
-                     int *jidx, int *jpairs, long long *st, long long *slots,
+    k_refine_out_few(long n, const long long *kDev, const int *pairs, PolyRefs p, long B, long O,
+                     RefineOut r, const long long *bOff, const long long *oOff, long long capB,
+                     long long capO, int *jidx, int *jpairs, long long *st, long long *slots,
                      const long long *lbErr) {
   __shared__ int lds[16];
   __shared__ long long lds64[16];
@@ -1196,10 +1206,11 @@ __global__ void __launch_bounds__(1024)
   long long all;
   block_excl_scan<long long>(acc, lds64, all);
   if (threadIdx.x != 0) return;
-  long long v[kJoinStats] = {K, K <= n ? bOff[K] : 0, K <= n ? oOff[K] : 0};
+  long long v[kJoinStats + 1] = {K, K <= n ? bOff[K] : 0, K <= n ? oOff[K] : 0};
   for (int i = 0; i < 4; i++) v[3 + i] = (all >> (16 * i)) & 0xffff;
-  for (int i = 0; i < kJoinStats; i++) st[i] = v[i];
-  put_slots(slots, v, kJoinStats, lbErr);
+  v[kJoinStats] = (B ? p.bVPSNum[B - 1] : 0) + (O ? p.oVPSNum[O - 1] : 0);
+  for (int i = 0; i <= kJoinStats; i++) st[i] = v[i];
+  put_slots(slots, v, kJoinStats + 1, lbErr);
 }
 
 // The same end in two launches: the pairs of the compacted list and each
@@ -1255,9 +1266,11 @@ constexpr double kCmfSmall = 32.0, kCmfTiny = 12.0;
 constexpr long long kEdgeGuess = 1LL << 26;
 
 // Stages 2 to 5 over n candidate places, *kDev of them candidates (null: all
-// n).  Returns false, nothing else valid, when there are more than n.
+// n); avg, the mean vertex count per polygon, is set by a small call.  Returns
+// false when there are more than n candidates: r.K is their number and nothing
+// else of r is valid.
 static bool refine(Context &c, const JoinInputs &in, long n, const long long *kDev, bool few,
-                   double avg, const int *pairs, JoinRefine &r) {
+                   double &avg, const int *pairs, JoinRefine &r) {
   const size_t n1 = (size_t)std::max(n, 1L);
   r.cmbr = (double *)c.ws.get("jr_cmbr", 32 * n1);
   r.pipFlag = (int *)c.ws.get("jr_pipFlag", 4 * n1);
@@ -1277,7 +1290,7 @@ static bool refine(Context &c, const JoinInputs &in, long n, const long long *kD
   const PolyRefs p = poly_refs(in);
   const RefineOut o{r.cmbr,   r.pipFlag, r.joinFlag, r.bCount,
                     r.oCount, r.segFlag, joined,     r.pipType};
-  long long *st = (long long *)c.ws.get("jr_stats", 8 * kJoinStats);
+  long long *st = (long long *)c.ws.get("jr_stats", 8 * (kJoinStats + 1));
   // Edge lists are given a place before their lengths are known: the polygons'
   // mean vertex count per candidate, within 8 to 32.  Totals beyond that (or
   // beyond what an earlier call left) cost the second pass again; above
@@ -1328,9 +1341,10 @@ static bool refine(Context &c, const JoinInputs &in, long n, const long long *kD
       HIP_CHECK(hipGetLastError());
     }
     if (few) {
-      hipLaunchKernelGGL(k_refine_out_few, dim3(1), dim3(1024), 0, c.stream, n, kDev, pairs, o,
-                         (const long long *)bOff, (const long long *)oOff, capB, capO, jidx,
-                         r.joinedPairs, st, slots_begin(c), (const long long *)c.lb_err);
+      hipLaunchKernelGGL(k_refine_out_few, dim3(1), dim3(1024), 0, c.stream, n, kDev, pairs, p,
+                         in.B, in.O, o, (const long long *)bOff, (const long long *)oOff, capB,
+                         capO, jidx, r.joinedPairs, st, slots_begin(c),
+                         (const long long *)c.lb_err);
       HIP_CHECK(hipGetLastError());
     } else {
       const long long *nj = compact_flags_dev(c, joined, n, jidx, "joined");
@@ -1346,10 +1360,15 @@ static bool refine(Context &c, const JoinInputs &in, long n, const long long *kD
       HIP_CHECK(hipGetLastError());
     }
     long long v[kHostSlots];
-    slots_end(c, {st, st + 1, st + 2, st + 3, st + 4, st + 5, st + 6}, v);
+    if (few) {
+      slots_end(c, {st, st + 1, st + 2, st + 3, st + 4, st + 5, st + 6, st + 7}, v);
+      avg = (double)v[kJoinStats] / (double)(in.B + in.O);
+    } else {
+      slots_end(c, {st, st + 1, st + 2, st + 3, st + 4, st + 5, st + 6}, v);
+    }
+    r.K = (long)v[0];
     if (v[0] > n) return false;
     if (v[1] <= capB && v[2] <= capO) {
-      r.K = (long)v[0];
       r.nbEdges = (long)v[1];
       r.noEdges = (long)v[2];
       r.pipNum = (long)v[3];
@@ -1381,22 +1400,26 @@ static_assert(kOptFew * kFewPolys <= 1L << 15, "16-bit sums of k_refine_out_few"
 long join_run(Context &c, const JoinInputs &in, int **counts_out, int **pairs_out,
               MbrSortView *sv, JoinRefine &r) {
   const long N = in.B + in.O;
+  MbrOrder m;
   if (N <= 0) {
-    refine(c, in, 0, nullptr, false, -1.0, nullptr, r);
+    refine(c, in, 0, nullptr, false, m.avg, nullptr, r);
     return 0;
   }
-  MbrOrder m;
   mbr_order(c, in.B, in.O, in.bMBR, in.oMBR, in.bVNum, in.oVNum, m);
   int *counts = (int *)c.ws.get("mbr_counts", 4 * (size_t)N);
   long long *offs = (long long *)c.ws.get("mbr_offs", 8 * (size_t)(N + 1));
-  bool done = false;
   if (!m.strips && N <= kOptPolys) {
     const long cap = (m.few ? kOptFew : kOptMid) * N;
     const long long *kDev = nullptr;
     mbr_candidates(c, m, cap, counts, offs, pairs_out, &kDev);
-    done = refine(c, in, cap, kDev, m.few, m.avg, *pairs_out, r);
-  }
-  if (!done) {
+    if (!refine(c, in, cap, kDev, m.few, m.avg, *pairs_out, r)) {
+      // counted by now: places for all, and the pairs once more
+      const long K = r.K;
+      if (m.few) scan_i32_to_i64(c, counts, offs, N);
+      mbr_write(c, m, K, false, counts, offs, pairs_out);
+      refine(c, in, K, nullptr, false, m.avg, *pairs_out, r);
+    }
+  } else {
     const long K = mbr_candidates(c, m, 0, counts, offs, pairs_out, nullptr);
     refine(c, in, K, nullptr, false, m.avg, *pairs_out, r);
   }
