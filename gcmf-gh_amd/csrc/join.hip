@@ -1034,7 +1034,8 @@ __global__ void __launch_bounds__(256)
 // chains per wave in flight.
 //
 // n is the length of the per-candidate arrays; the candidates are *kDev of
-// them (all n without it), and none is touched when *kDev exceeds n.
+// them (all n without it); when *kDev exceeds n, every count is 0 and nothing
+// else is touched.
 struct RefineOut {
   double *cmbr;
   int *pipFlag, *joinFlag, *bCount, *oCount, *segFlag, *joined;
@@ -1045,8 +1046,8 @@ template <int G>
 __global__ void __launch_bounds__(256)
     k_refine_count(long n, const long long *kDev, const int *pairs, PolyRefs p,
                    const double *bMBR2, const double *oMBR2, RefineOut r) {
-  const long K = kDev ? (long)*kDev : n;
-  if (K > n) return;
+  long K = kDev ? (long)*kDev : n;
+  if (K > n) K = 0;
   const int g = (int)__lane_id() & (G - 1);
   const long step = (long)gridDim.x * (256 / G);
   for (long k = (long)blockIdx.x * (256 / G) + threadIdx.x / G; k < n; k += step) {
@@ -1263,7 +1264,7 @@ __global__ void __launch_bounds__(256)
 // polygons of at most this many vertices on average take groups of 16 lanes
 // (one group per candidate, eight per wave, of at most kCmfTiny)
 constexpr double kCmfSmall = 32.0, kCmfTiny = 12.0;
-constexpr long long kEdgeGuess = 1LL << 26;
+constexpr long long kEdgeGuess = 1LL << 22;
 
 // Stages 2 to 5 over n candidate places, *kDev of them candidates (null: all
 // n); avg, the mean vertex count per polygon, is set by a small call.  Returns
@@ -1293,8 +1294,10 @@ static bool refine(Context &c, const JoinInputs &in, long n, const long long *kD
   long long *st = (long long *)c.ws.get("jr_stats", 8 * (kJoinStats + 1));
   // Edge lists are given a place before their lengths are known: the polygons'
   // mean vertex count per candidate, within 8 to 32.  Totals beyond that (or
-  // beyond what an earlier call left) cost the second pass again; above
-  // kEdgeGuess places the totals are read first.
+  // beyond what an earlier call left) cost the second pass again.  Above
+  // kEdgeGuess places that would cost more than the 12 us of a read-back, and
+  // memory; under capture a read-back costs nothing on replay: there the
+  // totals are read first, and the lists get what they need.
   const long long est = n * (avg < 0 ? 32 : (long long)std::min(std::max(avg, 8.0), 32.0));
   auto cap_of = [&](const char *name) {
     const long long have = c.replay ? 0 : (long long)(c.ws.slots[name].bytes / 4);
@@ -1321,7 +1324,7 @@ static bool refine(Context &c, const JoinInputs &in, long n, const long long *kD
     HIP_CHECK(hipGetLastError());
   }
   if (!few) scan_i32_to_i64_multi(c, {{r.bCount, bOff, n}, {r.oCount, oOff, n}});
-  if (!kDev && est > kEdgeGuess) {
+  if (!few && (c.replay || (!kDev && est > kEdgeGuess))) {
     long long tot[kHostSlots];
     read_scalars(c, {bOff + n, oOff + n}, tot);
     capB = std::max(tot[0], 1LL);
