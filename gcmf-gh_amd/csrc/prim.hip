@@ -1120,14 +1120,15 @@ __global__ void __launch_bounds__(kSortThreads)
 }
 
 // off[tile][d] = the keys of digit d in earlier tiles.  A block takes
-// kStartDigits digits, its groups of as many lanes a run of tiles each: summed
-// (kept in registers up to kStartKeep tiles a run, else read twice), the runs'
-// starts scanned over the block, then written.  It replaces a general scan
-// over the digit-major counts: 8.6 us a pass for 3 000 000 keys on one MI355X,
-// 4.9 this way, bound by its chain of load, scan and store.
+// kStartDigits digits, its groups of as many lanes a run of at most kStartKeep
+// tiles each, kept in registers: summed, the runs' starts scanned over the
+// block, then written.  It replaces a general scan over the digit-major counts:
+// 8.7 us a pass for 3 000 000 keys on one MI355X, 6.8 this way, 9.7 and 10.8
+// for 8 000 000, bound by its chain of load, scan and store.
 constexpr int kStartThreads = 1024;
-constexpr int kStartDigits = 8;
+constexpr int kStartDigits = 4;
 constexpr int kStartKeep = 8;
+constexpr long kStartTiles = (long)(kStartThreads / kStartDigits) * kStartKeep;
 __global__ void __launch_bounds__(kStartThreads)
     k_sort_starts(const int *hist, long tiles, long long *off) {
   constexpr int D = kStartDigits, R = kStartThreads / D, W = kStartThreads / 64;
@@ -1139,15 +1140,10 @@ __global__ void __launch_bounds__(kStartThreads)
   long long *o = off + blockIdx.x * D + d;
   int v[kStartKeep];
   long long c = 0;
-  if (per <= kStartKeep) {
 #pragma unroll
-    for (int u = 0; u < kStartKeep; u++) {
-      v[u] = t0 + u < t1 ? h[256 * (t0 + u)] : 0;
-      c += v[u];
-    }
-  } else {
-#pragma unroll 8
-    for (long t = t0; t < t1; t++) c += h[256 * t];
+  for (int u = 0; u < kStartKeep; u++) {
+    v[u] = t0 + u < t1 ? h[256 * (t0 + u)] : 0;
+    c += v[u];
   }
   // over the wave's runs of this digit, then over the waves
   long long inc = c;
@@ -1161,19 +1157,54 @@ __global__ void __launch_bounds__(kStartThreads)
   c = inc - c;
 #pragma unroll
   for (int x = 0; x < W; x++) c += x < w ? sum[x][d] : 0;
-  if (per <= kStartKeep) {
 #pragma unroll
-    for (int u = 0; u < kStartKeep; u++) {
-      if (t0 + u < t1) o[256 * (t0 + u)] = c;
-      c += v[u];
-    }
-  } else {
+  for (int u = 0; u < kStartKeep; u++) {
+    if (t0 + u < t1) o[256 * (t0 + u)] = c;
+    c += v[u];
+  }
+}
+
+// The same for more than kStartTiles tiles, in two launches of a block per run
+// of `per` tiles (at most kStartRuns runs), four threads per digit with a
+// quarter of the rows each: the runs' sums, then every run adds up the sums
+// before its own and writes its tiles'.  Whole rows are read, where the blocks
+// above read 16 bytes of each.  20 000 000 keys: 18 us a pass, 31 when the
+// blocks above took any number of tiles, reading them twice.
+constexpr long kStartRuns = 128;
+// the sum of rows [r0, r1) of a digit's column
+template <typename T>
+__device__ __forceinline__ long long sum_rows(const T *col, long r0, long r1) {
+  long long c = 0;
+#pragma unroll 16
+  for (long r = r0; r < r1; r++) c += col[256 * r];
+  return c;
+}
+__global__ void __launch_bounds__(1024)
+    k_sort_run_sums(const int *hist, long tiles, long per, long long *part) {
+  __shared__ long long sum[4][256];
+  const int q = threadIdx.x >> 8, d = threadIdx.x & 255;
+  const long t0 = (long)blockIdx.x * per, n = min(tiles, t0 + per) - t0;
+  sum[q][d] = sum_rows(hist + d, t0 + n * q / 4, t0 + n * (q + 1) / 4);
+  __syncthreads();
+  if (q == 0) part[256 * (long)blockIdx.x + d] = sum[0][d] + sum[1][d] + sum[2][d] + sum[3][d];
+}
+__global__ void __launch_bounds__(1024)
+    k_sort_run_starts(const int *hist, long tiles, long per, const long long *part,
+                      long long *off) {
+  __shared__ long long sum[2][4][256];
+  const int q = threadIdx.x >> 8, d = threadIdx.x & 255;
+  const long t0 = (long)blockIdx.x * per, n = min(tiles, t0 + per) - t0, x = blockIdx.x;
+  const long a = t0 + n * q / 4, z = t0 + n * (q + 1) / 4;
+  sum[0][q][d] = sum_rows(part + d, x * q / 4, x * (q + 1) / 4);
+  sum[1][q][d] = sum_rows(hist + d, a, z);
+  __syncthreads();
+  long long c = 0;
+  for (int y = 0; y < 4; y++) c += sum[0][y][d] + (y < q ? sum[1][y][d] : 0);
 #pragma unroll 8
-    for (long t = t0; t < t1; t++) {
-      const int x = h[256 * t];
-      o[256 * t] = c;
-      c += x;
-    }
+  for (long t = a; t < z; t++) {
+    const int v = hist[256 * t + d];
+    off[256 * t + d] = c;
+    c += v;
   }
 }
 
@@ -1315,10 +1346,20 @@ static void sort_pass(Context &c, const uint64_t *k, const int *v, long n, int s
                        n, shift, hist, tiles);
     HIP_CHECK(hipGetLastError());
   }
-  if (!fuse) {
+  if (!fuse && tiles <= kStartTiles) {
     LaunchTimer t(c, "sort_starts");
     hipLaunchKernelGGL(k_sort_starts, dim3(256 / kStartDigits), dim3(kStartThreads), 0, c.stream,
                        (const int *)hist, tiles, off);
+    HIP_CHECK(hipGetLastError());
+  } else if (!fuse) {
+    const long per = (tiles + kStartRuns - 1) / kStartRuns, runs = (tiles + per - 1) / per;
+    long long *part = (long long *)c.ws.get("sort_runs", 8 * 256 * (size_t)kStartRuns);
+    LaunchTimer t(c, "sort_starts");
+    hipLaunchKernelGGL(k_sort_run_sums, dim3((unsigned)runs), dim3(1024), 0, c.stream,
+                       (const int *)hist, tiles, per, part);
+    HIP_CHECK(hipGetLastError());
+    hipLaunchKernelGGL(k_sort_run_starts, dim3((unsigned)runs), dim3(1024), 0, c.stream,
+                       (const int *)hist, tiles, per, (const long long *)part, off);
     HIP_CHECK(hipGetLastError());
   }
   LaunchTimer t(c, "sort_scatter");
@@ -1409,6 +1450,7 @@ constexpr long kNoAllocRows = 256 * (kNoAllocSortMax / kSortTileOf<16>);  // no 
 static_assert(kSortSmall4 / kSortTileOf<4> <= kNoAllocRows / 256 &&
                   kSortSmall8 / kSortTileOf<8> <= kNoAllocRows / 256,
               "more tiles than rows");
+static_assert(kNoAllocRows / 256 <= kStartTiles, "more tiles than the form without scratch takes");
 constexpr size_t noalloc_round(size_t b) { return (b + 255) & ~(size_t)255; }
 constexpr size_t kNoAllocKeys = 0;
 constexpr size_t kNoAllocVals = kNoAllocKeys + noalloc_round(8 * kNoAllocSortMax);

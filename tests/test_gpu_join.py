@@ -252,9 +252,11 @@ def test_scan_and_compact_tile_limits(gctx, tiles, extra):
 
 
 # around the sizes where the tile of a sort changes (1024, 2048, 4096 keys), the
-# fused form ends (64 tiles) and a run of tiles is read twice (above 1024 tiles)
+# fused form ends (64 tiles), a run of tiles has more than four (1024 tiles) and
+# the runs' sums take a launch of their own (above 2048 tiles)
 @pytest.mark.parametrize("n", [8193, 64 * 1024, 64 * 1024 + 1, (1 << 18) - 1, (1 << 18) + 1,
-                               1 << 20, (1 << 20) + 1, 1024 * 4096 + 4097])
+                               1 << 20, (1 << 20) + 1, 1024 * 4096 + 4097, 2048 * 4096,
+                               2048 * 4096 + 1, 2203 * 4096 - 5])
 @pytest.mark.parametrize("bits", [8, 22])
 def test_radix_sort_tile_forms(gctx, n, bits):
     """Stable at every tile size and form of the passes, few and many ties."""
