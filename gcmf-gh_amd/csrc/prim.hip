@@ -1119,19 +1119,20 @@ __global__ void __launch_bounds__(kSortThreads)
   hist[T * 256 + threadIdx.x] = h[threadIdx.x];
 }
 
-// off[tile][d] = the keys of digit d in earlier tiles.  A block takes
-// kStartDigits digits, its groups of as many lanes a run of at most kStartKeep
-// tiles each, kept in registers: summed, the runs' starts scanned over the
-// block, then written.  It replaces a general scan over the digit-major counts:
-// 8.7 us a pass for 3 000 000 keys on one MI355X, 6.8 this way, 9.7 and 10.8
-// for 8 000 000, bound by its chain of load, scan and store.
+// off[tile][d] = the keys of digit d in earlier tiles.  A block takes D digits
+// (8 while that keeps the tiles in registers, then 4), its groups of as many
+// lanes a run of at most kStartKeep tiles each: summed, the runs' starts scanned
+// over the block, then written.  It replaces a general scan over the
+// digit-major counts: 8.6 us a pass for 3 000 000 keys on one MI355X, 4.8 this
+// way, the same for 8 000 000; bound by its chain of load, scan and store.
 constexpr int kStartThreads = 1024;
-constexpr int kStartDigits = 4;
 constexpr int kStartKeep = 8;
-constexpr long kStartTiles = (long)(kStartThreads / kStartDigits) * kStartKeep;
+template <int D>
+constexpr long kStartTiles = (long)(kStartThreads / D) * kStartKeep;
+template <int D>
 __global__ void __launch_bounds__(kStartThreads)
     k_sort_starts(const int *hist, long tiles, long long *off) {
-  constexpr int D = kStartDigits, R = kStartThreads / D, W = kStartThreads / 64;
+  constexpr int R = kStartThreads / D, W = kStartThreads / 64;
   __shared__ long long sum[W][D];
   const int lane = __lane_id(), w = threadIdx.x >> 6;
   const int d = threadIdx.x % D, s = threadIdx.x / D;
@@ -1140,9 +1141,13 @@ __global__ void __launch_bounds__(kStartThreads)
   long long *o = off + blockIdx.x * D + d;
   int v[kStartKeep];
   long long c = 0;
+  // (every load first, past the run's end the last tile's: a guarded load waits
+  // before the next)
+#pragma unroll
+  for (int u = 0; u < kStartKeep; u++) v[u] = h[256 * min(t0 + u, tiles - 1)];
 #pragma unroll
   for (int u = 0; u < kStartKeep; u++) {
-    v[u] = t0 + u < t1 ? h[256 * (t0 + u)] : 0;
+    if (t0 + u >= t1) v[u] = 0;
     c += v[u];
   }
   // over the wave's runs of this digit, then over the waves
@@ -1164,7 +1169,7 @@ __global__ void __launch_bounds__(kStartThreads)
   }
 }
 
-// The same for more than kStartTiles tiles, in two launches of a block per run
+// The same for more than kStartTiles<4> tiles, in two launches of a block per run
 // of `per` tiles (at most kStartRuns runs), four threads per digit with a
 // quarter of the rows each: the runs' sums, then every run adds up the sums
 // before its own and writes its tiles'.  Whole rows are read, where the blocks
@@ -1346,10 +1351,11 @@ static void sort_pass(Context &c, const uint64_t *k, const int *v, long n, int s
                        n, shift, hist, tiles);
     HIP_CHECK(hipGetLastError());
   }
-  if (!fuse && tiles <= kStartTiles) {
+  if (!fuse && tiles <= kStartTiles<4>) {
     LaunchTimer t(c, "sort_starts");
-    hipLaunchKernelGGL(k_sort_starts, dim3(256 / kStartDigits), dim3(kStartThreads), 0, c.stream,
-                       (const int *)hist, tiles, off);
+    const bool eight = tiles <= kStartTiles<8>;
+    hipLaunchKernelGGL(eight ? k_sort_starts<8> : k_sort_starts<4>, dim3(eight ? 32 : 64),
+                       dim3(kStartThreads), 0, c.stream, (const int *)hist, tiles, off);
     HIP_CHECK(hipGetLastError());
   } else if (!fuse) {
     const long per = (tiles + kStartRuns - 1) / kStartRuns, runs = (tiles + per - 1) / per;
@@ -1450,7 +1456,7 @@ constexpr long kNoAllocRows = 256 * (kNoAllocSortMax / kSortTileOf<16>);  // no 
 static_assert(kSortSmall4 / kSortTileOf<4> <= kNoAllocRows / 256 &&
                   kSortSmall8 / kSortTileOf<8> <= kNoAllocRows / 256,
               "more tiles than rows");
-static_assert(kNoAllocRows / 256 <= kStartTiles, "more tiles than the form without scratch takes");
+static_assert(kNoAllocRows / 256 <= kStartTiles<4>, "more tiles than the form without scratch takes");
 constexpr size_t noalloc_round(size_t b) { return (b + 255) & ~(size_t)255; }
 constexpr size_t kNoAllocKeys = 0;
 constexpr size_t kNoAllocVals = kNoAllocKeys + noalloc_round(8 * kNoAllocSortMax);
