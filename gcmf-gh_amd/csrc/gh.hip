@@ -5108,8 +5108,8 @@ enum {
 // alone does not decide returns CT_SLOW with nothing changed, and
 // label_and_trace then takes the pair: a ring without a crossing or without
 // an ordinary vertex, a chain (step 2) that leaves the intersection vertices,
-// a walk that starts without a status or closes after outgrowing its room.  A
-// walk that cannot close fails here as it would there (CT_FAILED).
+// a walk that closes after outgrowing its room.  A walk that cannot close fails
+// here as it would there (CT_FAILED).
 //
 // What bounds it: lane 0's chain of dependent accesses, so the list lies in
 // LDS where it fits.  Measured on one MI355X, a pair of 8001 x 2003 vertices
@@ -5236,12 +5236,8 @@ __device__ __forceinline__ int contracted_trace(const Nodes &N, OutBuf &O, doubl
       prv[nxt[c]] = v;
       nxt[c] = v;
     };
-    // the area at c on the list: a vertex that has a copy already (a Q vertex
-    // that a second P vertex links to, where P touches itself) is followed by
-    // that copy, which lies on it
-    auto turn = [&](int c) {
-      if (nxt[c] >= C) return 0.0;
-      const int u = pos[c], r0 = u < nP ? 0 : nP, z = u < nP ? nP : n;
+    auto turn = [&](int u) {
+      const int r0 = u < nP ? 0 : nP, z = u < nP ? nP : n;
       return triA(P_(N, u == r0 ? z - 1 : u - 1), P_(N, u), P_(N, u + 1 == z ? r0 : u + 1));
     };
     for (int i = 0; i < X[0] && ok; i++) {
@@ -5255,7 +5251,10 @@ __device__ __forceinline__ int contracted_trace(const Nodes &N, OutBuf &O, doubl
       const int VP = T++, VQ = T++;
       pos[VP] = pos[I];
       pos[VQ] = pos[IQ];
-      if (turn(I) * turn(IQ) > 0) {
+      // a Q vertex split before (for another P vertex that links to it, where P
+      // touches itself) is followed by its copy, which lies on it: no area
+      const bool again = lab(IQ) == L_CROSSING;
+      if (!again && turn(pos[I]) * turn(pos[IQ]) > 0) {
         nb[I] = VQ;
         nb[VQ] = I;
         nb[IQ] = VP;
@@ -5296,8 +5295,10 @@ __device__ __forceinline__ int contracted_trace(const Nodes &N, OutBuf &O, doubl
       }
       tot += len;
       const int r0 = ringdir & 2 ? nP : 0, nR = ringdir & 2 ? nQ : nP;
-      const int o = (ringdir & 1) ? (p - r0 + len) % nR : (p - r0 + nR - len % nR) % nR;
-      lastEnd = r0 + o;
+      int e = (ringdir & 1) ? p + len : p - len;  // len <= nR
+      if (e >= r0 + nR) e -= nR;
+      if (e < r0) e += nR;
+      lastEnd = e;
       lastKey = ringdir;
       return tot <= n;
     };
@@ -5315,7 +5316,6 @@ __device__ __forceinline__ int contracted_trace(const Nodes &N, OutBuf &O, doubl
         do {
           int status = enex(V);
           toggle(status);
-          if (status == NEITHER) ok = false;
           const bool fwd = status == EXIT;
           do {
             const int d = fwd ? nxt[V] : prv[V];
@@ -5332,6 +5332,9 @@ __device__ __forceinline__ int contracted_trace(const Nodes &N, OutBuf &O, doubl
             } else if (len <= 0) {
               len += nR;
             }
+            // without a status the walk goes back until it meets a vertex
+            // without one: at once, an ordinary vertex, which has no link
+            if (status == NEITHER && len > 1) failed = true;
             if (p >= r0 + nR) p -= nR;
             if (p < r0) p += nR;
             if (!full) full = !emit(p, len, (onQ ? 2 : 0) | (fwd ? 1 : 0));
