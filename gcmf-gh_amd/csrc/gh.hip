@@ -5306,7 +5306,8 @@ __device__ __forceinline__ int contracted_trace(const Nodes &N, OutBuf &O, doubl
     int I = 0;
     do {
       if (ok && has(I, F_INT) && lab(I) == L_CROSSING) {
-        if (nc >= O.capComp) ok = false;
+        // (the clean-up's scratch holds Dc / 2 + 2 components)
+        if (nc >= min(O.capComp, Dc / 2 + 2)) ok = false;
         const int start = tot;
         lastKey = -1;
         int V = I, savedV = -1, savedS = -1;
