@@ -1233,6 +1233,14 @@ __global__ void __launch_bounds__(kSortThreads)
   uint64_t kk[I];
   int vv[I];
   int pos[I];
+  // this tile's output start for digit threadIdx.x (256 threads, 256 digits):
+  // asked for before the keys, so that the digits' scan does not wait for them
+  const int *hrow = hist + threadIdx.x;
+  long long pre = 0, dtot = 0;
+  if (off) {
+    pre = off[T * 256 + threadIdx.x];
+    dtot = off[(tiles - 1) * 256 + threadIdx.x] + hrow[(tiles - 1) * 256];
+  }
   // all of the wave's loads in flight at once, before the ranking rounds
 #pragma unroll
   for (int r = 0; r < I; r++) {
@@ -1240,13 +1248,7 @@ __global__ void __launch_bounds__(kSortThreads)
     kk[r] = i < n ? keys[i] : 0;
     vv[r] = i < n ? vals[i] : 0;
   }
-  // this tile's output start for digit threadIdx.x (256 threads, 256 digits)
-  const int *hrow = hist + threadIdx.x;
-  long long pre = 0, dtot = 0;
-  if (off) {
-    pre = off[T * 256 + threadIdx.x];
-    dtot = off[(tiles - 1) * 256 + threadIdx.x] + hrow[(tiles - 1) * 256];
-  } else {
+  if (!off) {
 #pragma unroll 16
     for (int t = 0; t < (int)tiles; t++) {
       const int h = hrow[256 * t];
