@@ -58,11 +58,13 @@ struct KernelTimer {
 // workload's pairs.
 struct Tuning {
   long cullMin = 512;       // rings longer than this are walked through run boxes
-  long long bigNodes = 8192;  // pairs with this many nodes are labelled by a block
+  long long bigNodes = 8192;  // pairs with this many nodes are labelled by a block (512 at
+                              // most in calls of at most one pair per CU)
   long long gridNodes = 1LL << 20;  // ... and with this many by the whole GPU
   int gridClean = 16384;    // there, components longer than this are cleaned by the grid
   long long stripMin = 1LL << 17;  // joins of this many polygons sweep the MBRs in y strips
-  int cmfGroup = 0;         // lanes per pair in the CMF edge filter (16, 64; 0: by polygon size)
+  int cmfGroup = 0;         // lanes per candidate in the refine passes (16, 64; 0: 8, 16 or 64
+                            // by the mean ring)
   int labelSteal = 0;       // 1: labelling waves are persistent and take pairs from a counter
   int blockCap = 128;       // blocks of the block labelling (each takes pairs from a counter)
   int countStage = 0;       // 1: each count lane walks the whole Q ring (a wave's copy in

@@ -2170,7 +2170,10 @@ __global__ void __launch_bounds__(256, CULL ? 1 : 5)
 // wave walk, in us: 64 P edges 7 / 25, 2 000 12 / 111, 7 500 (37 pairs) 12 /
 // 50, 47 000 (200 pairs) 41 / 49, 107 000 (400 pairs) 82 / 52; 32 000 of
 // joined pairs 26 / 127, 316 000 204 / 217, 688 000 437 / 254.  The line lies
-// where the batches' two sides meet.
+// where the batches' two sides meet: what decides is the share of a ring's runs
+// that pass, which is not known before the pass.  Joined pairs, whose rings
+// have fewer of them, meet above 316 000 edges, so between the line and that
+// they take the wave walk though it is up to about a tenth slower.
 constexpr long kCountEdgeMax = 65536;
 
 __global__ void __launch_bounds__(256)
@@ -4365,8 +4368,8 @@ __device__ int segment_trace(const Nodes &N, OutBuf &O, double *xy, int *clen, i
   return SEG_DONE;
 }
 
-// The same for the whole grid, where a grid barrier (about 25 us) follows every
-// step and every round.
+// The same for the whole grid, where a grid barrier (under 20 us with
+// k_label_grid's blocks) follows every step and every round.
 __device__ int grid_segment_trace(const Nodes &N, OutBuf &O, double *xy, int *clen, int *rg,
                                   int nP, int nQ, int Dc, int *omap) {
   constexpr int W = kGrid;
@@ -5112,9 +5115,10 @@ enum {
 // here as it would there (CT_FAILED).
 //
 // What bounds it: lane 0's chain of dependent accesses, so the list lies in
-// LDS where it fits.  Measured on one MI355X, a pair of 8001 x 2003 vertices
-// snapped to a grid (about 400 intersection vertices): 10.1 -> 0.53 ms by one
-// block; 4849 x 1833 (160): 5.8 -> 0.51 ms by one wave.
+// LDS where it fits.  Measured on one MI355X against the sequential steps, pairs
+// snapped to a grid that do have degenerate labels: 8001 x 2003 vertices (about
+// 400 intersection vertices) 10.1 -> 0.53 ms by one block, 4849 x 1833 (160) 5.8
+// -> 0.51 ms by one wave, 3000 x 3000 (a failing walk) 3.8 -> 0.48 ms.
 enum { CT_SLOW = 0, CT_DONE = 1, CT_FAILED = 2 };
 template <int W>
 __device__ __forceinline__ int contracted_trace(const Nodes &N, OutBuf &O, double *xy, int *clen, int *rg,
@@ -5812,12 +5816,10 @@ __device__ __forceinline__ int label_pair(long k, int *status, const SlotArrays 
   return path;
 }
 
-// Pairs with at least TraceArgs::bigNodes nodes (Tuning::bigNodes) are
-// labelled by a block of kBigGroup
-// threads (k_label_block), the others by one wave each (k_label_wave).  At
-// 1024 threads the sequential fallback spills a few registers; the extra
-// parallelism of the block is worth more (the 1e6 x 1e5 pair labels in 113
-// ms at 1024 threads, 167 ms at 512).
+// Pairs with at least TraceArgs::bigNodes nodes (Tuning::bigNodes) are labelled
+// by a block of kBigGroup threads (k_label_block), the others by one wave each
+// (k_label_wave).  At 1024 threads the sequential fallback spills a few
+// registers; the extra parallelism of the block is worth more.
 constexpr int kBigGroup = 1024;
 // Pairs with at least Tuning::gridNodes nodes are labelled by the whole GPU,
 // one cooperative launch of kGridBlock-thread blocks each (k_label_grid).
@@ -6084,10 +6086,10 @@ __global__ void __launch_bounds__(W == 64 ? 256 : W)
 // kGlueMax edges per ring side one block does all of them that lie between
 // two such kernels, and stores the values the host waits for straight into
 // its staging buffer.  One such launch takes 7 to 18 us, the five to eight it
-// replaces 4 to 9 each with their gaps: on one MI355X a call of 64 x 48
-// vertices went from 36 launches to 17 and from 334 to 223 us, of 37 pairs
-// from 470 to 410, of 2000 x 1500 vertices from 675 to 593.  Above that the
-// many-block kernels are faster than one block: the offsets of 15 600 pairs
+// replaces 4 to 9 each with their gaps: with them a call of 64 x 48 vertices
+// takes 17 launches instead of 36 on one MI355X (223 us in place of 334), one of
+// 37 pairs 410 us in place of 470, one of 2000 x 1500 vertices 593 in place of
+// 675.  Above that the many-block kernels are faster than one block: the offsets of 15 600 pairs
 // took 27 us here and 20 there.
 constexpr int kGlueThreads = 1024;
 constexpr int kGlueItems = 4;  // per thread and round, one 16-byte load
@@ -7275,9 +7277,12 @@ void clip_pairs(Context &c, const JoinInputs &in, const int *pairs, long M,
       HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCu, k_label_grid, kGridBlock,
                                                              0));
       // (a block on every other CU: the grid barriers, which every block
-      // writes its caches back for, cost more than the idle CUs would save.  The
-      // wavy 1e6 x 1e5 pair: 7.9 ms in 512 blocks of 256 threads, 5.6 in 256 of
-      // 512, 5.15 in 128, 5.9 in 64)
+      // writes its caches back for, cost more than the idle CUs would save.
+      // Labelling with a block on every, every other and every fourth CU, ms:
+      // a wavy pair of 3.7 million nodes 3.10, 2.65 and 3.36; of 582 000 2.19,
+      // 1.38 and 1.07, of 129 000 1.93, 1.12 and 0.75, a star pair of 310 000
+      // 2.33, 1.53 and 1.19.  Pairs below the default of a million nodes come
+      // here only by the caller's grid_nodes)
       const int blocks = std::max(1, std::min(perCu * c.cu_count, c.cu_count / 2));
       long long *part = wsT<long long>(c, "gh_grid_part", 2L * blocks);
       for (int kp : gl) {

@@ -1024,8 +1024,9 @@ __global__ void __launch_bounds__(256)
 // polygons of 8 vertices on one MI355X the stages as passes of their own over
 // compacted lists, one wave per pair in the segment test, took 600 us of
 // kernel time in 13 launches: that test alone 331 us with 64 lanes on about
-// nine edge pairs.  The two passes take 88 and 131 us, and 110 and 170 with 16
-// lanes per candidate instead of 8.  What bounds both now is the chain of
+// nine edge pairs.  The two passes take 53 and 87 us (88 and 131 with a vertex
+// loaded as two numbers; then 110 and 170 with 16 lanes per candidate instead
+// of 8).  What bounds both now is the chain of
 // dependent loads (pair, ring bounds, vertices); groups of 8 lanes keep eight
 // chains per wave in flight.
 //

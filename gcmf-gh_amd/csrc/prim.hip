@@ -6,13 +6,14 @@
 //
 // Scan: reduce-then-scan over 4096-element tiles (256 threads x 16 items),
 // wave64 shuffles inside a wave, LDS across the 4 waves of a block.
-// Radix sort: 8-bit digits, LDS digit histograms per 4096-key tile, a
-// digit-major scan of the histograms, and a stable scatter ranked with
-// 8 wave ballots per 64 keys (peer mask = keys with the same digit).  The
-// scatter and the compaction's write pass take their tiles through
-// xcd_tile, so that neighbouring tiles, whose outputs share cache lines at
-// every digit run's ends, run on one XCD (measured on MI355X at 2^27 keys:
-// 1.57 -> 0.75 ms per scatter pass).
+// Radix sort: 8-bit digits, LDS digit histograms per tile of 1024, 2048 or 4096
+// keys (by the sort's size), written tile by tile, the tiles' starts inside
+// each digit, and a stable scatter ranked with 8 wave ballots per 64 keys (peer
+// mask = keys with the same digit).  Up to 8192 keys take one launch that
+// counts the keys before each.  The scatter and the compaction's write pass
+// take their tiles through xcd_tile, so that neighbouring tiles, whose outputs
+// share cache lines at every digit run's ends, run on one XCD (measured on
+// MI355X at 2^27 keys: 1.57 -> 0.75 ms per scatter pass).
 #include "gcmf_device.hpp"
 #include <algorithm>
 #include <cstring>

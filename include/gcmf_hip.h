@@ -212,7 +212,10 @@ int gcmf_clip_write(gcmf_ctx *ctx, const char *path, int format);
 typedef struct {
   long cull_min;       /* rings longer than this are walked through run boxes (512) */
   long long big_nodes; /* pairs with this many nodes are labelled by a
-                          1024-thread block instead of one wave (8192) */
+                          1024-thread block instead of one wave (8192).  A
+                          call of at most one pair per CU, which waits for its
+                          slowest pair, takes a block from min(big_nodes, 512)
+                          nodes on, unless label_steal is 1 */
   int count_block;     /* threads per block of the count kernel: 64, 128, 256 (128) */
   int lds_max_q;       /* pairs whose Q ring is longer than cull_min and has at
                           most this many vertices are counted with Q binned in
@@ -228,15 +231,18 @@ typedef struct {
                           wave or thread each (49.., 16384) */
   long long strip_min;  /* joins of at least this many polygons (both layers)
                           run the MBR sweep over y strips (2^17; 0: always) */
-  int cmf_group;        /* lanes per candidate pair in the CMF edge filter:
-                          16 (four pairs per wave), 64, or 0: 16 when the
-                          layers average at most 32 vertices per polygon (0) */
+  int cmf_group;        /* lanes per candidate pair in the join's refine passes:
+                          16 (four pairs per wave), 64, or 0: 8 when the
+                          layers average at most 12 vertices per polygon, 16
+                          at most 32, else 64; joins of up to 4096 polygons 64
+                          (0) */
   int label_steal;      /* 1: the labelling waves are a persistent launch that
                           takes the pairs from a device counter in turn
                           (work stealing); 0: one wave per pair (0) */
   int block_cap;        /* blocks of the 1024-thread labelling launch, each
                           taking the next listed pair from a device counter
-                          (1..65536, 128) */
+                          (1..65536, 128; a call of at most one pair per CU
+                          has a block per pair) */
   int count_stage;      /* 0: the edges of one pair in a count wave walk the
                           other ring together, 16-edge runs at a time, leaving
                           out the runs none of them can pair with; 1: every
@@ -249,7 +255,9 @@ int gcmf_set_tuning(gcmf_ctx *ctx, const gcmf_tuning *t);
 /* Chooses the tuning by measurement on one batch (the autotuner): clips the
  * pairs once per candidate value of each parameter in turn, times the
  * launches the parameter affects with HIP events, and keeps the fastest in
- * the context.  The chosen values are returned in *out.  No reference
+ * the context.  The chosen values are returned in *out.  A batch of at most
+ * one pair per CU says nothing about big_nodes, which it does not depend on
+ * from 512 up: tune on a batch of the size that will be clipped.  No reference
  * counterpart. */
 int gcmf_tune_clip(gcmf_ctx *ctx, const gcmf_dlayer *base, const gcmf_dlayer *over,
                    const int *d_pairs, long M, int flags, gcmf_tuning *out);
