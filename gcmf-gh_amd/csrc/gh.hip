@@ -5436,6 +5436,39 @@ __device__ void spill_nodes(Nodes &N, const Nodes &G, int nP, int nQ) {
   N.cap = cap;
 }
 
+// label_and_trace for label_pair's lane 0.  A block calls it out of line, with
+// copies on both sides of the call: inlined, the compiler keeps its scalars
+// across the parallel steps (211 spilled, 138 now); a call on the pair's own
+// Nodes has those steps read the arrays' addresses back from scratch memory,
+// and without the callee's copies its walks do.  Us for the call, inlined, on
+// the originals, copied by the caller only, copied by both: one pair of 250 000
+// x 25 000 vertices 10 220, 11 221, 9 997, 10 000; 700 000 x 5 000 19 311, 21
+// 028, 18 711, 18 882; 60 000 x 3 000 on a grid 1 981, -, 1 983, 1 962; 256
+// self-overlapping pairs of 2000 x 2000, some of which come here, 6 547, -,
+// 8 672, 6 580.
+__device__ __attribute__((noinline)) int label_and_trace_call(const Nodes *N, int rootP, int rootQ,
+                                                              OutBuf *O, const int *pinHint) {
+  Nodes n = *N;
+  OutBuf o = *O;
+  const int rc = label_and_trace(n, rootP, rootQ, o, true, pinHint);
+  *O = o;
+  return rc;
+}
+
+template <int W>
+__device__ __forceinline__ int sequential_trace(Nodes N, int rootP, int rootQ, OutBuf &O,
+                                                const int pinHint[4]) {
+  if constexpr (W == 64 || W == kGrid) {
+    return label_and_trace(N, rootP, rootQ, O, true, pinHint);
+  } else {
+    OutBuf o = O;
+    const int hint[4] = {pinHint[0], pinHint[1], pinHint[2], pinHint[3]};
+    const int rc = label_and_trace_call(&N, rootP, rootQ, &o, hint);
+    O = o;
+    return rc;
+  }
+}
+
 // arena / arenaBytes: the group's LDS for the pair's arrays (null: none)
 // (contracted_trace takes the LDS the arena has left, at least `spare` bytes
 // of it where the later arrays leave room for that)
@@ -5780,7 +5813,7 @@ __device__ __forceinline__ int label_pair(long k, int *status, const SlotArrays 
     if (lane != 0) return LP_SEQUENTIAL;
     O.n = 0;
     O.ncomp = 0;
-    int rc = label_and_trace(N, 0, nP, O, true, pinHint);
+    int rc = sequential_trace<W>(N, 0, nP, O, pinHint);
     if (rc != GH_OK) {
       status[k] = rc;
       a.outNComp[k] = 0;
